@@ -737,11 +737,13 @@ static int tridiag_launch(hipStream_t st, unsigned nb, size_t lds, int k, const 
                           const DiagDev& D, double* B, const double* bvec, double* tau,
                           double* dd, double* ee, double* U, int* nvec, int* status,
                           int reg, const int32_t* perm, const RatTab& R) {
-  // k >= 32 (K = 64), rows padded to a multiple of 8 (to 50 for k = 49 and
-  // 50): reg 2 the two-problem register kernel (k <= 50), reg 1 (or 2 past
-  // k = 50) the one-problem register kernel, reg 0 the LDS kernel
+  // rows padded to a multiple of 8 (to 50 for k = 49 and 50): reg 2 the DPP
+  // register kernel (two problems per wave, one past k = 50); reg 1 the
+  // one-problem register kernel (k >= 32); reg 0 the LDS kernel, and what
+  // reg 1 runs below k = 32.  2959 problems of k = 20 with the rational
+  // solve: 85 us from LDS, 24 us by DPP
   const int kq = (k == 49 || k == 50) ? 50 : (k + 7) / 8 * 8;
-  if (K == 64 && reg == 2) {
+  if (reg == 2) {
     const int rc = launch_tridiag_pair(st, (int64_t)nb, perm, kq, NV, k, K, L, S, V, C, D, B,
                                        bvec, tau, dd, ee, U, nvec, status, R.tab, R.n, R.nb);
     if (rc) return rc;

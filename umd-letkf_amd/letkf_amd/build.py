@@ -43,7 +43,7 @@ def hipcc() -> str:
 EXTRA = {f"tridiag_reg_kq{kq}.hip": ["-mllvm", "-pragma-unroll-threshold=2000000"]
          for kq in (32, 40, 48, 50, 56, 64)}
 EXTRA.update({f"tridiag_pair_kq{kq}.hip": ["-mllvm", "-pragma-unroll-threshold=2000000"]
-              for kq in (32, 40, 48, 50)})
+              for kq in (8, 16, 24, 32, 40, 48, 50, 56, 64)})
 
 
 def _compile(src: str) -> str:
