@@ -33,3 +33,25 @@ def test_edges(k, ns):
             e["state"] = rel(st, orc["state"])
         print(e, flush=True)
         assert max(e.values()) <= tol, e
+
+
+@pytest.mark.parametrize("rat", ["1", "0"])
+@pytest.mark.parametrize("err", [0.05, 3e-3, 3e-4])
+@pytest.mark.parametrize("k,ns", [(20, 1), (20, 12), (50, 1), (50, 12), (63, 2), (63, 12)])
+def test_conditioning(k, ns, err, rat, monkeypatch):
+    """The rational A^(-1/2) of the FP64 path with few and with many slabs a
+    group, at condition numbers of the local problems up to about 8e6, which
+    take more than one round of nodes (31) and more than one group of them
+    (16), and the QL eigensolve it replaced (LETKF_GPU_RAT=0): both within
+    1e-10 of the oracle."""
+    monkeypatch.setenv("LETKF_GPU_RAT", rat)
+    p = synth.random_problem(seed=1300 + k, nx=27, ny=13, k=k, ns=ns, nobs=1500, err=err, rtps=0.0)
+    orc = oracle_run(p)
+    print("conditioning k", k, "ns", ns, "err", err, "rat", rat, flush=True)
+    with LetkfGpuSolver(p, precision="fp64", path="plain") as s:
+        s.run()
+        st, mn, sp = s.state_f64()
+    e = dict(mean=rel(mn, orc["mean"]), sprd=rel(sp, orc["sprd"]), state=rel(st, orc["state"]),
+             inc=rel(mn - p.mean, orc["mean"] - p.mean))
+    print(e, flush=True)
+    assert max(e.values()) <= 1e-10, e

@@ -1,0 +1,313 @@
+// back_apply.hip -- the transform of a group of many slabs for k < 64 without
+// an eigensolve: M = sqrt(k-1) Tri^(-1/2) as a matrix, W = Q M Q^T from the
+// stored reflectors, wbar = W (W b) / (k-1), and x_a = W x_b + wbar . x_b for
+// every slab of the group (src/letkf_core.F90:100-141,
+// src/letkf_solver.F90:284-290), all in FP64.
+//
+//  k_small_rational  the lower triangle of M from the two-term recurrences of
+//                    the inverses (Tri + s_n I)^-1 (see kernels_transform.hip,
+//                    k_mat_rational), one wave per problem;
+//  k_back_apply      the two-sided back-transform and the apply with the
+//                    matrix one row a lane, as tridiag_pair.h keeps it.
+//
+// They take the place of implicit QL with recorded rotations, the replay of
+// the records into eigenvectors and two mat-vecs a slab (k_tql, k_replay,
+// k_vec_apply, still run with LETKF_GPU_RAT=0): QL is a serial chain per
+// problem, one lane each, and its records cross memory twice.  11 855
+// problems of k = 40 with 50 slabs: 5.2 ms then, 1.1 ms now; 33 problems
+// of k = 50 with 12 slabs: 540 us and 240 us.  The node table is the fine
+// one (5e-16): over condition numbers of 1e2 to 8e6 the analysis is no further
+// from the FP64 oracle than the eigensolve's (spread 2e-14 against 1e-13 at
+// 8e6, k = 50).
+#include <hip/hip_runtime.h>
+
+#include "dpp_common.h"
+#include "letkf_internal.h"
+
+namespace lk {
+
+constexpr int kGroupNodes = 16;   // nodes of one pass over the rows (17 KB of
+                                  // LDS: nine waves a CU; all 62 would be two)
+
+__global__ __launch_bounds__(64) void k_small_rational(int k, int K, ChunkDev C,
+                                                       double* __restrict__ B,
+                                                       const double* __restrict__ dd,
+                                                       const double* __restrict__ ee, RatTab R) {
+  constexpr int NG = kGroupNodes;
+  constexpr int LD = 65;
+  __shared__ double sd[64], se[64];
+  // U of the node's bottom-up pivots, and its top-down pivots, then the
+  // diagonal of the inverse
+  __shared__ double Us[NG][LD], Gs[NG][LD];
+  const int64_t pair = blockIdx.x;
+  if (!C.solve[pair]) return;
+  const int l = threadIdx.x;
+  const double m = (double)(k - 1);
+  sd[l] = l < k ? dd[pair * K + l] : 0.0;
+  se[l] = l < k - 1 ? ee[pair * K + l] : 0.0;
+  __syncthreads();
+  double gm = l < k ? sd[l] + (l > 0 ? fabs(se[l - 1]) : 0.0) + fabs(se[l]) : 0.0;
+  gm = p_max<64>(gm);
+  int bk = (int)ceil(log2(fmax(gm / m, 2.0)));
+  bk = bk < 1 ? 1 : (bk > R.nb - 1 ? R.nb - 1 : bk);
+  bk = __builtin_amdgcn_readfirstlane(bk);
+  const int nn = __builtin_amdgcn_readfirstlane(R.n[bk]);
+  const double* sn = R.tab + bk * kRatLd;
+  const double* wn = sn + kRatLd / 2;
+  double* Bp = B + pair * (int64_t)k * k;
+  for (int n0 = 0; n0 < nn; n0 += NG) {
+    // the pivots: lanes 0..15 top-down, lanes 16..31 bottom-up, a node each
+    // (a node past the last has a pivot of at least m and weight 0)
+    if (l < 2 * NG) {
+      const int n = l & (NG - 1);
+      const double sg = n0 + n < nn ? m * sn[n0 + n] : m;
+      double f = 0.0;
+      if (l < NG) {
+        for (int i = 0; i < k; ++i) {
+          const double D = sd[i] + sg - (i > 0 ? se[i - 1] * f : 0.0);
+          Gs[n][i] = D;
+          f = se[i] * rcp_cubic(D);
+        }
+      } else {
+        for (int i = k - 1; i >= 0; --i) {
+          const double D = fma(-se[i], f, sd[i] + sg);
+          f = i > 0 ? se[i - 1] * rcp_cubic(D) : 0.0;
+          Us[n][i] = f;
+        }
+      }
+    }
+    __syncthreads();
+    // the inverse's diagonal 1 / (D+_i + D-_i - (d_i + s)) = 1 / (D+_i - e_i U_(i+1))
+    if (l < k) {
+#pragma unroll 4
+      for (int n = 0; n < NG; ++n)
+        Gs[n][l] = rcp_cubic(fma(-se[l], l < k - 1 ? Us[n][l + 1] : 0.0, Gs[n][l]));
+    }
+    __syncthreads();
+    // column l from its diagonal down
+    double cf[NG], x[NG];
+#pragma unroll
+    for (int n = 0; n < NG; ++n) {
+      cf[n] = n0 + n < nn ? m * wn[n0 + n] : 0.0;
+      x[n] = Gs[n][l < k ? l : 0];
+    }
+    for (int r = 0; r < k; ++r) {
+      double acc[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int n = 0; n < NG; ++n) {
+        const double xn = -Us[n][r] * x[n];
+        x[n] = r > l ? xn : x[n];
+        acc[n & 3] = fma(cf[n], x[n], acc[n & 3]);
+      }
+      if (r >= l && l < k) {
+        const double s = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+        double* at = Bp + (int64_t)r * k + l;
+        *at = n0 > 0 ? *at + s : s;
+      }
+    }
+    __syncthreads();
+  }
+}
+
+// blocks of columns by 16: p += sum_c q(c) a[c], c = 16 T .. min(16 T + 15, KQ - 1)
+template <int KQ, int RPL, int T>
+__device__ __forceinline__ void block_prod(double (&p)[4], double q, const double (&a0)[KQ],
+                                           const double (&a1)[RPL == 2 ? KQ : 1]) {
+  constexpr int c0 = 16 * T, n = KQ - c0 < 16 ? KQ - c0 : 16;
+  static_for<n / 4>([&](auto I) __attribute__((always_inline)) {
+    constexpr int i = 4 * decltype(I)::value, c = c0 + i;
+    if constexpr (RPL == 2)
+      bfma42<i>(p[0], p[1], p[2], p[3], q, a0[c], a0[c + 1], a0[c + 2], a0[c + 3], a1[c],
+                a1[c + 1], a1[c + 2], a1[c + 3]);
+    else
+      bfma4<i>(p[0], p[1], q, a0[c], a0[c + 1], a0[c + 2], a0[c + 3]);
+  });
+  static_for<n % 4>([&](auto I) __attribute__((always_inline)) {
+    constexpr int i = n / 4 * 4 + decltype(I)::value, c = c0 + i;
+    if constexpr (RPL == 2) bfma2<i>(p[0], p[2], q, a0[c], a1[c]);
+    else bfma<i>(p[0], q, a0[c]);
+  });
+}
+
+// a[c] -= v_r w_c (+ w_r v_c with VC) on one block of columns
+template <int KQ, int T, bool VC>
+__device__ __forceinline__ void block_upd(double (&a)[KQ], double wq, double vq, double nv,
+                                          double nw) {
+  constexpr int c0 = 16 * T, n = KQ - c0 < 16 ? KQ - c0 : 16;
+  static_for<n / 4>([&](auto I) __attribute__((always_inline)) {
+    constexpr int i = 4 * decltype(I)::value, c = c0 + i;
+    if constexpr (VC) upd4<i>(a[c], a[c + 1], a[c + 2], a[c + 3], wq, vq, nv, nw);
+    else upd4v<i>(a[c], a[c + 1], a[c + 2], a[c + 3], wq, nv);
+  });
+  static_for<n % 4>([&](auto I) __attribute__((always_inline)) {
+    constexpr int i = n / 4 * 4 + decltype(I)::value, c = c0 + i;
+    if constexpr (VC) upd<i>(a[c], wq, vq, nv, nw);
+    else bfma<i>(a[c], wq, nv);
+  });
+}
+
+// P lanes a problem (two a wave for k <= 50), rows r and, with RPL = 2,
+// r + 32.  The reflectors are walked backwards; reflector j has zeros up to
+// entry j, so whole blocks of 16 columns below it need no product and only
+// the v_r w_c part of the update (a wave-uniform branch each).  Reflectors
+// are loaded four steps ahead.
+template <int KQ, int P, int RPL>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2)))
+void k_back_apply(int k, int K, int64_t np, const int32_t* __restrict__ perm, LocDev L, StateDev S,
+                  VarsDev V, ChunkDev C, DiagDev D, const double* __restrict__ B,
+                  const double* __restrict__ bvec, const double* __restrict__ tau,
+                  double* __restrict__ ana) {
+  constexpr int NPW = 64 / P;
+  constexpr int NT = (KQ + 15) / 16;
+  __shared__ unsigned short sl[NPW][2048];
+  const int lane = threadIdx.x;
+  const int hh = P == 32 ? lane >> 5 : 0;
+  const int r = lane & (P - 1), r1 = r + 32;
+  const int64_t q = NPW * (int64_t)blockIdx.x + hh;
+  int64_t pair = -1;
+  if (q < np) pair = perm ? (int64_t)perm[q] : q;
+  const bool act = pair >= 0 && C.solve[pair] != 0;
+  if (__ballot(act) == 0ull) return;   // wave-uniform
+  const int64_t pq = act ? pair : 0;
+  const double* Bp = B + pq * (int64_t)k * k;
+  const bool in0 = act && r < k, in1 = act && RPL == 2 && r1 < k;
+  // M, symmetric, from its lower triangle (row-major in B)
+  double a0[KQ], a1[RPL == 2 ? KQ : 1];
+#pragma unroll
+  for (int c = 0; c < KQ; ++c) {
+    a0[c] = (in0 && c < k) ? Bp[r >= c ? (int64_t)r * k + c : (int64_t)c * k + r] : 0.0;
+    if constexpr (RPL == 2)
+      a1[c] = (in1 && c < k) ? Bp[r1 >= c ? (int64_t)r1 * k + c : (int64_t)c * k + r1] : 0.0;
+  }
+  const double* tp = tau + pq * K;
+  double pv0[4], pv1[4], pt[4];
+  auto fetch = [&](int j, int u) __attribute__((always_inline)) {
+    pv0[u] = (in0 && r > j && j >= 0) ? Bp[(int64_t)j * k + r] : 0.0;
+    pv1[u] = (in1 && r1 > j && j >= 0) ? Bp[(int64_t)j * k + r1] : 0.0;
+    pt[u] = (act && j >= 0) ? tp[j] : 0.0;
+  };
+#pragma unroll
+  for (int u = 0; u < 4; ++u) fetch(k - 2 - u, u);
+  for (int jb = k - 2; jb >= 0; jb -= 4) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int j = jb - u;
+      if (j < 0) break;
+      // an unused reflector (t = 0) was not stored
+      const double t = pt[u];
+      const double v0 = t != 0.0 ? pv0[u] : 0.0, v1 = t != 0.0 ? pv1[u] : 0.0;
+      fetch(j - 4, u);
+      double vq[4], p[4] = {0.0, 0.0, 0.0, 0.0};
+      spread<P, RPL, NT>(v0, v1, vq);
+      static_for<NT>([&](auto T) __attribute__((always_inline)) {
+        constexpr int tt = decltype(T)::value;
+        if (j < 16 * tt + 15) block_prod<KQ, RPL, tt>(p, vq[tt], a0, a1);
+      });
+      const double p0 = t * (p[0] + p[1]), p1 = t * (p[2] + p[3]);
+      double pv = p0 * v0;
+      if constexpr (RPL == 2) pv = fma(p1, v1, pv);
+      const double kc = 0.5 * t * p_sum<P>(pv);
+      const double w0 = fma(-kc, v0, p0), w1 = fma(-kc, v1, p1);
+      double wq[4];
+      spread<P, RPL, NT>(w0, w1, wq);
+      static_for<NT>([&](auto T) __attribute__((always_inline)) {
+        constexpr int tt = decltype(T)::value;
+        if (j < 16 * tt + 15) {
+          block_upd<KQ, tt, true>(a0, wq[tt], vq[tt], -v0, -w0);
+          if constexpr (RPL == 2) block_upd<KQ, tt, true>(a1, wq[tt], vq[tt], -v1, -w1);
+        } else {
+          block_upd<KQ, tt, false>(a0, wq[tt], vq[tt], -v0, -w0);
+          if constexpr (RPL == 2) block_upd<KQ, tt, false>(a1, wq[tt], vq[tt], -v1, -w1);
+        }
+      });
+    }
+  }
+  // wbar = W (W b) / (k-1), added to every row: T = W + 1 wbar^T
+  auto mul = [&](double x0, double x1, double* o0, double* o1) __attribute__((always_inline)) {
+    double xq[4], p[4] = {0.0, 0.0, 0.0, 0.0};
+    spread<P, RPL, NT>(x0, x1, xq);
+    static_for<NT>([&](auto T) __attribute__((always_inline)) {
+      constexpr int tt = decltype(T)::value;
+      block_prod<KQ, RPL, tt>(p, xq[tt], a0, a1);
+    });
+    *o0 = p[0] + p[1];
+    *o1 = p[2] + p[3];
+  };
+  {
+    double w0, w1;
+    mul(in0 ? bvec[pq * (int64_t)k + r] : 0.0, in1 ? bvec[pq * (int64_t)k + r1] : 0.0, &w0, &w1);
+    mul(w0, w1, &w0, &w1);
+    const double m = (double)(k - 1);
+    double wq[4];
+    spread<P, RPL, NT>(w0 / m, w1 / m, wq);
+    static_for<NT>([&](auto T) __attribute__((always_inline)) {
+      constexpr int tt = decltype(T)::value;
+      block_upd<KQ, tt, false>(a0, wq[tt], 0.0, 1.0, 0.0);
+      if constexpr (RPL == 2) block_upd<KQ, tt, false>(a1, wq[tt], 0.0, 1.0, 0.0);
+    });
+  }
+  // slabs of each problem's group in ascending order
+  const int64_t t_gp = pq / C.G;
+  const int g = (int)(pq - t_gp * C.G);
+  const int64_t ij = C.i0 + t_gp;
+  const int mld = act ? D.mld[ij] : 0;
+  int nsl = 0;
+  for (int s0 = 0; s0 < S.ns; s0 += P) {
+    const int s = s0 + r;
+    const bool in = act && s < S.ns && slab_group(L, V, s, mld) == g;
+    const unsigned long long bal = __ballot(in);
+    const unsigned long long hb = P == 64 ? bal : (bal >> (32 * hh)) & 0xffffffffull;
+    if (in) sl[hh][nsl + __popcll(hb & ((1ull << r) - 1ull))] = (unsigned short)s;
+    nsl += __popcll(hb);
+  }
+  __syncthreads();
+  int nmax = nsl;
+  if constexpr (P == 32) nmax = max(nsl, __shfl_xor(nsl, 32, 64));
+  nmax = __builtin_amdgcn_readfirstlane(nmax);
+  const float* xb = S.state + (int64_t)S.k * S.ns * ij;
+  double* xa = ana + (int64_t)S.k * S.ns * ij;
+  auto slab = [&](int qs) { return (int64_t)k * (qs < nsl ? (int)sl[hh][qs] : 0); };
+  int64_t so = slab(0);
+  float x0 = (in0 && nsl > 0) ? xb[so + r] : 0.0f, x1 = (in1 && nsl > 0) ? xb[so + r1] : 0.0f;
+  for (int qs = 0; qs < nmax; ++qs) {
+    const int64_t sn = slab(qs + 1);
+    const bool more = qs + 1 < nsl;
+    const float n0 = (in0 && more) ? xb[sn + r] : 0.0f, n1 = (in1 && more) ? xb[sn + r1] : 0.0f;
+    double o0, o1;
+    mul((double)x0, (double)x1, &o0, &o1);
+    if (qs < nsl) {
+      if (in0) xa[so + r] = o0;
+      if (in1) xa[so + r1] = o1;
+    }
+    so = sn;
+    x0 = n0;
+    x1 = n1;
+  }
+}
+
+// the reduction has left T in dd and ee and the reflectors in B and tau (K
+// entries a problem); perm: the order of the problems, nullptr for 0..np-1
+void launch_back_apply(hipStream_t st, const LocDev& L, const StateDev& S, const VarsDev& V,
+                       const ChunkDev& C, const DiagDev& D, double* B, const double* bvec,
+                       const double* tau, const double* dd, const double* ee, int K,
+                       const RatTab& R, double* ana, const int32_t* perm) {
+  const int64_t np = C.ngp * C.G;
+  if (np <= 0) return;
+  const int k = (int)S.k;
+  k_small_rational<<<(unsigned)np, 64, 0, st>>>(k, K, C, B, dd, ee, R);
+  const unsigned two = (unsigned)((np + 1) / 2);
+#define LK_BACK(KQ, P, RPL, nb)                                                              \
+  k_back_apply<KQ, P, RPL><<<nb, 64, 0, st>>>(k, K, np, perm, L, S, V, C, D, B, bvec, tau, ana)
+  if (k <= 8) LK_BACK(8, 32, 1, two);
+  else if (k <= 16) LK_BACK(16, 32, 1, two);
+  else if (k <= 24) LK_BACK(24, 32, 1, two);
+  else if (k <= 32) LK_BACK(32, 32, 1, two);
+  else if (k <= 40) LK_BACK(40, 32, 2, two);
+  else if (k <= 48) LK_BACK(48, 32, 2, two);
+  else if (k <= 50) LK_BACK(50, 32, 2, two);
+  else if (k <= 56) LK_BACK(56, 64, 1, (unsigned)np);
+  else LK_BACK(64, 64, 1, (unsigned)np);
+#undef LK_BACK
+}
+
+}  // namespace lk

@@ -10,27 +10,25 @@
 //
 // which equals x_b^T T with T = W + wbar 1^T, W being symmetric.
 //
-// Kernels, each shaped for what it does:
+// By default no eigensolve is made for k < 64: A is reduced to tridiagonal form
+// (launch_tridiag_pair: by DPP, two problems per wave) and the transform
+// follows from the rational approximation of x^(-1/2), for the carried vectors
+// alone where every group has few slabs (NV > 0: rat_solve.h, then k_qapply),
+// else as a matrix (back_apply.hip).  Kernels here:
 //  k_tridiag  one wave per problem: Householder reduction A = Q Tri Q^T
-//             (LAPACK dsytd2, lower), A in LDS, lane r owns row r;
+//             (LAPACK dsytd2, lower), A in LDS, lane r owns row r (launch
+//             choice tridiag_reg 0);
+//  k_ratsolve the rational solve as a kernel of its own;
+//  k_qapply   one wave per problem: x_a = Q y + wbar . x_b.
+// With LETKF_GPU_RAT=0 the eigensolve, as a check of the above:
 //  k_tql      one LANE per problem: implicit QL with Wilkinson shift on the
 //             tridiagonal (Numerical Recipes tqli), d and e held in registers
 //             through a statically unrolled, predicated sweep; every rotation
 //             (c, s) and every sweep header (l, m, count) is recorded;
-// then, when a group has many slabs (full path):
-//  k_replay   one wave per problem: replays the recorded rotations into Z
-//             (lane r owns row r, registers; records prefetched two sweeps
-//             ahead and broadcast with readlane) and stores Z;
-//  k_vec_apply  one wave per problem: back-transforms V = Q Z (reflectors
-//             bulk-loaded into LDS) and applies the transform to the group's
-//             slabs with two matrix-vector products per slab (the k x k W is
-//             never formed);
-// or, when every group has few slabs (vector path), only the vectors that
-// the transform touches are carried, V^T x = Z^T Q^T x:
-//  k_tridiag  also applies each reflector to b and to the slabs' x_b;
-//  k_rot_fwd  one lane per (problem, vector): Z^T u from the records;
-//  k_rot_bwd  one lane per (problem, slab): y = f(lam) u, Z y, Q (Z y),
-//             plus wbar.x_b = (V^T b)^T lam^-1 (V^T x_b).
+//  k_replay   one wave per problem: replays the recorded rotations into Z;
+//  k_vec_apply  one wave per problem: V = Q Z and two mat-vecs per slab;
+//  k_rot_fwd, k_rot_bwd  one lane per (problem, vector): the rotations applied
+//             to the carried vectors only, V^T x = Z^T Q^T x.
 // Problems whose record space overflows or whose QL does not converge are
 // flagged and solved by the Jacobi kernel instead.
 #include <hip/hip_runtime.h>
@@ -39,6 +37,7 @@
 
 #include "eigen_common.h"
 #include "letkf_internal.h"
+#include "rat_solve.h"
 
 namespace lk {
 
@@ -571,99 +570,35 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
 // Gershgorin bound of the largest eigenvalue.  Each (T + sigma I) is an SPD
 // tridiagonal system solved by LDL^T in O(k).
 // ---------------------------------------------------------------------------
-constexpr int kRatLanes = 32;        // lanes per problem: 31 nodes + the T^-1 b lane
 
-// 1/x: the hardware estimate and one Newton step, which squares its
-// relative error (the pivots are >= k - 1 > 0 and the batched path's
-// tolerance is far above the result)
-__device__ __forceinline__ double rcp_nr(double x) {
-  const double y = __builtin_amdgcn_rcp(x);
-  return y * (2.0 - x * y);
-}
-
-// one wave = two problems x 32 lanes; lane j < 31 of a problem solves with
-// node j, lane 31 solves T x = Q^T b.  U holds Q^T b (vector 0) and Q^T x_b
-// (vectors 1..nvec); on exit vector q holds y = sqrt(k-1) T^(-1/2) u_q and its
-// last slot (index K-1 >= k) holds wbar . x_b.
+// the solves of rat_vectors (tridiag_pair.h) as a kernel of their own, one
+// wave for two problems: where the reduction has one problem per wave.  U
+// holds Q^T b (vector 0) and Q^T x_b (vectors 1..nvec); on exit vector q holds
+// y = sqrt(k-1) T^(-1/2) u_q and its last slot (index K-1 >= k) wbar . x_b.
 template <int KQ>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2)))
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(KQ > 50 ? 1 : 2)))
 void k_ratsolve(int k, int K, int NV, int64_t np, ChunkDev C, const double* __restrict__ dd,
                 const double* __restrict__ ee, const int* __restrict__ nvec,
-                const int* __restrict__ status, const double* __restrict__ tab,
-                const int* __restrict__ tabn, int nbucket, double* __restrict__ U) {
+                const int* __restrict__ status, RatTab R, double* __restrict__ U) {
+  constexpr int LDH = 66;
+  constexpr int kMaxNV = 9;
+  __shared__ double s_d[2 * LDH], s_e[2 * LDH], s_u[2 * kMaxNV * LDH];
   const int lane = threadIdx.x;
-  const int j = lane & (kRatLanes - 1);
-  const int64_t pair_raw = (int64_t)blockIdx.x * 2 + (lane >> 5);
+  const int r = lane & 31, hh = lane >> 5;
+  const int64_t pair_raw = (int64_t)blockIdx.x * 2 + hh;
   const bool valid = pair_raw < np && C.solve[pair_raw] && status[pair_raw] == 0;
+  if (__ballot(valid) == 0ull) return;
   const int64_t pair = valid ? pair_raw : 0;
-  const double* dp = dd + pair * K;
-  const double* ep = ee + pair * K;
-  // Gershgorin bound of the largest eigenvalue of T (SPD)
-  double gm = 0.0;
-  for (int i = j; i < k; i += kRatLanes) {
-    const double em = i > 0 ? fabs(ep[i - 1]) : 0.0;
-    gm = fmax(gm, dp[i] + em + fabs(ep[i]));
+  for (int i = r; i < 64; i += 32) {
+    s_d[hh * LDH + i] = valid && i < k ? dd[pair * K + i] : 1.0;
+    s_e[hh * LDH + i] = valid && i < k - 1 ? ee[pair * K + i] : 0.0;
+    for (int q = 0; q < NV; ++q)
+      s_u[(hh * kMaxNV + q) * LDH + i] = valid && i < k ? U[(pair * NV + q) * K + i] : 0.0;
   }
-#pragma unroll
-  for (int o = kRatLanes / 2; o >= 1; o >>= 1) gm = fmax(gm, __shfl_xor(gm, o, kRatLanes));
-  const double m = (double)(k - 1);
-  const double kappa = gm / m;
-  int b = (int)ceil(log2(fmax(kappa, 2.0)));
-  b = b < 1 ? 1 : (b > nbucket - 1 ? nbucket - 1 : b);
-  const int nn = tabn[b];
-  const bool node = j < kRatLanes - 1;
-  const double sigma = node ? (j < nn ? m * tab[b * 64 + j] : m) : 0.0;
-  const double coef = (node && j < nn) ? m * tab[b * 64 + 32 + j] : 0.0;
-  const int nsl = valid ? nvec[pair] : 0;
-  const int nsl_all = max(nsl, __shfl_xor(nsl, 32, 64));
-  for (int q = 1; q <= nsl_all; ++q) {
-    const bool act = valid && q <= nsl;
-    const double* ux = U + (pair * NV + (act ? q : 0)) * K;
-    const double* u = node ? ux : U + pair * NV * K;
-    // LDL^T of T + sigma I with the forward substitution, then back
-    double l[KQ], p[KQ];
-    double rprev = 0.0, zprev = 0.0, eprev = 0.0;
-#pragma unroll
-    for (int i = 0; i < KQ; ++i) {
-      if (i < k) {
-        const double li = eprev * rprev;
-        const double Di = dp[i] + sigma - li * eprev;
-        const double ri = rcp_nr(Di);
-        const double zi = u[i] - li * zprev;
-        l[i] = li;
-        p[i] = zi * ri;
-        rprev = ri;
-        zprev = zi;
-        eprev = ep[i];
-      } else {
-        l[i] = 0.0;
-        p[i] = 0.0;
-      }
-    }
-#pragma unroll
-    for (int i = KQ - 2; i >= 0; --i)
-      if (i + 1 < k) p[i] -= l[i + 1] * p[i + 1];
-    // lane 31: wbar . x_b = u_q . T^-1 u_b
-    double wx = 0.0;
-    if (!node) {
-#pragma unroll
-      for (int i = 0; i < KQ; ++i)
-        if (i < k) wx += ux[i] * p[i];
-    }
-    // y_i = sum over node lanes of coef * x_i, gathered by DPP in the last
-    // lane of each half (the T^-1 b lane, whose coef is 0); rows past k
-    // stay unused
-#pragma unroll
-    for (int i = 0; i < KQ; ++i)
-      if (i < k) p[i] = half_sum_dpp(coef * p[i]);
-    if (act && !node) {
-      double* uo = U + (pair * NV + q) * K;
-#pragma unroll
-      for (int i = 0; i < KQ; ++i)
-        if (i < k) uo[i] = p[i];
-      uo[K - 1] = wx;
-    }
-  }
+  __syncthreads();
+  const double* su = s_u + hh * kMaxNV * LDH;
+  rat_vectors<KQ>(k, K, NV, valid, pair, valid ? nvec[pair] : 0, r, s_d + hh * LDH,
+                  s_e + hh * LDH, [su](int q) { return su + q * LDH; }, U, R);
 }
 
 // x_a = Q y + wbar . x_b for every slab of a problem; one wave per problem,
@@ -745,7 +680,7 @@ static int tridiag_launch(hipStream_t st, unsigned nb, size_t lds, int k, const 
   const int kq = (k == 49 || k == 50) ? 50 : (k + 7) / 8 * 8;
   if (reg == 2) {
     const int rc = launch_tridiag_pair(st, (int64_t)nb, perm, kq, NV, k, K, L, S, V, C, D, B,
-                                       bvec, tau, dd, ee, U, nvec, status, R.tab, R.n, R.nb);
+                                       bvec, tau, dd, ee, U, nvec, status, R);
     if (rc) return rc;
   }
   if (K == 64 && reg != 0 &&
@@ -760,7 +695,7 @@ template <int KQ>
 static void ratsolve_launch(hipStream_t st, unsigned nb, int k, int K, int NV, int64_t np,
                             const ChunkDev& C, const double* dd, const double* ee,
                             const int* nvec, const int* status, const RatTab& R, double* U) {
-  k_ratsolve<KQ><<<nb, 64, 0, st>>>(k, K, NV, np, C, dd, ee, nvec, status, R.tab, R.n, R.nb, U);
+  k_ratsolve<KQ><<<nb, 64, 0, st>>>(k, K, NV, np, C, dd, ee, nvec, status, R, U);
 }
 
 template <int K>
@@ -805,6 +740,10 @@ static void pipeline(hipStream_t st, const LocDev& L, const StateDev& S, const V
       default: ratsolve_launch<64>(st, nr, k, K, NV, np, C, dd, ee, nvec, status, R, U); break;
     }
     k_qapply<K><<<nb, K, 0, st>>>(L, S, V, C, D, NV, B, tau, nvec, status, U, ana);
+    return;
+  }
+  if (R.nb > 0) {
+    launch_back_apply(st, L, S, V, C, D, B, bvec, tau, dd, ee, K, R, ana, perm);
     return;
   }
   tql_launch<K, K>(st, nl, k, np, C, dd, ee, rot, cap_rot, itr, cap_it, nit, status);

@@ -132,8 +132,8 @@ __global__ __launch_bounds__(128) void k_mat_rational(int k, ChunkDev C, double*
   bk = __builtin_amdgcn_readfirstlane(bk);
   const int nn = __builtin_amdgcn_readfirstlane(tabn[bk]);
   if (nn > NNL || nn <= NNLO) return;
-  const double* sn = tab + bk * 64;
-  const double* wn = sn + 32;
+  const double* sn = tab + bk * kRatLd;
+  const double* wn = sn + kRatLd / 2;
   // unused node rows stay 0, so that their chains stay 0
   for (int n = nn; n < NNL; ++n) { Us[n][tid] = 0.0; Gs[n][tid] = 0.0; }
   // one lane per node runs both pivot recurrences in one loop, step s

@@ -157,8 +157,7 @@ struct letkf_gpu_t {
   int tune_fuse = 1;      // rational solve inside the two-problem tridiagonalization
   int tune_matblk = 1;    // 64 <= k <= 128: 2D-block reduction and back-transform
   int tune_fusefin = 1;   // 64 <= k <= 128, mixed: post-processing inside the apply
-  int tune_rat = 1;       // vector path: rational A^(-1/2), no eigensolve (1 batched
-                          // path only, 2 the plain FP64 path too, 0 off)
+  int tune_rat = 1;       // k < 64: rational A^(-1/2), no eigensolve (0 off)
   int tune_mat = 1;       // batched, 64 <= k <= 128: explicit T applied on MFMA
   bool use_mat = false;
   int alloc_mat = -1;
@@ -167,6 +166,33 @@ struct letkf_gpu_t {
     return dims.path == LETKF_PATH_BATCHED && dims.precision != LETKF_PREC_FP64;
   }
 };
+
+// The node tables (RatTab): coarse (1e-12, at most 31 nodes) in rows
+// 0..kRatBuckets-1, fine (5e-16, at most 62) in the rows after; where no node
+// count meets the tolerance, the most.  Constants, built at first use: about
+// 30 ms, which every handle paid before.
+struct RatTables {
+  std::vector<double> tab;
+  std::vector<int> n;
+  RatTables() : tab((size_t)2 * kRatBuckets * kRatLd, 0.0), n((size_t)2 * kRatBuckets, 0) {
+    for (int b = 1; b < kRatBuckets; ++b) {
+      const double kappa = std::ldexp(1.0, b);
+      double* s = tab.data() + (size_t)b * kRatLd;
+      double* w = s + kRatLd / 2;
+      int m = rat::choose(kappa, 1e-12, 31, s, w, std::min(31, rat::fewest(kappa, 1e-12)));
+      if (m < 0) { m = 31; rat::nodes(kappa, m, s, w); }
+      n[(size_t)b] = m;
+      s += (size_t)kRatBuckets * kRatLd;
+      w += (size_t)kRatBuckets * kRatLd;
+      m = rat::choose_fine(kappa, 5e-16, 62, s, w);
+      n[(size_t)(kRatBuckets + b)] = m < 0 ? 62 : m;   // s and w hold 62 then
+    }
+  }
+};
+static const RatTables& rat_tables() {
+  static const RatTables t;
+  return t;
+}
 
 static std::string g_create_err;
 
@@ -856,11 +882,12 @@ static int ensure_outputs(letkf_gpu_t* h) {
   HIPCHK(h, dalloc(h, &h->d_lgloc, (size_t)(G * nij)));
   HIPCHK(h, dalloc(h, &h->d_lghash, (size_t)(G * nij)));
   // chunk sizing: bound the per-pair work arrays to about 32 GB
-  h->use_rat = nv > 0 && (h->batched() ? h->tune_rat != 0 : h->tune_rat == 2) && k >= 2;
+  h->use_rat = h->eigK && h->tune_rat != 0;
   h->cap_rot = h->cap_it = 0;
   if (h->eigK && !h->use_rat) eigen_caps((int)k, &h->cap_rot, &h->cap_it);
   const int64_t per_pair = 8 * k * k + 8 * k + 3 * 8 * (int64_t)(use_mat ? 128 : h->eigK) +
-                           (nv ? 8 * (int64_t)nv * h->eigK : 8 * (int64_t)h->eigK * h->eigK) +
+                           (nv ? 8 * (int64_t)nv * h->eigK
+                               : h->use_rat ? 0 : 8 * (int64_t)h->eigK * h->eigK) +
                            16 * (int64_t)h->cap_rot + 16 * (int64_t)h->cap_it + 40;
   int64_t pairs = std::max<int64_t>(
       1, std::min<int64_t>(1ll << h->tune_chunk_log2, (32ll << 30) / per_pair));
@@ -895,7 +922,7 @@ static int ensure_outputs(letkf_gpu_t* h) {
       HIPCHK(h, dalloc(h, &h->d_nvec, (size_t)np));
     } else {
       dfree(h, h->d_U);
-      HIPCHK(h, dalloc(h, &h->d_Z, (size_t)(np * h->eigK * h->eigK)));
+      if (!h->use_rat) HIPCHK(h, dalloc(h, &h->d_Z, (size_t)(np * h->eigK * h->eigK)));
     }
   }
   size_t tb = 0;
@@ -916,20 +943,11 @@ static int ensure_outputs(letkf_gpu_t* h) {
     h->stmp_bytes = sb;
   }
   if ((h->use_rat || h->use_mat) && !h->d_rat) {
-    // x^(-1/2) on [1, 2^b]: the fewest nodes (<= 31) for 1e-12 relative error,
-    // else 31 nodes
-    std::vector<double> tab((size_t)kRatBuckets * 64, 0.0);
-    std::vector<int> tn(kRatBuckets, 0);
-    for (int b = 1; b < kRatBuckets; ++b) {
-      double* sb = tab.data() + (size_t)b * 64;
-      int n = rat::choose(std::ldexp(1.0, b), 1e-12, 31, sb, sb + 32);
-      if (n < 0) { n = 31; rat::nodes(std::ldexp(1.0, b), n, sb, sb + 32); }
-      tn[b] = n;
-    }
-    HIPCHK(h, dalloc(h, &h->d_rat, tab.size()));
-    HIPCHK(h, dalloc(h, &h->d_ratn, tn.size()));
-    HIPCHK(h, hipMemcpy(h->d_rat, tab.data(), 8 * tab.size(), hipMemcpyHostToDevice));
-    HIPCHK(h, hipMemcpy(h->d_ratn, tn.data(), 4 * tn.size(), hipMemcpyHostToDevice));
+    const RatTables& T = rat_tables();
+    HIPCHK(h, dalloc(h, &h->d_rat, T.tab.size()));
+    HIPCHK(h, dalloc(h, &h->d_ratn, T.n.size()));
+    HIPCHK(h, hipMemcpy(h->d_rat, T.tab.data(), 8 * T.tab.size(), hipMemcpyHostToDevice));
+    HIPCHK(h, hipMemcpy(h->d_ratn, T.n.data(), 4 * T.n.size(), hipMemcpyHostToDevice));
   }
   h->alloc_G = G;
   h->alloc_nv = nv;
@@ -1009,7 +1027,12 @@ static hipError_t enqueue_solve(letkf_gpu_t* h, hipStream_t st, const RunViews& 
                          h->tune_matblk != 0, fin_fused(h) ? &F : nullptr);
   } else if (h->eigK) {
     RatTab R;
-    if (h->use_rat) { R.tab = h->d_rat; R.n = h->d_ratn; R.nb = kRatBuckets; }
+    if (h->use_rat) {
+      // the fine table where an eigensolve was exact to rounding: the plain
+      // path, and groups of many slabs
+      const int row = !h->batched() || h->vec_nv == 0 ? kRatBuckets : 0;
+      R = RatTab{h->d_rat + (size_t)row * kRatLd, h->d_ratn + row, kRatBuckets};
+    }
     launch_eigen_pipeline(st, h->loc, W.S, W.V, C, W.D, h->d_B, h->d_b, h->d_tau, h->d_dd,
                           h->d_ee, h->d_rot, h->cap_rot, h->d_itr, h->cap_it, h->d_nit,
                           h->d_status, h->d_Z, h->vec_nv, h->d_U, h->d_nvec, R, h->d_ana,
@@ -1018,7 +1041,7 @@ static hipError_t enqueue_solve(letkf_gpu_t* h, hipStream_t st, const RunViews& 
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     // problems the QL could not finish go to the Jacobi solver
-    e = launch_eigen_apply_f64(st, h->loc, W.S, W.V, C, W.D, h->d_B, h->d_b, h->d_status,
+    if (!h->use_rat) e = launch_eigen_apply_f64(st, h->loc, W.S, W.V, C, W.D, h->d_B, h->d_b, h->d_status,
                                h->d_ana);
     if (e != hipSuccess) return e;
   } else {

@@ -221,6 +221,17 @@ bool product_t16_supported(int prec, int k);
 void launch_bucket_keys(hipStream_t st, int mode, int bbits, int64_t np, int G, int64_t i0,
                         const int64_t* cnt, const uint8_t* solve, const float* lat,
                         const float* lon, uint32_t* keys, int32_t* vals);
+// node tables of the rational approximation of x^(-1/2) on [1, 2^b]: nodes
+// tab[b * kRatLd + j] and weights tab[b * kRatLd + kRatLd / 2 + j], j < n[b].
+// The coarse table has 1e-12 relative error and at most 31 nodes, the fine
+// one 5e-16 and at most 62 (RatTables in letkf_gpu.hip).
+struct RatTab {
+  const double* tab = nullptr;
+  const int* n = nullptr;
+  int nb = 0;                 // 0: not used
+};
+constexpr int kRatBuckets = 48;
+constexpr int kRatLd = 128;
 // register-resident tridiagonalization for rows of KQ (a multiple of 8,
 // k <= KQ <= 64); false if no kernel exists for (KQ, NV)
 bool launch_tridiag_reg(hipStream_t st, unsigned nb, int KQ, int NV, int k, int K,
@@ -228,33 +239,31 @@ bool launch_tridiag_reg(hipStream_t st, unsigned nb, int KQ, int NV, int k, int 
                         const ChunkDev& C, const DiagDev& D, double* B, const double* bvec,
                         double* tau, double* dd, double* ee, double* U, int* nvec,
                         int* status);
-// the same reduction for two problems per wave (rows of KQ <= 50, at most
-// 3 carried vectors), the problems taken in the order perm (nullptr:
-// 0..np-1).  With rnb > 0 (rational node tables) and carried vectors the
-// rational solve runs in the same kernel.  Returns 0 if no kernel exists
-// for (KQ, NV), 1 for the reduction alone, 2 with the rational solve.
+// the same reduction by DPP (rows of KQ, 8 to 64; two problems per wave up
+// to 50), the problems taken in the order perm (nullptr: 0..np-1).  With a
+// node table (R.nb > 0) and carried vectors the rational solve runs in the
+// same kernel up to rows of 50.  Returns 0 if no kernel exists for (KQ, NV),
+// 1 for the reduction alone, 2 with the rational solve.
 int launch_tridiag_pair(hipStream_t st, int64_t np, const int32_t* perm, int KQ, int NV, int k,
                         int K, const LocDev& L, const StateDev& S, const VarsDev& V,
                         const ChunkDev& C, const DiagDev& D, double* B, const double* bvec,
                         double* tau, double* dd, double* ee, double* U, int* nvec,
-                        int* status, const double* rtab, const int* rtabn, int rnb);
+                        int* status, const RatTab& R);
+// the transform of groups of many slabs from the reduction's T and
+// reflectors (k < 64): M, the back-transform and the apply (back_apply.hip)
+void launch_back_apply(hipStream_t st, const LocDev& L, const StateDev& S, const VarsDev& V,
+                       const ChunkDev& C, const DiagDev& D, double* B, const double* bvec,
+                       const double* tau, const double* dd, const double* ee, int K,
+                       const RatTab& R, double* ana, const int32_t* perm);
 int eigen_pipeline_K(int k);
 void eigen_caps(int k, int* cap_rot, int* cap_it);
 // vectors carried per problem on the vector path (b + slabs of a group,
 // rounded up to an instantiated count), 0 if maxslab is too large
 int eigen_vec_nv(int maxslab);
-// node tables of the rational approximation of x^(-1/2) on [1, 2^b]:
-// tab[b * 64 + j] = s_j, tab[b * 64 + 32 + j] = w_j (j < n[b] <= 31)
-struct RatTab {
-  const double* tab = nullptr;
-  const int* n = nullptr;
-  int nb = 0;                 // 0: not used
-};
-constexpr int kRatBuckets = 48;
-// NV == 0: eigenvectors formed (Z, V = QZ) and applied to every slab;
 // NV > 0: only the NV carried vectors are transformed (U: NV x K per
-// problem), by the QL rotations, or, with a node table (R.nb > 0), by the
-// rational approximation of A^(-1/2) without an eigensolve
+// problem); NV == 0: the whole transform is formed and applied to every slab.
+// With a node table (R.nb > 0) by the rational approximation of A^(-1/2),
+// without one by an eigensolve (the QL rotations, or Z and V = Q Z)
 void launch_eigen_pipeline(hipStream_t st, const LocDev& L, const StateDev& S,
                            const VarsDev& V, const ChunkDev& C, const DiagDev& D,
                            double* B, const double* bvec, double* tau, double* dd,

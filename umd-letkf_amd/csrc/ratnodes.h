@@ -19,91 +19,125 @@
 // the square of sc accurate when k is close to 1.
 #pragma once
 
+#include <algorithm>
 #include <cmath>
+#include <limits>
+#include <vector>
 
 namespace lk {
 namespace rat {
 
+template <typename T>
+constexpr T kPi = (T)3.141592653589793238462643383279502884L;
+
 // complete elliptic integral K(k) = pi / (2 AGM(1, k'))
-inline double ellipk_c(double kc) {
-  double a = 1.0, b = kc;
-  for (int i = 0; i < 64 && std::fabs(a - b) > 1e-17 * a; ++i) {
-    const double an = 0.5 * (a + b);
+template <typename T>
+inline T ellipk_c(T kc) {
+  T a = 1, b = kc;
+  for (int i = 0; i < 64 && std::fabs(a - b) > std::numeric_limits<T>::epsilon() / 16 * a; ++i) {
+    const T an = (a + b) / 2;
     b = std::sqrt(a * b);
     a = an;
   }
-  return M_PI / (2.0 * a);
+  return kPi<T> / (2 * a);
 }
 
 // sn, cn, dn of u for modulus k (k' = kc), AGM method
-inline void ellipj(double u, double k, double kc, double* sn, double* cn, double* dn) {
-  double a[40], c[40];
-  a[0] = 1.0;
-  double b = kc;
+template <typename T>
+inline void ellipj(T u, T k, T kc, T* sn, T* cn, T* dn) {
+  T a[40], c[40];
+  a[0] = 1;
+  T b = kc;
   c[0] = k;
   int n = 0;
-  while (n < 38 && std::fabs(c[n]) > 1e-17) {
-    a[n + 1] = 0.5 * (a[n] + b);
-    c[n + 1] = 0.5 * (a[n] - b);
+  while (n < 38 && std::fabs(c[n]) > std::numeric_limits<T>::epsilon() / 16) {
+    a[n + 1] = (a[n] + b) / 2;
+    c[n + 1] = (a[n] - b) / 2;
     b = std::sqrt(a[n] * b);
     ++n;
   }
-  double phi = std::ldexp(a[n] * u, n);
-  double phi_prev = phi;
+  T phi = std::ldexp(a[n] * u, n);
+  T phi_prev = phi;
   for (int i = n; i >= 1; --i) {
     phi_prev = phi;
-    phi = 0.5 * (phi + std::asin(c[i] * std::sin(phi) / a[i]));
+    phi = (phi + std::asin(c[i] * std::sin(phi) / a[i])) / 2;
   }
   *sn = std::sin(phi);
   *cn = std::cos(phi);
-  *dn = n >= 1 ? std::cos(phi) / std::cos(phi_prev - phi) : 1.0;
+  *dn = n >= 1 ? std::cos(phi) / std::cos(phi_prev - phi) : T(1);
 }
 
-// nodes for [1, kappa] with n points: s[j] = sc^2(u_j), w[j]
-inline void nodes(double kappa, int n, double* s, double* w) {
-  const double kc = 1.0 / std::sqrt(kappa);
-  const double k = std::sqrt((1.0 - kc) * (1.0 + kc));
-  const double K = ellipk_c(kc);
+// nodes for [1, kappa] with n points: s[j] = sc^2(u_j), w[j]; computed in T
+template <typename T>
+inline void nodes_in(T kappa, int n, T* s, T* w) {
+  const T kc = 1 / std::sqrt(kappa);
+  const T k = std::sqrt((1 - kc) * (1 + kc));
+  const T K = ellipk_c(kc);
   for (int j = 0; j < n; ++j) {
-    const double u = (j + 0.5) * K / n;
-    double sc2, dnc2;
-    if (u <= 0.5 * K) {
-      double sn, cn, dn;
+    const T u = (j + T(0.5)) * K / n;
+    T sc2, dnc2;
+    if (u <= K / 2) {
+      T sn, cn, dn;
       ellipj(u, k, kc, &sn, &cn, &dn);
       sc2 = (sn / cn) * (sn / cn);
       dnc2 = dn / (cn * cn);
     } else {
       // u = K - v: sn = cn(v)/dn(v), cn = k' sn(v)/dn(v), dn = k'/dn(v)
-      double sn, cn, dn;
+      T sn, cn, dn;
       ellipj(K - u, k, kc, &sn, &cn, &dn);
-      const double r = cn / (kc * sn);          // sc(u)
+      const T r = cn / (kc * sn);               // sc(u)
       sc2 = r * r;
       dnc2 = (kc / dn) * (dn / (kc * sn)) * (dn / (kc * sn));   // dn(u) nc(u)^2
     }
     s[j] = sc2;
-    w[j] = 2.0 * K / (M_PI * n) * dnc2;
+    w[j] = 2 * K / (kPi<T> * n) * dnc2;
   }
 }
+inline void nodes(double kappa, int n, double* s, double* w) { nodes_in<double>(kappa, n, s, w); }
 
 // largest relative error of the n-point approximation over [1, kappa]
-// (log-spaced samples; the error is a smooth function of log x)
+// (log-spaced samples; the error is a smooth function of log x), summed in T
+template <typename T>
+inline double max_rel_err_in(double kappa, int n, const double* s, const double* w,
+                             int samples) {
+  T e = 0;
+  for (int i = 0; i <= samples; ++i) {
+    const T x = std::exp(std::log((T)kappa) * i / samples);
+    T acc = 0;
+    for (int j = 0; j < n; ++j) acc += w[j] / (x + s[j]);
+    e = std::fmax(e, std::fabs(acc * std::sqrt(x) - 1));
+  }
+  return (double)e;
+}
 inline double max_rel_err(double kappa, int n, const double* s, const double* w,
                           int samples = 1500) {
-  double e = 0.0;
-  for (int i = 0; i <= samples; ++i) {
-    const double x = std::exp(std::log(kappa) * i / samples);
-    double acc = 0.0;
-    for (int j = 0; j < n; ++j) acc += w[j] / (x + s[j]);
-    e = std::fmax(e, std::fabs(acc * std::sqrt(x) - 1.0));
-  }
-  return e;
+  return max_rel_err_in<double>(kappa, n, s, w, samples);
 }
 
-// smallest n <= nmax meeting tol on [1, kappa]; fills s, w; returns n or -1
-inline int choose(double kappa, double tol, int nmax, double* s, double* w) {
-  for (int n = 2; n <= nmax; ++n) {
+// fewest nodes that can meet tol: the error falls like
+// exp(-2 pi^2 n / log(16 kappa)); two below, so that no smaller n does
+inline int fewest(double kappa, double tol) {
+  return std::max(2, (int)(-std::log(tol) * std::log(16.0 * kappa) / (2.0 * M_PI * M_PI)) - 2);
+}
+
+// smallest n in nmin..nmax meeting tol on [1, kappa]; fills s, w; returns n
+// or -1
+inline int choose(double kappa, double tol, int nmax, double* s, double* w, int nmin = 2) {
+  for (int n = nmin; n <= nmax; ++n) {
     nodes(kappa, n, s, w);
     if (max_rel_err(kappa, n, s, w) <= tol) return n;
+  }
+  return -1;
+}
+
+// the same for a tolerance at the rounding of the values themselves: nodes
+// and error in extended precision, the nodes rounded once
+inline int choose_fine(double kappa, double tol, int nmax, double* s, double* w) {
+  std::vector<long double> ls((size_t)nmax), lw((size_t)nmax);
+  for (int n = std::min(fewest(kappa, tol), nmax); n <= nmax; ++n) {
+    nodes_in<long double>(kappa, n, ls.data(), lw.data());
+    for (int j = 0; j < n; ++j) { s[j] = (double)ls[(size_t)j]; w[j] = (double)lw[(size_t)j]; }
+    if (max_rel_err_in<long double>(kappa, n, s, w, 200) <= tol) return n;
   }
   return -1;
 }

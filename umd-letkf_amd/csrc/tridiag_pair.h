@@ -7,11 +7,10 @@
 
 #include <hip/hip_runtime.h>
 
-#include <type_traits>
-#include <utility>
-
+#include "dpp_common.h"
 #include "eigen_common.h"
 #include "letkf_internal.h"
+#include "rat_solve.h"
 
 namespace lk {
 
@@ -44,282 +43,6 @@ namespace lk {
 // and 8.3 ms.
 // ---------------------------------------------------------------------------
 
-template <typename F, int... I>
-__device__ __forceinline__ void static_for_(F&& f, std::integer_sequence<int, I...>) {
-  (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-  static_for_(f, std::make_integer_sequence<int, N>{});
-}
-
-// the value of lane N of each 16-lane row
-template <int N>
-__device__ __forceinline__ double row_bcast(double v) {
-  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), 0x150 + N, 0xf, 0xf, true);
-  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), 0x150 + N, 0xf, 0xf, true);
-  return __hiloint2double(hi, lo);
-}
-
-// rows (0, 1, 2, 3) of 16 lanes -> e = (0, 0, 2, 2), o = (1, 1, 3, 3)
-__device__ __forceinline__ void rows16(double v, double* e, double* o) {
-  const unsigned l = (unsigned)__double2loint(v), h = (unsigned)__double2hiint(v);
-  const auto sl = __builtin_amdgcn_permlane16_swap(l, l, false, false);
-  const auto sh = __builtin_amdgcn_permlane16_swap(h, h, false, false);
-  *e = __hiloint2double((int)sh[0], (int)sl[0]);
-  *o = __hiloint2double((int)sh[1], (int)sl[1]);
-}
-
-// halves (0, 1) of the wave -> e = (0, 0), o = (1, 1)
-__device__ __forceinline__ void rows32(double v, double* e, double* o) {
-  const unsigned l = (unsigned)__double2loint(v), h = (unsigned)__double2hiint(v);
-  const auto sl = __builtin_amdgcn_permlane32_swap(l, l, false, false);
-  const auto sh = __builtin_amdgcn_permlane32_swap(h, h, false, false);
-  *e = __hiloint2double((int)sh[0], (int)sl[0]);
-  *o = __hiloint2double((int)sh[1], (int)sl[1]);
-}
-
-template <int CTRL>
-__device__ __forceinline__ double dpp_mov(double v) {
-  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xf, 0xf, true);
-  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xf, 0xf, true);
-  return __hiloint2double(hi, lo);
-}
-
-// sum over the P lanes of a problem, the same bits in every lane: rotations
-// by 8, 4, 2 and 1 within the 16-lane rows (each stage adds the same two
-// values in both lanes of a pair), then the rows' sums
-template <int P>
-__device__ __forceinline__ double p_sum(double x) {
-  x += dpp_mov<0x128>(x);
-  x += dpp_mov<0x124>(x);
-  x += dpp_mov<0x122>(x);
-  x += dpp_mov<0x121>(x);
-  double e, o;
-  rows16(x, &e, &o);
-  x = e + o;
-  if constexpr (P == 64) {
-    rows32(x, &e, &o);
-    x = e + o;
-  }
-  return x;
-}
-
-// largest value over the P lanes, in every lane
-template <int P>
-__device__ __forceinline__ double p_max(double x) {
-  x = fmax(x, dpp_mov<0x128>(x));
-  x = fmax(x, dpp_mov<0x124>(x));
-  x = fmax(x, dpp_mov<0x122>(x));
-  x = fmax(x, dpp_mov<0x121>(x));
-  double e, o;
-  rows16(x, &e, &o);
-  x = fmax(e, o);
-  if constexpr (P == 64) {
-    rows32(x, &e, &o);
-    x = fmax(e, o);
-  }
-  return x;
-}
-
-// q[t], t < NT: entry 16 t + i of a problem's vector in lane i of each of
-// its 16-lane rows, from the lanes that own rows r (v0) and r + 32 (v1)
-template <int P, int RPL, int NT>
-__device__ __forceinline__ void spread(double v0, double v1, double (&q)[4]) {
-  if constexpr (P == 32) {
-    rows16(v0, &q[0], &q[1]);
-    if constexpr (RPL == 2 && NT > 2) rows16(v1, &q[2], &q[3]);
-  } else {
-    double e, o;
-    rows16(v0, &e, &o);
-    rows32(e, &q[0], &q[2]);
-    rows32(o, &q[1], &q[3]);
-  }
-}
-
-// acc += q(lane N of the row) * x.  A VALU write of a register needs two
-// wait states before DPP reads it, which the compiler does not see inside
-// an asm statement: each one starts with them.
-#define LK_FD(acc, q, x, n) \
-  "v_fmac_f64_dpp " acc ", " q ", " x " row_newbcast:" n " row_mask:0xf bank_mask:0xf\n\t"
-template <int N>
-__device__ __forceinline__ void bfma(double& p, double q, double a) {
-  asm("s_nop 1\n\t" LK_FD("%0", "%1", "%2", "%3") : "+&v"(p) : "v"(q), "v"(a), "n"(N));
-}
-template <int N>
-__device__ __forceinline__ void bfma2(double& p0, double& p1, double q, double a0, double a1) {
-  asm("s_nop 1\n\t" LK_FD("%0", "%2", "%3", "%5") LK_FD("%1", "%2", "%4", "%5")
-      : "+&v"(p0), "+&v"(p1)
-      : "v"(q), "v"(a0), "v"(a1), "n"(N));
-}
-// four columns N..N+3 of the product, two partial sums a row
-template <int N>
-__device__ __forceinline__ void bfma4(double& pa, double& pb, double q, double x0, double x1,
-                                      double x2, double x3) {
-  asm("s_nop 1\n\t" LK_FD("%0", "%2", "%3", "%7") LK_FD("%1", "%2", "%4", "%8")
-      LK_FD("%0", "%2", "%5", "%9") LK_FD("%1", "%2", "%6", "%10")
-      : "+&v"(pa), "+&v"(pb)
-      : "v"(q), "v"(x0), "v"(x1), "v"(x2), "v"(x3), "n"(N), "n"(N + 1), "n"(N + 2), "n"(N + 3));
-}
-template <int N>
-__device__ __forceinline__ void bfma42(double& p0a, double& p0b, double& p1a, double& p1b,
-                                       double q, double x0, double x1, double x2, double x3,
-                                       double y0, double y1, double y2, double y3) {
-  asm("s_nop 1\n\t" LK_FD("%0", "%4", "%5", "%13") LK_FD("%2", "%4", "%9", "%13")
-      LK_FD("%1", "%4", "%6", "%14") LK_FD("%3", "%4", "%10", "%14")
-      LK_FD("%0", "%4", "%7", "%15") LK_FD("%2", "%4", "%11", "%15")
-      LK_FD("%1", "%4", "%8", "%16") LK_FD("%3", "%4", "%12", "%16")
-      : "+&v"(p0a), "+&v"(p0b), "+&v"(p1a), "+&v"(p1b)
-      : "v"(q), "v"(x0), "v"(x1), "v"(x2), "v"(x3), "v"(y0), "v"(y1), "v"(y2), "v"(y3), "n"(N),
-        "n"(N + 1), "n"(N + 2), "n"(N + 3));
-}
-// column N of the rank-2 update, a -= v_r w_c + w_r v_c (nv = -v_r, nw = -w_r)
-template <int N>
-__device__ __forceinline__ void upd(double& a, double wq, double vq, double nv, double nw) {
-  asm("s_nop 1\n\t" LK_FD("%0", "%1", "%3", "%5") LK_FD("%0", "%2", "%4", "%5")
-      : "+&v"(a)
-      : "v"(wq), "v"(vq), "v"(nv), "v"(nw), "n"(N));
-}
-// four columns N..N+3 of it
-template <int N>
-__device__ __forceinline__ void upd4(double& a, double& b, double& c, double& d, double wq,
-                                     double vq, double nv, double nw) {
-  asm("s_nop 1\n\t" LK_FD("%0", "%4", "%6", "%8") LK_FD("%1", "%4", "%6", "%9")
-      LK_FD("%2", "%4", "%6", "%10") LK_FD("%3", "%4", "%6", "%11")
-      LK_FD("%0", "%5", "%7", "%8") LK_FD("%1", "%5", "%7", "%9")
-      LK_FD("%2", "%5", "%7", "%10") LK_FD("%3", "%5", "%7", "%11")
-      : "+&v"(a), "+&v"(b), "+&v"(c), "+&v"(d)
-      : "v"(wq), "v"(vq), "v"(nv), "v"(nw), "n"(N), "n"(N + 1), "n"(N + 2), "n"(N + 3));
-}
-#undef LK_FD
-
-// 1/x by the hardware estimate e0 and 1/x = e0 (1 + d + d^2 + ...), d = 1 -
-// x e0 (at most 2^-22): cubic, so within rounding of a division.  The pivots
-// of the rational solve are >= k - 1 > 0.
-__device__ __forceinline__ double rcp_cubic(double x) {
-  const double y = __builtin_amdgcn_rcp(x);
-  const double d = fma(-x, y, 1.0);
-  return fma(y, fma(d, d, d), y);
-}
-
-// One stage of the sums of p[0..n) over the lanes: lanes with `bit` go on
-// with the odd entries, the others with the even ones, so n values of all
-// lanes become (n + 1) / 2; CTRL brings the partner lane's value.
-template <int CTRL, int N>
-__device__ __forceinline__ void fold_stage(double (&p)[N], int n, bool bit) {
-#pragma unroll
-  for (int i = 0; i < N; i += 2) {
-    if (i >= n) break;
-    const double a = p[i], b = i + 1 < n ? p[i + 1] : 0.0;
-    const double keep = bit ? b : a, send = bit ? a : b;
-    p[i / 2] = keep + dpp_mov<CTRL>(send);
-  }
-}
-
-// sums over each 32-lane half of p[0..KQ): entry 32 s + rev5(lane) is left
-// in p[s] of lane `lane` (rev5: the five bits reversed).  3 to 7
-// instructions a sum where one DPP sum chain for each takes 15.
-template <int KQ>
-__device__ __forceinline__ void half_sums_spread(double (&p)[KQ], int lane) {
-#pragma unroll
-  for (int i = 0; i < KQ; i += 2) {
-    const double a = p[i], b = i + 1 < KQ ? p[i + 1] : 0.0;
-    const auto l = __builtin_amdgcn_permlane16_swap((unsigned)__double2loint(a),
-                                                    (unsigned)__double2loint(b), false, false);
-    const auto h = __builtin_amdgcn_permlane16_swap((unsigned)__double2hiint(a),
-                                                    (unsigned)__double2hiint(b), false, false);
-    p[i / 2] = __hiloint2double((int)h[0], (int)l[0]) + __hiloint2double((int)h[1], (int)l[1]);
-  }
-  constexpr int n1 = (KQ + 1) / 2, n2 = (n1 + 1) / 2, n3 = (n2 + 1) / 2, n4 = (n3 + 1) / 2;
-  fold_stage<0x140>(p, n1, (lane & 8) != 0);   // row_mirror
-  fold_stage<0x141>(p, n2, (lane & 4) != 0);   // row_half_mirror
-  fold_stage<0x1b>(p, n3, (lane & 2) != 0);    // quad_perm 3 2 1 0
-  fold_stage<0xb1>(p, n4, (lane & 1) != 0);    // quad_perm 1 0 3 2
-}
-
-// The rational solve of one problem per half (see k_tridiag_pair, RAT); all
-// lanes of the wave take part (barrier, DPP sums), lanes of an inactive half
-// or of a problem with more slabs than carried vectors store nothing.
-// s_d, s_e and s_u hold T and the carried vectors of both halves, 0 past
-// row k (1 on the diagonal).
-template <int KQ, int NV>
-__device__ __forceinline__ void rat_tail(int k, int K, bool act, int64_t pq, int nsl, int r,
-                                         bool upper, const double* s_d, const double* s_e,
-                                         const double* s_u, double* __restrict__ U,
-                                         const double* __restrict__ rtab,
-                                         const int* __restrict__ rtabn, int rnb) {
-  constexpr int LDH = 66;
-  const int hh = upper ? 1 : 0;
-  const double* sdh = s_d + hh * LDH;
-  const double* seh = s_e + hh * LDH;
-  const bool valid = act && nsl <= NV - 1;
-  // Gershgorin bound of the largest eigenvalue of T (SPD)
-  double gm = 0.0;
-#pragma unroll
-  for (int i = r; i < KQ; i += 32)
-    if (i < k) gm = fmax(gm, sdh[i] + (i > 0 ? fabs(seh[i - 1]) : 0.0) + fabs(seh[i]));
-  gm = p_max<32>(gm);
-  const double m = (double)(k - 1);
-  const double kappa = gm / m;
-  int b = (int)ceil(log2(fmax(kappa, 2.0)));
-  b = b < 1 ? 1 : (b > rnb - 1 ? rnb - 1 : b);
-  const int nn = rtabn[b];
-  const bool node = r < 31;
-  const double sigma = node ? (r < nn ? m * rtab[b * 64 + r] : m) : 0.0;
-  const double coef = (node && r < nn) ? m * rtab[b * 64 + 32 + r] : 0.0;
-  const int nv_h = valid ? nsl : 0;
-  const int nsl_all = max(nv_h, __shfl_xor(nv_h, 32, 64));
-  const int i0 = (int)(__brev((unsigned)r) >> 27);
-  for (int q = 1; q <= nsl_all; ++q) {
-    const bool actq = valid && q <= nsl;
-    const double* ux = s_u + (hh * NV + (actq ? q : 0)) * LDH;
-    const double* u = node ? ux : s_u + hh * NV * LDH;
-    // LDL^T of T + sigma I with the forward substitution, then back; rows
-    // past k are 1 on the diagonal and 0 elsewhere
-    double l[KQ], p[KQ];
-    double rprev = 0.0, zprev = 0.0, eprev = 0.0;
-#pragma unroll
-    for (int i = 0; i < KQ; ++i) {
-      const double li = eprev * rprev;
-      const double Di = fma(-li, eprev, sdh[i] + sigma);
-      const double ri = rcp_cubic(Di);
-      const double zi = fma(-li, zprev, u[i]);
-      l[i] = li;
-      p[i] = zi * ri;
-      rprev = ri;
-      zprev = zi;
-      eprev = seh[i];
-      // bounds how far the LDS reads are hoisted (their registers)
-      if ((i & 7) == 7) asm volatile("" ::: "memory");
-    }
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int i = KQ - 2; i >= 0; --i) p[i] = fma(-l[i + 1], p[i + 1], p[i]);
-    // lane 31: wbar . x_b = u_q . T^-1 u_b
-    double wx = 0.0;
-    if (!node) {
-#pragma unroll
-      for (int i = 0; i < KQ; ++i) {
-        wx = fma(ux[i], p[i], wx);
-        if ((i & 7) == 7) asm volatile("" ::: "memory");
-      }
-    }
-    // y_i = sum over the node lanes of coef * x_i
-#pragma unroll
-    for (int i = 0; i < KQ; ++i) p[i] *= coef;
-    __builtin_amdgcn_sched_barrier(0);
-    half_sums_spread<KQ>(p, r);
-    if (actq) {
-      double* uo = U + (pq * NV + q) * K;
-      if (i0 < k) uo[i0] = p[0];
-      if constexpr (KQ > 32) {
-        if (i0 + 32 < k) uo[i0 + 32] = p[1];
-      }
-      if (!node) uo[K - 1] = wx;
-    }
-  }
-}
-
 // RAT: the rational solve of the vector path runs in the same kernel after
 // the reduction (P = 32 only), in the layout of k_ratsolve: lane j < 31 of
 // a half solves (T + sigma_j I) x = Q^T x_b by LDL^T, lane 31 solves
@@ -335,8 +58,7 @@ void k_tridiag_pair(int k, int K, int64_t np, const int32_t* __restrict__ perm, 
                     StateDev S, VarsDev V, ChunkDev C, DiagDev D, double* __restrict__ B,
                     const double* __restrict__ bvec, double* __restrict__ tau,
                     double* __restrict__ dd, double* __restrict__ ee, double* __restrict__ U,
-                    int* __restrict__ nvec, int* __restrict__ status,
-                    const double* __restrict__ rtab, const int* __restrict__ rtabn, int rnb) {
+                    int* __restrict__ nvec, int* __restrict__ status, RatTab R) {
   static_assert(P == 32 || (P == 64 && RPL == 1 && !RAT), "");
   static_assert(!XS || (P == 64 && NV > 0), "");
   constexpr int NPW = 64 / P;             // problems per wave
@@ -566,7 +288,9 @@ void k_tridiag_pair(int k, int K, int64_t np, const int32_t* __restrict__ perm, 
     s_d[hh * LDH + r1] = r1 < k ? dg1 : 1.0;
     s_e[hh * LDH + r1] = r1 < k - 1 ? e1 : 0.0;
     __syncthreads();
-    rat_tail<KQ, NV>(k, K, act, pq, nsl, r, upper, s_d, s_e, s_u, U, rtab, rtabn, rnb);
+    const double* su = s_u + hh * NV * LDH;
+    rat_vectors<KQ>(k, K, NV, act && nsl <= NV - 1, pq, nsl, r, s_d + hh * LDH, s_e + hh * LDH,
+                    [su](int qv) { return su + qv * LDH; }, U, R);
   } else if constexpr (NV > 0) {
     __syncthreads();
   }
@@ -609,17 +333,17 @@ int launch_tridiag_pair_nv(hipStream_t st, int64_t np, const int32_t* perm, int 
                            const LocDev& L, const StateDev& S, const VarsDev& V,
                            const ChunkDev& C, const DiagDev& D, double* B, const double* bvec,
                            double* tau, double* dd, double* ee, double* U, int* nvec,
-                           int* status, const double* rtab, const int* rtabn, int rnb) {
+                           int* status, const RatTab& R) {
   const unsigned nb = P == 32 ? (unsigned)((np + 1) / 2) : (unsigned)np;
   if constexpr (NV > 0 && P == 32) {
-    if (rnb > 0) {
+    if (R.nb > 0) {
       k_tridiag_pair<KQ, NV, true, P, RPL, XS><<<nb, 64, 0, st>>>(
-          k, K, np, perm, L, S, V, C, D, B, bvec, tau, dd, ee, U, nvec, status, rtab, rtabn, rnb);
+          k, K, np, perm, L, S, V, C, D, B, bvec, tau, dd, ee, U, nvec, status, R);
       return 2;
     }
   }
   k_tridiag_pair<KQ, NV, false, P, RPL, XS><<<nb, 64, 0, st>>>(
-      k, K, np, perm, L, S, V, C, D, B, bvec, tau, dd, ee, U, nvec, status, rtab, rtabn, rnb);
+      k, K, np, perm, L, S, V, C, D, B, bvec, tau, dd, ee, U, nvec, status, R);
   return 1;
 }
 
@@ -628,11 +352,10 @@ int launch_tridiag_pair_kq(hipStream_t st, int64_t np, const int32_t* perm, int 
                            const LocDev& L, const StateDev& S, const VarsDev& V,
                            const ChunkDev& C, const DiagDev& D, double* B, const double* bvec,
                            double* tau, double* dd, double* ee, double* U, int* nvec,
-                           int* status, const double* rtab, const int* rtabn, int rnb) {
+                           int* status, const RatTab& R) {
 #define LK_GO(NV, P, RPL, XS)                                                               \
   return launch_tridiag_pair_nv<KQ, NV, P, RPL, XS>(st, np, perm, k, K, L, S, V, C, D, B, bvec, \
-                                                    tau, dd, ee, U, nvec, status, rtab, rtabn, \
-                                                    rnb)
+                                                    tau, dd, ee, U, nvec, status, R)
 #define LK_NV(P, RPL, XS)          \
   switch (NV) {                    \
     case 2: LK_GO(2, P, RPL, XS);  \

@@ -7,9 +7,9 @@ int launch_tridiag_pair_24(hipStream_t st, int64_t np, const int32_t* perm, int 
                            const LocDev& L, const StateDev& S, const VarsDev& V,
                            const ChunkDev& C, const DiagDev& D, double* B, const double* bvec,
                            double* tau, double* dd, double* ee, double* U, int* nvec,
-                           int* status, const double* rtab, const int* rtabn, int rnb) {
+                           int* status, const RatTab& R) {
   return launch_tridiag_pair_kq<24>(st, np, perm, NV, k, K, L, S, V, C, D, B, bvec, tau, dd, ee,
-                                     U, nvec, status, rtab, rtabn, rnb);
+                                     U, nvec, status, R);
 }
 
 }  // namespace lk
