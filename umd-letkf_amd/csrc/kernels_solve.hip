@@ -16,6 +16,7 @@
 
 #include <algorithm>
 
+#include "dpp_common.h"
 #include "eigen_common.h"
 #include "letkf_internal.h"
 
@@ -24,98 +25,195 @@ namespace lk {
 typedef double double4_t __attribute__((ext_vector_type(4)));
 
 // ---------------------------------------------------------------------------
-// products: one workgroup (4 waves) per (gridpoint, group).  The kept obs
-// are gathered 64 at a time into LDS as FP64 rows y_j (k values, then d_j in
-// row k, zero padding to KP).  The upper-triangle 16x16 blocks of the
-// (KP x KP) result are spread over the 4 waves; column k of the result is
-// Yb^T R^-1 d.
+// products: Yb^T R^-1 Yb and Yb^T R^-1 d of one (gridpoint, group) on FP64 MFMA
+// (16x16x4), from the padded operand columns (hx in rows 0..k-1, the
+// departure in row k, zeros above).  A wave keeps its 16x16 tiles of the
+// upper triangle in registers and takes four observations a step: lane l
+// holds row 16 b + l % 16 of observation l / 16 for every row block b its
+// tiles touch, which is both MFMA operands' layout, so a step loads each
+// value once, converts it once, and feeds NB (NB + 1) / 2 products of 64
+// cycles from NB loads.  Indices and scaled weights of 64 observations are
+// read one lane each (one division an observation), a batch ahead, and
+// passed on by lane shuffles; columns are loaded one step ahead.
+//
+// Up to k = 63 one wave holds all (at most 10) tiles: one wave a problem, or
+// four that share its observations and add up through LDS where the chunk
+// has too few problems to fill the chip (below 4096: 256 CUs x 4 SIMDs x 4
+// waves).  Above, four waves share the tiles and each reads the columns its
+// own tiles need.
+//
+// The kernel is bound by the matrix units: 5.5 ms at 160 600
+// problems of k = 50 with 6.6e7 kept observations (4.6 ms at the rate of a
+// large FP64 matrix product), where staging 64 converted observations in LDS
+// for four waves, two LDS reads a product, took 18.9 ms.
 // ---------------------------------------------------------------------------
-template <int KP>
-__global__ __launch_bounds__(256) void k_product_f64(ObsDev O, int k, ChunkDev C,
-                                                     double* __restrict__ B,
-                                                     double* __restrict__ bvec) {
-  constexpr int NB = KP / 16;
-  constexpr int NBLK = NB * (NB + 1) / 2;
-  constexpr int PER = (NBLK + 3) / 4;
-  constexpr int LD = KP + 16;
-  __shared__ double Ys[64 * LD];
-  __shared__ double sc[64];
-  const int64_t pair = xcd_order(C.xcd, blockIdx.x, gridDim.x);
-  if (!C.solve[pair]) return;
-  const int64_t m = C.cnt[pair];
-  const int64_t off = C.off[pair];
-  const int tid = threadIdx.x, wid = tid >> 6, lane = tid & 63;
+constexpr int kFewProblems = 4096;
 
-  int bi[PER], bj[PER];
-#pragma unroll
-  for (int p = 0; p < PER; ++p) {
-    int idx = wid + 4 * p, r = 0;
-    bi[p] = -1; bj[p] = -1;
-    if (idx < NBLK) {
-      while (idx >= NB - r) { idx -= NB - r; ++r; }
-      bi[p] = r;
-      bj[p] = r + idx;
-    }
-  }
-  double4_t acc[PER];
-#pragma unroll
-  for (int p = 0; p < PER; ++p) acc[p] = (double4_t){0.0, 0.0, 0.0, 0.0};
+template <int NB>
+__device__ constexpr int tile_row(int idx) {
+  int r = 0;
+  while (idx >= NB - r) { idx -= NB - r; ++r; }
+  return r;
+}
+template <int NB>
+__device__ constexpr int tile_col(int idx) {
+  int r = 0;
+  while (idx >= NB - r) { idx -= NB - r; ++r; }
+  return r + idx;
+}
+// some tile of T0 .. T0 + N - 1 reads row block b
+template <int NB, int T0, int N>
+__device__ constexpr bool tile_reads(int b) {
+  for (int i = T0; i < T0 + N; ++i)
+    if (tile_row<NB>(i) == b || tile_col<NB>(i) == b) return true;
+  return false;
+}
 
-  for (int64_t j0 = 0; j0 < m; j0 += 64) {
-    __syncthreads();
-    for (int e = tid; e < 64 * KP; e += 256) {
-      const int j = e / KP, a = e - j * KP;
-      const int64_t jj = j0 + j;
-      double v = 0.0;
-      if (jj < m) {
-        const int32_t s = C.list_idx[off + jj];
-        if (a < k) v = (double)O.hx[(int64_t)s * k + a];
-        else if (a == k) v = (double)O.dep[s];
-      }
-      Ys[j * LD + a] = v;
-    }
-    if (tid < 64) {
-      const int64_t jj = j0 + tid;
-      double v = 0.0;
-      if (jj < m) v = (double)C.list_w[off + jj] / (double)O.err[C.list_idx[off + jj]];
-      sc[tid] = v;
-    }
-    __syncthreads();
-#pragma unroll 4
-    for (int kk = 0; kk < 16; ++kk) {
-      const int jr = kk * 4 + (lane >> 4);
-      const double s = sc[jr];
-      const double* row = &Ys[jr * LD + (lane & 15)];
-#pragma unroll
-      for (int p = 0; p < PER; ++p) {
-        if (bi[p] >= 0) {
-          const double a = row[16 * bi[p]] * s;
-          const double b = row[16 * bj[p]];
-          acc[p] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc[p], 0, 0, 0);
+// tiles T0 .. T0 + N - 1 over the observations ow, ow + OW, .. (in batches of 64)
+template <int NB, int T0, int N, int OW>
+__device__ __forceinline__ void product_tiles(const ObsDev& O, const int32_t* __restrict__ li,
+                                              const float* __restrict__ lw, int64_t m, int ow,
+                                              int lane, double4_t (&acc)[N]) {
+  const int q = lane >> 4;
+  const float* __restrict__ col = O.hxp + (lane & 15);
+  const int64_t kp = O.kp;
+  auto idx_at = [&](int64_t j) { return li[j + lane < m ? j + lane : 0]; };
+  auto load = [&](int32_t id, float (&y)[NB]) __attribute__((always_inline)) {
+    const float* c = col + (int64_t)id * kp;
+    static_for<NB>([&](auto I) __attribute__((always_inline)) {
+      constexpr int b = decltype(I)::value;
+      if constexpr (tile_reads<NB, T0, N>(b)) y[b] = c[16 * b];
+    });
+  };
+  int64_t j0 = 64 * (int64_t)ow;
+  if (j0 >= m) return;
+  // an entry past the list reads the list's first observation with weight 0
+  int32_t idx = idx_at(j0);
+  double sc = j0 + lane < m ? (double)lw[j0 + lane] / (double)O.err[idx] : 0.0;
+  float y[NB] = {};
+  load(__shfl(idx, q), y);
+  for (; j0 < m; j0 += 64 * OW) {
+    const int64_t jn = j0 + 64 * OW;
+    const bool more = jn < m;
+    const int32_t idx_n = more ? idx_at(jn) : idx;
+    const bool on = jn + lane < m;
+    const float w_n = on ? lw[jn + lane] : 0.0f;
+    const float e_n = on ? O.err[idx_n] : 1.0f;
+    const int nst = (int)min((int64_t)16, (m - j0 + 3) / 4);
+#pragma unroll 2
+    for (int st = 0; st < nst; ++st) {
+      float yn[NB];
+      const int nxt = 4 * (st + 1) + q;
+      load(st + 1 < nst ? __shfl(idx, nxt) : __shfl(idx_n, q), yn);
+      const double s = __shfl(sc, 4 * st + q);
+      double u[NB], v[NB];
+      static_for<NB>([&](auto I) __attribute__((always_inline)) {
+        constexpr int b = decltype(I)::value;
+        if constexpr (tile_reads<NB, T0, N>(b)) {
+          u[b] = (double)y[b];
+          v[b] = u[b] * s;
         }
-      }
+      });
+      static_for<N>([&](auto I) __attribute__((always_inline)) {
+        constexpr int i = decltype(I)::value;
+        constexpr int r = tile_row<NB>(T0 + i), c = tile_col<NB>(T0 + i);
+        acc[i] = __builtin_amdgcn_mfma_f64_16x16x4f64(v[r], u[c], acc[i], 0, 0, 0);
+      });
+      static_for<NB>([&](auto I) __attribute__((always_inline)) {
+        constexpr int b = decltype(I)::value;
+        if constexpr (tile_reads<NB, T0, N>(b)) y[b] = yn[b];
+      });
     }
+    idx = idx_n;
+    sc = on ? (double)w_n / (double)e_n : 0.0;
   }
+}
 
-  double* Bp = B + pair * (int64_t)k * k;
-  double* bp = bvec + pair * (int64_t)k;
-#pragma unroll
-  for (int p = 0; p < PER; ++p) {
-    if (bi[p] < 0) continue;
+// register r of lane l of a tile: row 4r + l/16, column l%16; column k of the
+// result is Yb^T R^-1 d.  A diagonal tile is complete, the others are mirrored.
+template <int NB, int T0, int N>
+__device__ __forceinline__ void product_store(const double4_t (&acc)[N], int k, int lane,
+                                              double* __restrict__ Bp, double* __restrict__ bp) {
+  static_for<N>([&](auto I) __attribute__((always_inline)) {
+    constexpr int i = decltype(I)::value;
+    constexpr int tr = tile_row<NB>(T0 + i), tc = tile_col<NB>(T0 + i);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      // v_mfma_f64_16x16x4f64: register r of lane l holds row 4r + l/16
-      const int row = 16 * bi[p] + 4 * r + (lane >> 4);
-      const int col = 16 * bj[p] + (lane & 15);
-      const double v = acc[p][r];
+      const int row = 16 * tr + 4 * r + (lane >> 4);
+      const int col = 16 * tc + (lane & 15);
+      const double v = acc[i][r];
       if (row < k && col < k) {
-        Bp[row + (int64_t)k * col] = v;
         Bp[col + (int64_t)k * row] = v;
+        if constexpr (tr != tc) Bp[row + (int64_t)k * col] = v;
       } else if (col == k && row < k) {
         bp[row] = v;
       }
     }
+  });
+}
+
+// all tiles in one wave; OW waves share the observations
+template <int NB, int OW>
+__global__ __launch_bounds__(64 * OW) __attribute__((amdgpu_waves_per_eu(3)))
+void k_product_f64(ObsDev O, int k, ChunkDev C, double* __restrict__ B,
+                   double* __restrict__ bvec) {
+  constexpr int N = NB * (NB + 1) / 2;
+  __shared__ double red[OW > 1 ? 2 * N * 4 * 64 : 1];
+  const int64_t pair = xcd_order(C.xcd, blockIdx.x, gridDim.x);
+  if (!C.solve[pair]) return;
+  const int64_t m = C.cnt[pair], off = C.off[pair];
+  const int lane = threadIdx.x & 63;
+  const int ow = OW > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
+  double4_t acc[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) acc[i] = (double4_t){0.0, 0.0, 0.0, 0.0};
+  product_tiles<NB, 0, N, OW>(O, C.list_idx + off, C.list_w + off, m, ow, lane, acc);
+  if constexpr (OW == 4) {
+    // waves 2 and 3 into 0 and 1, then 1 into 0
+#pragma unroll
+    for (int h = 2; h >= 1; h >>= 1) {
+      if (ow >= h && ow < 2 * h) {
+        double* to = red + (ow - h) * (N * 256);
+#pragma unroll
+        for (int i = 0; i < 4 * N; ++i) to[i * 64 + lane] = acc[i >> 2][i & 3];
+      }
+      __syncthreads();
+      if (ow < h) {
+        const double* from = red + ow * (N * 256);
+#pragma unroll
+        for (int i = 0; i < 4 * N; ++i) acc[i >> 2][i & 3] += from[i * 64 + lane];
+      }
+      __syncthreads();
+    }
+    if (ow != 0) return;
   }
+  product_store<NB, 0, N>(acc, k, lane, B + pair * (int64_t)k * k, bvec + pair * (int64_t)k);
+}
+
+// four waves share the tiles (k >= 64)
+template <int NB>
+__global__ __launch_bounds__(256) void k_product_f64_wide(ObsDev O, int k, ChunkDev C,
+                                                          double* __restrict__ B,
+                                                          double* __restrict__ bvec) {
+  constexpr int NBLK = NB * (NB + 1) / 2, PER = (NBLK + 3) / 4;
+  const int64_t pair = xcd_order(C.xcd, blockIdx.x, gridDim.x);
+  if (!C.solve[pair]) return;
+  const int64_t m = C.cnt[pair], off = C.off[pair];
+  const int lane = threadIdx.x & 63;
+  const int tw = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  double* Bp = B + pair * (int64_t)k * k;
+  double* bp = bvec + pair * (int64_t)k;
+  static_for<4>([&](auto W) __attribute__((always_inline)) {
+    constexpr int w = decltype(W)::value;
+    constexpr int T0 = w * PER, N = NBLK - T0 < PER ? NBLK - T0 : PER;
+    if (tw == w) {
+      double4_t acc[N];
+#pragma unroll
+      for (int i = 0; i < N; ++i) acc[i] = (double4_t){0.0, 0.0, 0.0, 0.0};
+      product_tiles<NB, T0, N, 1>(O, C.list_idx + off, C.list_w + off, m, 0, lane, acc);
+      product_store<NB, T0, N>(acc, k, lane, Bp, bp);
+    }
+  });
 }
 
 void launch_product_f64(hipStream_t st, const ObsDev& O, const StateDev& S,
@@ -123,18 +221,23 @@ void launch_product_f64(hipStream_t st, const ObsDev& O, const StateDev& S,
   const int64_t np = C.ngp * C.G;
   if (np <= 0) return;
   const int k = (int)S.k;
-  const int kp = ((k + 1 + 15) / 16) * 16;
   const unsigned nb = (unsigned)np;
-  switch (kp) {
-    case 16: k_product_f64<16><<<nb, 256, 0, st>>>(O, k, C, B, bvec); break;
-    case 32: k_product_f64<32><<<nb, 256, 0, st>>>(O, k, C, B, bvec); break;
-    case 48: k_product_f64<48><<<nb, 256, 0, st>>>(O, k, C, B, bvec); break;
-    case 64: k_product_f64<64><<<nb, 256, 0, st>>>(O, k, C, B, bvec); break;
-    case 80: k_product_f64<80><<<nb, 256, 0, st>>>(O, k, C, B, bvec); break;
-    case 96: k_product_f64<96><<<nb, 256, 0, st>>>(O, k, C, B, bvec); break;
-    case 112: k_product_f64<112><<<nb, 256, 0, st>>>(O, k, C, B, bvec); break;
-    default: k_product_f64<128><<<nb, 256, 0, st>>>(O, k, C, B, bvec); break;
+  const bool few = np < kFewProblems;
+#define LK_PROD(NB)                                               \
+  if (few) k_product_f64<NB, 4><<<nb, 256, 0, st>>>(O, k, C, B, bvec); \
+  else k_product_f64<NB, 1><<<nb, 64, 0, st>>>(O, k, C, B, bvec);      \
+  break
+  switch ((k + 1 + 15) / 16) {
+    case 1: LK_PROD(1);
+    case 2: LK_PROD(2);
+    case 3: LK_PROD(3);
+    case 4: LK_PROD(4);
+    case 5: k_product_f64_wide<5><<<nb, 256, 0, st>>>(O, k, C, B, bvec); break;
+    case 6: k_product_f64_wide<6><<<nb, 256, 0, st>>>(O, k, C, B, bvec); break;
+    case 7: k_product_f64_wide<7><<<nb, 256, 0, st>>>(O, k, C, B, bvec); break;
+    default: k_product_f64_wide<8><<<nb, 256, 0, st>>>(O, k, C, B, bvec); break;
   }
+#undef LK_PROD
 }
 
 // ---------------------------------------------------------------------------
