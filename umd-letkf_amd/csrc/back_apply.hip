@@ -14,8 +14,8 @@
 // the records into eigenvectors and two mat-vecs a slab (k_tql, k_replay,
 // k_vec_apply, still run with LETKF_GPU_RAT=0): QL is a serial chain per
 // problem, one lane each, and its records cross memory twice.  11 855
-// problems of k = 40 with 50 slabs: 5.2 ms then, 1.1 ms now; 33 problems
-// of k = 50 with 12 slabs: 540 us and 240 us.  The node table is the fine
+// problems of k = 40 with 50 slabs: 5.2 ms then, 0.64 ms now; 33 problems
+// of k = 50 with 12 slabs: 540 us and 100 us.  The node table is the fine
 // one (5e-16): over condition numbers of 1e2 to 8e6 the analysis is no further
 // from the FP64 oracle than the eigensolve's (spread 2e-14 against 1e-13 at
 // 8e6, k = 50).
@@ -148,9 +148,10 @@ __device__ __forceinline__ void block_upd(double (&a)[KQ], double wq, double vq,
 
 // P lanes a problem (two a wave for k <= 50), rows r and, with RPL = 2,
 // r + 32.  The reflectors are walked backwards; reflector j has zeros up to
-// entry j, so whole blocks of 16 columns below it need no product and only
-// the v_r w_c part of the update (a wave-uniform branch each).  Reflectors
-// are loaded four steps ahead.
+// entry j, so the blocks of 16 columns below it need no product and only the
+// v_r w_c part of the update.  That is one loop for each block, not a branch
+// in the step: the matrix stays in place in its registers (with the branch
+// the compiler kept two copies of it and spilled).
 template <int KQ, int P, int RPL>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2)))
 void k_back_apply(int k, int K, int64_t np, const int32_t* __restrict__ perm, LocDev L, StateDev S,
@@ -171,37 +172,47 @@ void k_back_apply(int k, int K, int64_t np, const int32_t* __restrict__ perm, Lo
   const int64_t pq = act ? pair : 0;
   const double* Bp = B + pq * (int64_t)k * k;
   const bool in0 = act && r < k, in1 = act && RPL == 2 && r1 < k;
+  // every load is made, from an address inside the problem, and masked after
+  const int rc = min(r, k - 1), rc1 = min(r1, k - 1);
+  __shared__ double st[NPW][64];
+  for (int i = r; i < 64; i += P) st[hh][i] = act && i < k - 1 ? tau[pq * K + i] : 0.0;
   // M, symmetric, from its lower triangle (row-major in B)
   double a0[KQ], a1[RPL == 2 ? KQ : 1];
 #pragma unroll
   for (int c = 0; c < KQ; ++c) {
-    a0[c] = (in0 && c < k) ? Bp[r >= c ? (int64_t)r * k + c : (int64_t)c * k + r] : 0.0;
-    if constexpr (RPL == 2)
-      a1[c] = (in1 && c < k) ? Bp[r1 >= c ? (int64_t)r1 * k + c : (int64_t)c * k + r1] : 0.0;
+    const int cc = min(c, k - 1);
+    a0[c] = Bp[max(rc, cc) * k + min(rc, cc)];
+    if constexpr (RPL == 2) a1[c] = Bp[max(rc1, cc) * k + min(rc1, cc)];
   }
-  const double* tp = tau + pq * K;
-  double pv0[4], pv1[4], pt[4];
-  auto fetch = [&](int j, int u) __attribute__((always_inline)) {
-    pv0[u] = (in0 && r > j && j >= 0) ? Bp[(int64_t)j * k + r] : 0.0;
-    pv1[u] = (in1 && r1 > j && j >= 0) ? Bp[(int64_t)j * k + r1] : 0.0;
-    pt[u] = (act && j >= 0) ? tp[j] : 0.0;
+#pragma unroll
+  for (int c = 0; c < KQ; ++c) {
+    a0[c] = in0 && c < k ? a0[c] : 0.0;
+    if constexpr (RPL == 2) a1[c] = in1 && c < k ? a1[c] : 0.0;
+  }
+  __syncthreads();
+  double n0 = 0.0, n1 = 0.0;
+  auto fetch = [&](int j) __attribute__((always_inline)) {
+    const double* row = Bp + max(j, 0) * k;
+    n0 = row[rc];
+    if constexpr (RPL == 2) n1 = row[rc1];
   };
-#pragma unroll
-  for (int u = 0; u < 4; ++u) fetch(k - 2 - u, u);
-  for (int jb = k - 2; jb >= 0; jb -= 4) {
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int j = jb - u;
-      if (j < 0) break;
+  fetch(k - 2);
+  // reflectors 16 B - 1 .. 16 B + 14 have zeros in the columns of blocks 0 .. B - 1
+  static_for<NT>([&](auto I) __attribute__((always_inline)) {
+    constexpr int blk = NT - 1 - decltype(I)::value;
+    const int jlo = blk > 0 ? 16 * blk - 1 : 0;
+    for (int j = min(k - 2, 16 * blk + 14); j >= jlo; --j) {
       // an unused reflector (t = 0) was not stored
-      const double t = pt[u];
-      const double v0 = t != 0.0 ? pv0[u] : 0.0, v1 = t != 0.0 ? pv1[u] : 0.0;
-      fetch(j - 4, u);
+      const double t = st[hh][j];
+      const double v0 = in0 && r > j && t != 0.0 ? n0 : 0.0;
+      double v1 = 0.0;
+      if constexpr (RPL == 2) v1 = in1 && r1 > j && t != 0.0 ? n1 : 0.0;
+      fetch(j - 1);
       double vq[4], p[4] = {0.0, 0.0, 0.0, 0.0};
       spread<P, RPL, NT>(v0, v1, vq);
-      static_for<NT>([&](auto T) __attribute__((always_inline)) {
-        constexpr int tt = decltype(T)::value;
-        if (j < 16 * tt + 15) block_prod<KQ, RPL, tt>(p, vq[tt], a0, a1);
+      static_for<NT - blk>([&](auto T) __attribute__((always_inline)) {
+        constexpr int tt = blk + decltype(T)::value;
+        block_prod<KQ, RPL, tt>(p, vq[tt], a0, a1);
       });
       const double p0 = t * (p[0] + p[1]), p1 = t * (p[2] + p[3]);
       double pv = p0 * v0;
@@ -212,16 +223,11 @@ void k_back_apply(int k, int K, int64_t np, const int32_t* __restrict__ perm, Lo
       spread<P, RPL, NT>(w0, w1, wq);
       static_for<NT>([&](auto T) __attribute__((always_inline)) {
         constexpr int tt = decltype(T)::value;
-        if (j < 16 * tt + 15) {
-          block_upd<KQ, tt, true>(a0, wq[tt], vq[tt], -v0, -w0);
-          if constexpr (RPL == 2) block_upd<KQ, tt, true>(a1, wq[tt], vq[tt], -v1, -w1);
-        } else {
-          block_upd<KQ, tt, false>(a0, wq[tt], vq[tt], -v0, -w0);
-          if constexpr (RPL == 2) block_upd<KQ, tt, false>(a1, wq[tt], vq[tt], -v1, -w1);
-        }
+        block_upd<KQ, tt, (tt >= blk)>(a0, wq[tt], vq[tt], -v0, -w0);
+        if constexpr (RPL == 2) block_upd<KQ, tt, (tt >= blk)>(a1, wq[tt], vq[tt], -v1, -w1);
       });
     }
-  }
+  });
   // wbar = W (W b) / (k-1), added to every row: T = W + 1 wbar^T
   auto mul = [&](double x0, double x1, double* o0, double* o1) __attribute__((always_inline)) {
     double xq[4], p[4] = {0.0, 0.0, 0.0, 0.0};
@@ -272,7 +278,7 @@ void k_back_apply(int k, int K, int64_t np, const int32_t* __restrict__ perm, Lo
   for (int qs = 0; qs < nmax; ++qs) {
     const int64_t sn = slab(qs + 1);
     const bool more = qs + 1 < nsl;
-    const float n0 = (in0 && more) ? xb[sn + r] : 0.0f, n1 = (in1 && more) ? xb[sn + r1] : 0.0f;
+    const float y0 = (in0 && more) ? xb[sn + r] : 0.0f, y1 = (in1 && more) ? xb[sn + r1] : 0.0f;
     double o0, o1;
     mul((double)x0, (double)x1, &o0, &o1);
     if (qs < nsl) {
@@ -280,8 +286,8 @@ void k_back_apply(int k, int K, int64_t np, const int32_t* __restrict__ perm, Lo
       if (in1) xa[so + r1] = o1;
     }
     so = sn;
-    x0 = n0;
-    x1 = n1;
+    x0 = y0;
+    x1 = y1;
   }
 }
 
