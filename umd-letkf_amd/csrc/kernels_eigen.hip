@@ -19,7 +19,7 @@
 //             (LAPACK dsytd2, lower), A in LDS, lane r owns row r (launch
 //             choice tridiag_reg 0);
 //  k_ratsolve the rational solve as a kernel of its own;
-//  k_qapply   one wave per problem: x_a = Q y + wbar . x_b.
+//  k_qapply   four problems per wave: x_a = Q y + wbar . x_b.
 // With LETKF_GPU_RAT=0 the eigensolve, as a check of the above:
 //  k_tql      one LANE per problem: implicit QL with Wilkinson shift on the
 //             tridiagonal (Numerical Recipes tqli), d and e held in registers
@@ -601,53 +601,129 @@ void k_ratsolve(int k, int K, int NV, int64_t np, ChunkDev C, const double* __re
                   s_e + hh * LDH, [su](int q) { return su + q * LDH; }, U, R);
 }
 
-// x_a = Q y + wbar . x_b for every slab of a problem; one wave per problem,
-// lane r owns row r
-template <int K>
-__global__ __launch_bounds__(64) void k_qapply(LocDev L, StateDev S, VarsDev V, ChunkDev C,
-                                               DiagDev D, int NV, const double* __restrict__ B,
-                                               const double* __restrict__ tau,
-                                               const int* __restrict__ nvec,
-                                               const int* __restrict__ status,
-                                               const double* __restrict__ U,
-                                               double* __restrict__ ana) {
-  const int64_t pair = blockIdx.x;
-  if (!C.solve[pair] || status[pair] != 0) return;
+// x_a = Q y + wbar . x_b for every slab of a problem, Q y = H_0 H_1 ... H_(k-2) y.
+// Four problems a wave, one in each 16-lane row: lane i holds entries 16 b + i
+// of y for the RB blocks of 16 rows, so v . y is RB products and four DPP
+// rotations for four problems (one problem a wave spent six DPP stages and a
+// readlane on one), and the NS slabs' chains are independent.  What is left
+// is reading the reflectors once (blocks above the pivot row are skipped),
+// the next step's while this one is applied.  592 000 problems of k = 40 with
+// two slabs: 4.7 ms with one problem a wave, 1.85 ms this way; 620 000 of
+// k = 50 with one: 2.7 and 2.4 (their rows fill half of each line they touch).
+template <int RB, int NS>
+__global__ __launch_bounds__(256) void k_qapply(LocDev L, StateDev S, VarsDev V, ChunkDev C,
+                                                DiagDev D, int K, int NV, int64_t np,
+                                                const int32_t* __restrict__ perm,
+                                                const double* __restrict__ B,
+                                                const double* __restrict__ tau,
+                                                const int* __restrict__ nvec,
+                                                const int* __restrict__ status,
+                                                const double* __restrict__ U,
+                                                double* __restrict__ ana) {
+  const int i = threadIdx.x & 15;
+  const int64_t q = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4);
+  int64_t pair = -1;
+  if (q < np) pair = perm ? (int64_t)perm[q] : q;
+  const bool act = pair >= 0 && C.solve[pair] && status[pair] == 0;
+  if (__ballot(act) == 0ull) return;   // wave-uniform
+  const int64_t pq = act ? pair : 0;
   const int k = (int)S.k;
-  const int r = threadIdx.x;
-  const double* Bp = B + pair * (int64_t)k * k;
-  const double* tp = tau + pair * K;
-  const int64_t t_gp = pair / C.G;
-  const int g = (int)(pair - t_gp * C.G);
+  const double* Bp = B + pq * (int64_t)k * k;
+  const double* tp = tau + pq * K;
+  const int nsl = act ? min(nvec[pq], NS) : 0;
+  double y[NS][RB], wx[NS];
+#pragma unroll
+  for (int n = 0; n < NS; ++n) {
+    const double* up = U + (pq * NV + min(n + 1, NV - 1)) * K;
+#pragma unroll
+    for (int b = 0; b < RB; ++b) {
+      const int r = 16 * b + i;
+      const double u = up[min(r, k - 1)];
+      y[n][b] = n < nsl && r < k ? u : 0.0;
+    }
+    wx[n] = up[K - 1];
+  }
+  // reflector j: every load is made, from inside the problem, and masked
+  // (a reflector with tau = 0 was not stored)
+  double vn[RB], tn;
+  auto fetch = [&](int j) __attribute__((always_inline)) {
+    const double* row = Bp + max(j, 0) * k;
+    tn = act && j >= 0 ? tp[j] : 0.0;
+#pragma unroll
+    for (int b = 0; b < RB; ++b)
+      if (16 * b + 15 > j) vn[b] = row[min(16 * b + i, k - 1)];   // wave-uniform
+  };
+#pragma unroll
+  for (int b = 0; b < RB; ++b) vn[b] = 0.0;
+  fetch(k - 2);
+  for (int j = k - 2; j >= 0; --j) {
+    const double t = tn;
+    double v[RB];
+#pragma unroll
+    for (int b = 0; b < RB; ++b) {
+      const int r = 16 * b + i;
+      v[b] = r > j && r < k && t != 0.0 ? vn[b] : 0.0;
+    }
+    fetch(j - 1);
+#pragma unroll
+    for (int n = 0; n < NS; ++n) {
+      double d = v[0] * y[n][0];
+#pragma unroll
+      for (int b = 1; b < RB; ++b) d = fma(v[b], y[n][b], d);
+      d += dpp_mov<0x128>(d);
+      d += dpp_mov<0x124>(d);
+      d += dpp_mov<0x122>(d);
+      d += dpp_mov<0x121>(d);
+      d *= -t;
+#pragma unroll
+      for (int b = 0; b < RB; ++b) y[n][b] = fma(d, v[b], y[n][b]);
+    }
+  }
+  if (!act) return;
+  const int64_t t_gp = pq / C.G;
+  const int g = (int)(pq - t_gp * C.G);
   const int64_t ij = C.i0 + t_gp;
   const int mld = D.mld[ij];
-  const int nsl = nvec[pair];
-  // every reflector's row r and tau (lane jj holds tau_jj) are loaded once,
-  // up front, so the chain of wave sums below never waits on memory; the
-  // step loop is unrolled so that the reflectors stay in registers
-  double hv[K - 1];
-#pragma unroll
-  for (int c = 0; c < K - 1; ++c)
-    hv[c] = (c <= k - 2 && r > c && r < k) ? Bp[(int64_t)c * k + r] : 0.0;
-  const double tv = tp[r];
   int s = -1;
-  for (int q = 1; q <= nsl; ++q) {
+#pragma unroll
+  for (int n = 0; n < NS; ++n) {
+    if (n >= nsl) break;
     for (++s; s < S.ns && slab_group(L, V, s, mld) != g; ++s) {
     }
     if (s >= S.ns) return;
-    const double* up = U + (pair * NV + q) * K;
-    double y = r < k ? up[r] : 0.0;
-    const double wx = up[K - 1];
+    double* xa = ana + (int64_t)S.k * S.ns * ij + (int64_t)k * s;
 #pragma unroll
-    for (int jj = K - 2; jj >= 0; --jj) {
-      if (jj > k - 2) continue;
-      const double tj = bcast(tv, jj);
-      if (tj == 0.0) continue;
-      const double dot = K == 64 ? wave_sum_dpp(hv[jj] * y) : wsumK<K>(hv[jj] * y);
-      y -= (tj * dot) * hv[jj];
+    for (int b = 0; b < RB; ++b) {
+      const int r = 16 * b + i;
+      if (r < k) xa[r] = y[n][b] + wx[n];
     }
-    if (r < k) ana[(int64_t)S.k * S.ns * ij + (int64_t)k * s + r] = y + wx;
   }
+}
+
+static void qapply_launch(hipStream_t st, const LocDev& L, const StateDev& S, const VarsDev& V,
+                          const ChunkDev& C, const DiagDev& D, int K, int NV, int64_t np,
+                          const int32_t* perm, const double* B, const double* tau,
+                          const int* nvec, const int* status, const double* U, double* ana) {
+  const unsigned nb = (unsigned)((np + 15) / 16);
+#define LK_QA(RB, NS)                                                                           \
+  k_qapply<RB, NS><<<nb, 256, 0, st>>>(L, S, V, C, D, K, NV, np, perm, B, tau, nvec, status, U, \
+                                       ana)
+#define LK_QA_NS(RB)              \
+  switch (NV) {                   \
+    case 2: LK_QA(RB, 1); break;  \
+    case 3: LK_QA(RB, 2); break;  \
+    case 5: LK_QA(RB, 4); break;  \
+    default: LK_QA(RB, 8); break; \
+  }                               \
+  break
+  switch (((int)S.k + 15) / 16) {
+    case 1: LK_QA_NS(1);
+    case 2: LK_QA_NS(2);
+    case 3: LK_QA_NS(3);
+    default: LK_QA_NS(4);
+  }
+#undef LK_QA_NS
+#undef LK_QA
 }
 
 int eigen_pipeline_K(int k) { return k <= 31 ? 32 : (k <= 63 ? 64 : 0); }
@@ -724,7 +800,7 @@ static void pipeline(hipStream_t st, const LocDev& L, const StateDev& S, const V
     // rational T^(-1/2): no QL, no eigenvectors
     const unsigned nr = (unsigned)((np + 1) / 2);
     if (tri == 2) {   // solved inside the tridiagonalization
-      k_qapply<K><<<nb, K, 0, st>>>(L, S, V, C, D, NV, B, tau, nvec, status, U, ana);
+      qapply_launch(st, L, S, V, C, D, K, NV, np, perm, B, tau, nvec, status, U, ana);
       return;
     }
     // rows of 50 for k = 49 and 50 (as the register tridiagonalization)
@@ -739,7 +815,7 @@ static void pipeline(hipStream_t st, const LocDev& L, const StateDev& S, const V
       case 50: ratsolve_launch<50>(st, nr, k, K, NV, np, C, dd, ee, nvec, status, R, U); break;
       default: ratsolve_launch<64>(st, nr, k, K, NV, np, C, dd, ee, nvec, status, R, U); break;
     }
-    k_qapply<K><<<nb, K, 0, st>>>(L, S, V, C, D, NV, B, tau, nvec, status, U, ana);
+    qapply_launch(st, L, S, V, C, D, K, NV, np, perm, B, tau, nvec, status, U, ana);
     return;
   }
   if (R.nb > 0) {
