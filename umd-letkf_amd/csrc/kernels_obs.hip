@@ -3,8 +3,8 @@
 //
 // Observations are binned into 1 x 1 degree lat/lon cells, sorted by cell
 // (stable radix sort, so the order inside a cell is the original order) and
-// stored as structure-of-arrays in that order together with their unit
-// vectors and the hx perturbation columns (k floats, contiguous per obs).
+// stored in that order together with their unit vectors (one 32-byte record
+// an observation, with the hash of its index) and the hx perturbation columns (k floats, contiguous per obs).
 // A gridpoint's radius search then reads a handful of contiguous obs ranges.
 #include <hip/hip_runtime.h>
 
@@ -50,8 +50,7 @@ __global__ void k_obs_gather_fields(int64_t n, const int32_t* __restrict__ perm,
                                     const int32_t* __restrict__ obsid,
                                     const int32_t* __restrict__ platid,
                                     const float* __restrict__ hxmean,
-                                    double* x, double* y, double* z,
-                                    float* ozdim, float* oerr, float* odep,
+                                    double2* pos, float* ozdim, float* oerr, float* odep,
                                     int32_t* oidx, int32_t* oobsid,
                                     int32_t* oplatid, float* otime) {
   int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -59,9 +58,8 @@ __global__ void k_obs_gather_fields(int64_t n, const int32_t* __restrict__ perm,
   const int32_t o = perm[s];
   double a, b, c;
   dm::xyz(lat[o], lon[o], &a, &b, &c);
-  x[s] = a;
-  y[s] = b;
-  z[s] = c;
+  pos[2 * s] = make_double2(a, b);
+  pos[2 * s + 1] = make_double2(c, __longlong_as_double((long long)dm::mix64((uint64_t)o)));
   ozdim[s] = zdim[o];
   oerr[s] = err[o];
   {
@@ -122,15 +120,14 @@ void launch_obs_gather(hipStream_t st, int64_t n, int k, const int32_t* perm,
                        const float* time, const float* val, const float* err,
                        const int32_t* obsid, const int32_t* platid,
                        const float* hx, const float* hxmean,
-                       const int32_t* sorted_cell, double* x, double* y,
-                       double* z, float* ozdim, float* oerr, float* odep,
+                       const int32_t* sorted_cell, double2* pos, float* ozdim,
+                       float* oerr, float* odep,
                        int32_t* oidx, int32_t* oobsid, int32_t* oplatid,
                        float* otime, float* ohx, int32_t* cell_start) {
   if (n > 0) {
     unsigned nb = (unsigned)((n + 255) / 256);
-    k_obs_gather_fields<<<nb, 256, 0, st>>>(n, perm, lat, lon, zdim, time, val,
-                                            err, obsid, platid, hxmean, x, y, z,
-                                            ozdim, oerr, odep, oidx, oobsid,
+    k_obs_gather_fields<<<nb, 256, 0, st>>>(n, perm, lat, lon, zdim, time, val, err, obsid,
+                                            platid, hxmean, pos, ozdim, oerr, odep, oidx, oobsid,
                                             oplatid, otime);
     k_obs_gather_hx<<<(unsigned)((n + 63) / 64), 256, 0, st>>>(n, k, perm, hx, ohx);
   }
@@ -173,6 +170,25 @@ void launch_obs_flags(hipStream_t st, const LocDev& L, int64_t n,
   k_obs_flags<<<(unsigned)((n + 255) / 256), 256, 0, st>>>(
       L, n, obsid, platid, time, sat_obs, n_sat_obs, sat_plats, n_sat_plats,
       surf, tw_prof, tw_sat);
+}
+
+// LOC_VGAUSS: the vertical weight of every (level, observation), the same
+// float for every gridpoint
+__global__ void k_obs_vt(int64_t n, int64_t ld, float vt_scale, const float* __restrict__ zdim,
+                         const float* __restrict__ lev_depth, float* vt) {
+#pragma clang fp contract(off)
+  const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (s >= n) return;
+  const double dz = (double)zdim[s] - (double)lev_depth[blockIdx.y];
+  const double sc = (double)vt_scale;
+  vt[blockIdx.y * ld + s] = (float)dm::exp_neg(-(dz * dz) / (2.0 * sc * sc));
+}
+
+void launch_obs_vt(hipStream_t st, int64_t n, int64_t ld, int nlev, float vt_scale,
+                   const float* zdim, const float* lev_depth, float* vt) {
+  if (n <= 0) return;
+  k_obs_vt<<<dim3((unsigned)((n + 255) / 256), (unsigned)nlev), 256, 0, st>>>(
+      n, ld, vt_scale, zdim, lev_depth, vt);
 }
 
 __global__ void k_grid_xyz(int64_t n, const float* __restrict__ lat,

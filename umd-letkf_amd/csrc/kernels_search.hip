@@ -23,21 +23,30 @@
 #include <hip/hip_runtime.h>
 
 #include "det_math.h"
+#include "eigen_common.h"
 #include "letkf_internal.h"
 
 namespace lk {
 
 constexpr double kRad2Deg = 57.295779513082320876;
 
-__device__ __forceinline__ double wave_sum_f64(double v) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
+__device__ __forceinline__ double wave_sum_f64(double v) { return wave_sum_dpp(v); }
+template <int CTRL, int ROWMASK>
+__device__ __forceinline__ uint64_t dpp_u64(uint64_t v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)v, CTRL, ROWMASK, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(v >> 32), CTRL, ROWMASK, 0xf, false);
+  return ((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo;
 }
 __device__ __forceinline__ uint64_t wave_sum_u64(uint64_t v) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
+  v += dpp_u64<0x111, 0xf>(v);
+  v += dpp_u64<0x112, 0xf>(v);
+  v += dpp_u64<0x114, 0xf>(v);
+  v += dpp_u64<0x118, 0xf>(v);
+  v += dpp_u64<0x142, 0xa>(v);
+  v += dpp_u64<0x143, 0xc>(v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, 63);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(v >> 32), 63);
+  return ((uint64_t)hi << 32) | lo;
 }
 // exclusive prefix sum over the wave's lanes, and the total
 __device__ __forceinline__ int wave_excl_scan(int v, int lane, int* total) {
@@ -55,36 +64,12 @@ __device__ __forceinline__ int lane_rank(uint64_t mask) {
                                    __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
 }
 
-// the localizer's scalars that the weights use (copied out of the kernel
-// arguments, so that no reference to them is held)
-struct LocScalars {
-  float tloc_prof, tloc_sat, vt_scale;
-};
-
-// localization weight of one kept-candidate obs for group g (FP32 result)
-__device__ __forceinline__ float loc_weight(int cls, const LocScalars& L, int g, float hz,
-                                            float d, float Lp, float Ls,
-                                            uint8_t surf, float twp, float tws,
-                                            float zdim, const float* lev_depth) {
+// vertical weight of one observation at level g (FP32 result)
+__device__ __forceinline__ float vertical_weight(float vt_scale, float zdim, float depth) {
 #pragma clang fp contract(off)
-  if (cls == LETKF_LOC_OCEAN) {
-    if (surf) {
-      if (g == 1) return 0.0f;
-      float r = dm::gc(d, Ls);
-      if (L.tloc_sat > 0.0f) r = r * tws;
-      return r;
-    }
-    float r = dm::gc(d, Lp);
-    if (L.tloc_prof > 0.0f) r = r * twp;
-    return r;
-  }
-  if (cls == LETKF_LOC_VGAUSS) {
-    const double dz = (double)zdim - (double)lev_depth[g];
-    const double sc = (double)L.vt_scale;
-    const double v = dm::exp_neg(-(dz * dz) / (2.0 * sc * sc));
-    return hz * (float)v;
-  }
-  return hz;
+  const double dz = (double)zdim - (double)depth;
+  const double sc = (double)vt_scale;
+  return (float)dm::exp_neg(-(dz * dz) / (2.0 * sc * sc));
 }
 
 __device__ __forceinline__ bool group_has_slabs(int cls, const LocDev& L, int g, int mld) {
@@ -149,6 +134,14 @@ struct CapCover {
   bool all_lon;   // the cap reaches a pole: whole bands
 };
 
+// cosine of a latitude in degrees, by det_math.h's polynomials (the
+// library's sin, cos and asin carry range reductions that no argument here
+// needs; the cover has margins far above the rounding)
+__device__ __forceinline__ double cos_lat(double deg) {
+  const double x = fabs(deg) / kRad2Deg;
+  return x <= dm::kPIO4 ? dm::cos_core(x) : dm::sin_core(dm::kPIO2 - x);
+}
+
 __device__ __forceinline__ CapCover cap_cover(float rs, float lat, float lon) {
 #pragma clang fp contract(off)
   CapCover cv;
@@ -168,9 +161,9 @@ __device__ __forceinline__ CapCover cap_cover(float rs, float lat, float lon) {
     cv.b1 = b1 < 0 ? 0 : (b1 >= kBands ? kBands - 1 : b1);
     cv.all_lon = !(cv.lat0 + cv.thd < 90.0 && cv.lat0 - cv.thd > -90.0);
   }
-  const double sh = sin(0.5 * theta);
+  const double sh = dm::sin_rad(fmin(0.5 * theta, 1.5));   // not used past a pole
   cv.hav_cap = sh * sh;
-  cv.cos_lat0 = cos(cv.lat0 / kRad2Deg);
+  cv.cos_lat0 = cos_lat(cv.lat0);
   return cv;
 }
 
@@ -185,14 +178,14 @@ __device__ __forceinline__ double cover_halfwidth(const CapCover& cv, int b) {
   if (cv.all_lon || b - cv.b0 >= 64) return 180.0;
   const double la = (double)b - 90.0, lb = la + 1.0;
   const double dmin = cv.lat0 < la ? la - cv.lat0 : (cv.lat0 > lb ? cv.lat0 - lb : 0.0);
-  const double sd = sin(0.5 * dmin / kRad2Deg);
+  const double sd = dm::sin_rad(0.5 * dmin / kRad2Deg);
   const double num = cv.hav_cap - sd * sd;
   if (num <= 0.0) return -1.0;
   const double lo = fmax(la, cv.lat0 - cv.thd), hi = fmin(lb, cv.lat0 + cv.thd);
   const double amax = lo <= hi ? fmax(fabs(lo), fabs(hi)) : fmax(fabs(la), fabs(lb));
-  const double q = num / (cv.cos_lat0 * cos(amax / kRad2Deg));
+  const double q = num / (cv.cos_lat0 * cos_lat(amax));
   if (!(q < 1.0)) return 180.0;
-  return 2.0 * asin(sqrt(q)) * kRad2Deg * (1.0 + 1e-9) + 1e-6;
+  return 2.0 * dm::asin01(sqrt(q)) * kRad2Deg * (1.0 + 1e-9) + 1e-6;
 }
 
 // the one or two longitude cell ranges [rc0, rc1] of half-width dl (< 180)
@@ -218,6 +211,7 @@ __device__ __forceinline__ int cover_ranges(const CapCover& cv, double dl, int r
 //                flag, the search-set size and the other diagnostics
 constexpr int kCountExact = 0, kFill = 1, kFillDiag = 3;
 constexpr int kQueue = 128;   // per-wave candidate ring (two batches)
+constexpr int kSeg = 256;     // several groups: localized candidates held back
 
 // orders this wave's LDS stores and loads on either side (the queue is
 // private to one wave; the block's waves retire independently, so no
@@ -227,11 +221,17 @@ __device__ __forceinline__ void wave_lds_fence() {
   __builtin_amdgcn_wave_barrier();
 }
 
+// sqrt(w / err) of the mixed products' lists, by the hardware reciprocal and
+// square root (1 ulp each; the products round far more)
+__device__ __forceinline__ float list_weight(float w, float err) {
+  return __builtin_amdgcn_sqrtf(w * __builtin_amdgcn_rcpf(err));
+}
+
 // the one-group fill pass (the common case) keeps one group in LDS, which
 // leaves six waves per SIMD to hide the candidates' load latency
 template <int PASS, int CLS>
 __global__ __launch_bounds__(256)
-__attribute__((amdgpu_waves_per_eu(PASS == 3 ? 6 : 1, 8))) void k_search(LocDev L, ObsDev O, StateDev S,
+__attribute__((amdgpu_waves_per_eu(PASS == 3 ? 5 : 1, 8))) void k_search(LocDev L, ObsDev O, StateDev S,
                                                 VarsDev V, ChunkDev C, DiagDev D) {
   constexpr bool FILL = PASS == kFill || PASS == kFillDiag;
   constexpr bool STATS = PASS == kCountExact || PASS == kFillDiag;   // sums, hash
@@ -243,7 +243,14 @@ __attribute__((amdgpu_waves_per_eu(PASS == 3 ? 6 : 1, 8))) void k_search(LocDev 
   __shared__ int32_t s_qs[4][kQueue];             // queued candidates: obs index,
   __shared__ double s_qc[4][kQueue];              //   squared chord,
   __shared__ float s_qe[4][kQueue];               //   error variance
-  __shared__ int32_t s_qo[4][kQueue];             //   and original index
+  __shared__ uint64_t s_qh[4][STATS ? kQueue : 1];   //   and index hash
+  // several groups: horizontally localized candidates (observation, surface
+  // flag in bit 31; weight; error variance or hash), in scan order
+  constexpr bool SEG = PASS != kFillDiag;
+  __shared__ int32_t s_gs[4][SEG ? kSeg : 1];
+  __shared__ float s_gw[4][SEG ? kSeg : 1];
+  __shared__ float s_ge[4][SEG && FILL ? kSeg : 1];
+  __shared__ uint64_t s_gh[4][SEG && !FILL ? kSeg : 1];
   __shared__ int32_t s_rsb[4][129];               // cover ranges: first obs
   __shared__ int32_t s_roff[4][130];              //   and offset in the candidate stream
   const int wid = threadIdx.x >> 6;
@@ -280,9 +287,14 @@ __attribute__((amdgpu_waves_per_eu(PASS == 3 ? 6 : 1, 8))) void k_search(LocDev 
 
   const float lat_ij = S.lat[ij];
   const Radii R = search_radii(CLS, L, lat_ij);
-  const LocScalars LS{L.tloc_prof, L.tloc_sat, L.vt_scale};
-  const float Lh = R.Lh, Lp = R.Lp, Ls = R.Ls, maxhz = R.maxhz, rs = R.rs;
+  const float tloc_prof = L.tloc_prof, tloc_sat = L.tloc_sat, vt_scale = L.vt_scale;
+  const float maxhz = R.maxhz, rs = R.rs;
   const double thr2 = dm::thr2(rs);
+  // length scale of the weights (LOC_OCEAN: profile, and that of surface obs)
+  const float L0 = CLS == LETKF_LOC_OCEAN ? R.Lp : R.Lh;
+  const dm::GcScale gs0 = dm::gc_scale(L0);
+  const dm::GcScale gs1 = CLS == LETKF_LOC_OCEAN ? dm::gc_scale(R.Ls) : gs0;
+  const bool near_cap = 0.25 * thr2 <= dm::kFastHalf2;   // wave-uniform
 
   int mld = 0;                                        // calc_mldlvl_bkgt
   if (CLS == LETKF_LOC_OCEAN && L.vtloc_surf == 1) {
@@ -315,73 +327,123 @@ __attribute__((amdgpu_waves_per_eu(PASS == 3 ? 6 : 1, 8))) void k_search(LocDev 
     fd_cur = C.off[t];
     fd_lim = fd_cur + C.cnt[t];
   }
+  int sn = 0;                  // several groups: candidates held back (wave-uniform)
+  // Several groups: the candidates held back go through the groups 64 at a
+  // time, with one reduction of the sums for each group and up to kSeg of
+  // them (a reduction costs as much as 50 weights).  The count pass of 50
+  // levels on 16 200 gridpoints: 3.6 ms with a reduction for every 64
+  // candidates and the vertical weights evaluated each time, 1.7 ms now.
+  auto flush = [&]() __attribute__((always_inline)) {
+    wave_lds_fence();
+    for (int g = 0; g < G; ++g) {
+      const float depth = CLS == LETKF_LOC_VGAUSS ? V.lev_depth[g] : 0.0f;
+      const float* vt = CLS == LETKF_LOC_VGAUSS && O.vt ? O.vt + g * O.n : nullptr;
+      int64_t cur = 0, lim = 0;
+      if (FILL) { cur = s_cnt[wid][g]; lim = s_lim[wid][g]; }
+      int64_t kept = 0;
+      double sum = 0.0;
+      uint64_t hash = 0;
+      for (int e0 = 0; e0 < sn; e0 += 64) {
+        const int e = e0 + lane;
+        const bool in = e < sn;
+        const int32_t sv = in ? s_gs[wid][e] : 0;
+        float w = in ? s_gw[wid][e] : 0.0f;
+        const int32_t o = sv & 0x7fffffff;
+        if (CLS == LETKF_LOC_VGAUSS) {
+          // the same product as hz * (float)v of the weight function
+          const float v = vt ? vt[o] : vertical_weight(vt_scale, O.zdim[o], depth);
+          w = w * v;
+        }
+        if (CLS == LETKF_LOC_OCEAN && g == 1 && sv < 0) w = 0.0f;   // surface obs: SURF only
+        const bool keep = in && (w > 1.0e-4f);   // src/letkf_solver.F90:251
+        const uint64_t kmask = __ballot(keep);
+        if (kmask == 0) continue;
+        if (STATS) {
+          sum += keep ? (double)w : 0.0;
+          hash += keep ? s_gh[wid][in ? e : 0] : 0ull;
+        }
+        if (FILL && keep) {
+          // writes never pass the end of this pair's list space
+          const int64_t pos = cur + kept + lane_rank(kmask);
+          if (pos < lim) {
+            C.list_idx[pos] = C.list_mode ? (int32_t)((int64_t)o * O.kp * 4) : o;
+            C.list_w[pos] = C.list_mode ? list_weight(w, s_ge[wid][e]) : w;
+          }
+        }
+        kept += __popcll(kmask);
+      }
+      if (kept == 0) continue;
+      if (STATS) {
+        sum = wave_sum_f64(sum);
+        hash = wave_sum_u64(hash);
+      }
+      if (lane == 0) {
+        s_cnt[wid][g] += kept;
+        if (STATS) {
+          s_sum[wid][g] += sum;
+          s_hash[wid][g] += hash;
+        }
+      }
+    }
+    sn = 0;
+    wave_lds_fence();
+  };
   auto localize = [&](int cnt) __attribute__((always_inline)) {
     wave_lds_fence();
     const bool inside = lane < cnt;
-    int64_t s = 0;
-    double c2 = 9.0;
-    float oerr = 1.0f;
-    int32_t oid = 0;
-    if (inside) {
-      const int e = (qh + lane) & (kQueue - 1);
-      s = s_qs[wid][e];
-      c2 = s_qc[wid][e];
-      oerr = s_qe[wid][e];
-      oid = s_qo[wid][e];
+    const int e = (qh + lane) & (kQueue - 1);
+    const int32_t s = inside ? s_qs[wid][e] : 0;
+    const double c2 = inside ? s_qc[wid][e] : 1e-4;
+    const float oerr = inside ? s_qe[wid][e] : 1.0f;
+    const uint64_t mix = STATS && inside ? s_qh[wid][STATS ? e : 0] : 0ull;
+    bool surf = false;
+    float tw = 1.0f;
+    if (CLS == LETKF_LOC_OCEAN) {
+      surf = inside && O.surf[s] != 0;
+      if (surf && tloc_sat > 0.0f) tw = O.tw_sat[s];
+      if (!surf && tloc_prof > 0.0f) tw = O.tw_prof[s];
     }
     wave_lds_fence();
-    float d = 0.0f, hz = 0.0f, zd = 0.0f, twp = 1.0f, tws = 1.0f;
-    uint8_t sf = 0;
-    uint64_t mix = 0;
-    if (inside) {
-      d = dm::dist(c2);
-      if (CLS != LETKF_LOC_OCEAN) hz = dm::gc(d, Lh);
-      if (CLS == LETKF_LOC_OCEAN) { sf = O.surf[s]; twp = O.tw_prof[s]; tws = O.tw_sat[s]; }
-      if (CLS == LETKF_LOC_VGAUSS) zd = O.zdim[s];
-      if (STATS) mix = dm::mix64((uint64_t)oid);
+    // the short forms, and the full ones where a lane is not sure of its float
+    bool sure = false;
+    float d = dm::dist_fast(c2, &sure);
+    sure = sure && near_cap;
+    if (__ballot(inside && !sure) != 0ull) {
+      if (!sure) d = dm::dist(c2);
     }
-    for (int g = 0; g < G; ++g) {
-      float w = 0.0f;
-      if (inside) w = loc_weight(CLS, LS, g, hz, d, Lp, Ls, sf, twp, tws, zd, V.lev_depth);
-      const bool keep = inside && (w > 1.0e-4f);   // src/letkf_solver.F90:251
-      const uint64_t kmask = __ballot(keep);
-      if (kmask == 0) continue;
-      if (PASS == kFillDiag) {
-        // one group: per-lane partial sums, reduced once per gridpoint
-        lsum += keep ? (double)w : 0.0;
-        lhash += keep ? mix : 0ull;
-      } else if (STATS) {
-        const double sr = wave_sum_f64(keep ? (double)w : 0.0);
-        const uint64_t hs = wave_sum_u64(keep ? mix : 0ull);
-        if (lane == 0) {
-          if (!FILL) s_cnt[wid][g] += __popcll(kmask);
-          s_sum[wid][g] += sr;
-          s_hash[wid][g] += hs;
-        }
-      }
-      if (FILL) {
+    dm::GcScale gs = gs0;
+    if (CLS == LETKF_LOC_OCEAN && surf) gs = gs1;
+    float hz = dm::gc_fast(d, gs, &sure);
+    if (__ballot(inside && !sure) != 0ull) {
+      if (!sure) hz = dm::gc(d, CLS == LETKF_LOC_OCEAN && surf ? R.Ls : L0);
+    }
+    if (CLS == LETKF_LOC_OCEAN && (surf ? tloc_sat : tloc_prof) > 0.0f) hz = hz * tw;
+    const bool keep = inside && (hz > 1.0e-4f);   // src/letkf_solver.F90:251
+    const uint64_t kmask = __ballot(keep);
+    if (PASS == kFillDiag) {
+      // one group: per-lane partial sums, reduced once per gridpoint
+      lsum += keep ? (double)hz : 0.0;
+      lhash += keep ? mix : 0ull;
+      if (keep) {
         // writes never pass the end of this pair's list space
-        int64_t cur = fd_cur, lim = fd_lim;
-        if (PASS != kFillDiag) {
-          if (lane == 0) { cur = s_cnt[wid][g]; lim = s_lim[wid][g]; }
-          cur = __shfl(cur, 0, 64);
-          lim = __shfl(lim, 0, 64);
+        const int64_t pos = fd_cur + lane_rank(kmask);
+        if (pos < fd_lim) {
+          C.list_idx[pos] = C.list_mode ? (int32_t)((int64_t)s * O.kp * 4) : s;
+          C.list_w[pos] = C.list_mode ? list_weight(hz, oerr) : hz;
         }
-        if (keep) {
-          const int64_t pos = cur + lane_rank(kmask);
-          if (pos < lim) {
-            // mixed products: byte offset of the padded operand column and
-            // sqrt(w / err) by the hardware reciprocal and square root
-            // (1 ulp each; the products round far more)
-            C.list_idx[pos] = C.list_mode ? (int32_t)(s * O.kp * 4) : (int32_t)s;
-            C.list_w[pos] = C.list_mode
-                                ? __builtin_amdgcn_sqrtf(w * __builtin_amdgcn_rcpf(oerr))
-                                : w;
-          }
-        }
-        if (PASS == kFillDiag) fd_cur = cur + __popcll(kmask);
-        else if (lane == 0) s_cnt[wid][g] = cur + __popcll(kmask);
       }
+      fd_cur += __popcll(kmask);
+    } else if (kmask != 0) {
+      // a group's weight is at most hz: what hz drops, every group drops
+      if (sn + 64 > kSeg) flush();
+      if (keep) {
+        const int at = sn + lane_rank(kmask);
+        s_gs[wid][at] = s | (surf ? (int32_t)0x80000000 : 0);
+        s_gw[wid][at] = hz;
+        if (FILL) s_ge[wid][FILL ? at : 0] = oerr;
+        else s_gh[wid][FILL ? 0 : at] = mix;
+      }
+      sn += __popcll(kmask);
     }
     qh = (qh + cnt) & (kQueue - 1);
     qn -= cnt;
@@ -396,9 +458,9 @@ __attribute__((amdgpu_waves_per_eu(PASS == 3 ? 6 : 1, 8))) void k_search(LocDev 
   // two batches ahead.
   const bool need_err = FILL && C.list_mode;
   struct Cand {
-    double x, y, z;
+    double2 xy, zh;     // position, and the index hash
     float e;
-    int32_t o, s;       // s < 0: past the stream
+    int32_t s;          // < 0: past the stream
   };
   {
     const int b = b0 + lane;
@@ -452,15 +514,13 @@ __attribute__((amdgpu_waves_per_eu(PASS == 3 ? 6 : 1, 8))) void k_search(LocDev 
         so = s_rsb[wid][rl] + (p - s_roff[wid][rl]);
       }
       c.s = p < T ? so : -1;
-      c.x = O.x[so];
-      c.y = O.y[so];
-      c.z = O.z[so];
+      c.xy = O.pos[2 * (int64_t)so];
+      c.zh = O.pos[2 * (int64_t)so + 1];
       if (FILL) c.e = O.err[so];
-      if (STATS) c.o = O.oidx[so];
     };
     auto scan = [&](const Cand& c) __attribute__((always_inline)) {
       double c2 = 9.0;
-      if (c.s >= 0) c2 = dm::chord2(c.x, c.y, c.z, gx, gy, gz);
+      if (c.s >= 0) c2 = dm::chord2(c.xy.x, c.xy.y, c.zh.x, gx, gy, gz);
       const bool inside = c2 <= thr2;
       const uint64_t imask = __ballot(inside);
       if (imask == 0) return;
@@ -471,7 +531,7 @@ __attribute__((amdgpu_waves_per_eu(PASS == 3 ? 6 : 1, 8))) void k_search(LocDev 
         s_qs[wid][e] = c.s;
         s_qc[wid][e] = c2;
         s_qe[wid][e] = need_err ? c.e : 1.0f;
-        s_qo[wid][e] = STATS ? c.o : 0;
+        if (STATS) s_qh[wid][STATS ? e : 0] = (uint64_t)__double_as_longlong(c.zh.y);
       }
       qn += __popcll(imask);
       if (qn >= 64) localize(64);
@@ -497,6 +557,7 @@ __attribute__((amdgpu_waves_per_eu(PASS == 3 ? 6 : 1, 8))) void k_search(LocDev 
     wave_lds_fence();
   }
   if (qn > 0) localize(qn);
+  if (PASS != kFillDiag && sn > 0) flush();
 
   if (PASS == kFillDiag) {
     const double sr = wave_sum_f64(lsum);
@@ -555,16 +616,19 @@ __attribute__((amdgpu_waves_per_eu(PASS == 3 ? 6 : 1, 8))) void k_search(LocDev 
   }
 }
 
-// One-group count pass, one thread per gridpoint: the number of
+// One-group count pass, eight lanes per gridpoint (a band each; on a small
+// grid one lane walking the bands was a 45 us chain): the number of
 // observations in the cells of the cap's cover, an upper bound of the kept
 // count that sizes the list (the fill pass scans the same cells).  Masked
 // gridpoints get zero counts and diagnostics.
 __global__ __launch_bounds__(256) void k_count_cover(LocDev L, ObsDev O, StateDev S,
                                                      ChunkDev C, DiagDev D) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int64_t t = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 3;
+  const int l8 = threadIdx.x & 7;
   if (t >= C.ngp) return;
   const int64_t ij = C.i0 + t;
   if (S.mask[ij]) {                                   // src/letkf_solver.F90:207
+    if (l8 != 0) return;
     C.cnt[t] = 0;
     C.solve[t] = 0;
     D.lg_m[ij] = 0;
@@ -577,8 +641,8 @@ __global__ __launch_bounds__(256) void k_count_cover(LocDev L, ObsDev O, StateDe
   }
   const float lat_ij = S.lat[ij];
   const CapCover cv = cap_cover(search_radii(L.cls, L, lat_ij).rs, lat_ij, S.lon[ij]);
-  int64_t ncand = 0;
-  for (int b = cv.b0; b <= cv.b1; ++b) {
+  int ncand = 0;
+  for (int b = cv.b0 + l8; b <= cv.b1; b += 8) {
     const double dl = cover_halfwidth(cv, b);
     if (dl < 0.0) continue;
     int rc0[2], rc1[2];
@@ -586,7 +650,10 @@ __global__ __launch_bounds__(256) void k_count_cover(LocDev L, ObsDev O, StateDe
     for (int r = 0; r < nr; ++r)
       ncand += O.cell_start[b * kLonCells + rc1[r] + 1] - O.cell_start[b * kLonCells + rc0[r]];
   }
-  C.cnt[t] = ncand;
+  ncand += __shfl_xor(ncand, 1, 8);
+  ncand += __shfl_xor(ncand, 2, 8);
+  ncand += __shfl_xor(ncand, 4, 8);
+  if (l8 == 0) C.cnt[t] = ncand;
 }
 
 // The graph-captured analysis.  Its counters are cleared by a kernel (a
@@ -640,7 +707,7 @@ void launch_search(hipStream_t st, bool fill, const LocDev& L, const ObsDev& O,
   // one group: size the lists by the search set (chord test only) and count
   // the kept observations while writing them
   if (C.G == 1 && !fill) {
-    k_count_cover<<<(unsigned)((C.ngp + 255) / 256), 256, 0, st>>>(L, O, S, C, D);
+    k_count_cover<<<(unsigned)((C.ngp + 31) / 32), 256, 0, st>>>(L, O, S, C, D);
     return;
   }
   const int pass = C.G == 1 ? kFillDiag : (fill ? kFill : kCountExact);

@@ -49,7 +49,7 @@ struct letkf_gpu_t {
 
   // observations (raw copies, then sorted)
   int64_t nobs = 0;
-  double *d_ox = nullptr, *d_oy = nullptr, *d_oz = nullptr;
+  double2* d_opos = nullptr;   // unit vectors and index hashes, 2 per obs
   float *d_ozdim = nullptr, *d_oerr = nullptr, *d_odep = nullptr, *d_otime = nullptr;
   int32_t *d_oidx = nullptr, *d_oobsid = nullptr, *d_oplatid = nullptr;
   float* d_ohx = nullptr;
@@ -58,6 +58,8 @@ struct letkf_gpu_t {
   int32_t* d_cell_start = nullptr;
   uint8_t* d_osurf = nullptr;
   float *d_otwp = nullptr, *d_otws = nullptr;
+  float* d_ovt = nullptr;      // LOC_VGAUSS vertical weights (obs_cap, nlev)
+  int64_t ovt_n = 0;
 
   // variables / localizer / solver
   int nvars = 0;
@@ -378,7 +380,7 @@ int letkf_gpu_destroy(letkf_gpu_t* h) {
   if (h->graph) hipGraphDestroy(h->graph);
   dfree(h, h->d_state); dfree(h, h->d_mean); dfree(h, h->d_sprd); dfree(h, h->d_lat); dfree(h, h->d_lon);
   dfree(h, h->d_mask); dfree(h, h->d_gx); dfree(h, h->d_gy); dfree(h, h->d_gz);
-  dfree(h, h->d_ox); dfree(h, h->d_oy); dfree(h, h->d_oz); dfree(h, h->d_ozdim); dfree(h, h->d_oerr);
+  dfree(h, h->d_opos); dfree(h, h->d_ovt); dfree(h, h->d_ozdim); dfree(h, h->d_oerr);
   dfree(h, h->d_odep); dfree(h, h->d_otime); dfree(h, h->d_oidx); dfree(h, h->d_oobsid);
   dfree(h, h->d_oplatid); dfree(h, h->d_ohx); dfree(h, h->d_ohxp); dfree(h, h->d_cell_start); dfree(h, h->d_osurf);
   dfree(h, h->d_otwp); dfree(h, h->d_otws);
@@ -597,7 +599,7 @@ static int set_obs_impl(letkf_gpu_t* h, int64_t n, const float* lat, const float
     const int64_t cap = std::max<int64_t>((int64_t)nn,
                                           std::min<int64_t>((int64_t)nn + (int64_t)nn / 4, lim));
     const size_t c = (size_t)cap;
-    OBSCHK(dalloc(h, &h->d_ox, c)); OBSCHK(dalloc(h, &h->d_oy, c)); OBSCHK(dalloc(h, &h->d_oz, c));
+    OBSCHK(dalloc(h, &h->d_opos, 2 * c));
     OBSCHK(dalloc(h, &h->d_ozdim, c)); OBSCHK(dalloc(h, &h->d_oerr, c)); OBSCHK(dalloc(h, &h->d_odep, c));
     OBSCHK(dalloc(h, &h->d_otime, c)); OBSCHK(dalloc(h, &h->d_oidx, c)); OBSCHK(dalloc(h, &h->d_oobsid, c));
     OBSCHK(dalloc(h, &h->d_oplatid, c)); OBSCHK(dalloc(h, &h->d_ohx, c * k));
@@ -617,8 +619,7 @@ static int set_obs_impl(letkf_gpu_t* h, int64_t n, const float* lat, const float
     OBSCHK(hipcub::DeviceRadixSort::SortPairs(tmp, tb, cell, scell, iota, perm, (int)n, 0, 17, st));
   }
   launch_obs_gather(st, n, (int)k, perm, r_lat, r_lon, r_zdim, r_time, r_val, r_err,
-                    r_obsid, r_platid, r_hx, r_hxm, scell, h->d_ox, h->d_oy, h->d_oz,
-                    h->d_ozdim, h->d_oerr, h->d_odep, h->d_oidx, h->d_oobsid,
+                    r_obsid, r_platid, r_hx, r_hxm, scell, h->d_opos, h->d_ozdim, h->d_oerr, h->d_odep, h->d_oidx, h->d_oobsid,
                     h->d_oplatid, h->d_otime, h->d_ohx, h->d_cell_start);
   OBSCHK(hipGetLastError());
   launch_obs_pad_hx(st, n, (int)k, h->kp, h->d_ohx, h->d_odep, h->d_ohxp);
@@ -721,10 +722,35 @@ static int upload_flags(letkf_gpu_t* h) {
                    (int)h->sat_obs.size(), sp, (int)h->sat_plats.size(), h->d_osurf,
                    h->d_otwp, h->d_otws);
   hipError_t e = hipGetLastError();
+  // LOC_VGAUSS: a table of the vertical weights, up to 1 GiB of it (the
+  // search evaluates them otherwise)
+  const int64_t nvt = h->loc.cls == LETKF_LOC_VGAUSS ? h->obs_cap * h->loc.nlev : 0;
+  if (nvt > 0 && nvt <= (1ll << 28)) {
+    if (nvt != h->ovt_n) {
+      const hipError_t ea = dalloc(h, &h->d_ovt, (size_t)nvt);
+      if (ea != hipSuccess) {      // a full device: evaluated by the search
+        (void)hipGetLastError();
+        h->d_ovt = nullptr;
+      }
+      h->ovt_n = h->d_ovt ? nvt : 0;
+    }
+    if (h->d_ovt && e == hipSuccess) {
+      launch_obs_vt(h->stream, h->nobs, h->obs_cap, h->loc.nlev, h->loc.vt_scale, h->d_ozdim,
+                    h->d_lev_depth, h->d_ovt);
+      e = hipGetLastError();
+    }
+  } else if (h->d_ovt) {
+    hipStreamSynchronize(h->stream);
+    dfree(h, h->d_ovt);
+    h->ovt_n = 0;
+    ++h->gen;
+  }
   hipStreamSynchronize(h->stream);
   dfree(h, so);
   dfree(h, sp);
-  if (e != hipSuccess) return fail(h, LETKF_EHIP, "obs flags: %s", hipGetErrorString(e));
+  if (e != hipSuccess)
+    return fail(h, e == hipErrorOutOfMemory ? LETKF_ENOMEM : LETKF_EHIP, "obs flags: %s",
+                hipGetErrorString(e));
   return LETKF_OK;
 }
 
@@ -996,9 +1022,8 @@ static RunViews run_views(const letkf_gpu_t* h) {
   return RunViews{
       StateDev{h->k, h->ns, h->nij, h->d_state, h->d_mean, h->d_sprd, h->d_lat, h->d_lon,
                h->d_mask, h->d_gx, h->d_gy, h->d_gz},
-      ObsDev{h->obs_cap, h->d_ox, h->d_oy, h->d_oz, h->d_ozdim, h->d_oerr, h->d_odep,
-             h->d_oidx, h->d_osurf, h->d_otwp, h->d_otws, h->d_ohx, h->d_cell_start,
-             h->d_ohxp, h->kp},
+      ObsDev{h->obs_cap, h->d_opos, h->d_ozdim, h->d_oerr, h->d_odep, h->d_osurf, h->d_otwp,
+             h->d_otws, h->d_ohx, h->d_cell_start, h->d_ovt, h->d_ohxp, h->kp},
       VarsDev{h->nvars, h->d_slab_var, h->d_slab_lev, h->d_inc_max, h->d_bounds,
               h->d_lev_depth},
       DiagDev{h->d_maxhz, h->d_obscount, h->d_lgm, h->d_lgloc, h->d_lghash, h->d_mld,
@@ -1558,14 +1583,11 @@ int letkf_gpu_get_selection(letkf_gpu_t* h, int64_t ij, int32_t group, int32_t* 
   // re-run the search of the chunk that holds ij
   const int64_t i0 = ij;
   ChunkDev C{i0, 1, h->G, h->d_cnt, h->d_off, h->d_solve, h->d_list_idx, h->d_list_w, 0, 0};
-  StateDev S{h->k, h->ns, h->nij, h->d_state, h->d_mean, h->d_sprd, h->d_lat, h->d_lon,
-             h->d_mask, h->d_gx, h->d_gy, h->d_gz};
-  ObsDev O{h->nobs, h->d_ox, h->d_oy, h->d_oz, h->d_ozdim, h->d_oerr, h->d_odep,
-           h->d_oidx, h->d_osurf, h->d_otwp, h->d_otws, h->d_ohx, h->d_cell_start,
-           h->d_ohxp, h->kp};
-  VarsDev V{h->nvars, h->d_slab_var, h->d_slab_lev, h->d_inc_max, h->d_bounds, h->d_lev_depth};
-  DiagDev D{h->d_maxhz, h->d_obscount, h->d_lgm, h->d_lgloc, h->d_lghash, h->d_mld,
-            h->d_ctr};
+  const RunViews W = run_views(h);
+  const ObsDev& O = W.O;
+  const StateDev& S = W.S;
+  const VarsDev& V = W.V;
+  const DiagDev& D = W.D;
   hipStream_t st = h->stream;
   launch_search(st, false, h->loc, O, S, V, C, D);
   size_t tb = h->tmp_bytes;

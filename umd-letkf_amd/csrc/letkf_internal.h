@@ -37,16 +37,16 @@ struct LocDev {
 // sorted observations (search order) and their per-localizer factors
 struct ObsDev {
   int64_t n;
-  const double* x; const double* y; const double* z;
+  const double2* pos;        // 2 per obs: (x, y), (z, bits of mix64(original index))
   const float* zdim;
   const float* err;
   const float* dep;          // val - hx_mean in FP32
-  const int32_t* oidx;       // original index
   const uint8_t* surf;       // LOC_OCEAN surface flag
   const float* tw_prof;      // GC(time, tloc_prof) or 1
   const float* tw_sat;
   const float* hx;           // (k, n) perturbations, sorted columns
   const int32_t* cell_start; // kCells + 1
+  const float* vt;           // LOC_VGAUSS (n, nlev): vertical weights, or nullptr
   const float* hxp;          // (kp, n): hx rows, departure in row k, zero rows
   int kp;                    // 32-multiple >= k + 1
 };
@@ -169,8 +169,8 @@ void launch_obs_gather(hipStream_t st, int64_t n, int k, const int32_t* perm,
                        const float* time, const float* val, const float* err,
                        const int32_t* obsid, const int32_t* platid,
                        const float* hx, const float* hxmean,
-                       const int32_t* sorted_cell, double* x, double* y,
-                       double* z, float* ozdim, float* oerr, float* odep,
+                       const int32_t* sorted_cell, double2* pos, float* ozdim,
+                       float* oerr, float* odep,
                        int32_t* oidx, int32_t* oobsid, int32_t* oplatid,
                        float* otime, float* ohx, int32_t* cell_start);
 void launch_obs_flags(hipStream_t st, const LocDev& L, int64_t n,
@@ -178,6 +178,9 @@ void launch_obs_flags(hipStream_t st, const LocDev& L, int64_t n,
                       const float* time, const int32_t* sat_obs, int n_sat_obs,
                       const int32_t* sat_plats, int n_sat_plats, uint8_t* surf,
                       float* tw_prof, float* tw_sat);
+// vertical weights of LOC_VGAUSS: vt[g * ld + s] for every level g
+void launch_obs_vt(hipStream_t st, int64_t n, int64_t ld, int nlev, float vt_scale,
+                   const float* zdim, const float* lev_depth, float* vt);
 void launch_obs_pad_hx(hipStream_t st, int64_t n, int k, int kp, const float* ohx,
                        const float* odep, float* hxp);
 // observation arrays of set_obs in input order: lat, lon, zdim, time, val,
