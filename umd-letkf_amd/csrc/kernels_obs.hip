@@ -83,15 +83,17 @@ __global__ void k_obs_gather_hx(int64_t n, int k, const int32_t* __restrict__ pe
   }
 }
 
-// operand columns of the mixed-precision products: hxp(kp, n) in search
-// order, rows 0..k-1 the hx perturbations, row k the departure, rows above
-// zero, so a column can be read without row tests
+// operand columns of the products: hxp(kp, n) in search order, rows 0..k-1
+// the hx perturbations, row k the departure, rows above zero, so a column can
+// be read without row tests.  Entry (kp / 16) i + t holds row 16 t + i: lane i
+// of a 16-row operand reads its rows of all row tiles as one run.
 __global__ void k_obs_pad_hx(int64_t n, int k, int kp, const float* __restrict__ ohx,
                              const float* __restrict__ odep, float* hxp) {
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= n * kp) return;
   const int64_t s = e / kp;
-  const int a = (int)(e - s * kp);
+  const int at = (int)(e - s * kp), kt = kp >> 4;
+  const int a = 16 * (at % kt) + at / kt;
   hxp[e] = a < k ? ohx[s * k + a] : (a == k ? odep[s] : 0.0f);
 }
 

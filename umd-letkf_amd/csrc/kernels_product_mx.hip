@@ -63,8 +63,11 @@ __device__ __forceinline__ int obs_slot(int half, int e) {
 // descriptors whose range ends there, so entries past the list read as
 // (0, 0): column 0 with weight 0.  The padded columns carry the departure in
 // row k and zeros above it, so no row or range test is needed.
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned int u32x3 __attribute__((ext_vector_type(3)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef double f64x2 __attribute__((ext_vector_type(2), aligned(8)));
 
 // column byte offsets of the lane's 8 observations of a step
 struct ListRegs {
@@ -97,6 +100,29 @@ __device__ __forceinline__ void load_list(ListRegs& Lr, __amdgpu_buffer_rsrc_t i
   }
 }
 
+// y[0 .. N - 1][e] from N consecutive values of a column, N <= 7
+template <int N>
+__device__ __forceinline__ void load_run(float (&y)[N][8], int e, __amdgpu_buffer_rsrc_t hxr,
+                                         uint32_t vo) {
+  constexpr int T0 = N >= 4 ? 4 : 0, L = N - T0;
+  if constexpr (N >= 4) {
+    const u32x4 c = __builtin_amdgcn_raw_buffer_load_b128(hxr, vo, 0, 0);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) y[t][e] = __uint_as_float(c[t]);
+  }
+  if constexpr (L == 1) {
+    y[T0][e] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(hxr, vo, 4 * T0, 0));
+  } else if constexpr (L == 2) {
+    const u32x2 c = __builtin_amdgcn_raw_buffer_load_b64(hxr, vo, 4 * T0, 0);
+#pragma unroll
+    for (int t = 0; t < 2; ++t) y[T0 + t][e] = __uint_as_float(c[t]);
+  } else if constexpr (L == 3) {
+    const u32x3 c = __builtin_amdgcn_raw_buffer_load_b96(hxr, vo, 4 * T0, 0);
+#pragma unroll
+    for (int t = 0; t < 3; ++t) y[T0 + t][e] = __uint_as_float(c[t]);
+  }
+}
+
 // the step's columns (at the list's offsets) and its weights, which are
 // loaded here rather than with the offsets so that no copy of them has to
 // outlive the offsets' registers
@@ -119,13 +145,11 @@ __device__ __forceinline__ void load_cols(MxFrag<NB>& F, __amdgpu_buffer_rsrc_t 
       F.w[4 + e] = __uint_as_float(b1[e]);
     }
   }
+  // row slot i of block rb is row 16 (NB (i / 16) + rb) + i % 16 (mx_row): a
+  // lane's NB rows follow one another in a column
+  const uint32_t i4 = 4u * NB * (uint32_t)(2 * (i & 15) + (i >> 4));
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    const uint32_t vo = Lr.sidx[e] + 4u * (uint32_t)i;
-#pragma unroll
-    for (int rb = 0; rb < NB; ++rb)
-      F.y[rb][e] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(hxr, vo, 128 * rb, 0));
-  }
+  for (int e = 0; e < 8; ++e) load_run<NB>(F.y, e, hxr, Lr.sidx[e] + i4);
 }
 
 // acc += the products of one 16-observation step
@@ -204,6 +228,12 @@ __device__ __forceinline__ void mx_fold(f32x16* acc, f32x4* Sl) {
     }
 }
 
+// the row in slot i of row block rb (load_cols)
+template <int NB>
+__device__ __forceinline__ int mx_row(int rb, int i) {
+  return 16 * (NB * (i >> 4) + rb) + (i & 15);
+}
+
 template <int KP, int PREC>
 __global__ __launch_bounds__(64) void k_product_mx(ObsDev O, int k, ChunkDev C,
                                                    const int32_t* __restrict__ perm,
@@ -277,8 +307,8 @@ __global__ __launch_bounds__(64) void k_product_mx(ObsDev O, int k, ChunkDev C,
     for (int cb = rb; cb < NB; ++cb, ++b) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const int row = 32 * rb + 8 * (r >> 2) + 4 * half + (r & 3);
-        const int col = 32 * cb + i;
+        const int row = mx_row<NB>(rb, 8 * (r >> 2) + 4 * half + (r & 3));
+        const int col = mx_row<NB>(cb, i);
         double v = (double)acc[b][r];
         if (COMP) v += (double)Ssh[64 * (4 * b + (r >> 2)) + lane][r & 3];
         if (row < k && col < k) {
@@ -286,6 +316,8 @@ __global__ __launch_bounds__(64) void k_product_mx(ObsDev O, int k, ChunkDev C,
           Bp[col + (int64_t)k * row] = v;
         } else if (col == k && row < k) {
           bp[row] = v;
+        } else if (row == k && col < k) {
+          bp[col] = v;
         }
       }
     }
@@ -298,51 +330,87 @@ __global__ __launch_bounds__(64) void k_product_mx(ObsDev O, int k, ChunkDev C,
 // 1,536 products per observation, against 3 blocks of 32x32, 3,072; k = 50:
 // 2,560 against 3,072).  One step is 32 observations: lane l holds
 // observations 8 (l / 16) + e (e = 0..7) of row 16 t + l % 16 of every row
-// tile t, so each lane reads 8 list entries per 32 observations (half the
-// 32x32 kernel's).  The columns of a step are loaded into one register set
+// tile t, which follow one another in a column, so an observation is one
+// load of NT values (two at NT > 4); a dword a row tile kept the address
+// unit busy in 82% of the cycles.  Of the list, a lane holds one entry of
+// its row's eight.  The columns of a step are loaded into one register set
 // right after the previous step's were converted to BF16, and are in flight
 // during that step's MFMAs; lists are loaded two steps ahead.  Split-BF16
 // precisions and compensated accumulation as above (PREC_FP32 keeps the
 // 32x32 kernel).
+//
+// Bound by power: at 620 000 problems of k = 50 with 1e9 kept observations
+// in bf16x4 the cycles are 35 million, near what the instructions cost (an
+// MFMA takes 16 cycles of the matrix unit and 8 of issue, the others 4 of
+// issue: about 1016 a step), and the clock falls to 1.75 GHz.  23.9 ms with
+// dword loads, list entries in every lane, accumulators in AGPRs that each
+// fold copied to VGPRs and back (46 million cycles
+// at 1.88 GHz); 19.6 ms this way.  k = 40, 592 000 problems: 6.6 and
+// 5.5 ms; k = 63 in bf16x3: 1.38 and 1.11; k = 100 in bf16x3: 559 and 451 us.
+// The split by v_dot2_f32_bf16 has a quarter fewer instructions in the
+// conversion but shares the matrix unit with the MFMAs: the same time.
 // ---------------------------------------------------------------------------
 
 template <int NT>
 struct T16Frag {
   float y[NT][8];   // y_j[16 t + lane%16] of the lane's 8 obs, as loaded
-  float w[8];       // their sqrt(rloc_j/err_j)
+  float w;          // sqrt(rloc_j/err_j) of obs lane%8 of the lane's 8
 };
 
-__device__ __forceinline__ void t16_list(ListRegs& Lr, __amdgpu_buffer_rsrc_t ir, int j0,
-                                         int lane) {
-  const uint32_t vo = (uint32_t)(j0 + 8 * (lane >> 4)) * 4u;
-  const u32x4 a0 = __builtin_amdgcn_raw_buffer_load_b128(ir, vo, 0, 0);
-  const u32x4 a1 = __builtin_amdgcn_raw_buffer_load_b128(ir, vo, 16, 0);
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    Lr.sidx[e] = a0[e];
-    Lr.sidx[4 + e] = a1[e];
-  }
+// The eight list entries of a 16-lane row are held by its lanes 0..7 and
+// passed on by row_newbcast in the instructions that use them (the compiler
+// would move each to a register first).  The two wait states are those of a
+// DPP operand that a vector instruction wrote.
+#define LK_ROW8(op, b) \
+  "s_nop 1\n\t" \
+  op " %0, %8, " b(0) " row_newbcast:0 row_mask:0xf bank_mask:0xf\n\t" \
+  op " %1, %8, " b(1) " row_newbcast:1 row_mask:0xf bank_mask:0xf\n\t" \
+  op " %2, %8, " b(2) " row_newbcast:2 row_mask:0xf bank_mask:0xf\n\t" \
+  op " %3, %8, " b(3) " row_newbcast:3 row_mask:0xf bank_mask:0xf\n\t" \
+  op " %4, %8, " b(4) " row_newbcast:4 row_mask:0xf bank_mask:0xf\n\t" \
+  op " %5, %8, " b(5) " row_newbcast:5 row_mask:0xf bank_mask:0xf\n\t" \
+  op " %6, %8, " b(6) " row_newbcast:6 row_mask:0xf bank_mask:0xf\n\t" \
+  op " %7, %8, " b(7) " row_newbcast:7 row_mask:0xf bank_mask:0xf\n\t"
+#define LK_ROW8_OWN(e) "%" #e
+#define LK_ROW8_ADD(e) "%9"
+
+// c[e] *= entry e of w
+__device__ __forceinline__ void row8_mul(float (&c)[8], float w) {
+  asm(LK_ROW8("v_mul_f32_dpp", LK_ROW8_OWN)
+      : "+v"(c[0]), "+v"(c[1]), "+v"(c[2]), "+v"(c[3]), "+v"(c[4]), "+v"(c[5]), "+v"(c[6]),
+        "+v"(c[7])
+      : "v"(w));
+}
+
+// vo[e] = entry e of idx + add
+__device__ __forceinline__ void row8_add(uint32_t (&vo)[8], uint32_t idx, uint32_t add) {
+  asm(LK_ROW8("v_add_u32_dpp", LK_ROW8_ADD)
+      : "=&v"(vo[0]), "=&v"(vo[1]), "=&v"(vo[2]), "=&v"(vo[3]), "=&v"(vo[4]), "=&v"(vo[5]),
+        "=&v"(vo[6]), "=&v"(vo[7])
+      : "v"(idx), "v"(add));
+}
+#undef LK_ROW8
+#undef LK_ROW8_OWN
+#undef LK_ROW8_ADD
+
+// one list entry a lane: a 16-byte load of the eight that a row shares
+// returns 1 KB to the registers and takes as long as the columns' own loads
+__device__ __forceinline__ uint32_t t16_list(__amdgpu_buffer_rsrc_t r, int j0, int lane) {
+  return __builtin_amdgcn_raw_buffer_load_b32(
+      r, (uint32_t)(j0 + 8 * (lane >> 4) + (lane & 7)) * 4u, 0, 0);
 }
 
 template <int NT>
 __device__ __forceinline__ void t16_cols(T16Frag<NT>& F, __amdgpu_buffer_rsrc_t hxr,
-                                         __amdgpu_buffer_rsrc_t wr, const ListRegs& Lr, int j0,
+                                         __amdgpu_buffer_rsrc_t wr, uint32_t idx, int j0,
                                          int lane) {
-  const uint32_t vo = (uint32_t)(j0 + 8 * (lane >> 4)) * 4u;
-  const u32x4 b0 = __builtin_amdgcn_raw_buffer_load_b128(wr, vo, 0, 0);
-  const u32x4 b1 = __builtin_amdgcn_raw_buffer_load_b128(wr, vo, 16, 0);
+  F.w = __uint_as_float(t16_list(wr, j0, lane));
+  constexpr uint32_t KT = (NT + 1) & ~1;                // rows 16 t + i are entries KT i + t
+  const uint32_t i4 = 4u * KT * (uint32_t)(lane & 15);
+  uint32_t vo[8];
+  row8_add(vo, idx, i4);
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    F.w[e] = __uint_as_float(b0[e]);
-    F.w[4 + e] = __uint_as_float(b1[e]);
-  }
-  const uint32_t i4 = 4u * (uint32_t)(lane & 15);
-#pragma unroll
-  for (int e = 0; e < 8; ++e)
-#pragma unroll
-    for (int t = 0; t < NT; ++t)
-      F.y[t][e] = __uint_as_float(
-          __builtin_amdgcn_raw_buffer_load_b32(hxr, Lr.sidx[e] + i4, 64 * t, 0));
+  for (int e = 0; e < 8; ++e) load_run<NT>(F.y, e, hxr, vo[e]);
 }
 
 // weighted operands of a step, split (or rounded) to BF16
@@ -352,7 +420,8 @@ __device__ __forceinline__ void t16_convert(const T16Frag<NT>& F, bf16x8* hi, bf
   for (int t = 0; t < NT; ++t) {
     float c[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) c[e] = F.y[t][e] * F.w[e];
+    for (int e = 0; e < 8; ++e) c[e] = F.y[t][e];
+    row8_mul(c, F.w);
     if (PREC == LETKF_PREC_BF16) hi[t] = to_bf16(c);
     else split_bf16(c, hi[t], lo[t]);
   }
@@ -394,7 +463,7 @@ __device__ __forceinline__ void t16_mfma(f32x4* acc, const bf16x8* hi, const bf1
 
 // compensated accumulation on 16x16 tiles (4 values per lane per tile); the
 // running sums of tile b are the lane's own LDS slot Sl[64 b], which keeps
-// them out of the registers (two waves per SIMD become three at NT = 4)
+// them out of the registers (four waves per SIMD at NT = 4)
 template <int NTILE>
 __device__ __forceinline__ void t16_fold(f32x4* acc, f32x4* Sl) {
 #pragma clang fp contract(off)
@@ -416,7 +485,8 @@ __device__ __forceinline__ void t16_fold(f32x4* acc, f32x4* Sl) {
 }
 
 template <int NT, int PREC>
-__global__ __launch_bounds__(64) void k_product_t16(ObsDev O, int k, ChunkDev C,
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(NT <= 4 ? 3 : 2)))
+void k_product_t16(ObsDev O, int k, ChunkDev C,
                                                     const int32_t* __restrict__ perm,
                                                     double* __restrict__ B,
                                                     double* __restrict__ bvec, int fold_mask) {
@@ -447,26 +517,28 @@ __global__ __launch_bounds__(64) void k_product_t16(ObsDev O, int k, ChunkDev C,
   // f: the columns of the step in flight; la, lb: lists two and one steps
   // ahead (steps past m load zeros and add nothing)
   T16Frag<NT> f;
-  ListRegs la, lb;
   bf16x8 hi[NT], lo[PREC == LETKF_PREC_BF16 ? 1 : NT];
-  t16_list(la, ir, 0, lane);
-  t16_list(lb, ir, 32, lane);
+  uint32_t la = t16_list(ir, 0, lane), lb = t16_list(ir, 32, lane);
   t16_cols<NT>(f, hxr, wr, la, 0, lane);
-  t16_list(la, ir, 64, lane);
+  la = t16_list(ir, 64, lane);
   for (int j0 = 0; j0 < m; j0 += 32) {
     __builtin_amdgcn_sched_barrier(0);
     t16_convert<NT, PREC>(f, hi, lo);
     __builtin_amdgcn_sched_barrier(0);
     t16_cols<NT>(f, hxr, wr, lb, j0 + 32, lane);
     lb = la;
-    t16_list(la, ir, j0 + 96, lane);
+    la = t16_list(ir, j0 + 96, lane);
     __builtin_amdgcn_sched_barrier(0);
     t16_mfma<NT, PREC>(acc, hi, lo);
     if (COMP && ((j0 + 32) & fold_mask) == 0) t16_fold<NTILE>(acc, Ssh + lane);
   }
 
   // 16x16 f32 accumulator: register r of lane l holds row 4 (l / 16) + r,
-  // column l % 16
+  // column l % 16.  A tile off the diagonal goes to its columns as 16-byte
+  // stores of two rows each and, mirrored, to its rows as whole 128-byte
+  // runs; a diagonal tile, which holds (row, col) and (col, row), takes the
+  // second form alone.  16 (NT - 1) <= k, so only the last row tile and the
+  // last column tile pass the end.
   double* Bp = B + pair * (int64_t)k * k;
   double* bp = bvec + pair * (int64_t)k;
   const int g = lane >> 4, i = lane & 15;
@@ -476,18 +548,26 @@ __global__ __launch_bounds__(64) void k_product_t16(ObsDev O, int k, ChunkDev C,
 #pragma unroll
     for (int ct = rt; ct < NT; ++ct, ++b) {
       const f32x4 sb = COMP ? Ssh[64 * b + lane] : (f32x4){};
+      const int row = 16 * rt + 4 * g, col = 16 * ct + i;
+      double v[4];
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int row = 16 * rt + 4 * g + r;
-        const int col = 16 * ct + i;
-        double v = (double)acc[b][r];
-        if (COMP) v += (double)sb[r];
-        if (row < k && col < k) {
-          Bp[row + (int64_t)k * col] = v;
-          Bp[col + (int64_t)k * row] = v;
-        } else if (col == k && row < k) {
-          bp[row] = v;
+        v[r] = (double)acc[b][r];
+        if (COMP) v[r] += (double)sb[r];
+      }
+      if (ct < NT - 1 || col < k) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (rt < NT - 1 || row + r < k) Bp[col + (int64_t)k * (row + r)] = v[r];
+        if (rt != ct) {
+          double* to = Bp + row + (int64_t)k * col;
+          *(f64x2*)to = (f64x2){v[0], v[1]};
+          *(f64x2*)(to + 2) = (f64x2){v[2], v[3]};
         }
+      } else if (col == k) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (rt < NT - 1 || row + r < k) bp[row + r] = v[r];
       }
     }
 }

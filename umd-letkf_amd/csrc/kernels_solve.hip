@@ -32,7 +32,7 @@ typedef double double4_t __attribute__((ext_vector_type(4)));
 // holds row 16 b + l % 16 of observation l / 16 for every row block b its
 // tiles touch, which is both MFMA operands' layout, so a step loads each
 // value once, converts it once, and feeds NB (NB + 1) / 2 products of 64
-// cycles from NB loads.  Indices and scaled weights of 64 observations are
+// cycles from one run of loads.  Indices and scaled weights of 64 observations are
 // read one lane each (one division an observation), a batch ahead, and
 // passed on by lane shuffles; columns are loaded one step ahead.
 //
@@ -75,14 +75,20 @@ __device__ __forceinline__ void product_tiles(const ObsDev& O, const int32_t* __
                                               const float* __restrict__ lw, int64_t m, int ow,
                                               int lane, double4_t (&acc)[N]) {
   const int q = lane >> 4;
-  const float* __restrict__ col = O.hxp + (lane & 15);
+  // entry KT i + b of a column is row 16 b + i: a lane's rows are one run
+  constexpr int KT = (NB + 1) & ~1;
+  const float* __restrict__ col = O.hxp + KT * (lane & 15);
   const int64_t kp = O.kp;
   auto idx_at = [&](int64_t j) { return li[j + lane < m ? j + lane : 0]; };
   auto load = [&](int32_t id, float (&y)[NB]) __attribute__((always_inline)) {
     const float* c = col + (int64_t)id * kp;
-    static_for<NB>([&](auto I) __attribute__((always_inline)) {
-      constexpr int b = decltype(I)::value;
-      if constexpr (tile_reads<NB, T0, N>(b)) y[b] = c[16 * b];
+    static_for<KT / 2>([&](auto I) __attribute__((always_inline)) {
+      constexpr int b = 2 * decltype(I)::value;
+      if constexpr (tile_reads<NB, T0, N>(b) || (b + 1 < NB && tile_reads<NB, T0, N>(b + 1))) {
+        const float2 f = *(const float2*)(c + b);
+        y[b] = f.x;
+        if constexpr (b + 1 < NB) y[b + 1] = f.y;
+      }
     });
   };
   int64_t j0 = 64 * (int64_t)ow;

@@ -47,7 +47,8 @@ struct ObsDev {
   const float* hx;           // (k, n) perturbations, sorted columns
   const int32_t* cell_start; // kCells + 1
   const float* vt;           // LOC_VGAUSS (n, nlev): vertical weights, or nullptr
-  const float* hxp;          // (kp, n): hx rows, departure in row k, zero rows
+  const float* hxp;          // (kp, n): hx rows, departure in row k, zero rows;
+                             // entry (kp / 16) i + t is row 16 t + i
   int kp;                    // 32-multiple >= k + 1
 };
 
