@@ -109,43 +109,6 @@ __global__ __launch_bounds__(64) void k_small_rational(int k, int K, ChunkDev C,
   }
 }
 
-// blocks of columns by 16: p += sum_c q(c) a[c], c = 16 T .. min(16 T + 15, KQ - 1)
-template <int KQ, int RPL, int T>
-__device__ __forceinline__ void block_prod(double (&p)[4], double q, const double (&a0)[KQ],
-                                           const double (&a1)[RPL == 2 ? KQ : 1]) {
-  constexpr int c0 = 16 * T, n = KQ - c0 < 16 ? KQ - c0 : 16;
-  static_for<n / 4>([&](auto I) __attribute__((always_inline)) {
-    constexpr int i = 4 * decltype(I)::value, c = c0 + i;
-    if constexpr (RPL == 2)
-      bfma42<i>(p[0], p[1], p[2], p[3], q, a0[c], a0[c + 1], a0[c + 2], a0[c + 3], a1[c],
-                a1[c + 1], a1[c + 2], a1[c + 3]);
-    else
-      bfma4<i>(p[0], p[1], q, a0[c], a0[c + 1], a0[c + 2], a0[c + 3]);
-  });
-  static_for<n % 4>([&](auto I) __attribute__((always_inline)) {
-    constexpr int i = n / 4 * 4 + decltype(I)::value, c = c0 + i;
-    if constexpr (RPL == 2) bfma2<i>(p[0], p[2], q, a0[c], a1[c]);
-    else bfma<i>(p[0], q, a0[c]);
-  });
-}
-
-// a[c] -= v_r w_c (+ w_r v_c with VC) on one block of columns
-template <int KQ, int T, bool VC>
-__device__ __forceinline__ void block_upd(double (&a)[KQ], double wq, double vq, double nv,
-                                          double nw) {
-  constexpr int c0 = 16 * T, n = KQ - c0 < 16 ? KQ - c0 : 16;
-  static_for<n / 4>([&](auto I) __attribute__((always_inline)) {
-    constexpr int i = 4 * decltype(I)::value, c = c0 + i;
-    if constexpr (VC) upd4<i>(a[c], a[c + 1], a[c + 2], a[c + 3], wq, vq, nv, nw);
-    else upd4v<i>(a[c], a[c + 1], a[c + 2], a[c + 3], wq, nv);
-  });
-  static_for<n % 4>([&](auto I) __attribute__((always_inline)) {
-    constexpr int i = n / 4 * 4 + decltype(I)::value, c = c0 + i;
-    if constexpr (VC) upd<i>(a[c], wq, vq, nv, nw);
-    else bfma<i>(a[c], wq, nv);
-  });
-}
-
 // P lanes a problem (two a wave for k <= 50), rows r and, with RPL = 2,
 // r + 32.  The reflectors are walked backwards; reflector j has zeros up to
 // entry j, so the blocks of 16 columns below it need no product and only the

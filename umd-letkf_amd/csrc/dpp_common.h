@@ -1,6 +1,6 @@
 // dpp_common.h -- broadcasts and sums by DPP and lane swaps, in FP64, of the
 // kernels that keep a problem's matrix one row a lane (tridiag_pair.h,
-// back_apply.h).
+// back_apply.hip, transform_row.h).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -167,6 +167,43 @@ __device__ __forceinline__ void upd4v(double& a, double& b, double& c, double& d
       : "v"(wq), "v"(nv), "n"(N), "n"(N + 1), "n"(N + 2), "n"(N + 3));
 }
 #undef LK_FD
+
+// blocks of columns by 16: p += sum_c q(c) a[c], c = 16 T .. min(16 T + 15, KQ - 1)
+template <int KQ, int RPL, int T>
+__device__ __forceinline__ void block_prod(double (&p)[4], double q, const double (&a0)[KQ],
+                                           const double (&a1)[RPL == 2 ? KQ : 1]) {
+  constexpr int c0 = 16 * T, n = KQ - c0 < 16 ? KQ - c0 : 16;
+  static_for<n / 4>([&](auto I) __attribute__((always_inline)) {
+    constexpr int i = 4 * decltype(I)::value, c = c0 + i;
+    if constexpr (RPL == 2)
+      bfma42<i>(p[0], p[1], p[2], p[3], q, a0[c], a0[c + 1], a0[c + 2], a0[c + 3], a1[c],
+                a1[c + 1], a1[c + 2], a1[c + 3]);
+    else
+      bfma4<i>(p[0], p[1], q, a0[c], a0[c + 1], a0[c + 2], a0[c + 3]);
+  });
+  static_for<n % 4>([&](auto I) __attribute__((always_inline)) {
+    constexpr int i = n / 4 * 4 + decltype(I)::value, c = c0 + i;
+    if constexpr (RPL == 2) bfma2<i>(p[0], p[2], q, a0[c], a1[c]);
+    else bfma<i>(p[0], q, a0[c]);
+  });
+}
+
+// a[c] -= v_r w_c (+ w_r v_c with VC) on one block of columns
+template <int KQ, int T, bool VC>
+__device__ __forceinline__ void block_upd(double (&a)[KQ], double wq, double vq, double nv,
+                                          double nw) {
+  constexpr int c0 = 16 * T, n = KQ - c0 < 16 ? KQ - c0 : 16;
+  static_for<n / 4>([&](auto I) __attribute__((always_inline)) {
+    constexpr int i = 4 * decltype(I)::value, c = c0 + i;
+    if constexpr (VC) upd4<i>(a[c], a[c + 1], a[c + 2], a[c + 3], wq, vq, nv, nw);
+    else upd4v<i>(a[c], a[c + 1], a[c + 2], a[c + 3], wq, nv);
+  });
+  static_for<n % 4>([&](auto I) __attribute__((always_inline)) {
+    constexpr int i = n / 4 * 4 + decltype(I)::value, c = c0 + i;
+    if constexpr (VC) upd<i>(a[c], wq, vq, nv, nw);
+    else bfma<i>(a[c], wq, nv);
+  });
+}
 
 // 1/x by the hardware estimate e0 and 1/x = e0 (1 + d + d^2 + ...), d = 1 -
 // x e0 (at most 2^-22): cubic, so within rounding of a division.  The pivots

@@ -33,8 +33,16 @@ LK_NR(40) LK_NR(48) LK_NR(56) LK_NR(64)
                                 double* B, double* tau, double* dd, double* ee);          \
   void launch_blk_back_bs##n(hipStream_t st, unsigned nb, int k, const ChunkDev& C,       \
                              double* B, const double* bvec, const double* tau);
-LK_BS(4) LK_BS(5) LK_BS(6) LK_BS(7) LK_BS(8)
+LK_BS(7) LK_BS(8)
 #undef LK_BS
+// k_row_tridiag / k_row_back launchers (one file per row length)
+#define LK_KQ(n)                                                                          \
+  void launch_row_tridiag_kq##n(hipStream_t st, unsigned nb, int k, const ChunkDev& C,    \
+                                double* B, double* tau, double* dd, double* ee);          \
+  void launch_row_back_kq##n(hipStream_t st, unsigned nb, int k, const ChunkDev& C,       \
+                             double* B, const double* bvec, const double* tau);
+LK_KQ(72) LK_KQ(80) LK_KQ(88) LK_KQ(96) LK_KQ(104)
+#undef LK_KQ
 
 // M below the diagonal, one thread per column c; the rows are visited in the
 // same order by every lane (x starts at g_c in row c, is 0 above it), so the
@@ -589,18 +597,18 @@ void launch_transform_mat(hipStream_t st, int prec, const LocDev& L, const State
   if (np <= 0) return;
   const int k = (int)S.k;
   const unsigned nb = (unsigned)np;
-  // blk: the 2D-block kernels, BS x BS blocks with 16 BS >= k; else the
+  // blk: one row a lane, whose KQ >= k columns fill the registers at 104;
+  // above, the 2D-block kernels, BS x BS blocks with 16 BS >= k.  Else the
   // column-half kernels, rows per half k <= 2 NR
-  const int bs = (k + 15) / 16;
   const int nr = (k + 1) / 2;
   if (blk) {
-    switch (bs) {
-      case 4: launch_blk_tridiag_bs4(st, nb, k, C, B, tau, dd, ee); break;
-      case 5: launch_blk_tridiag_bs5(st, nb, k, C, B, tau, dd, ee); break;
-      case 6: launch_blk_tridiag_bs6(st, nb, k, C, B, tau, dd, ee); break;
-      case 7: launch_blk_tridiag_bs7(st, nb, k, C, B, tau, dd, ee); break;
-      default: launch_blk_tridiag_bs8(st, nb, k, C, B, tau, dd, ee); break;
-    }
+    if (k <= 72) launch_row_tridiag_kq72(st, nb, k, C, B, tau, dd, ee);
+    else if (k <= 80) launch_row_tridiag_kq80(st, nb, k, C, B, tau, dd, ee);
+    else if (k <= 88) launch_row_tridiag_kq88(st, nb, k, C, B, tau, dd, ee);
+    else if (k <= 96) launch_row_tridiag_kq96(st, nb, k, C, B, tau, dd, ee);
+    else if (k <= 104) launch_row_tridiag_kq104(st, nb, k, C, B, tau, dd, ee);
+    else if (k <= 112) launch_blk_tridiag_bs7(st, nb, k, C, B, tau, dd, ee);
+    else launch_blk_tridiag_bs8(st, nb, k, C, B, tau, dd, ee);
   } else if (nr <= 40) launch_mat_tridiag_nr40(st, nb, k, C, B, tau, dd, ee);
   else if (nr <= 48) launch_mat_tridiag_nr48(st, nb, k, C, B, tau, dd, ee);
   else if (nr <= 56) launch_mat_tridiag_nr56(st, nb, k, C, B, tau, dd, ee);
@@ -609,13 +617,13 @@ void launch_transform_mat(hipStream_t st, int prec, const LocDev& L, const State
   k_mat_rational<24, 16><<<nb, 128, 0, st>>>(k, C, B, dd, ee, R.tab, R.n, R.nb);
   k_mat_rational<kMaxNodes, 24><<<nb, 128, 0, st>>>(k, C, B, dd, ee, R.tab, R.n, R.nb);
   if (blk) {
-    switch (bs) {
-      case 4: launch_blk_back_bs4(st, nb, k, C, B, bvec, tau); break;
-      case 5: launch_blk_back_bs5(st, nb, k, C, B, bvec, tau); break;
-      case 6: launch_blk_back_bs6(st, nb, k, C, B, bvec, tau); break;
-      case 7: launch_blk_back_bs7(st, nb, k, C, B, bvec, tau); break;
-      default: launch_blk_back_bs8(st, nb, k, C, B, bvec, tau); break;
-    }
+    if (k <= 72) launch_row_back_kq72(st, nb, k, C, B, bvec, tau);
+    else if (k <= 80) launch_row_back_kq80(st, nb, k, C, B, bvec, tau);
+    else if (k <= 88) launch_row_back_kq88(st, nb, k, C, B, bvec, tau);
+    else if (k <= 96) launch_row_back_kq96(st, nb, k, C, B, bvec, tau);
+    else if (k <= 104) launch_row_back_kq104(st, nb, k, C, B, bvec, tau);
+    else if (k <= 112) launch_blk_back_bs7(st, nb, k, C, B, bvec, tau);
+    else launch_blk_back_bs8(st, nb, k, C, B, bvec, tau);
   } else if (nr <= 40) launch_mat_back_nr40(st, nb, k, C, B, bvec, tau);
   else if (nr <= 48) launch_mat_back_nr48(st, nb, k, C, B, bvec, tau);
   else if (nr <= 56) launch_mat_back_nr56(st, nb, k, C, B, bvec, tau);

@@ -1,6 +1,6 @@
 // transform_blk.h -- the reduction and the back-transform of the explicit
-// transform matrix (64 <= k <= 128, see transform_mat.h) with A distributed
-// over a 256-thread block in 2D: the matrix, padded to N = 16 BS, is a 16 x 16
+// transform matrix (105 <= k <= 128, see transform_mat.h; transform_row.h
+// serves smaller ones) with A distributed over a 256-thread block in 2D: the matrix, padded to N = 16 BS, is a 16 x 16
 // grid of BS x BS blocks, and thread t holds block (I, J) = (t / 16, t % 16)
 // in registers.  Per step a thread needs v and w only for its BS rows and
 // its BS columns (4 BS values from LDS), where the column layout of
