@@ -61,12 +61,14 @@ __device__ __forceinline__ double p_sum(double x) {
   x += dpp_mov<0x124>(x);
   x += dpp_mov<0x122>(x);
   x += dpp_mov<0x121>(x);
-  double e, o;
-  rows16(x, &e, &o);
-  x = e + o;
-  if constexpr (P == 64) {
-    rows32(x, &e, &o);
+  if constexpr (P >= 32) {
+    double e, o;
+    rows16(x, &e, &o);
     x = e + o;
+    if constexpr (P == 64) {
+      rows32(x, &e, &o);
+      x = e + o;
+    }
   }
   return x;
 }

@@ -7,7 +7,7 @@
 //                   + V L^-1 V^T Yb^T R^-1 d 1^T, x_a = x_b^T T for each slab of
 //                   the group (src/letkf_core.F90:100-141,
 //                   src/letkf_solver.F90:284-290)
-//   k_finalize      recenter, increment clip, RTPS, RTPP, multiplicative
+//   k_finalize<NJ>  recenter, increment clip, RTPS, RTPP, multiplicative
 //                   inflation, member bounds, spread
 //                   (src/letkf_solver.F90:299-379)
 #include <hip/hip_runtime.h>
@@ -452,108 +452,92 @@ hipError_t launch_eigen_apply_f64(hipStream_t st, const LocDev& L, const StateDe
 }
 
 // ---------------------------------------------------------------------------
-// post-processing: one wave per gridpoint, lanes over members (2 per lane
-// for k > 64).  Every step of src/letkf_solver.F90:299-379 acts slab by slab,
-// so each slab is carried through all of them in turn.
+// post-processing.  Every step of src/letkf_solver.F90:299-379 acts slab by
+// slab, and the slabs of all gridpoints follow one another: a wave takes four
+// at a time, one in each of its 16-lane rows with members i + 16 j in lane i.
+// A sum is NJ - 1 additions and four DPP rotations, and the roots and
+// divisions serve four slabs (with one slab a wave, 250 instructions each,
+// the instructions bounded it: 684 us at 1.04e6 slabs of k = 50, 397 us at
+// 810 000 of k = 40, against 150 and 80 us of memory traffic; now 267 and
+// 198 us).  Small grids: one slab's latency instead of a gridpoint's slabs
+// in turn.
+//
+// A run of slabs is looked over first, a lane each: which are solved,
+// masked (the background unchanged) or, with skip_solved, done already by
+// the apply.  A run is the four slabs of one pass, or 16 where the apply has
+// done most of millions of slabs and the waves' launch counts.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ double wsum(double v) { return wave_sum_dpp(v); }
-
-__global__ __launch_bounds__(256) void k_finalize(LocDev L, StateDev S, VarsDev V,
-                                                  ChunkDev C, DiagDev D, float rtps,
-                                                  float rtpp, float mul,
+template <int NJ>
+__global__ __launch_bounds__(256) void k_finalize(LocDev L, StateDev S, VarsDev V, ChunkDev C,
+                                                  DiagDev D, float rtps, float rtpp, float mul,
                                                   double* __restrict__ ana,
                                                   double* __restrict__ amean,
-                                                  double* __restrict__ asprd,
-                                                  bool skip_solved) {
+                                                  double* __restrict__ asprd, bool skip_solved,
+                                                  uint32_t n, int run) {
   const int wid = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int64_t t = (int64_t)blockIdx.x * 4 + wid;
-  if (t >= C.ngp) return;
-  const int64_t ij = C.i0 + t;
+  const int64_t u64 = ((int64_t)blockIdx.x * 4 + wid) * run;
+  if (u64 >= n) return;
+  const uint32_t u0 = (uint32_t)u64;
   const int k = (int)S.k;
-  const int64_t ns = S.ns;
-  const float* xb0 = S.state + (int64_t)k * ns * ij;
-  double* xa0 = ana + (int64_t)k * ns * ij;
-  const bool m0 = lane < k, m1 = lane + 64 < k;
-  if (S.mask[ij]) {
-    // the background unchanged: the gridpoint's k x ns block is contiguous,
-    // copied 512 elements per round with 8 loads of a lane in flight
-    const int64_t n = (int64_t)k * ns;
-    for (int64_t e0 = 0; e0 < n; e0 += 512) {
-      float v[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) v[u] = xb0[min(e0 + 64 * u + lane, n - 1)];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int64_t e = e0 + 64 * u + lane;
-        if (e < n) xa0[e] = (double)v[u];
-      }
-    }
-    for (int64_t s = lane; s < ns; s += 64) {
-      amean[ns * ij + s] = (double)S.mean[ns * ij + s];
-      asprd[ns * ij + s] = (double)S.sprd[ns * ij + s];
-    }
-    return;
+  int s_own = 0;
+  bool solved = false, masked = false, need = false;
+  if (lane < run && u0 + lane < n) {
+    const uint32_t t = (u0 + lane) / (uint32_t)S.ns;
+    s_own = (int)(u0 + lane - t * (uint32_t)S.ns);
+    const int64_t ij = C.i0 + t;
+    masked = S.mask[ij] != 0;
+    const int g = slab_group(L, V, s_own, D.mld[ij]);
+    solved = !masked && g >= 0 && C.solve[(int64_t)t * C.G + g];
+    need = !(skip_solved && solved);
   }
-  const int mld = D.mld[ij];
-  if (skip_solved) {
-    // nothing to do where every slab's group was solved (and post-processed
-    // by the apply): the slabs' flags are checked 64 at a time
-    bool any = false;
-    for (int64_t s0 = 0; s0 < ns && !any; s0 += 64) {
-      bool need = false;
-      if (s0 + lane < ns) {
-        const int g = slab_group(L, V, (int)(s0 + lane), mld);
-        need = !(g >= 0 && C.solve[t * C.G + g]);
-      }
-      any = __ballot(need) != 0;
-    }
-    if (!any) return;
-  }
+  const uint64_t b_solved = __ballot(solved), b_masked = __ballot(masked), b_need = __ballot(need);
   const double dk = (double)k, dk1 = (double)(k - 1);
-  // a slab's inputs are loaded two slabs ahead of its post-processing, so
-  // that the loads of later slabs are in flight during the wave sums
-  struct SlabIn {
-    double x0, x1;      // transformed perturbation, or background member
-    float b0, b1;       // background member
-    float bm, bs;       // background mean and spread
-    bool skip;          // post-processed elsewhere
-  };
-  auto fetch = [&](int64_t s) {
-    SlabIn r;
-    const int g = slab_group(L, V, (int)s, mld);
-    const bool solved = g >= 0 && C.solve[t * C.G + g];
-    r.skip = skip_solved && solved;
-    if (r.skip) return r;
-    r.b0 = m0 ? xb0[k * s + lane] : 0.0f;
-    r.b1 = m1 ? xb0[k * s + lane + 64] : 0.0f;
-    r.x0 = solved ? (m0 ? xa0[k * s + lane] : 0.0) : (double)r.b0;
-    r.x1 = solved ? (m1 ? xa0[k * s + lane + 64] : 0.0) : (double)r.b1;
-    r.bm = S.mean[ns * ij + s];
-    r.bs = S.sprd[ns * ij + s];
-    return r;
-  };
-  SlabIn cur = fetch(0);
-  SlabIn nxt = ns > 1 ? fetch(1) : cur;
-  for (int64_t s = 0; s < ns; ++s) {
-    const SlabIn in = cur;
-    cur = nxt;
-    if (s + 2 < ns) nxt = fetch(s + 2);
-    if (in.skip) continue;
-    const double xb_0 = (double)in.b0;
-    const double xb_1 = (double)in.b1;
-    double x0 = in.x0;
-    double x1 = in.x1;
-    const double bm = (double)in.bm;
-    const double bs = (double)in.bs;
+  const int i = lane & 15;
+  for (int q = 0; q < run; q += 4) {
+    if (((b_need >> q) & 15) == 0) continue;          // wave-uniform
+    const int at = q + (lane >> 4);
+    const bool on = (b_need >> at) & 1, sol = (b_solved >> at) & 1, msk = (b_masked >> at) & 1;
+    const int s = __shfl(s_own, at, 64);
+    const int64_t e = C.i0 * S.ns + u0 + at;          // slab of the whole grid
+    const float* xb = S.state + e * k;
+    double* xa = ana + e * k;
+    double x[NJ];
+    float b[NJ];
+    if (on) {
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+        b[j] = (!sol || rtpp > 0.0f) && i + 16 * j < k ? xb[i + 16 * j] : 0.0f;
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+        x[j] = sol && i + 16 * j < k ? xa[i + 16 * j] : (double)b[j];
+    } else {
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) { b[j] = 0.0f; x[j] = 0.0; }
+    }
+    const double bm = on ? (double)S.mean[e] : 0.0, bs = on ? (double)S.sprd[e] : 0.0;
+    const int v = on ? V.slab_var[s] : -1;
+    double blo = 0.0, bhi = 0.0, inc = 0.0;
+    if (v >= 0) {
+      inc = (double)V.inc_max[v];
+      blo = (double)V.bounds[2 * v];
+      bhi = (double)V.bounds[2 * v + 1];
+    }
+    auto sum = [&](auto f) __attribute__((always_inline)) {
+      double p = 0.0;
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) p += i + 16 * j < k ? f(x[j]) : 0.0;
+      return p_sum<16>(p);
+    };
+    auto self = [](double y) { return y; };
+    auto sq = [](double y) { return y * y; };
     // recenter (:299-303)
-    x0 += bm; x1 += bm;
-    double mean = wsum((m0 ? x0 : 0.0) + (m1 ? x1 : 0.0)) / dk;
-    x0 -= mean; x1 -= mean;
-    const int v = V.slab_var[s];
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) x[j] += bm;
+    double mean = sum(self) / dk;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) x[j] -= mean;
     // increment clipping (:308-318)
     if (v >= 0) {
-      const double inc = (double)V.inc_max[v];
-      const double blo = (double)V.bounds[2 * v], bhi = (double)V.bounds[2 * v + 1];
       double r = mean - bm;
       r = fmax(r, -inc);
       r = fmin(r, inc);
@@ -563,43 +547,79 @@ __global__ __launch_bounds__(256) void k_finalize(LocDev L, StateDev S, VarsDev 
     }
     // RTPS (:322-335)
     if (rtps > 0.0f) {
-      const double sa = sqrt(wsum((m0 ? x0 * x0 : 0.0) + (m1 ? x1 * x1 : 0.0)) / dk1);
-      if (sa > 0.0) {
-        const double f = (double)rtps * (bs - sa) / sa + 1.0;
-        x0 *= f; x1 *= f;
-      }
+      const double sa = sqrt(sum(sq) / dk1);
+      const double f = sa > 0.0 ? (double)rtps * (bs - sa) / sa + 1.0 : 1.0;
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) x[j] *= f;
     }
     // RTPP (:339-343)
     if (rtpp > 0.0f) {
       const double a = (double)rtpp;
-      x0 = a * xb_0 + (1.0 - a) * x0;
-      x1 = a * xb_1 + (1.0 - a) * x1;
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) x[j] = a * (double)b[j] + (1.0 - a) * x[j];
     }
     // multiplicative (:347-349)
-    if (mul != 1.0f) { x0 *= (double)mul; x1 *= (double)mul; }
+    if (mul != 1.0f) {
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) x[j] *= (double)mul;
+    }
     // member bounds and re-mean (:357-371)
-    if (v >= 0) {
-      const double blo = (double)V.bounds[2 * v], bhi = (double)V.bounds[2 * v + 1];
-      x0 = fmin(fmax(x0, blo - mean), bhi - mean);
-      x1 = fmin(fmax(x1, blo - mean), bhi - mean);
-      const double r = wsum((m0 ? x0 : 0.0) + (m1 ? x1 : 0.0)) / dk;
-      x0 -= r; x1 -= r;
-      mean += r;
+    if (__ballot(v >= 0)) {
+      if (v >= 0) {
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) x[j] = fmin(fmax(x[j], blo - mean), bhi - mean);
+      }
+      const double r = sum(self) / dk;
+      if (v >= 0) {
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) x[j] -= r;
+        mean += r;
+      }
     }
     // final spread and members (:375-379)
-    const double sp = sqrt(wsum((m0 ? x0 * x0 : 0.0) + (m1 ? x1 * x1 : 0.0)) / dk1);
-    if (m0) xa0[k * s + lane] = x0 + mean;
-    if (m1) xa0[k * s + lane + 64] = x1 + mean;
-    if (lane == 0) { amean[ns * ij + s] = mean; asprd[ns * ij + s] = sp; }
+    const double sp = sqrt(sum(sq) / dk1);
+    if (on) {
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+        if (i + 16 * j < k) xa[i + 16 * j] = msk ? (double)b[j] : x[j] + mean;
+      if (i == 0) {
+        amean[e] = msk ? bm : mean;
+        asprd[e] = msk ? bs : sp;
+      }
+    }
   }
 }
 
 void launch_finalize(hipStream_t st, const LocDev& L, const StateDev& S,
                      const VarsDev& V, const ChunkDev& C, const DiagDev& D,
                      const FinArgs& F, double* ana, bool skip_solved) {
-  if (C.ngp <= 0) return;
-  k_finalize<<<(unsigned)((C.ngp + 3) / 4), 256, 0, st>>>(
-      L, S, V, C, D, F.rtps, F.rtpp, F.mul, ana, F.amean, F.asprd, skip_solved);
+  // slabs are numbered in 32 bits: gridpoints in parts of at most 2^31 slabs
+  const int64_t part = std::max<int64_t>(1, (1ll << 31) / std::max<int64_t>(S.ns, 1) - 1);
+  for (int64_t t0 = 0; t0 < C.ngp && S.ns > 0; t0 += part) {
+    ChunkDev P = C;
+    P.i0 = C.i0 + t0;
+    P.ngp = std::min(part, C.ngp - t0);
+    P.solve = C.solve + t0 * C.G;
+    const int64_t n = P.ngp * S.ns;
+    const int run = skip_solved && n > (4 << 20) ? 16 : 4;
+    const int64_t waves = (n + run - 1) / run;
+    const unsigned nb = (unsigned)((waves + 3) / 4);
+#define LK_FIN(NJ)                                                                          \
+  k_finalize<NJ><<<nb, 256, 0, st>>>(L, S, V, P, D, F.rtps, F.rtpp, F.mul, ana, F.amean,    \
+                                     F.asprd, skip_solved, (uint32_t)n, run);               \
+  break
+    switch (((int)S.k + 15) / 16) {
+      case 1: LK_FIN(1);
+      case 2: LK_FIN(2);
+      case 3: LK_FIN(3);
+      case 4: LK_FIN(4);
+      case 5: LK_FIN(5);
+      case 6: LK_FIN(6);
+      case 7: LK_FIN(7);
+      default: LK_FIN(8);
+    }
+#undef LK_FIN
+  }
 }
 
 }  // namespace lk
