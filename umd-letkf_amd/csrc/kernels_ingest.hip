@@ -15,6 +15,8 @@
 //  k_obs_compact         the QC compaction of :479-489 (qc > 0 dropped, order
 //                        kept) as a gather through the selected indices
 //  k_f64_to_f32          the FP32 view of the analysis (state_ij's REAL kind)
+//  k_state_to_host, k_diag_to_host, k_counters_to_host
+//                        results written into page-locked host memory
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -103,6 +105,104 @@ __global__ void k_f64_to_f32(int64_t n, const double* __restrict__ in, float* __
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride)
     out[i] = (float)in[i];
+}
+
+// The analysis straight into the caller's page-locked arrays, in one launch:
+// state, mean and spread converted to O (float rounds to nearest, double is a
+// copy) and written over the bus by the lanes, four values each where the
+// array starts on 16 bytes.  A staging buffer, a conversion and a copy for
+// each array, each waited for, cost 100 us on a grid whose copies take 12;
+// on large ones the conversion now runs in the copy's time.
+struct ToHost {
+  const double* src[3];
+  void* dst[3];
+  int64_t n[3];
+};
+template <typename O>
+__global__ __launch_bounds__(256) void k_state_to_host(ToHost T) {
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  const int64_t i0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  typedef O Ox __attribute__((ext_vector_type(16 / sizeof(O))));
+  constexpr int W = 16 / sizeof(O);
+#pragma unroll
+  for (int f = 0; f < 3; ++f) {
+    const double* __restrict__ in = T.src[f];
+    O* __restrict__ out = (O*)T.dst[f];
+    const int64_t n = T.n[f];
+    int64_t done = 0;
+    if ((reinterpret_cast<uintptr_t>(out) & 15) == 0) {
+      const int64_t nv = n / W;
+      for (int64_t i = i0; i < nv; i += stride) {
+        Ox v;
+#pragma unroll
+        for (int e = 0; e < W; ++e) v[e] = (O)in[W * i + e];
+        __builtin_nontemporal_store(v, reinterpret_cast<Ox*>(out) + i);
+      }
+      done = nv * W;
+    }
+    for (int64_t i = done + i0; i < n; i += stride) out[i] = (O)in[i];
+  }
+}
+
+void launch_state_to_host(hipStream_t st, bool f64, const double* const* src, void* const* dst,
+                          const int64_t* n) {
+  ToHost T;
+  int64_t most = 0;
+  for (int f = 0; f < 3; ++f) {
+    T.src[f] = src[f];
+    T.dst[f] = dst[f];
+    T.n[f] = dst[f] ? n[f] : 0;
+    most = std::max(most, T.n[f]);
+  }
+  if (most <= 0) return;
+  const unsigned nb = (unsigned)std::min<int64_t>((most + 1023) / 1024, 1024);
+  if (f64) k_state_to_host<double><<<nb, 256, 0, st>>>(T);
+  else k_state_to_host<float><<<nb, 256, 0, st>>>(T);
+}
+
+// The diagnostics fields of an analysis as letkf_gpu_get_diag returns them,
+// in page-locked memory: maxhz, obscount (nij), then per (group, gridpoint)
+// kept count, weight sum (FP32) and hash
+__global__ __launch_bounds__(256) void k_diag_to_host(int64_t nij, int64_t G, DiagDev D,
+                                                      uint64_t* __restrict__ hash,
+                                                      float* __restrict__ f) {
+  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= nij * G) return;
+  const int64_t g = e / nij, i = e - g * nij;
+  if (g == 0) {
+    f[i] = D.maxhz[i];
+    f[nij + i] = (float)D.obscount[i];
+  }
+  hash[e] = D.lg_hash[i * G + g];
+  f[2 * nij + e] = (float)D.lg_m[i * G + g];
+  f[(2 + G) * nij + e] = (float)D.lg_obsloc[i * G + g];
+}
+
+void launch_diag_to_host(hipStream_t st, int64_t nij, int64_t G, const DiagDev& D,
+                         uint64_t* hash, float* f) {
+  if (nij * G <= 0) return;
+  k_diag_to_host<<<(unsigned)((nij * G + 255) / 256), 256, 0, st>>>(nij, G, D, hash, f);
+}
+
+// the search counters (every kCtrStep-th word of a slot) and, where tot is
+// given, the last pair's list offset and count, into page-locked memory
+__global__ __launch_bounds__(256) void k_counters_to_host(const unsigned long long* ctr,
+                                                          unsigned long long* h_ctr,
+                                                          const int64_t* off, const int64_t* cnt,
+                                                          int64_t* tot) {
+  const int e = blockIdx.x * 256 + threadIdx.x;
+  if (e < kCtrSlots * kCtrStride / kCtrStep) h_ctr[e * kCtrStep] = ctr[e * kCtrStep];
+  if (tot && e == 0) {
+    tot[0] = *off;
+    tot[1] = *cnt;
+  }
+}
+
+void launch_counters_to_host(hipStream_t st, const unsigned long long* ctr,
+                             unsigned long long* h_ctr, const int64_t* off, const int64_t* cnt,
+                             int64_t* tot) {
+  k_counters_to_host<<<(kCtrSlots * kCtrStride / kCtrStep + 255) / 256, 256, 0, st>>>(
+      ctr, h_ctr, off, cnt, tot);
 }
 
 void launch_f64_to_f32(hipStream_t st, int64_t n, const double* in, float* out) {

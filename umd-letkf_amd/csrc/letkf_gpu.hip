@@ -126,6 +126,8 @@ struct letkf_gpu_t {
   void* d_tmp = nullptr;
   size_t tmp_bytes = 0;
   int64_t* h_tot = nullptr;    // pinned
+  void* h_diag = nullptr;      // pinned: diagnostics on their way out
+  size_t diag_bytes = 0;
 
   letkf_gpu_timing timing{};
   // device address of this device's no-allocation staging array
@@ -208,6 +210,7 @@ static std::string g_create_err;
 // address is handed to kernels and copies.  All calls on one device share
 // the array: calls that overlap in time on one GPU race.
 // ---------------------------------------------------------------------------
+static constexpr size_t kDiagBytes = 2ull << 20;   // 80 000 gridpoints of one group
 static constexpr size_t kNoAllocScratchBytes = 64ull << 20;
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 
@@ -400,6 +403,7 @@ int letkf_gpu_destroy(letkf_gpu_t* h) {
   if (h->h_tot) hipHostFree(h->h_tot);
   if (h->h_tot2) hipHostFree(h->h_tot2);
   if (h->h_ctr) hipHostFree(h->h_ctr);
+  if (h->h_diag) hipHostFree(h->h_diag);
   hipStreamDestroy(h->stream);
   hipStreamDestroy(h->stream2);
   delete h;
@@ -1079,11 +1083,9 @@ static hipError_t enqueue_solve(letkf_gpu_t* h, hipStream_t st, const RunViews& 
 
 // The search counters of the last analysis (work counts into T), the
 // max_obs capacity check and, for a replayed graph, the pairs refused list
-// space (*overflow; nullptr: not looked at).
+// space (*overflow; nullptr: not looked at).  The analysis' last kernel has
+// put them into h_ctr, and its stream has been waited for.
 static int read_counters(letkf_gpu_t* h, letkf_gpu_timing* T, int64_t* overflow) {
-  const size_t ctr_bytes = sizeof(unsigned long long) * kCtrSlots * kCtrStride;
-  HIPCHK(h, hipMemcpyAsync(h->h_ctr, h->d_ctr, ctr_bytes, hipMemcpyDeviceToHost, h->stream));
-  HIPCHK(h, hipStreamSynchronize(h->stream));
   unsigned long long maxc = 0;
   for (int sl = 0; sl < kCtrSlots; ++sl) {
     T->n_problems += (int64_t)h->h_ctr[sl * kCtrStride + kCtrSolves];
@@ -1170,9 +1172,8 @@ static int run_eager(letkf_gpu_t* h) {
     size_t tb = h->tmp_bytes;
     RUNCHK(hipcub::DeviceScan::ExclusiveSum(b_tmp, tb, padded_counts(b_cnt), b_off, (int)np,
                                             sst));
-    RUNCHK(hipMemcpyAsync(b_tot, b_off + (np - 1), 8, hipMemcpyDeviceToHost, sst));
-    RUNCHK(hipMemcpyAsync(b_tot + 1, b_cnt + (np - 1), 8, hipMemcpyDeviceToHost, sst));
-    RUNCHK(hipMemcpyAsync(h->h_ctr, h->d_ctr, ctr_bytes, hipMemcpyDeviceToHost, sst));
+    launch_counters_to_host(sst, h->d_ctr, h->h_ctr, b_off + (np - 1), b_cnt + (np - 1), b_tot);
+    RUNCHK(hipGetLastError());
     RUNCHK(hipStreamSynchronize(sst));
     // list space: padded offsets, plus one alignment unit of slack for the
     // vector loads past the last list
@@ -1232,6 +1233,8 @@ static int run_eager(letkf_gpu_t* h) {
   }
   RUNCHK(mk(&e_last));
   RUNCHK(hipEventRecord(e_last, st));
+  launch_counters_to_host(st, h->d_ctr, h->h_ctr, nullptr, nullptr, nullptr);
+  RUNCHK(hipGetLastError());
   RUNCHK(hipStreamSynchronize(st));
   RUNCHK(hipStreamSynchronize(h->stream2));
   for (const auto& ce : cev) {
@@ -1305,6 +1308,10 @@ static hipError_t enqueue_analysis(letkf_gpu_t* h) {
     if (e == hipSuccess) e = enqueue_solve(h, st, W, C);
     if (e != hipSuccess) break;
     launch_finalize(st, h->loc, W.S, W.V, C, W.D, fin_args(h), h->d_ana, fin_fused(h));
+    e = hipGetLastError();
+  }
+  if (e == hipSuccess) {
+    launch_counters_to_host(st, h->d_ctr, h->h_ctr, nullptr, nullptr, nullptr);
     e = hipGetLastError();
   }
   return e;
@@ -1398,6 +1405,43 @@ static int run_graph(letkf_gpu_t* h) {
   return LETKF_OK;
 }
 
+// the device's address of n bytes of page-locked host memory, or nullptr for
+// anything else: the first and the last byte must be page-locked and as far
+// apart there as here
+static void* locked_view(const void* p, size_t n) {
+  hipPointerAttribute_t a{}, b{};
+  const char* last = (const char*)p + n - 1;
+  if (hipPointerGetAttributes(&a, p) != hipSuccess || a.type != hipMemoryTypeHost ||
+      hipPointerGetAttributes(&b, last) != hipSuccess || b.type != hipMemoryTypeHost) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  if (!a.devicePointer || (char*)b.devicePointer - (char*)a.devicePointer != last - (const char*)p)
+    return nullptr;
+  return a.devicePointer;
+}
+
+// state, mean and spread of the analysis into the caller's arrays by one
+// kernel, where all that are asked for are page-locked (*done)
+static hipError_t state_to_host(letkf_gpu_t* h, bool f64, void* const* to, bool* done) {
+  const int64_t n = h->ns * h->nij;
+  const double* const src[3] = {h->d_ana, h->d_amean, h->d_asprd};
+  const int64_t cnt[3] = {h->k * n, n, n};
+  void* dst[3] = {};
+  *done = false;
+  if (n <= 0) return hipSuccess;
+  for (int f = 0; f < 3; ++f) {
+    if (!to[f]) continue;
+    dst[f] = locked_view(to[f], (size_t)cnt[f] * (f64 ? 8 : 4));
+    if (!dst[f]) return hipSuccess;
+  }
+  launch_state_to_host(h->stream, f64, src, dst, cnt);
+  hipError_t e = hipGetLastError();
+  if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
+  *done = e == hipSuccess;
+  return e;
+}
+
 extern "C" {
 
 int letkf_gpu_run(letkf_gpu_t* h) {
@@ -1422,6 +1466,10 @@ int letkf_gpu_get_state_f64(letkf_gpu_t* h, double* state, double* mean, double*
   if (!h) return LETKF_EINVAL;
   if (!h->have_run) return fail(h, LETKF_ESTATE, "no analysis: call letkf_gpu_run first");
   const int64_t k = h->k, ns = h->ns, nij = h->nij;
+  void* const dst[3] = {state, mean, sprd};
+  bool done = false;
+  HIPCHK(h, state_to_host(h, true, dst, &done));
+  if (done) return LETKF_OK;
   if (state) HIPCHK(h, hipMemcpy(state, h->d_ana, 8 * k * ns * nij, hipMemcpyDeviceToHost));
   if (mean) HIPCHK(h, hipMemcpy(mean, h->d_amean, 8 * ns * nij, hipMemcpyDeviceToHost));
   if (sprd) HIPCHK(h, hipMemcpy(sprd, h->d_asprd, 8 * ns * nij, hipMemcpyDeviceToHost));
@@ -1516,7 +1564,11 @@ int letkf_gpu_get_state(letkf_gpu_t* h, float* state, float* mean, float* sprd) 
   const int64_t k = h->k, ns = h->ns, nij = h->nij;
   const int64_t n_max = std::max(k * ns * nij, ns * nij);
   if (n_max <= 0) return LETKF_OK;
-  // converted on the device, then copied down in slices of at most 16M
+  void* const dst[3] = {state, mean, sprd};
+  bool done = false;
+  HIPCHK(h, state_to_host(h, false, dst, &done));
+  if (done) return LETKF_OK;
+  // pageable arrays: converted on the device, then copied down in slices of at most 16M
   // values through one staging buffer (host memory holds only the caller's
   // FP32 arrays)
   const int64_t slice = std::min<int64_t>(n_max, 1ll << 24);
@@ -1545,6 +1597,30 @@ int letkf_gpu_get_diag(letkf_gpu_t* h, const letkf_gpu_diag* d) {
   if (!h || !d) return LETKF_EINVAL;
   if (!h->have_run) return fail(h, LETKF_ESTATE, "no analysis: call letkf_gpu_run first");
   const int64_t nij = h->nij, G = h->G;
+  // small fields: put in the reference's layout by one kernel that writes
+  // them to page-locked memory, where five copies would each be waited for.
+  // Above kDiagBytes the copies' own time counts, and the memory they need.
+  const size_t bytes = (size_t)nij * (8 + 16 * (size_t)G);
+  if (nij * G > 0 && bytes <= kDiagBytes) {
+    if (h->diag_bytes < bytes) {
+      if (h->h_diag) hipHostFree(h->h_diag);
+      h->h_diag = nullptr;
+      h->diag_bytes = 0;
+      HIPCHK(h, hipHostMalloc(&h->h_diag, bytes, hipHostMallocDefault));
+      h->diag_bytes = bytes;
+    }
+    uint64_t* hash = (uint64_t*)h->h_diag;
+    float* f = (float*)(hash + nij * G);
+    launch_diag_to_host(h->stream, nij, G, run_views(h).D, hash, f);
+    HIPCHK(h, hipGetLastError());
+    HIPCHK(h, hipStreamSynchronize(h->stream));
+    if (d->maxhz) memcpy(d->maxhz, f, 4 * nij);
+    if (d->obscount) memcpy(d->obscount, f + nij, 4 * nij);
+    if (d->lg_obscount) memcpy(d->lg_obscount, f + 2 * nij, 4 * nij * G);
+    if (d->lg_obsloc) memcpy(d->lg_obsloc, f + (2 + G) * nij, 4 * nij * G);
+    if (d->lg_selhash) memcpy(d->lg_selhash, hash, 8 * nij * G);
+    return LETKF_OK;
+  }
   if (d->maxhz) HIPCHK(h, hipMemcpy(d->maxhz, h->d_maxhz, 4 * nij, hipMemcpyDeviceToHost));
   std::vector<int32_t> ib;
   if (d->obscount) {

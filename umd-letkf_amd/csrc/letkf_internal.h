@@ -133,6 +133,7 @@ constexpr int kCtrSlots = 64;
 constexpr int kCtrStride = 64;        // 512 B per slot
 constexpr int kCtrSolves = 0, kCtrCand = 16, kCtrPairs = 32, kCtrMax = 48;
 constexpr int kCtrOverflow = 8;       // slot 0 only: pairs refused list space
+constexpr int kCtrStep = 8;           // all of them are multiples of it
 
 // group of slab s at a gridpoint (letkf_loc_ocean.F90:360-375 for bkg_t)
 __device__ __forceinline__ int slab_group(const LocDev& L, const VarsDev& V,
@@ -193,6 +194,13 @@ struct ObsFields {
   float* hx;
 };
 void launch_f64_to_f32(hipStream_t st, int64_t n, const double* in, float* out);
+void launch_state_to_host(hipStream_t st, bool f64, const double* const* src, void* const* dst,
+                          const int64_t* n);
+void launch_diag_to_host(hipStream_t st, int64_t nij, int64_t G, const DiagDev& D,
+                         uint64_t* hash, float* f);
+void launch_counters_to_host(hipStream_t st, const unsigned long long* ctr,
+                             unsigned long long* h_ctr, const int64_t* off, const int64_t* cnt,
+                             int64_t* tot);
 void launch_state_from_members(hipStream_t st, int64_t nij, int64_t ns, int k,
                                const float* members, float* state, float* mean, float* sprd);
 void launch_members_from_state(hipStream_t st, int64_t nij, int64_t ns, int k,
