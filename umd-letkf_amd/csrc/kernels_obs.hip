@@ -83,6 +83,12 @@ __global__ void k_obs_gather_hx(int64_t n, int k, const int32_t* __restrict__ pe
   }
 }
 
+void launch_gather_cols(hipStream_t st, int64_t n, int k, const int32_t* perm, const float* hx,
+                        float* ohx) {
+  if (n <= 0) return;
+  k_obs_gather_hx<<<(unsigned)((n + 63) / 64), 256, 0, st>>>(n, k, perm, hx, ohx);
+}
+
 // operand columns of the products: hxp(kp, n) in search order, rows 0..k-1
 // the hx perturbations, row k the departure, rows above zero, so a column can
 // be read without row tests.  Entry (kp / 16) i + t holds row 16 t + i: lane i
@@ -131,7 +137,7 @@ void launch_obs_gather(hipStream_t st, int64_t n, int k, const int32_t* perm,
     k_obs_gather_fields<<<nb, 256, 0, st>>>(n, perm, lat, lon, zdim, time, val, err, obsid,
                                             platid, hxmean, pos, ozdim, oerr, odep, oidx, oobsid,
                                             oplatid, otime);
-    k_obs_gather_hx<<<(unsigned)((n + 63) / 64), 256, 0, st>>>(n, k, perm, hx, ohx);
+    launch_gather_cols(st, n, k, perm, hx, ohx);
   }
   k_cell_start<<<(kCells + 1 + 255) / 256, 256, 0, st>>>(n, sorted_cell, cell_start);
 }

@@ -208,6 +208,9 @@ void launch_members_from_state(hipStream_t st, int64_t nij, int64_t ns, int k,
                                float* members, float* mean, float* sprd);
 void launch_obs_hx_split(hipStream_t st, int64_t n, int k, const float* hx, const int32_t* qc,
                          float* pert, float* hmean, uint8_t* keep);
+// columns of k values: out's column s is in's column perm[s]
+void launch_gather_cols(hipStream_t st, int64_t n, int k, const int32_t* perm, const float* hx,
+                        float* ohx);
 void launch_obs_compact(hipStream_t st, int64_t nsel, int k, const int32_t* sel,
                         const ObsFields& in, const ObsFields& out);
 void launch_grid_xyz(hipStream_t st, int64_t n, const float* lat,
