@@ -647,18 +647,6 @@ __device__ __forceinline__ uint32_t spread_bits(uint32_t x) {   // 16 -> 32 bits
   return x;
 }
 
-__device__ __forceinline__ uint32_t bucket_desc(int64_t m, int bbits) {
-  // 0 for the largest bucket; unsolved problems (m = 0) last
-  const uint32_t nb = 32u << bbits;
-  if (m <= 0) return nb - 1u;
-  const uint32_t L = 63u - (uint32_t)__clzll((unsigned long long)m);   // floor(log2 m)
-  const uint32_t Lc = L > 30u ? 30u : L;
-  const uint32_t mask = (1u << bbits) - 1u;
-  const uint32_t sub = L >= (uint32_t)bbits ? (uint32_t)(m >> (L - bbits)) & mask
-                                            : (uint32_t)(m << (bbits - L)) & mask;
-  return nb - 2u - ((Lc << bbits) | sub);
-}
-
 __global__ void k_bucket_keys(int mode, int bbits, int64_t np, int G, int64_t i0,
                               const int64_t* __restrict__ cnt,
                               const uint8_t* __restrict__ solve,

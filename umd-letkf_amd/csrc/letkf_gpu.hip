@@ -1314,10 +1314,14 @@ static int run_eager(letkf_gpu_t* h) {
     RUNCHK(hipEventRecord(ce[0], sst));
     launch_search(sst, false, h->loc, O, S, V, C, D);
     RUNCHK(hipGetLastError());
-    size_t tb = h->tmp_bytes;
-    RUNCHK(hipcub::DeviceScan::ExclusiveSum(b_tmp, tb, padded_counts(b_cnt), b_off, (int)np,
-                                            sst));
-    launch_counters_to_host(sst, h->d_ctr, h->h_ctr, b_off + (np - 1), b_cnt + (np - 1), b_tot);
+    if (np <= kSmallChunk) {
+      launch_scan_small(sst, np, b_cnt, b_off, b_solve, -1, h->d_ctr, h->h_ctr, b_tot);
+    } else {
+      size_t tb = h->tmp_bytes;
+      RUNCHK(hipcub::DeviceScan::ExclusiveSum(b_tmp, tb, padded_counts(b_cnt), b_off, (int)np,
+                                              sst));
+      launch_counters_to_host(sst, h->d_ctr, h->h_ctr, b_off + (np - 1), b_cnt + (np - 1), b_tot);
+    }
     RUNCHK(hipGetLastError());
     RUNCHK(hipStreamSynchronize(sst));
     // list space: padded offsets, plus one alignment unit of slack for the
@@ -1355,11 +1359,15 @@ static int run_eager(letkf_gpu_t* h) {
     if (overlap) RUNCHK(hipStreamWaitEvent(st, ce[1], 0));
     RUNCHK(hipEventRecord(ce[2], st));
     if (h->batched()) {
-      launch_bucket_keys(st, h->tune_bucket, h->tune_bbits, np, (int)G, i0, b_cnt, b_solve,
-                         h->d_lat, h->d_lon, h->d_bkey, h->d_bval);
-      size_t sb = h->stmp_bytes;
-      RUNCHK(hipcub::DeviceRadixSort::SortPairs(h->d_stmp, sb, h->d_bkey, h->d_bkey2,
-                                                h->d_bval, h->d_perm, (int)np, 0, 32, st));
+      if (np <= kSmallOrder && h->tune_bucket >= 2) {
+        launch_order_small(st, np, h->tune_bbits, b_cnt, b_solve, h->d_perm);
+      } else {
+        launch_bucket_keys(st, h->tune_bucket, h->tune_bbits, np, (int)G, i0, b_cnt, b_solve,
+                           h->d_lat, h->d_lon, h->d_bkey, h->d_bval);
+        size_t sb = h->stmp_bytes;
+        RUNCHK(hipcub::DeviceRadixSort::SortPairs(h->d_stmp, sb, h->d_bkey, h->d_bkey2,
+                                                  h->d_bval, h->d_perm, (int)np, 0, 32, st));
+      }
       RUNCHK(hipEventRecord(ce[3], st));
       launch_product_mx(st, h->dims.precision, O, S, C, h->d_perm, h->d_B, h->d_b,
                         h->fold_log2, h->tune_tile);
@@ -1429,21 +1437,30 @@ static hipError_t enqueue_analysis(letkf_gpu_t* h) {
     launch_search(st, false, h->loc, W.O, W.S, W.V, C, W.D);
     e = hipGetLastError();
     if (e != hipSuccess) break;
-    size_t tb = h->tmp_bytes;
-    e = hipcub::DeviceScan::ExclusiveSum(h->d_tmp, tb, padded_counts(h->d_cnt), h->d_off,
-                                         (int)np, st);
-    if (e != hipSuccess) break;
-    launch_list_guard(st, np, h->d_cnt, h->d_off, h->d_solve, h->list_cap, h->d_ctr);
+    if (np <= kSmallChunk) {
+      launch_scan_small(st, np, h->d_cnt, h->d_off, h->d_solve, h->list_cap, h->d_ctr, nullptr,
+                        nullptr);
+    } else {
+      size_t tb = h->tmp_bytes;
+      e = hipcub::DeviceScan::ExclusiveSum(h->d_tmp, tb, padded_counts(h->d_cnt), h->d_off,
+                                           (int)np, st);
+      if (e != hipSuccess) break;
+      launch_list_guard(st, np, h->d_cnt, h->d_off, h->d_solve, h->list_cap, h->d_ctr);
+    }
     launch_search(st, true, h->loc, W.O, W.S, W.V, C, W.D);
     e = hipGetLastError();
     if (e != hipSuccess) break;
     if (h->batched()) {
-      launch_bucket_keys(st, h->tune_bucket, h->tune_bbits, np, (int)G, i0, h->d_cnt,
-                         h->d_solve, h->d_lat, h->d_lon, h->d_bkey, h->d_bval);
-      size_t sb = h->stmp_bytes;
-      e = hipcub::DeviceRadixSort::SortPairs(h->d_stmp, sb, h->d_bkey, h->d_bkey2, h->d_bval,
-                                             h->d_perm, (int)np, 0, 32, st);
-      if (e != hipSuccess) break;
+      if (np <= kSmallOrder && h->tune_bucket >= 2) {
+        launch_order_small(st, np, h->tune_bbits, h->d_cnt, h->d_solve, h->d_perm);
+      } else {
+        launch_bucket_keys(st, h->tune_bucket, h->tune_bbits, np, (int)G, i0, h->d_cnt,
+                           h->d_solve, h->d_lat, h->d_lon, h->d_bkey, h->d_bval);
+        size_t sb = h->stmp_bytes;
+        e = hipcub::DeviceRadixSort::SortPairs(h->d_stmp, sb, h->d_bkey, h->d_bkey2, h->d_bval,
+                                               h->d_perm, (int)np, 0, 32, st);
+        if (e != hipSuccess) break;
+      }
       launch_product_mx(st, h->dims.precision, W.O, W.S, C, h->d_perm, h->d_B, h->d_b,
                         h->fold_log2, h->tune_tile);
     } else {

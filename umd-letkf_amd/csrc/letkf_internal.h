@@ -135,6 +135,19 @@ constexpr int kCtrSolves = 0, kCtrCand = 16, kCtrPairs = 32, kCtrMax = 48;
 constexpr int kCtrOverflow = 8;       // slot 0 only: pairs refused list space
 constexpr int kCtrStep = 8;           // all of them are multiples of it
 
+// bucket of a kept count in the problem order: floor(log2 m) with the next
+// bbits bits, 0 for the largest; unsolved problems (m = 0) last
+__device__ __forceinline__ uint32_t bucket_desc(int64_t m, int bbits) {
+  const uint32_t nb = 32u << bbits;
+  if (m <= 0) return nb - 1u;
+  const uint32_t L = 63u - (uint32_t)__clzll((unsigned long long)m);   // floor(log2 m)
+  const uint32_t Lc = L > 30u ? 30u : L;
+  const uint32_t mask = (1u << bbits) - 1u;
+  const uint32_t sub = L >= (uint32_t)bbits ? (uint32_t)(m >> (L - bbits)) & mask
+                                            : (uint32_t)(m << (bbits - L)) & mask;
+  return nb - 2u - ((Lc << bbits) | sub);
+}
+
 // group of slab s at a gridpoint (letkf_loc_ocean.F90:360-375 for bkg_t)
 __device__ __forceinline__ int slab_group(const LocDev& L, const VarsDev& V,
                                           int s, int mld) {
@@ -216,6 +229,15 @@ void launch_obs_compact(hipStream_t st, int64_t nsel, int k, const int32_t* sel,
 void launch_grid_xyz(hipStream_t st, int64_t n, const float* lat,
                      const float* lon, double* x, double* y, double* z);
 void launch_clear_u64(hipStream_t st, int64_t n, unsigned long long* p);
+// chunks of few pairs (kernels_order.hip): at most kSmallChunk for the offsets,
+// and for the order at most kSmallOrder, two rounds of the problems that the
+// products have in flight, whose neighbourhood in L2 counts beyond
+constexpr int64_t kSmallChunk = 16384, kSmallOrder = 8192;
+void launch_scan_small(hipStream_t st, int64_t np, int64_t* cnt, int64_t* off, uint8_t* solve,
+                       int64_t cap, unsigned long long* ctr, unsigned long long* h_ctr,
+                       int64_t* tot);
+void launch_order_small(hipStream_t st, int64_t np, int bbits, const int64_t* cnt,
+                        const uint8_t* solve, int32_t* perm);
 void launch_list_guard(hipStream_t st, int64_t np, int64_t* cnt, const int64_t* off,
                        uint8_t* solve, int64_t cap, unsigned long long* ctr);
 void launch_search(hipStream_t st, bool fill, const LocDev& L,
