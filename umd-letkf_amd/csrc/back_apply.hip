@@ -14,8 +14,8 @@
 // the records into eigenvectors and two mat-vecs a slab (k_tql, k_replay,
 // k_vec_apply, still run with LETKF_GPU_RAT=0): QL is a serial chain per
 // problem, one lane each, and its records cross memory twice.  11 855
-// problems of k = 40 with 50 slabs: 5.2 ms then, 0.64 ms now; 33 problems
-// of k = 50 with 12 slabs: 540 us and 100 us.  The node table is the fine
+// problems of k = 40 with 50 slabs: 5.2 ms then, 0.51 ms now; 33 problems
+// of k = 50 with 12 slabs: 540 us and 75 us.  The node table is the fine
 // one (5e-16): over condition numbers of 1e2 to 8e6 the analysis is no further
 // from the FP64 oracle than the eigensolve's (spread 2e-14 against 1e-13 at
 // 8e6, k = 50).
@@ -26,25 +26,31 @@
 
 namespace lk {
 
-constexpr int kGroupNodes = 16;   // nodes of one pass over the rows (17 KB of
-                                  // LDS: nine waves a CU; all 62 would be two)
+constexpr int kGroupNodes = 16;   // nodes of one pass over the rows (18 KB of
+                                  // LDS: eight waves a CU; all 62 would be two)
 
+// Few problems or many, a wave's own latency is what this takes: the pivots'
+// recurrence, and in the rows the reads of U (all lanes the same 16 values,
+// two a read) and, from the second group of nodes on, of the entry to add to.
+// Those are made a row and two rows ahead, and a row's multiplications run on
+// the lanes below the diagonal alone instead of a select for each node: 342 ->
+// 199 us at 11 855 problems of k = 40, 44 -> 24 us at 33 problems of k = 50.
 __global__ __launch_bounds__(64) void k_small_rational(int k, int K, ChunkDev C,
                                                        double* __restrict__ B,
                                                        const double* __restrict__ dd,
                                                        const double* __restrict__ ee, RatTab R) {
   constexpr int NG = kGroupNodes;
-  constexpr int LD = 65;
-  __shared__ double sd[64], se[64];
-  // U of the node's bottom-up pivots, and its top-down pivots, then the
-  // diagonal of the inverse
-  __shared__ double Us[NG][LD], Gs[NG][LD];
+  constexpr int LD = NG + 2;        // 16-byte rows, lanes' own rows in different banks
+  __shared__ double sd[66], se[66];
+  // by row: U of the nodes' bottom-up pivots, and their top-down pivots
+  __shared__ __align__(16) double Us[66][LD], Gs[64][LD];
   const int64_t pair = blockIdx.x;
   if (!C.solve[pair]) return;
   const int l = threadIdx.x;
   const double m = (double)(k - 1);
   sd[l] = l < k ? dd[pair * K + l] : 0.0;
   se[l] = l < k - 1 ? ee[pair * K + l] : 0.0;
+  if (l < 2) { sd[64 + l] = 0.0; se[64 + l] = 0.0; }
   __syncthreads();
   double gm = l < k ? sd[l] + (l > 0 ? fabs(se[l - 1]) : 0.0) + fabs(se[l]) : 0.0;
   gm = p_max<64>(gm);
@@ -61,49 +67,64 @@ __global__ __launch_bounds__(64) void k_small_rational(int k, int K, ChunkDev C,
     if (l < 2 * NG) {
       const int n = l & (NG - 1);
       const double sg = n0 + n < nn ? m * sn[n0 + n] : m;
-      double f = 0.0;
+      double f = 0.0, e0 = 0.0;           // e0: the row before's off-diagonal
       if (l < NG) {
+        double d = sd[0], e1 = se[0];
         for (int i = 0; i < k; ++i) {
-          const double D = sd[i] + sg - (i > 0 ? se[i - 1] * f : 0.0);
-          Gs[n][i] = D;
-          f = se[i] * rcp_cubic(D);
+          const double d2 = sd[i + 1], e2 = se[i + 1];
+          const double D = fma(-e0, f, d + sg);
+          Gs[i][n] = D;
+          f = e1 * rcp_cubic(D);
+          e0 = e1;
+          d = d2;
+          e1 = e2;
         }
       } else {
+        double d = sd[k - 1], e1 = se[k - 2];
         for (int i = k - 1; i >= 0; --i) {
-          const double D = fma(-se[i], f, sd[i] + sg);
-          f = i > 0 ? se[i - 1] * rcp_cubic(D) : 0.0;
-          Us[n][i] = f;
+          const double d2 = sd[max(i - 1, 0)], e2 = se[max(i - 2, 0)];
+          const double D = fma(-e0, f, d + sg);
+          f = i > 0 ? e1 * rcp_cubic(D) : 0.0;
+          Us[i][n] = f;
+          e0 = e1;
+          d = d2;
+          e1 = e2;
         }
       }
     }
     __syncthreads();
-    // the inverse's diagonal 1 / (D+_i + D-_i - (d_i + s)) = 1 / (D+_i - e_i U_(i+1))
-    if (l < k) {
-#pragma unroll 4
-      for (int n = 0; n < NG; ++n)
-        Gs[n][l] = rcp_cubic(fma(-se[l], l < k - 1 ? Us[n][l + 1] : 0.0, Gs[n][l]));
-    }
-    __syncthreads();
-    // column l from its diagonal down
-    double cf[NG], x[NG];
+    // the inverse's diagonal 1 / (D+_i + D-_i - (d_i + s)) = 1 / (D+_i - e_i U_(i+1)),
+    // where column l starts
+    double cf[NG], x[NG], u[NG];
+    const int lr = l < k ? l : 0;
 #pragma unroll
     for (int n = 0; n < NG; ++n) {
       cf[n] = n0 + n < nn ? m * wn[n0 + n] : 0.0;
-      x[n] = Gs[n][l < k ? l : 0];
+      x[n] = rcp_cubic(fma(-se[lr], lr < k - 1 ? Us[lr + 1][n] : 0.0, Gs[lr][n]));
+      u[n] = Us[0][n];
     }
+    const bool more = n0 > 0 && l < k;
+    auto old = [&](int r) { return more && r >= l && r < k ? Bp[r * k + l] : 0.0; };
+    double o0 = old(0), o1 = old(1);
+    // column l from its diagonal down
     for (int r = 0; r < k; ++r) {
+      const double o2 = old(r + 2);
+      double un[NG];
+      const int rn = r + 1 < k ? r + 1 : r;
+#pragma unroll
+      for (int n = 0; n < NG; ++n) un[n] = Us[rn][n];
+      if (r > l) {
+#pragma unroll
+        for (int n = 0; n < NG; ++n) x[n] = -u[n] * x[n];
+      }
       double acc[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-      for (int n = 0; n < NG; ++n) {
-        const double xn = -Us[n][r] * x[n];
-        x[n] = r > l ? xn : x[n];
-        acc[n & 3] = fma(cf[n], x[n], acc[n & 3]);
-      }
-      if (r >= l && l < k) {
-        const double s = (acc[0] + acc[1]) + (acc[2] + acc[3]);
-        double* at = Bp + (int64_t)r * k + l;
-        *at = n0 > 0 ? *at + s : s;
-      }
+      for (int n = 0; n < NG; ++n) acc[n & 3] = fma(cf[n], x[n], acc[n & 3]);
+      if (r >= l && l < k) Bp[r * k + l] = o0 + ((acc[0] + acc[1]) + (acc[2] + acc[3]));
+      o0 = o1;
+      o1 = o2;
+#pragma unroll
+      for (int n = 0; n < NG; ++n) u[n] = un[n];
     }
     __syncthreads();
   }
