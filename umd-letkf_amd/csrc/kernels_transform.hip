@@ -13,6 +13,7 @@
 //                  path).
 #include <hip/hip_runtime.h>
 
+#include "dpp_common.h"
 #include "letkf_internal.h"
 #include "mx_common.h"
 #include "transform_mat.h"
@@ -48,7 +49,6 @@ LK_KQ(72) LK_KQ(80) LK_KQ(88) LK_KQ(96) LK_KQ(104)
 // same order by every lane (x starts at g_c in row c, is 0 above it), so the
 // pivot reads are broadcasts and the stores of a row are contiguous
 constexpr int kMaxNodes = 32;
-constexpr int kNodeLd = 129;        // LDS row length of the node arrays
 
 // a wave-uniform double in scalar registers
 __device__ __forceinline__ double uniform_f64(double v) {
@@ -57,56 +57,19 @@ __device__ __forceinline__ double uniform_f64(double v) {
   return __hiloint2double(hi, lo);
 }
 
-// rows rfirst..k-1 of column c of M for the first NN nodes (nn <= NN).  x
-// starts at g_c (the inverse's diagonal) and follows x <- -U_r x from row
-// c + 1 on; rows above c are not stored.  The node weights are uniform
-// (scalar registers), and each row's U values are read 8 at a time before
-// they are used, all lanes reading the same entries.
-template <int NN>
-__device__ __forceinline__ void mat_rational_rows(int k, int c, int rfirst, int nn, double m,
-                                                  const double* __restrict__ wn,
-                                                  const double (*Us)[kNodeLd],
-                                                  const double (*Gs)[kNodeLd], double* Bp) {
-  double cf[NN], x[NN];
-#pragma unroll
-  for (int n = 0; n < NN; ++n) {
-    cf[n] = uniform_f64(n < nn ? m * wn[n] : 0.0);
-    x[n] = Gs[n][c];
-  }
-  for (int r = rfirst; r < k; ++r) {
-    // four partial sums: the node chains are independent, the sum need not
-    // be one dependent chain
-    double acc[4] = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-    for (int n0 = 0; n0 < NN; n0 += 8) {
-      double u[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) u[e] = Us[n0 + e][r];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int n = n0 + e;
-        double xn = -u[e] * x[n];
-        asm volatile("" : "+v"(xn));   // computed on every lane, then selected
-        x[n] = r > c ? xn : x[n];
-        acc[n & 3] = fma(cf[n], x[n], acc[n & 3]);
-      }
-    }
-    if (r >= c) Bp[(int64_t)r * k + c] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
-  }
-}
-
-// 1/x: the hardware estimate and one Newton step, which squares its
-// relative error (as the vector path's rational solve)
-__device__ __forceinline__ double mat_rcp(double x) {
-  const double y = __builtin_amdgcn_rcp(x);
-  return y * (2.0 - x * y);
-}
 // One launch per class of node counts NNLO < nn <= NNL: the node arrays are
 // sized for the class, so the problems that need few nodes (the better
-// conditioned ones) run four blocks per CU (16 nodes, 35 KB of LDS) or three
+// conditioned ones) run four blocks per CU (16 nodes, 37 KB of LDS) or three
 // (24 nodes) where 32 nodes allow two; a problem of another class leaves once
-// its node count is known (uniform over the block).  Each problem takes the
-// same steps in its class's launch as in a single launch sized for 32 nodes.
+// its node count is known (uniform over the block).
+//
+// The first wave's lanes run the nodes' top-down pivots, the second's the
+// bottom-up ones, a node each.  Then a thread takes a column: x starts at the
+// inverse's diagonal in row c and follows x <- -U_r x below; a row's U values,
+// the same for all lanes, are read two at a time and a row ahead, and the
+// multiplications run on the lanes below the diagonal alone.  11 900 problems
+// of k = 100 with at most 16 nodes: 807 us with both recurrences in one lane,
+// U read node by node and a select for each, 456 us now.
 template <int NNL, int NNLO>
 __global__ __launch_bounds__(128) void k_mat_rational(int k, ChunkDev C, double* __restrict__ B,
                                                       const double* __restrict__ dd,
@@ -115,10 +78,10 @@ __global__ __launch_bounds__(128) void k_mat_rational(int k, ChunkDev C, double*
                                                       const int* __restrict__ tabn,
                                                       int nbucket) {
   static_assert(NNL % 8 == 0 && NNL <= kMaxNodes, "node class");
-  __shared__ double sd[128], se[128];
-  // rows of 129: lane n of the pivot recurrences writes row n, and the
-  // lanes' entries then fall in different banks (with 128, all in one)
-  __shared__ double Us[NNL][kNodeLd], Gs[NNL][kNodeLd];
+  constexpr int LD = NNL + 2;       // 16-byte rows, lanes' own rows in different banks
+  __shared__ double sd[130], se[130];
+  // by row: U of the nodes' bottom-up pivots, and their top-down pivots
+  __shared__ __align__(16) double Us[128][LD], Gs[128][LD];
   __shared__ double sgm[2];
   const int64_t pair = blockIdx.x;
   if (!C.solve[pair]) return;
@@ -126,6 +89,7 @@ __global__ __launch_bounds__(128) void k_mat_rational(int k, ChunkDev C, double*
   const double m = (double)(k - 1);
   sd[tid] = tid < k ? dd[pair * kMatStride + tid] : 0.0;
   se[tid] = tid < k - 1 ? ee[pair * kMatStride + tid] : 0.0;
+  if (tid < 2) { sd[128 + tid] = 0.0; se[128 + tid] = 0.0; }
   __syncthreads();
   double gm = 0.0;
   if (tid < k)
@@ -142,47 +106,64 @@ __global__ __launch_bounds__(128) void k_mat_rational(int k, ChunkDev C, double*
   if (nn > NNL || nn <= NNLO) return;
   const double* sn = tab + bk * kRatLd;
   const double* wn = sn + kRatLd / 2;
-  // unused node rows stay 0, so that their chains stay 0
-  for (int n = nn; n < NNL; ++n) { Us[n][tid] = 0.0; Gs[n][tid] = 0.0; }
-  // one lane per node runs both pivot recurrences in one loop, step s
-  // taking the top-down pivot D+ of row s and the bottom-up pivot D- of row
-  // k-1-s (two independent chains).  U_i = e_(i-1) / D-_i goes to Us; the
-  // diagonal of the inverse, 1 / g_i with g_i = D+_i + D-_i - (d_i + s),
-  // goes to Gs once both pivots of row i are known (the first of the two
-  // waits in Gs[n][i], written and read by the same lane)
-  if (tid < nn) {
-    const int n = tid;
-    const double sg = m * sn[n];
-    double Lp = 0.0, Up = 0.0;
-#pragma unroll 2
-    for (int st = 0; st < k; ++st) {
-      const int it = st, ib = k - 1 - st;
-      const double Dp = sd[it] + sg - (it > 0 ? se[it - 1] * Lp : 0.0);
-      const double Dm = sd[ib] + sg - (ib < k - 1 ? se[ib] * Up : 0.0);
-      Lp = it < k - 1 ? se[it] * mat_rcp(Dp) : 0.0;
-      const double Ui = ib > 0 ? se[ib - 1] * mat_rcp(Dm) : 0.0;
-      Us[n][ib] = Ui;
-      Up = Ui;
-      if (it < ib) {            // first half: park the pivots
-        Gs[n][it] = Dp;
-        Gs[n][ib] = Dm;
-      } else if (it == ib) {    // middle row (k odd)
-        Gs[n][it] = mat_rcp(Dp + Dm - (sd[it] + sg));
-      } else {                  // second half: the other pivot is parked
-        const double dmt = Gs[n][it];   // D- of row it
-        const double dpb = Gs[n][ib];   // D+ of row ib
-        Gs[n][it] = mat_rcp(Dp + dmt - (sd[it] + sg));
-        Gs[n][ib] = mat_rcp(dpb + Dm - (sd[ib] + sg));
+  // a node past the last has a pivot of at least m and weight 0
+  if (l < NNL) {
+    const double sg = l < nn ? m * sn[l] : m;
+    double f = 0.0, e0 = 0.0;             // e0: the row before's off-diagonal
+    if (tid < 64) {
+      double d = sd[0], e1 = se[0];
+      for (int i = 0; i < k; ++i) {
+        const double d2 = sd[i + 1], e2 = se[i + 1];
+        const double D = fma(-e0, f, d + sg);
+        Gs[i][l] = D;
+        f = e1 * rcp_cubic(D);
+        e0 = e1;
+        d = d2;
+        e1 = e2;
+      }
+    } else {
+      double d = sd[k - 1], e1 = se[k - 2];
+      for (int i = k - 1; i >= 0; --i) {
+        const double d2 = sd[max(i - 1, 0)], e2 = se[max(i - 2, 0)];
+        const double D = fma(-e0, f, d + sg);
+        f = i > 0 ? e1 * rcp_cubic(D) : 0.0;
+        Us[i][l] = f;
+        e0 = e1;
+        d = d2;
+        e1 = e2;
       }
     }
   }
   __syncthreads();
   const int c = tid;
   if (c >= k) return;
-  // rows above a wave's first column hold zeros in every lane of the wave
+  // the inverse's diagonal 1 / (D+_c + D-_c - (d_c + s)) = 1 / (D+_c - e_c U_(c+1))
+  double cf[NNL], x[NNL], u[NNL];
+  // rows above a wave's first column are not stored
   const int rfirst = __builtin_amdgcn_readfirstlane(tid & ~63);
+#pragma unroll
+  for (int n = 0; n < NNL; ++n) {
+    cf[n] = uniform_f64(n < nn ? m * wn[n] : 0.0);
+    x[n] = rcp_cubic(fma(-se[c], c < k - 1 ? Us[c + 1][n] : 0.0, Gs[c][n]));
+    u[n] = Us[rfirst][n];
+  }
   double* Bp = B + pair * (int64_t)k * k;
-  mat_rational_rows<NNL>(k, c, rfirst, nn, m, wn, Us, Gs, Bp);
+  for (int r = rfirst; r < k; ++r) {
+    double un[NNL];
+    const int rn = r + 1 < k ? r + 1 : r;
+#pragma unroll
+    for (int n = 0; n < NNL; ++n) un[n] = Us[rn][n];
+    if (r > c) {
+#pragma unroll
+      for (int n = 0; n < NNL; ++n) x[n] = -u[n] * x[n];
+    }
+    double acc[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int n = 0; n < NNL; ++n) acc[n & 3] = fma(cf[n], x[n], acc[n & 3]);
+    if (r >= c) Bp[r * k + c] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+#pragma unroll
+    for (int n = 0; n < NNL; ++n) u[n] = un[n];
+  }
 }
 
 // sum over a slab of the tile: the lane's registers (summed by the caller),
