@@ -73,6 +73,35 @@ __device__ __forceinline__ double p_sum(double x) {
   return x;
 }
 
+// sums of four values over the wave, uniform: the halves' sums of two values
+// take one swap and addition for both, so do the rows', and one chain of
+// rotations serves the four rows that then hold a value each (29 instructions
+// where four sums of their own take 104)
+__device__ __forceinline__ double swap_sum32(double a, double b) {
+  const auto l = __builtin_amdgcn_permlane32_swap((unsigned)__double2loint(a),
+                                                  (unsigned)__double2loint(b), false, false);
+  const auto h = __builtin_amdgcn_permlane32_swap((unsigned)__double2hiint(a),
+                                                  (unsigned)__double2hiint(b), false, false);
+  return __hiloint2double((int)h[0], (int)l[0]) + __hiloint2double((int)h[1], (int)l[1]);
+}
+__device__ __forceinline__ double swap_sum16(double a, double b) {
+  const auto l = __builtin_amdgcn_permlane16_swap((unsigned)__double2loint(a),
+                                                  (unsigned)__double2loint(b), false, false);
+  const auto h = __builtin_amdgcn_permlane16_swap((unsigned)__double2hiint(a),
+                                                  (unsigned)__double2hiint(b), false, false);
+  return __hiloint2double((int)h[0], (int)l[0]) + __hiloint2double((int)h[1], (int)l[1]);
+}
+__device__ __forceinline__ void wave_sums4(double (&q)[4]) {
+  // rows: q0, q2, q1, q3
+  const double x = p_sum<16>(swap_sum16(swap_sum32(q[0], q[1]), swap_sum32(q[2], q[3])));
+  const int lo = __double2loint(x), hi = __double2hiint(x);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int at = 16 * ((i & 1) * 2 + (i >> 1));
+    q[i] = __hiloint2double(__builtin_amdgcn_readlane(hi, at), __builtin_amdgcn_readlane(lo, at));
+  }
+}
+
 // largest value over the P lanes, in every lane
 template <int P>
 __device__ __forceinline__ double p_max(double x) {
