@@ -458,15 +458,16 @@ hipError_t launch_eigen_apply_f64(hipStream_t st, const LocDev& L, const StateDe
 // A sum is NJ - 1 additions and four DPP rotations, and the roots and
 // divisions serve four slabs (with one slab a wave, 250 instructions each,
 // the instructions bounded it: 684 us at 1.04e6 slabs of k = 50, 397 us at
-// 810 000 of k = 40, against 150 and 80 us of memory traffic; now 267 and
-// 198 us).  Small grids: one slab's latency instead of a gridpoint's slabs
+// 810 000 of k = 40, against 150 and 80 us of memory traffic; now 286 and
+// 186 us).  Small grids: one slab's latency instead of a gridpoint's slabs
 // in turn.
 //
 // A run of slabs is looked over first, a lane each: which are solved,
 // masked (the background unchanged) or, with skip_solved, done already by
 // the apply.  A run is the four slabs of one pass, or 16 where the apply has
 // done most of them and the waves' launch counts (972 000 slabs of k = 100, 30%
-// of them masked: 131 us with four, 104 with 16).
+// of them masked: 131 us with four, 104 with 16, 79 with masked slabs copied
+// without the sums).
 // ---------------------------------------------------------------------------
 template <int NJ>
 __global__ __launch_bounds__(256) void k_finalize(LocDev L, StateDev S, VarsDev V, ChunkDev C,
@@ -502,6 +503,22 @@ __global__ __launch_bounds__(256) void k_finalize(LocDev L, StateDev S, VarsDev 
     const int64_t e = C.i0 * S.ns + u0 + at;          // slab of the whole grid
     const float* xb = S.state + e * k;
     double* xa = ana + e * k;
+    if ((((b_need & ~b_masked) >> q) & 15) == 0) {    // masked gridpoints alone: a copy
+      if (on) {
+        float c[NJ];
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) c[j] = xb[min(i + 16 * j, k - 1)];
+        const float cm = S.mean[e], cs = S.sprd[e];
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+          if (i + 16 * j < k) xa[i + 16 * j] = (double)c[j];
+        if (i == 0) {
+          amean[e] = (double)cm;
+          asprd[e] = (double)cs;
+        }
+      }
+      continue;
+    }
     double x[NJ];
     float b[NJ];
     if (on) {
