@@ -26,6 +26,7 @@
 #include <vector>
 
 #include "det_math.h"
+#include "host_memory.h"
 #include "letkf_internal.h"
 #include "ratnodes.h"
 
@@ -460,23 +461,21 @@ int letkf_gpu_destroy(letkf_gpu_t* h) {
 
 }  // extern "C"
 
-// background buffers: sizes fixed by the handle's dims, allocated by the
-// first set_state* and reused by later ones (a new cycle's background keeps
-// the device addresses a captured analysis was recorded with)
 // the device's address of n bytes of page-locked host memory, or nullptr for
-// anything else: the first and the last byte must be page-locked and as far
-// apart there as here
+// anything else (locked_span)
 static void* locked_view(const void* p, size_t n) {
-  hipPointerAttribute_t a{}, b{};
-  const char* last = (const char*)p + n - 1;
-  if (hipPointerGetAttributes(&a, p) != hipSuccess || a.type != hipMemoryTypeHost ||
-      hipPointerGetAttributes(&b, last) != hipSuccess || b.type != hipMemoryTypeHost) {
-    (void)hipGetLastError();
-    return nullptr;
-  }
-  if (!a.devicePointer || (char*)b.devicePointer - (char*)a.devicePointer != last - (const char*)p)
-    return nullptr;
-  return a.devicePointer;
+  return locked_span(p, n, [](const void* q, LockedPiece* out) {
+    hipPointerAttribute_t a{};
+    hipDeviceptr_t base = nullptr;
+    size_t size = 0;
+    if (hipPointerGetAttributes(&a, q) != hipSuccess || a.type != hipMemoryTypeHost ||
+        hipMemGetAddressRange(&base, &size, (hipDeviceptr_t)a.devicePointer) != hipSuccess) {
+      (void)hipGetLastError();
+      return false;
+    }
+    *out = {(char*)a.devicePointer, (const char*)base, size};
+    return true;
+  });
 }
 
 // A large copy between pageable host memory and the device on h->stream.
@@ -559,6 +558,9 @@ static hipError_t bulk_copy(letkf_gpu_t* h, void* dst, const void* src, size_t b
   return (hipError_t)err.load();
 }
 
+// background buffers: sizes fixed by the handle's dims, allocated by the
+// first set_state* and reused by later ones (a new cycle's background keeps
+// the device addresses a captured analysis was recorded with)
 static hipError_t alloc_state(letkf_gpu_t* h) {
   const size_t k = (size_t)h->k, ns = (size_t)h->ns, nij = (size_t)h->nij;
   hipError_t e = hipSuccess;
