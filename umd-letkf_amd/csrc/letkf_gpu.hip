@@ -478,14 +478,26 @@ static void* locked_view(const void* p, size_t n) {
   });
 }
 
+// whether the runtime knows the memory at p: device, managed or page-locked
+static bool runtime_knows(const void* p) {
+  hipPointerAttribute_t a{};
+  if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return a.type != hipMemoryTypeUnregistered;
+}
+
 // A large copy between pageable host memory and the device on h->stream.
 // The runtime's own way is one thread's: 28 GB/s up, and 54 MB down into
 // memory touched for the first time took 5.3 ms, 2.6 of them page faults.
 // Here kRingThreads threads take the array's pieces in turn, each through two
 // page-locked slots of its own, so that copies in host memory, page faults and
 // the bus overlap.  The copies up are in the stream when it returns; those
-// down have arrived.  Small or page-locked arrays, and a machine that gives
-// no threads or slots, take the runtime's way.
+// down have arrived.  Small arrays, memory that the runtime knows (page-locked
+// or managed, or a device's own: the threads would read that over the bus, or
+// not at all), and a machine that gives no threads or slots, take the
+// runtime's way.
 static constexpr int kRingThreads = 6, kRingSlots = 2;
 static constexpr size_t kRingBytes = 1ull << 20;       // a slot
 static constexpr size_t kRingLeast = 8ull << 20;       // a smaller copy gains nothing
@@ -494,7 +506,8 @@ static hipError_t bulk_copy(letkf_gpu_t* h, void* dst, const void* src, size_t b
   hipStream_t st = h->stream;
   const hipMemcpyKind kind = up ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost;
   int dev = 0;
-  if (bytes < kRingLeast || locked_view(up ? src : dst, bytes) ||
+  const char* host = (const char*)(up ? src : dst);
+  if (bytes < kRingLeast || runtime_knows(host) || runtime_knows(host + bytes - 1) ||
       hipGetDevice(&dev) != hipSuccess)
     return hipMemcpyAsync(dst, src, bytes, kind, st);
   if (!h->h_ring && hipHostMalloc((void**)&h->h_ring, kRingThreads * kRingSlots * kRingBytes,
