@@ -130,7 +130,7 @@ struct letkf_gpu_t {
   void* d_tmp = nullptr;
   size_t tmp_bytes = 0;
   int64_t* h_tot = nullptr;    // pinned
-  char* h_ring = nullptr;      // pinned: slots of the threads of bulk_copy
+  char* h_ring = nullptr;      // pinned: slots of the threads of bulk_fetch
   void* h_diag = nullptr;      // pinned: diagnostics on their way out
   size_t diag_bytes = 0;
 
@@ -488,33 +488,32 @@ static bool runtime_knows(const void* p) {
   return a.type != hipMemoryTypeUnregistered;
 }
 
-// A large copy between pageable host memory and the device on h->stream.
-// The runtime's own way is one thread's: 28 GB/s up, and 54 MB down into
-// memory touched for the first time took 5.3 ms, 2.6 of them page faults.
-// Here kRingThreads threads take the array's pieces in turn, each through two
-// page-locked slots of its own, so that copies in host memory, page faults and
-// the bus overlap.  The copies up are in the stream when it returns; those
-// down have arrived.  Small arrays, memory that the runtime knows (page-locked
-// or managed, or a device's own: the threads would read that over the bus, or
-// not at all), and a machine that gives no threads or slots, take the
-// runtime's way.
+// A large copy from the device on h->stream to pageable host memory.  The
+// runtime's own way is one thread's: 54 MB into memory touched for the first
+// time took 5.3 ms, 2.6 of them page faults.  Here kRingThreads threads take
+// the array's pieces in turn, each through two page-locked slots of its own,
+// so that copies in host memory, page faults and the bus overlap.  The data
+// have arrived when it returns.  Small arrays, memory that the runtime knows
+// (page-locked or managed, or a device's own: the threads would write that
+// over the bus, or not at all), and a machine that gives no threads or slots,
+// take the runtime's way.  So do all copies up: 36 and 52 MB took the same time
+// either way (1.4 and 2.0 ms), 200 MB 7.4 ms by the threads and 7.9 without,
+// and the slots cost a handle's first copy 1.1 ms.
 static constexpr int kRingThreads = 6, kRingSlots = 2;
 static constexpr size_t kRingBytes = 1ull << 20;       // a slot
 static constexpr size_t kRingLeast = 8ull << 20;       // a smaller copy gains nothing
 
-static hipError_t bulk_copy(letkf_gpu_t* h, void* dst, const void* src, size_t bytes, bool up) {
+static hipError_t bulk_fetch(letkf_gpu_t* h, void* dst, const void* src, size_t bytes) {
   hipStream_t st = h->stream;
-  const hipMemcpyKind kind = up ? hipMemcpyHostToDevice : hipMemcpyDeviceToHost;
   int dev = 0;
-  const char* host = (const char*)(up ? src : dst);
-  if (bytes < kRingLeast || runtime_knows(host) || runtime_knows(host + bytes - 1) ||
+  if (bytes < kRingLeast || runtime_knows(dst) || runtime_knows((char*)dst + bytes - 1) ||
       hipGetDevice(&dev) != hipSuccess)
-    return hipMemcpyAsync(dst, src, bytes, kind, st);
+    return hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st);
   if (!h->h_ring && hipHostMalloc((void**)&h->h_ring, kRingThreads * kRingSlots * kRingBytes,
                                   hipHostMallocDefault) != hipSuccess) {
     (void)hipGetLastError();
     h->h_ring = nullptr;
-    return hipMemcpyAsync(dst, src, bytes, kind, st);
+    return hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st);
   }
   const size_t np = (bytes + kRingBytes - 1) / kRingBytes;
   std::atomic<size_t> next{0};
@@ -524,7 +523,7 @@ static hipError_t bulk_copy(letkf_gpu_t* h, void* dst, const void* src, size_t b
     hipError_t e = hipSetDevice(dev);
     char* slot[kRingSlots];
     hipEvent_t ev[kRingSlots] = {};
-    size_t held[kRingSlots];               // down: the piece that is on its way
+    size_t held[kRingSlots];               // the piece that is on its way
     bool busy[kRingSlots] = {};
     for (int s = 0; s < kRingSlots; ++s) {
       slot[s] = h->h_ring + (size_t)(w * kRingSlots + s) * kRingBytes;
@@ -535,18 +534,15 @@ static hipError_t bulk_copy(letkf_gpu_t* h, void* dst, const void* src, size_t b
       busy[s] = false;
       const hipError_t es = hipEventSynchronize(ev[s]);
       if (e == hipSuccess) e = es;
-      if (!up && e == hipSuccess)
-        memcpy((char*)dst + held[s] * kRingBytes, slot[s], piece(held[s]));
+      if (e == hipSuccess) memcpy((char*)dst + held[s] * kRingBytes, slot[s], piece(held[s]));
     };
     int s = 0;
     while (e == hipSuccess && err.load() == (int)hipSuccess) {
       settle(s);
       const size_t p = next.fetch_add(1);
       if (p >= np || e != hipSuccess) break;
-      const size_t at = p * kRingBytes, n = piece(p);
-      if (up) memcpy(slot[s], (const char*)src + at, n);
-      e = up ? hipMemcpyAsync((char*)dst + at, slot[s], n, kind, st)
-             : hipMemcpyAsync(slot[s], (const char*)src + at, n, kind, st);
+      e = hipMemcpyAsync(slot[s], (const char*)src + p * kRingBytes, piece(p),
+                         hipMemcpyDeviceToHost, st);
       if (e == hipSuccess) e = hipEventRecord(ev[s], st);
       if (e == hipSuccess) { busy[s] = true; held[s] = p; }
       s = (s + 1) % kRingSlots;
@@ -603,7 +599,8 @@ int letkf_gpu_set_state_members(letkf_gpu_t* h, const float* members, const floa
   if (nij > 0) {
     float* raw = nullptr;
     HIPCHK(h, dalloc(h, &raw, (size_t)(k * ns * nij)));
-    hipError_t e = bulk_copy(h, raw, members, sizeof(float) * k * ns * nij, true);
+    hipError_t e = hipMemcpyAsync(raw, members, sizeof(float) * k * ns * nij,
+                                  hipMemcpyHostToDevice, h->stream);
     if (e == hipSuccess) {
       launch_state_from_members(h->stream, nij, ns, (int)k, raw, h->d_state, h->d_mean,
                                 h->d_sprd);
@@ -634,7 +631,7 @@ int letkf_gpu_set_state(letkf_gpu_t* h, const float* state_ij, const float* mean
   h->have_run = false;
   HIPCHK(h, alloc_state(h));
   if (nij > 0) {
-    HIPCHK(h, bulk_copy(h, h->d_state, state_ij, sizeof(float) * k * ns * nij, true));
+    HIPCHK(h, hipMemcpyAsync(h->d_state, state_ij, sizeof(float) * k * ns * nij, hipMemcpyHostToDevice, h->stream));
     HIPCHK(h, hipMemcpyAsync(h->d_mean, mean_ij, sizeof(float) * ns * nij, hipMemcpyHostToDevice, h->stream));
     HIPCHK(h, hipMemcpyAsync(h->d_sprd, sprd_ij, sizeof(float) * ns * nij, hipMemcpyHostToDevice, h->stream));
     HIPCHK(h, hipMemcpyAsync(h->d_lat, lat_ij, sizeof(float) * nij, hipMemcpyHostToDevice, h->stream));
@@ -715,7 +712,7 @@ static int set_obs_impl(letkf_gpu_t* h, int64_t n, const float* lat, const float
     OBSCHK(hipMemcpyAsync(r_obsid, obsid, 4 * n, hipMemcpyHostToDevice, st));
     OBSCHK(hipMemcpyAsync(r_platid, platid, 4 * n, hipMemcpyHostToDevice, st));
     if (!members) {
-      OBSCHK(bulk_copy(h, r_hx, hx_pert, 4 * n * k, true));
+      OBSCHK(hipMemcpyAsync(r_hx, hx_pert, 4 * n * k, hipMemcpyHostToDevice, st));
       OBSCHK(hipMemcpyAsync(r_hxm, hx_mean, 4 * n, hipMemcpyHostToDevice, st));
     }
   }
@@ -723,7 +720,7 @@ static int set_obs_impl(letkf_gpu_t* h, int64_t n, const float* lat, const float
     // obs_hx_mean, perturbations and the qc <= 0 flags (src/letkf_obs.F90:459-466)
     OBSCHK(dalloc(h, &r_full, nn * k)); OBSCHK(dalloc(h, &r_qc, nn)); OBSCHK(dalloc(h, &keep, nn));
     OBSCHK(dalloc(h, &sel, nn)); OBSCHK(dalloc(h, &nsel_d, 1));
-    OBSCHK(bulk_copy(h, r_full, hx_full, 4 * n * k, true));
+    OBSCHK(hipMemcpyAsync(r_full, hx_full, 4 * n * k, hipMemcpyHostToDevice, st));
     OBSCHK(hipMemcpyAsync(r_qc, qc, 4 * n, hipMemcpyHostToDevice, st));
     launch_obs_hx_split(st, n, (int)k, r_full, r_qc, r_hx, r_hxm, keep);
     OBSCHK(hipGetLastError());
@@ -1657,7 +1654,7 @@ int letkf_gpu_get_state_members(letkf_gpu_t* h, float* members, float* mean, flo
                               dmu, dsp);
     e = hipGetLastError();
   }
-  if (e == hipSuccess && members) e = bulk_copy(h, members, dm, 4 * k * ns * nij, false);
+  if (e == hipSuccess && members) e = bulk_fetch(h, members, dm, 4 * k * ns * nij);
   if (e == hipSuccess && mean)
     e = hipMemcpyAsync(mean, dmu, 4 * ns * nij, hipMemcpyDeviceToHost, h->stream);
   if (e == hipSuccess && sprd)
@@ -1742,7 +1739,7 @@ int letkf_gpu_get_state(letkf_gpu_t* h, float* state, float* mean, float* sprd) 
       launch_f64_to_f32(h->stream, c, src + i, stage);
       e = hipGetLastError();
       if (e == hipSuccess)
-        e = bulk_copy(h, dst + i, stage, 4 * c, false);
+        e = bulk_fetch(h, dst + i, stage, 4 * c);
       if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
     }
   };
