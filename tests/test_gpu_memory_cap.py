@@ -1,0 +1,43 @@
+"""LETKF_GPU_MEM_LIMIT bounds all that a handle holds, the blocks it keeps
+between calls among it, and an analysis that fits the cap runs: the kept
+blocks make room for the lists and work arrays."""
+import numpy as np
+import pytest
+import torch
+
+from letkf_amd import synth
+from letkf_amd.solver import LetkfGpuSolver
+
+pytestmark = pytest.mark.gpu
+
+
+def _analyse(s):
+    s.run()
+    return (*s.state_f64(), s.diag())
+
+
+def _same(a, b):
+    for x, y in zip(a[:3], b[:3]):
+        assert np.array_equal(x, y)
+    for n in a[3]:
+        assert np.array_equal(a[3][n], b[3][n])
+
+
+def test_kept_blocks_count(monkeypatch):
+    """About 130 MB of observations and 125 MB of their upload's temporaries, which
+    are kept; then 130 MB of the run's arrays, for which they make room."""
+    cap = 340 << 20
+    p = synth.random_problem(seed=6, nx=100, ny=50, k=50, ns=10, nobs=200000, radius=60e3)
+    g = np.random.default_rng(6)
+    hx = np.asfortranarray(p.hx + p.hxmean[None])
+    qc = (g.random(p.nobs) < 0.1).astype(np.int32)
+    with LetkfGpuSolver(p, precision="fp64", path="plain", obs_members=(qc, hx)) as s:
+        ref = _analyse(s)
+    monkeypatch.setenv("LETKF_GPU_MEM_LIMIT", str(cap))
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    with LetkfGpuSolver(p, precision="fp64", path="plain", obs_members=(qc, hx)) as s:
+        _same(_analyse(s), ref)
+        held = free - torch.cuda.mem_get_info()[0]
+        print("held", held >> 20, "of", cap >> 20, "MB", flush=True)
+        assert held <= cap + (32 << 20)                # the driver's own rounding

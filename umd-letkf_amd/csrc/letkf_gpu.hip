@@ -20,7 +20,6 @@
 #include <mutex>
 #include <string>
 #include <atomic>
-#include <map>
 #include <thread>
 #include <unordered_map>
 #include <vector>
@@ -29,6 +28,7 @@
 #include "host_memory.h"
 #include "letkf_internal.h"
 #include "ratnodes.h"
+#include "spare_blocks.h"
 
 using namespace lk;
 
@@ -148,11 +148,10 @@ struct letkf_gpu_t {
   int64_t obs_cap = 0;     // columns allocated for the observation buffers
   int list_headroom_div = 4;   // lists grow to total + total / div
   // device memory of the handle: live allocations and an optional cap
-  struct Block { size_t asked, size; };
-  std::unordered_map<void*, Block> live;
-  std::multimap<size_t, void*> spare;   // blocks of temporaries kept for the next call
-  size_t spare_bytes = 0;
+  std::unordered_map<void*, size_t> live;
   size_t live_bytes = 0;
+  // blocks of temporaries kept for the next call
+  SpareBlocks spare{[](void* p) { hipFree(p); }};
   size_t mem_limit = 0;   // 0 = none
   int tune_xcd = 4;       // product kernels: runs of 256 problems per XCD
   int tune_tile = 1;      // batched product: 0 32x32 MFMA blocks, 1 16x16 tiles
@@ -270,41 +269,33 @@ static int fail(letkf_gpu_t* h, int code, const char* fmt, ...) {
 // exercised on a GPU with memory to spare.
 //
 // Blocks of a call's temporaries (upload and staging arrays) are kept for
-// later calls, at most kSpareBytes of them: 45 allocations and releases of an
-// observation set took 3.5 ms of the 7.6 that handing over 500 000
-// observations of k = 50 takes.  They don't count as live, are given back when
-// an allocation fails and with the handle, and are only kept once the
-// handle's stream is idle (a release waits for the device, so every call
-// waits for its stream before it lets go of them).
-static constexpr size_t kSpareBytes = 1ull << 30;
-
-static void release_spare(letkf_gpu_t* h) {
-  for (const auto& b : h->spare) hipFree(b.second);
-  h->spare.clear();
-  h->spare_bytes = 0;
+// later calls (SpareBlocks): 45 allocations and releases of an observation set
+// took 3.5 ms of the 7.6 that handing over 500 000 observations of k = 50
+// takes.  They count towards the limit, under which a block is only taken
+// again for its own size.  They are only kept once the handle's stream is
+// idle (a release waits for the device, so every call waits for its stream
+// before it lets go of them).  An allocation that fails takes back what the
+// handles on the device keep.
+static hipError_t fresh_alloc(letkf_gpu_t* h, void** p, size_t bytes) {
+  if (h->mem_limit && h->live_bytes + h->spare.bytes() + bytes > h->mem_limit) {
+    h->spare.release();
+    if (h->live_bytes + bytes > h->mem_limit) return hipErrorOutOfMemory;
+  }
+  hipError_t e = hipMalloc(p, bytes);
+  if (e != hipSuccess && SpareBlocks::release_device(h->device)) e = hipMalloc(p, bytes);
+  if (e != hipSuccess) (void)hipGetLastError();   // the caller has it
+  return e;
 }
 static hipError_t raw_alloc(letkf_gpu_t* h, void** p, size_t bytes, bool temp) {
-  if (h->mem_limit && h->live_bytes + bytes > h->mem_limit) return hipErrorOutOfMemory;
   size_t size = bytes;
   hipError_t e = hipSuccess;
-  // a kept block at most twice as large
-  auto it = temp ? h->spare.lower_bound(bytes) : h->spare.end();
-  if (it != h->spare.end() && it->first <= 2 * bytes + 4096) {
-    size = it->first;
-    *p = it->second;
-    h->spare_bytes -= size;
-    h->spare.erase(it);
-  } else {
-    e = hipMalloc(p, bytes);
-    if (e != hipSuccess && !h->spare.empty()) {
-      (void)hipGetLastError();
-      release_spare(h);
-      e = hipMalloc(p, bytes);
-    }
-  }
+  *p = temp ? h->spare.take(bytes, h->mem_limit ? bytes : 2 * bytes + 4096, &size) : nullptr;
+  if (!*p) e = fresh_alloc(h, p, bytes);
   if (e == hipSuccess) {
-    h->live[*p] = {bytes, size};
-    h->live_bytes += bytes;
+    h->live[*p] = size;
+    h->live_bytes += size;
+  } else {
+    *p = nullptr;
   }
   return e;
 }
@@ -313,16 +304,12 @@ static void raw_free(letkf_gpu_t* h, void* p, bool temp) {
   size_t size = 0;
   auto it = h->live.find(p);
   if (it != h->live.end()) {
-    size = it->second.size;
-    h->live_bytes -= it->second.asked;
+    size = it->second;
+    h->live_bytes -= size;
     h->live.erase(it);
   }
-  if (temp && size > 0 && h->spare_bytes + size <= kSpareBytes) {
-    h->spare.emplace(size, p);
-    h->spare_bytes += size;
-    return;
-  }
-  hipFree(p);
+  if (temp && size > 0) h->spare.keep(p, size);
+  else hipFree(p);
 }
 // a buffer pointer stored in the handle itself (not a local temporary)
 static bool handle_member(const letkf_gpu_t* h, const void* p) {
@@ -396,6 +383,7 @@ int letkf_gpu_create(const letkf_gpu_dims* d, letkf_gpu_t** out) {
   if (const char* e = getenv("LETKF_GPU_CHUNK_LOG2"))
     h->tune_chunk_log2 = std::min(20, std::max(17, atoi(e)));
   hipGetDevice(&h->device);
+  h->spare.set_device(h->device);
   h->d_scratch = scratch_address(h->device, &h->scratch_err);
   // both streams at the default priority
   if (hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking) != hipSuccess) {
@@ -454,7 +442,6 @@ int letkf_gpu_destroy(letkf_gpu_t* h) {
   if (h->h_ring) hipHostFree(h->h_ring);
   hipStreamDestroy(h->stream);
   hipStreamDestroy(h->stream2);
-  release_spare(h);
   delete h;
   return LETKF_OK;
 }
@@ -888,11 +875,7 @@ static int upload_flags(letkf_gpu_t* h) {
   const int64_t nvt = h->loc.cls == LETKF_LOC_VGAUSS ? h->obs_cap * h->loc.nlev : 0;
   if (nvt > 0 && nvt <= (1ll << 28)) {
     if (nvt != h->ovt_n) {
-      const hipError_t ea = dalloc(h, &h->d_ovt, (size_t)nvt);
-      if (ea != hipSuccess) {      // a full device: evaluated by the search
-        (void)hipGetLastError();
-        h->d_ovt = nullptr;
-      }
+      (void)dalloc(h, &h->d_ovt, (size_t)nvt);   // a full device: evaluated by the search
       h->ovt_n = h->d_ovt ? nvt : 0;
     }
     if (h->d_ovt && e == hipSuccess) {
