@@ -1,6 +1,8 @@
 """LETKF_GPU_MEM_LIMIT bounds all that a handle holds, the blocks it keeps
 between calls among it, and an analysis that fits the cap runs: the kept
-blocks make room for the lists and work arrays."""
+blocks and the table of vertical weights make room for the lists and work
+arrays.  Without the table the search evaluates the weights: the same lists
+and analysis bit for bit."""
 import numpy as np
 import pytest
 import torch
@@ -21,6 +23,27 @@ def _same(a, b):
         assert np.array_equal(x, y)
     for n in a[3]:
         assert np.array_equal(a[3][n], b[3][n])
+
+
+def test_weight_table_makes_room(monkeypatch):
+    """120 000 observations on 50 levels: 30 MB of weights, 235 MB of lists, 33 MB
+    of the rest and 15 MB of an upload's temporaries.  The cap holds all but the table."""
+    p = synth.random_problem(seed=5, nx=18, ny=9, k=4, ns=50, nobs=120000, radius=900e3,
+                             loc_cls="LOC_VGAUSS")
+    with LetkfGpuSolver(p, precision="fp64", path="plain") as s:
+        ref = _analyse(s)
+        ref_sel = s.selection(40, 7)
+    monkeypatch.setenv("LETKF_GPU_MEM_LIMIT", str(285 << 20))
+    with LetkfGpuSolver(p, precision="fp64", path="plain") as s:
+        print("capped", flush=True)
+        _same(_analyse(s), ref)
+        for a, b in zip(s.selection(40, 7), ref_sel):
+            assert np.array_equal(a, b)
+        s.cycle(p)
+        _same(_analyse(s), ref)
+        s.run_graph()
+        s.run_graph()
+        _same((*s.state_f64(), s.diag()), ref)
 
 
 def test_kept_blocks_count(monkeypatch):

@@ -274,8 +274,9 @@ static int fail(letkf_gpu_t* h, int code, const char* fmt, ...) {
 // takes.  They count towards the limit, under which a block is only taken
 // again for its own size.  They are only kept once the handle's stream is
 // idle (a release waits for the device, so every call waits for its stream
-// before it lets go of them).  An allocation that fails takes back what the
-// handles on the device keep.
+// before it lets go of them).  An allocation that fails takes back, in this
+// order, what the handles on the device keep, and this handle's table of
+// vertical weights, which the search can do without.
 static hipError_t fresh_alloc(letkf_gpu_t* h, void** p, size_t bytes) {
   if (h->mem_limit && h->live_bytes + h->spare.bytes() + bytes > h->mem_limit) {
     h->spare.release();
@@ -286,11 +287,15 @@ static hipError_t fresh_alloc(letkf_gpu_t* h, void** p, size_t bytes) {
   if (e != hipSuccess) (void)hipGetLastError();   // the caller has it
   return e;
 }
+static bool drop_weight_table(letkf_gpu_t* h);
 static hipError_t raw_alloc(letkf_gpu_t* h, void** p, size_t bytes, bool temp) {
   size_t size = bytes;
   hipError_t e = hipSuccess;
   *p = temp ? h->spare.take(bytes, h->mem_limit ? bytes : 2 * bytes + 4096, &size) : nullptr;
-  if (!*p) e = fresh_alloc(h, p, bytes);
+  if (!*p) {
+    e = fresh_alloc(h, p, bytes);
+    if (e != hipSuccess && drop_weight_table(h)) e = fresh_alloc(h, p, bytes);
+  }
   if (e == hipSuccess) {
     h->live[*p] = size;
     h->live_bytes += size;
@@ -333,6 +338,17 @@ template <typename T>
 static void dfree(letkf_gpu_t* h, T*& p) {
   raw_free(h, p, !handle_member(h, &p));
   p = nullptr;
+}
+// false if there was none; a search that is running has ended then, and what
+// is launched after takes the views' pointer anew
+static bool drop_weight_table(letkf_gpu_t* h) {
+  if (!h->d_ovt) return false;
+  hipStreamSynchronize(h->stream);
+  hipStreamSynchronize(h->stream2);
+  dfree(h, h->d_ovt);
+  h->ovt_n = 0;
+  ++h->gen;
+  return true;
 }
 
 extern "C" {
@@ -883,11 +899,8 @@ static int upload_flags(letkf_gpu_t* h) {
                     h->d_lev_depth, h->d_ovt);
       e = hipGetLastError();
     }
-  } else if (h->d_ovt) {
-    hipStreamSynchronize(h->stream);
-    dfree(h, h->d_ovt);
-    h->ovt_n = 0;
-    ++h->gen;
+  } else {
+    drop_weight_table(h);
   }
   hipStreamSynchronize(h->stream);
   dfree(h, so);
@@ -1246,7 +1259,7 @@ static int run_eager(letkf_gpu_t* h) {
   hipStream_t st = h->stream;
   const int64_t k = h->k, G = h->G;
 
-  const RunViews W = run_views(h);
+  RunViews W = run_views(h);
   const StateDev& S = W.S;
   const ObsDev& O = W.O;
   const VarsDev& V = W.V;
@@ -1347,6 +1360,7 @@ static int run_eager(letkf_gpu_t* h) {
       b_list_cap = cap;
       C.list_idx = b_list_idx;
       C.list_w = b_list_w;
+      W.O.vt = h->d_ovt;   // the lists may have taken its place
     }
     launch_search(sst, true, h->loc, O, S, V, C, D);
     RUNCHK(hipGetLastError());
@@ -1801,7 +1815,7 @@ int letkf_gpu_get_selection(letkf_gpu_t* h, int64_t ij, int32_t group, int32_t* 
   // re-run the search of the chunk that holds ij
   const int64_t i0 = ij;
   ChunkDev C{i0, 1, h->G, h->d_cnt, h->d_off, h->d_solve, h->d_list_idx, h->d_list_w, 0, 0};
-  const RunViews W = run_views(h);
+  RunViews W = run_views(h);
   const ObsDev& O = W.O;
   const StateDev& S = W.S;
   const VarsDev& V = W.V;
@@ -1825,6 +1839,7 @@ int letkf_gpu_get_selection(letkf_gpu_t* h, int64_t ij, int32_t group, int32_t* 
     h->list_cap = c2;
     C.list_idx = h->d_list_idx;
     C.list_w = h->d_list_w;
+    W.O.vt = h->d_ovt;
   }
   launch_search(st, true, h->loc, O, S, V, C, D);
   HIPCHK(h, hipGetLastError());
