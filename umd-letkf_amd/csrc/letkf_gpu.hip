@@ -753,6 +753,10 @@ static int set_obs_impl(letkf_gpu_t* h, int64_t n, const float* lat, const float
     n = nsel;
     nn = ns1;
   }
+  // from here on the old set is gone: have_obs is set again once the new one
+  // is whole (as have_vars and have_loc), and no run meets a buffer that an
+  // allocation failed for
+  h->have_obs = false;
   h->nobs = n;
   h->kp = (int)(((k + 1) + 31) / 32 * 32);
   if ((int64_t)nn > h->obs_cap) {
@@ -763,6 +767,7 @@ static int set_obs_impl(letkf_gpu_t* h, int64_t n, const float* lat, const float
     const int64_t cap = std::max<int64_t>((int64_t)nn,
                                           std::min<int64_t>((int64_t)nn + (int64_t)nn / 4, lim));
     const size_t c = (size_t)cap;
+    h->obs_cap = 0;
     OBSCHK(dalloc(h, &h->d_opos, 2 * c));
     OBSCHK(dalloc(h, &h->d_ozdim, c)); OBSCHK(dalloc(h, &h->d_oerr, c)); OBSCHK(dalloc(h, &h->d_odep, c));
     OBSCHK(dalloc(h, &h->d_otime, c)); OBSCHK(dalloc(h, &h->d_oidx, c)); OBSCHK(dalloc(h, &h->d_oobsid, c));
@@ -791,8 +796,8 @@ static int set_obs_impl(letkf_gpu_t* h, int64_t n, const float* lat, const float
   OBSCHK(hipStreamSynchronize(st));
   cleanup();
 #undef OBSCHK
+  if (h->have_loc && (rc = upload_flags(h)) != LETKF_OK) return rc;
   h->have_obs = true;
-  if (h->have_loc) return upload_flags(h);
   return LETKF_OK;
 }
 
@@ -829,6 +834,7 @@ static void build_interp(const letkf_linearinterp_lat& c, int* n, float* lat, fl
 }
 
 static int rebuild_slabs(letkf_gpu_t* h) {
+  h->have_vars = false;
   std::vector<int32_t> sv(h->ns, -1), sl(h->ns, 0);
   int maxlev = 1;
   for (int v = 0; v < h->nvars; ++v) {
@@ -843,6 +849,7 @@ static int rebuild_slabs(letkf_gpu_t* h) {
   HIPCHK(h, dalloc(h, &h->d_slab_lev, (size_t)h->ns));
   HIPCHK(h, hipMemcpy(h->d_slab_var, sv.data(), 4 * h->ns, hipMemcpyHostToDevice));
   HIPCHK(h, hipMemcpy(h->d_slab_lev, sl.data(), 4 * h->ns, hipMemcpyHostToDevice));
+  h->have_vars = true;
   return LETKF_OK;
 }
 
@@ -858,6 +865,7 @@ int letkf_gpu_set_statevars(letkf_gpu_t* h, int32_t nvars, const int32_t* s_idx,
                   s_idx[v], s_idx[v] + levels[v], (long long)h->ns);
   }
   h->have_run = false;
+  h->have_vars = false;
   ++h->gen;
   h->nvars = nvars;
   h->var_s.assign(s_idx, s_idx + nvars);
@@ -868,24 +876,23 @@ int letkf_gpu_set_statevars(letkf_gpu_t* h, int32_t nvars, const int32_t* s_idx,
     HIPCHK(h, hipMemcpy(h->d_inc_max, inc_max, 4 * nvars, hipMemcpyHostToDevice));
     HIPCHK(h, hipMemcpy(h->d_bounds, bounds, 8 * nvars, hipMemcpyHostToDevice));
   }
-  int rc = rebuild_slabs(h);
-  if (rc) return rc;
-  h->have_vars = true;
-  return LETKF_OK;
+  return rebuild_slabs(h);
 }
 
 static int upload_flags(letkf_gpu_t* h) {
   int32_t *so = nullptr, *sp = nullptr;
-  HIPCHK(h, dalloc(h, &so, std::max<size_t>(h->sat_obs.size(), 1)));
-  HIPCHK(h, dalloc(h, &sp, std::max<size_t>(h->sat_plats.size(), 1)));
-  if (!h->sat_obs.empty())
-    HIPCHK(h, hipMemcpy(so, h->sat_obs.data(), 4 * h->sat_obs.size(), hipMemcpyHostToDevice));
-  if (!h->sat_plats.empty())
-    HIPCHK(h, hipMemcpy(sp, h->sat_plats.data(), 4 * h->sat_plats.size(), hipMemcpyHostToDevice));
-  launch_obs_flags(h->stream, h->loc, h->nobs, h->d_oobsid, h->d_oplatid, h->d_otime, so,
-                   (int)h->sat_obs.size(), sp, (int)h->sat_plats.size(), h->d_osurf,
-                   h->d_otwp, h->d_otws);
-  hipError_t e = hipGetLastError();
+  hipError_t e = dalloc(h, &so, std::max<size_t>(h->sat_obs.size(), 1));
+  if (e == hipSuccess) e = dalloc(h, &sp, std::max<size_t>(h->sat_plats.size(), 1));
+  if (e == hipSuccess && !h->sat_obs.empty())
+    e = hipMemcpy(so, h->sat_obs.data(), 4 * h->sat_obs.size(), hipMemcpyHostToDevice);
+  if (e == hipSuccess && !h->sat_plats.empty())
+    e = hipMemcpy(sp, h->sat_plats.data(), 4 * h->sat_plats.size(), hipMemcpyHostToDevice);
+  if (e == hipSuccess) {
+    launch_obs_flags(h->stream, h->loc, h->nobs, h->d_oobsid, h->d_oplatid, h->d_otime, so,
+                     (int)h->sat_obs.size(), sp, (int)h->sat_plats.size(), h->d_osurf,
+                     h->d_otwp, h->d_otws);
+    e = hipGetLastError();
+  }
   // LOC_VGAUSS: a table of the vertical weights, up to 1 GiB of it (the
   // search evaluates them otherwise)
   const int64_t nvt = h->loc.cls == LETKF_LOC_VGAUSS ? h->obs_cap * h->loc.nlev : 0;
@@ -968,15 +975,16 @@ int letkf_gpu_set_localizer(letkf_gpu_t* h, const letkf_loc_desc* d) {
   L.max_var_lev = h->loc.max_var_lev > 0 ? h->loc.max_var_lev : 1;
   h->sat_obs.assign(d->sat_obs, d->sat_obs + (d->cls == LETKF_LOC_OCEAN ? d->n_sat_obs : 0));
   h->sat_plats.assign(d->sat_plats, d->sat_plats + (d->cls == LETKF_LOC_OCEAN ? d->n_sat_plats : 0));
+  h->have_loc = false;
   if (d->cls == LETKF_LOC_VGAUSS) {
     HIPCHK(h, dalloc(h, &h->d_lev_depth, (size_t)d->nlev));
     HIPCHK(h, hipMemcpy(h->d_lev_depth, d->lev_depth, 4 * d->nlev, hipMemcpyHostToDevice));
   }
   h->loc = L;
   h->G = L.maxgroups;
+  if (h->have_vars && (rc = rebuild_slabs(h)) != LETKF_OK) return rc;
+  if (h->have_obs && (rc = upload_flags(h)) != LETKF_OK) return rc;
   h->have_loc = true;
-  if (h->have_vars) { rc = rebuild_slabs(h); if (rc) return rc; }
-  if (h->have_obs) return upload_flags(h);
   return LETKF_OK;
 }
 
@@ -1037,15 +1045,13 @@ static hipcub::TransformInputIterator<int64_t, PadCount, const int64_t*> padded_
 
 static int ensure_outputs(letkf_gpu_t* h) {
   const int64_t k = h->k, ns = h->ns, nij = h->nij, G = h->G;
-  if (!h->d_ana) {
-    HIPCHK(h, dalloc(h, &h->d_ana, (size_t)(k * ns * nij)));
-    HIPCHK(h, dalloc(h, &h->d_amean, (size_t)(ns * nij)));
-    HIPCHK(h, dalloc(h, &h->d_asprd, (size_t)(ns * nij)));
-    HIPCHK(h, dalloc(h, &h->d_maxhz, (size_t)nij));
-    HIPCHK(h, dalloc(h, &h->d_obscount, (size_t)nij));
-    HIPCHK(h, dalloc(h, &h->d_mld, (size_t)nij));
-    HIPCHK(h, dalloc(h, &h->d_ctr, (size_t)kCtrSlots * kCtrStride));
-  }
+  HIPCHK(h, dalloc_once(h, &h->d_ana, (size_t)(k * ns * nij)));
+  HIPCHK(h, dalloc_once(h, &h->d_amean, (size_t)(ns * nij)));
+  HIPCHK(h, dalloc_once(h, &h->d_asprd, (size_t)(ns * nij)));
+  HIPCHK(h, dalloc_once(h, &h->d_maxhz, (size_t)nij));
+  HIPCHK(h, dalloc_once(h, &h->d_obscount, (size_t)nij));
+  HIPCHK(h, dalloc_once(h, &h->d_mld, (size_t)nij));
+  HIPCHK(h, dalloc_once(h, &h->d_ctr, (size_t)kCtrSlots * kCtrStride));
   // LETKF_GPU_EIGEN=jacobi selects the parallel Jacobi solver for every
   // problem (reference solver for tests); default: tridiagonal QL pipeline
   const char* ev = getenv("LETKF_GPU_EIGEN");
@@ -1058,6 +1064,7 @@ static int ensure_outputs(letkf_gpu_t* h) {
   if (h->alloc_G == G && h->eigK == eigK && h->alloc_nv == nv && h->alloc_mat == (int)use_mat &&
       h->alloc_chunk == h->tune_chunk_log2)
     return LETKF_OK;
+  h->alloc_G = -1;   // until every buffer below is there
   h->eigK = eigK;
   h->vec_nv = nv;
   h->use_mat = use_mat;
@@ -1125,10 +1132,10 @@ static int ensure_outputs(letkf_gpu_t* h) {
     HIPCHK(h, dalloc(h, (char**)&h->d_stmp, sb));
     h->stmp_bytes = sb;
   }
-  if ((h->use_rat || h->use_mat) && !h->d_rat) {
+  if ((h->use_rat || h->use_mat) && (!h->d_rat || !h->d_ratn)) {
     const RatTables& T = rat_tables();
-    HIPCHK(h, dalloc(h, &h->d_rat, T.tab.size()));
-    HIPCHK(h, dalloc(h, &h->d_ratn, T.n.size()));
+    HIPCHK(h, dalloc_once(h, &h->d_rat, T.tab.size()));
+    HIPCHK(h, dalloc_once(h, &h->d_ratn, T.n.size()));
     HIPCHK(h, hipMemcpy(h->d_rat, T.tab.data(), 8 * T.tab.size(), hipMemcpyHostToDevice));
     HIPCHK(h, hipMemcpy(h->d_ratn, T.n.data(), 4 * T.n.size(), hipMemcpyHostToDevice));
   }
@@ -1355,6 +1362,7 @@ static int run_eager(letkf_gpu_t* h) {
       // this set's previous chunk is finished (the search stream waited for it);
       // a quarter of headroom, half for a run that sizes a graph capture
       const int64_t cap = total + total / (h->list_headroom_div) + 1024;
+      b_list_cap = 0;
       RUNCHK(dalloc(h, &b_list_idx, (size_t)cap));
       RUNCHK(dalloc(h, &b_list_w, (size_t)cap));
       b_list_cap = cap;
@@ -1834,6 +1842,7 @@ int letkf_gpu_get_selection(letkf_gpu_t* h, int64_t ij, int32_t group, int32_t* 
   const int64_t total = h->h_tot[2] + PadCount()(h->h_tot[3]) + kListAlign;
   if (total > h->list_cap) {
     const int64_t c2 = total + 1024;
+    h->list_cap = 0;
     HIPCHK(h, dalloc(h, &h->d_list_idx, (size_t)c2));
     HIPCHK(h, dalloc(h, &h->d_list_w, (size_t)c2));
     h->list_cap = c2;
