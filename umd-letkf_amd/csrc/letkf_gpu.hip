@@ -153,6 +153,8 @@ struct letkf_gpu_t {
   // blocks of temporaries kept for the next call
   SpareBlocks spare{[](void* p) { hipFree(p); }};
   size_t mem_limit = 0;   // 0 = none
+  size_t locked_limit = ~(size_t)0;   // page-locked memory that can be done without
+  size_t locked_bytes = 0;            // h_ring and h_diag
   int tune_xcd = 4;       // product kernels: runs of 256 problems per XCD
   int tune_tile = 1;      // batched product: 0 32x32 MFMA blocks, 1 16x16 tiles
                           // (where that kernel exists)
@@ -383,6 +385,7 @@ int letkf_gpu_create(const letkf_gpu_dims* d, letkf_gpu_t** out) {
   h->ns = d->grid_ns;
   h->nij = d->ij_count;
   if (const char* e = getenv("LETKF_GPU_MEM_LIMIT")) h->mem_limit = strtoull(e, nullptr, 10);
+  if (const char* e = getenv("LETKF_GPU_LOCKED_LIMIT")) h->locked_limit = strtoull(e, nullptr, 10);
   if (const char* e = getenv("LETKF_GPU_XCD")) h->tune_xcd = std::min(kXcdModes - 1, std::max(0, atoi(e)));
   if (const char* e = getenv("LETKF_GPU_FOLD")) h->fold_log2 = std::min(10, std::max(5, atoi(e)));
   if (const char* e = getenv("LETKF_GPU_TILE")) h->tune_tile = atoi(e) != 0;
@@ -491,6 +494,21 @@ static bool runtime_knows(const void* p) {
   return a.type != hipMemoryTypeUnregistered;
 }
 
+// bytes of page-locked memory for *p, or false: the caller has a way without
+// it.  LETKF_GPU_LOCKED_LIMIT (bytes, read at create) bounds what a handle
+// takes, as a machine that gives no more would.
+static bool locked_alloc(letkf_gpu_t* h, void** p, size_t bytes) {
+  *p = nullptr;
+  if (bytes > h->locked_limit - std::min(h->locked_limit, h->locked_bytes)) return false;
+  if (hipHostMalloc(p, bytes, hipHostMallocDefault) != hipSuccess) {
+    (void)hipGetLastError();
+    *p = nullptr;
+    return false;
+  }
+  h->locked_bytes += bytes;
+  return true;
+}
+
 // A large copy from the device on h->stream to pageable host memory.  The
 // runtime's own way is one thread's: 54 MB into memory touched for the first
 // time took 5.3 ms, 2.6 of them page faults.  Here kRingThreads threads take
@@ -512,12 +530,8 @@ static hipError_t bulk_fetch(letkf_gpu_t* h, void* dst, const void* src, size_t 
   if (bytes < kRingLeast || runtime_knows(dst) || runtime_knows((char*)dst + bytes - 1) ||
       hipGetDevice(&dev) != hipSuccess)
     return hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st);
-  if (!h->h_ring && hipHostMalloc((void**)&h->h_ring, kRingThreads * kRingSlots * kRingBytes,
-                                  hipHostMallocDefault) != hipSuccess) {
-    (void)hipGetLastError();
-    h->h_ring = nullptr;
+  if (!h->h_ring && !locked_alloc(h, (void**)&h->h_ring, kRingThreads * kRingSlots * kRingBytes))
     return hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st);
-  }
   const size_t np = (bytes + kRingBytes - 1) / kRingBytes;
   std::atomic<size_t> next{0};
   std::atomic<int> err{(int)hipSuccess};
@@ -1764,15 +1778,15 @@ int letkf_gpu_get_diag(letkf_gpu_t* h, const letkf_gpu_diag* d) {
   // small fields: put in the reference's layout by one kernel that writes
   // them to page-locked memory, where five copies would each be waited for.
   // Above kDiagBytes the copies' own time counts, and the memory they need.
+  // Without the page-locked memory the copies serve small fields too.
   const size_t bytes = (size_t)nij * (8 + 16 * (size_t)G);
-  if (nij * G > 0 && bytes <= kDiagBytes) {
-    if (h->diag_bytes < bytes) {
-      if (h->h_diag) hipHostFree(h->h_diag);
-      h->h_diag = nullptr;
-      h->diag_bytes = 0;
-      HIPCHK(h, hipHostMalloc(&h->h_diag, bytes, hipHostMallocDefault));
-      h->diag_bytes = bytes;
-    }
+  const bool small = nij * G > 0 && bytes <= kDiagBytes;
+  if (small && h->diag_bytes < bytes) {
+    if (h->h_diag) hipHostFree(h->h_diag);
+    h->locked_bytes -= h->diag_bytes;
+    h->diag_bytes = locked_alloc(h, &h->h_diag, bytes) ? bytes : 0;
+  }
+  if (small && h->h_diag) {
     uint64_t* hash = (uint64_t*)h->h_diag;
     float* f = (float*)(hash + nij * G);
     launch_diag_to_host(h->stream, nij, G, run_views(h).D, hash, f);
