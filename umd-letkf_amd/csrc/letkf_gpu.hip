@@ -27,7 +27,7 @@
 #include "det_math.h"
 #include "host_memory.h"
 #include "letkf_internal.h"
-#include "ratnodes.h"
+#include "ratnodes_table.h"
 #include "spare_blocks.h"
 
 using namespace lk;
@@ -179,33 +179,6 @@ struct letkf_gpu_t {
     return dims.path == LETKF_PATH_BATCHED && dims.precision != LETKF_PREC_FP64;
   }
 };
-
-// The node tables (RatTab): coarse (1e-12, at most 31 nodes) in rows
-// 0..kRatBuckets-1, fine (5e-16, at most 62) in the rows after; where no node
-// count meets the tolerance, the most.  Constants, built at first use: about
-// 30 ms, which every handle paid before.
-struct RatTables {
-  std::vector<double> tab;
-  std::vector<int> n;
-  RatTables() : tab((size_t)2 * kRatBuckets * kRatLd, 0.0), n((size_t)2 * kRatBuckets, 0) {
-    for (int b = 1; b < kRatBuckets; ++b) {
-      const double kappa = std::ldexp(1.0, b);
-      double* s = tab.data() + (size_t)b * kRatLd;
-      double* w = s + kRatLd / 2;
-      int m = rat::choose(kappa, 1e-12, 31, s, w, std::min(31, rat::fewest(kappa, 1e-12)));
-      if (m < 0) { m = 31; rat::nodes(kappa, m, s, w); }
-      n[(size_t)b] = m;
-      s += (size_t)kRatBuckets * kRatLd;
-      w += (size_t)kRatBuckets * kRatLd;
-      m = rat::choose_fine(kappa, 5e-16, 62, s, w);
-      n[(size_t)(kRatBuckets + b)] = m < 0 ? 62 : m;   // s and w hold 62 then
-    }
-  }
-};
-static const RatTables& rat_tables() {
-  static const RatTables t;
-  return t;
-}
 
 static std::string g_create_err;
 
@@ -1147,11 +1120,10 @@ static int ensure_outputs(letkf_gpu_t* h) {
     h->stmp_bytes = sb;
   }
   if ((h->use_rat || h->use_mat) && (!h->d_rat || !h->d_ratn)) {
-    const RatTables& T = rat_tables();
-    HIPCHK(h, dalloc_once(h, &h->d_rat, T.tab.size()));
-    HIPCHK(h, dalloc_once(h, &h->d_ratn, T.n.size()));
-    HIPCHK(h, hipMemcpy(h->d_rat, T.tab.data(), 8 * T.tab.size(), hipMemcpyHostToDevice));
-    HIPCHK(h, hipMemcpy(h->d_ratn, T.n.data(), 4 * T.n.size(), hipMemcpyHostToDevice));
+    HIPCHK(h, dalloc_once(h, &h->d_rat, sizeof kRatTab / sizeof kRatTab[0]));
+    HIPCHK(h, dalloc_once(h, &h->d_ratn, sizeof kRatN / sizeof kRatN[0]));
+    HIPCHK(h, hipMemcpy(h->d_rat, kRatTab, sizeof kRatTab, hipMemcpyHostToDevice));
+    HIPCHK(h, hipMemcpy(h->d_ratn, kRatN, sizeof kRatN, hipMemcpyHostToDevice));
   }
   h->alloc_G = G;
   h->alloc_nv = nv;

@@ -6,6 +6,7 @@
 #include <stdint.h>
 
 #include "../../include/letkf_gpu.h"
+#include "rat_table.h"
 
 namespace lk {
 
@@ -258,17 +259,12 @@ bool product_t16_supported(int prec, int k);
 void launch_bucket_keys(hipStream_t st, int mode, int bbits, int64_t np, int G, int64_t i0,
                         const int64_t* cnt, const uint8_t* solve, const float* lat,
                         const float* lon, uint32_t* keys, int32_t* vals);
-// node tables of the rational approximation of x^(-1/2) on [1, 2^b]: nodes
-// tab[b * kRatLd + j] and weights tab[b * kRatLd + kRatLd / 2 + j], j < n[b].
-// The coarse table has 1e-12 relative error and at most 31 nodes, the fine
-// one 5e-16 and at most 62 (RatTables in letkf_gpu.hip).
+// a node table on the device (rat_table.h)
 struct RatTab {
   const double* tab = nullptr;
   const int* n = nullptr;
   int nb = 0;                 // 0: not used
 };
-constexpr int kRatBuckets = 48;
-constexpr int kRatLd = 128;
 // register-resident tridiagonalization for rows of KQ (a multiple of 8,
 // k <= KQ <= 64); false if no kernel exists for (KQ, NV)
 bool launch_tridiag_reg(hipStream_t st, unsigned nb, int KQ, int NV, int k, int K,

@@ -1,6 +1,8 @@
 """Build libletkf_gpu.so in-tree with hipcc for gfx950, and the Fortran host.
 
-Every .hip source under ``umd-letkf_amd/csrc`` is compiled to an object in
+``gen_ratnodes.cpp`` is compiled and run first: it writes the node tables as
+constants into ``umd-letkf_amd/_build/ratnodes_table.h``.  Then every .hip
+source under ``umd-letkf_amd/csrc`` is compiled to an object in
 ``umd-letkf_amd/_build`` (in parallel) and linked into
 ``umd-letkf_amd/letkf_amd/libletkf_gpu.so``.  ``build_fortran`` compiles the
 iso_c_binding module, the solver host module and the stand-alone driver in
@@ -27,6 +29,7 @@ FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wno-unused-command-line-argument",
     "-munsafe-fp-atomics",
+    f"-I{BUILD}",
 ]
 
 
@@ -44,6 +47,25 @@ EXTRA = {f"tridiag_reg_kq{kq}.hip": ["-mllvm", "-pragma-unroll-threshold=2000000
          for kq in (32, 40, 48, 50, 56, 64)}
 EXTRA.update({f"tridiag_pair_kq{kq}.hip": ["-mllvm", "-pragma-unroll-threshold=2000000"]
               for kq in (8, 16, 24, 32, 40, 48, 50, 56, 64)})
+
+
+def generate(build_dir: str = BUILD) -> str:
+    """Write the node tables (ratnodes_table.h); the file is left alone where
+    it would not change, so that nothing is compiled again for it."""
+    os.makedirs(build_dir, exist_ok=True)
+    exe = os.path.join(build_dir, "gen_ratnodes")
+    r = subprocess.run([hipcc(), "-x", "c++", "-O2", "-std=c++17",
+                        os.path.join(CSRC, "gen_ratnodes.cpp"), "-o", exe],
+                       capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"gen_ratnodes.cpp:\n{r.stderr[-4000:]}")
+    text = subprocess.run([exe], check=True, capture_output=True, text=True).stdout
+    out = os.path.join(build_dir, "ratnodes_table.h")
+    if not os.path.exists(out) or open(out).read() != text:
+        with open(out + ".tmp", "w") as f:
+            f.write(text)
+        os.replace(out + ".tmp", out)
+    return out
 
 
 def _compile(src: str) -> str:
@@ -64,9 +86,9 @@ def _stale(src: str, newest_header: float) -> bool:
 def build(verbose: bool = True, force: bool = True) -> str:
     """Compile and link the library; force=False recompiles only sources
     older than their object or than the newest header."""
-    os.makedirs(BUILD, exist_ok=True)
+    table = generate()
     srcs = sorted(glob.glob(os.path.join(CSRC, "*.hip")))
-    headers = glob.glob(os.path.join(CSRC, "*.h")) + glob.glob(
+    headers = [table] + glob.glob(os.path.join(CSRC, "*.h")) + glob.glob(
         os.path.join(ROOT, "..", "include", "*.h"))
     newest = max((os.path.getmtime(h) for h in headers), default=0.0)
     todo = [s for s in srcs if force or _stale(s, newest)]
