@@ -458,8 +458,8 @@ hipError_t launch_eigen_apply_f64(hipStream_t st, const LocDev& L, const StateDe
 // A sum is NJ - 1 additions and four DPP rotations, and the roots and
 // divisions serve four slabs (with one slab a wave, 250 instructions each,
 // the instructions bounded it: 684 us at 1.04e6 slabs of k = 50, 397 us at
-// 810 000 of k = 40, against 150 and 80 us of memory traffic; now 286 and
-// 186 us).  Small grids: one slab's latency instead of a gridpoint's slabs
+// 810 000 of k = 40, against 150 and 80 us of memory traffic; now 279 and
+// 173 us).  Small grids: one slab's latency instead of a gridpoint's slabs
 // in turn.
 //
 // A run of slabs is looked over first, a lane each: which are solved,
@@ -495,30 +495,40 @@ __global__ __launch_bounds__(256) void k_finalize(LocDev L, StateDev S, VarsDev 
   const uint64_t b_solved = __ballot(solved), b_masked = __ballot(masked), b_need = __ballot(need);
   const double dk = (double)k, dk1 = (double)(k - 1);
   const int i = lane & 15;
-  for (int q = 0; q < run; q += 4) {
-    if (((b_need >> q) & 15) == 0) continue;          // wave-uniform
+  // passes of masked slabs alone are a copy, and out of the loop below, where
+  // the copy cost every other pass 5% (1.04e6 slabs of k = 50 without masks 293 us;
+  // 277 without the copy, 279 this way; 810 000 of k = 40, 30% masked: 184, 195 and
+  // 173)
+  uint64_t todo = b_need;
+  for (int q = 0; q < run && (b_need & b_masked) != 0; q += 4) {
+    const uint32_t nd = (uint32_t)(b_need >> q) & 15u, mk = (uint32_t)(b_masked >> q) & 15u;
+    if (nd == 0 || (nd & ~mk) != 0) continue;         // wave-uniform
+    todo &= ~(15ull << q);
     const int at = q + (lane >> 4);
-    const bool on = (b_need >> at) & 1, sol = (b_solved >> at) & 1, msk = (b_masked >> at) & 1;
+    if (((b_need >> at) & 1) == 0) continue;
+    const int64_t e = C.i0 * S.ns + u0 + at;
+    const float* xb = S.state + e * k;
+    double* xa = ana + e * k;
+    float c[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) c[j] = xb[min(i + 16 * j, k - 1)];
+    const float cm = S.mean[e], cs = S.sprd[e];
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+      if (i + 16 * j < k) xa[i + 16 * j] = (double)c[j];
+    if (i == 0) {
+      amean[e] = (double)cm;
+      asprd[e] = (double)cs;
+    }
+  }
+  for (int q = 0; q < run; q += 4) {
+    if (((todo >> q) & 15) == 0) continue;            // wave-uniform
+    const int at = q + (lane >> 4);
+    const bool on = (todo >> at) & 1, sol = (b_solved >> at) & 1, msk = (b_masked >> at) & 1;
     const int s = __shfl(s_own, at, 64);
     const int64_t e = C.i0 * S.ns + u0 + at;          // slab of the whole grid
     const float* xb = S.state + e * k;
     double* xa = ana + e * k;
-    if ((((b_need & ~b_masked) >> q) & 15) == 0) {    // masked gridpoints alone: a copy
-      if (on) {
-        float c[NJ];
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) c[j] = xb[min(i + 16 * j, k - 1)];
-        const float cm = S.mean[e], cs = S.sprd[e];
-#pragma unroll
-        for (int j = 0; j < NJ; ++j)
-          if (i + 16 * j < k) xa[i + 16 * j] = (double)c[j];
-        if (i == 0) {
-          amean[e] = (double)cm;
-          asprd[e] = (double)cs;
-        }
-      }
-      continue;
-    }
     double x[NJ];
     float b[NJ];
     if (on) {
