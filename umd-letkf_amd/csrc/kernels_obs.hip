@@ -91,23 +91,45 @@ void launch_gather_cols(hipStream_t st, int64_t n, int k, const int32_t* perm, c
 
 // operand columns of the products: hxp(kp, n) in search order, rows 0..k-1
 // the hx perturbations, row k the departure, rows above zero, so a column can
-// be read without row tests.  Entry (kp / 16) i + t holds row 16 t + i: lane i
-// of a 16-row operand reads its rows of all row tiles as one run.
-__global__ void k_obs_pad_hx(int64_t n, int k, int kp, const float* __restrict__ ohx,
+// be read without row tests; their order in a column: column_entry
+__global__ void k_obs_pad_hx(int64_t n, int k, int kp, int kt, const float* __restrict__ ohx,
                              const float* __restrict__ odep, float* hxp) {
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= n * kp) return;
   const int64_t s = e / kp;
-  const int at = (int)(e - s * kp), kt = kp >> 4;
-  const int a = 16 * (at % kt) + at / kt;
+  const int at = (int)(e - s * kp);
+  const int a = kt == 1 ? at : 16 * (at % kt) + at / kt;
   hxp[e] = a < k ? ohx[s * k + a] : (a == k ? odep[s] : 0.0f);
 }
 
-void launch_obs_pad_hx(hipStream_t st, int64_t n, int k, int kp, const float* ohx,
+void launch_obs_pad_hx(hipStream_t st, int64_t n, int k, int kp, int kt, const float* ohx,
                        const float* odep, float* hxp) {
   if (n <= 0) return;
   const int64_t tot = n * kp;
-  k_obs_pad_hx<<<(unsigned)((tot + 255) / 256), 256, 0, st>>>(n, k, kp, ohx, odep, hxp);
+  k_obs_pad_hx<<<(unsigned)((tot + 255) / 256), 256, 0, st>>>(n, k, kp, kt, ohx, odep, hxp);
+}
+
+// a block's columns through LDS; only a change of the launch choices between
+// two runs on the same observations calls for it
+constexpr int kReorderCols = 32;
+__global__ __launch_bounds__(256) void k_obs_reorder(int64_t n, int kp, int from, int to,
+                                                     float* __restrict__ hxp) {
+  __shared__ float col[kReorderCols * kMaxK];
+  const int64_t s0 = (int64_t)blockIdx.x * kReorderCols;
+  const int m = (int)min((int64_t)kReorderCols, n - s0) * kp;
+  float* p = hxp + s0 * kp;
+  for (int e = threadIdx.x; e < m; e += 256) col[e] = p[e];
+  __syncthreads();
+  for (int e = threadIdx.x; e < m; e += 256) {
+    const int c = e / kp, row = e % kp;
+    p[c * kp + column_entry(row, to)] = col[c * kp + column_entry(row, from)];
+  }
+}
+
+void launch_obs_reorder(hipStream_t st, int64_t n, int kp, int from, int to, float* hxp) {
+  if (n <= 0 || from == to) return;
+  k_obs_reorder<<<(unsigned)((n + kReorderCols - 1) / kReorderCols), 256, 0, st>>>(n, kp, from, to,
+                                                                                 hxp);
 }
 
 // cell_start[c] = first sorted obs with cell >= c (c = 0..kCells)

@@ -145,11 +145,14 @@ __device__ __forceinline__ void load_cols(MxFrag<NB>& F, __amdgpu_buffer_rsrc_t 
       F.w[4 + e] = __uint_as_float(b1[e]);
     }
   }
-  // row slot i of block rb is row 16 (NB (i / 16) + rb) + i % 16 (mx_row): a
-  // lane's NB rows follow one another in a column
-  const uint32_t i4 = 4u * NB * (uint32_t)(2 * (i & 15) + (i >> 4));
+  // row 32 rb + i in lane i of a half: columns row by row
 #pragma unroll
-  for (int e = 0; e < 8; ++e) load_run<NB>(F.y, e, hxr, Lr.sidx[e] + i4);
+  for (int e = 0; e < 8; ++e) {
+    const uint32_t vo = Lr.sidx[e] + 4u * (uint32_t)i;
+#pragma unroll
+    for (int rb = 0; rb < NB; ++rb)
+      F.y[rb][e] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(hxr, vo, 128 * rb, 0));
+  }
 }
 
 // acc += the products of one 16-observation step
@@ -228,12 +231,6 @@ __device__ __forceinline__ void mx_fold(f32x16* acc, f32x4* Sl) {
     }
 }
 
-// the row in slot i of row block rb (load_cols)
-template <int NB>
-__device__ __forceinline__ int mx_row(int rb, int i) {
-  return 16 * (NB * (i >> 4) + rb) + (i & 15);
-}
-
 template <int KP, int PREC>
 __global__ __launch_bounds__(64) void k_product_mx(ObsDev O, int k, ChunkDev C,
                                                    const int32_t* __restrict__ perm,
@@ -307,8 +304,8 @@ __global__ __launch_bounds__(64) void k_product_mx(ObsDev O, int k, ChunkDev C,
     for (int cb = rb; cb < NB; ++cb, ++b) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const int row = mx_row<NB>(rb, 8 * (r >> 2) + 4 * half + (r & 3));
-        const int col = mx_row<NB>(cb, i);
+        const int row = 32 * rb + 8 * (r >> 2) + 4 * half + (r & 3);
+        const int col = 32 * cb + i;
         double v = (double)acc[b][r];
         if (COMP) v += (double)Ssh[64 * (4 * b + (r >> 2)) + lane][r & 3];
         if (row < k && col < k) {
@@ -316,8 +313,6 @@ __global__ __launch_bounds__(64) void k_product_mx(ObsDev O, int k, ChunkDev C,
           Bp[col + (int64_t)k * row] = v;
         } else if (col == k && row < k) {
           bp[row] = v;
-        } else if (row == k && col < k) {
-          bp[col] = v;
         }
       }
     }
@@ -405,7 +400,7 @@ __device__ __forceinline__ void t16_cols(T16Frag<NT>& F, __amdgpu_buffer_rsrc_t 
                                          __amdgpu_buffer_rsrc_t wr, uint32_t idx, int j0,
                                          int lane) {
   F.w = __uint_as_float(t16_list(wr, j0, lane));
-  constexpr uint32_t KT = (NT + 1) & ~1;                // rows 16 t + i are entries KT i + t
+  constexpr uint32_t KT = NT == 1 ? 1 : (NT + 1) & ~1;   // rows 16 t + i are entries KT i + t
   const uint32_t i4 = 4u * KT * (uint32_t)(lane & 15);
   uint32_t vo[8];
   row8_add(vo, idx, i4);

@@ -76,12 +76,13 @@ __device__ __forceinline__ void product_tiles(const ObsDev& O, const int32_t* __
                                               int lane, double4_t (&acc)[N]) {
   const int q = lane >> 4;
   // entry KT i + b of a column is row 16 b + i: a lane's rows are one run
-  constexpr int KT = (NB + 1) & ~1;
+  constexpr int KT = NB == 1 ? 1 : (NB + 1) & ~1;
   const float* __restrict__ col = O.hxp + KT * (lane & 15);
   const int64_t kp = O.kp;
   auto idx_at = [&](int64_t j) { return li[j + lane < m ? j + lane : 0]; };
   auto load = [&](int32_t id, float (&y)[NB]) __attribute__((always_inline)) {
     const float* c = col + (int64_t)id * kp;
+    if constexpr (NB == 1) y[0] = *c;
     static_for<KT / 2>([&](auto I) __attribute__((always_inline)) {
       constexpr int b = 2 * decltype(I)::value;
       if constexpr (tile_reads<NB, T0, N>(b) || (b + 1 < NB && tile_reads<NB, T0, N>(b + 1))) {

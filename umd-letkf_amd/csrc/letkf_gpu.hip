@@ -59,6 +59,7 @@ struct letkf_gpu_t {
   float* d_ohx = nullptr;
   float* d_ohxp = nullptr;   // padded operand columns (kp, n)
   int kp = 0;
+  int cols_kt = 0;           // the order of its rows (column_entry)
   int32_t* d_cell_start = nullptr;
   uint8_t* d_osurf = nullptr;
   float *d_otwp = nullptr, *d_otws = nullptr;
@@ -637,6 +638,14 @@ int letkf_gpu_set_state(letkf_gpu_t* h, const float* state_ij, const float* mean
 
 static int upload_flags(letkf_gpu_t* h);
 
+// the order of a column's rows that the products of the next run read
+static int columns_wanted(const letkf_gpu_t* h) {
+  const int k = (int)h->k;
+  const bool rows = h->batched() &&
+                    !(h->tune_tile == 1 && product_t16_supported(h->dims.precision, k));
+  return rows ? 1 : tiled_columns(k);
+}
+
 // n input observations from host arrays.  With qc and hx_full (the members'
 // hx, (k, n)) the mean / perturbation split and the QC compaction of
 // letkf_obs_read run on the device first; otherwise hx_pert and hx_mean are
@@ -778,7 +787,8 @@ static int set_obs_impl(letkf_gpu_t* h, int64_t n, const float* lat, const float
                     r_obsid, r_platid, r_hx, r_hxm, scell, h->d_opos, h->d_ozdim, h->d_oerr, h->d_odep, h->d_oidx, h->d_oobsid,
                     h->d_oplatid, h->d_otime, h->d_ohx, h->d_cell_start);
   OBSCHK(hipGetLastError());
-  launch_obs_pad_hx(st, n, (int)k, h->kp, h->d_ohx, h->d_odep, h->d_ohxp);
+  h->cols_kt = columns_wanted(h);
+  launch_obs_pad_hx(st, n, (int)k, h->kp, h->cols_kt, h->d_ohx, h->d_odep, h->d_ohxp);
   OBSCHK(hipGetLastError());
   OBSCHK(hipStreamSynchronize(st));
   cleanup();
@@ -1156,7 +1166,14 @@ static int run_prepare(letkf_gpu_t* h) {
   if (h->batched() && h->obs_cap * (int64_t)h->kp * 4 >= (1ll << 31))
     return fail(h, LETKF_EUNSUPPORTED, "batched path: n_obs x %d rows above 2^29 values",
                 h->kp);
-  return ensure_outputs(h);
+  const int rc = ensure_outputs(h);
+  if (rc) return rc;
+  if (h->cols_kt != columns_wanted(h)) {   // the tile choice has changed since set_obs
+    launch_obs_reorder(h->stream, h->nobs, h->kp, h->cols_kt, columns_wanted(h), h->d_ohxp);
+    HIPCHK(h, hipGetLastError());
+    h->cols_kt = columns_wanted(h);
+  }
+  return LETKF_OK;
 }
 
 // the device views of the handle's buffers that every kernel takes
