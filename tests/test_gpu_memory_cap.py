@@ -47,9 +47,9 @@ def test_weight_table_makes_room(monkeypatch):
 
 
 def test_kept_blocks_count(monkeypatch):
-    """About 130 MB of observations and 125 MB of their upload's temporaries, which
+    """About 90 MB of observations and 125 MB of their upload's temporaries, which
     are kept; then 130 MB of the run's arrays, for which they make room."""
-    cap = 340 << 20
+    cap = 290 << 20
     p = synth.random_problem(seed=6, nx=100, ny=50, k=50, ns=10, nobs=200000, radius=60e3)
     g = np.random.default_rng(6)
     hx = np.asfortranarray(p.hx + p.hxmean[None])

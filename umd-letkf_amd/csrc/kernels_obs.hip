@@ -92,21 +92,23 @@ void launch_gather_cols(hipStream_t st, int64_t n, int k, const int32_t* perm, c
 // operand columns of the products: hxp(kp, n) in search order, rows 0..k-1
 // the hx perturbations, row k the departure, rows above zero, so a column can
 // be read without row tests; their order in a column: column_entry
-__global__ void k_obs_pad_hx(int64_t n, int k, int kp, int kt, const float* __restrict__ ohx,
-                             const float* __restrict__ odep, float* hxp) {
+__global__ void k_obs_pad_hx(int64_t n, int k, int kp, int kt, const int32_t* __restrict__ perm,
+                             const float* __restrict__ hx, const float* __restrict__ odep,
+                             float* hxp) {
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= n * kp) return;
   const int64_t s = e / kp;
   const int at = (int)(e - s * kp);
   const int a = kt == 1 ? at : 16 * (at % kt) + at / kt;
-  hxp[e] = a < k ? ohx[s * k + a] : (a == k ? odep[s] : 0.0f);
+  hxp[e] = a < k ? hx[(int64_t)perm[s] * k + a] : (a == k ? odep[s] : 0.0f);
 }
 
-void launch_obs_pad_hx(hipStream_t st, int64_t n, int k, int kp, int kt, const float* ohx,
-                       const float* odep, float* hxp) {
+void launch_obs_pad_hx(hipStream_t st, int64_t n, int k, int kp, int kt, const int32_t* perm,
+                       const float* hx, const float* odep, float* hxp) {
   if (n <= 0) return;
   const int64_t tot = n * kp;
-  k_obs_pad_hx<<<(unsigned)((tot + 255) / 256), 256, 0, st>>>(n, k, kp, kt, ohx, odep, hxp);
+  k_obs_pad_hx<<<(unsigned)((tot + 255) / 256), 256, 0, st>>>(n, k, kp, kt, perm, hx,
+                                                            odep, hxp);
 }
 
 // a block's columns through LDS; only a change of the launch choices between
@@ -149,17 +151,16 @@ void launch_obs_gather(hipStream_t st, int64_t n, int k, const int32_t* perm,
                        const float* lat, const float* lon, const float* zdim,
                        const float* time, const float* val, const float* err,
                        const int32_t* obsid, const int32_t* platid,
-                       const float* hx, const float* hxmean,
+                       const float* hxmean,
                        const int32_t* sorted_cell, double2* pos, float* ozdim,
                        float* oerr, float* odep,
                        int32_t* oidx, int32_t* oobsid, int32_t* oplatid,
-                       float* otime, float* ohx, int32_t* cell_start) {
+                       float* otime, int32_t* cell_start) {
   if (n > 0) {
     unsigned nb = (unsigned)((n + 255) / 256);
     k_obs_gather_fields<<<nb, 256, 0, st>>>(n, perm, lat, lon, zdim, time, val, err, obsid,
                                             platid, hxmean, pos, ozdim, oerr, odep, oidx, oobsid,
                                             oplatid, otime);
-    launch_gather_cols(st, n, k, perm, hx, ohx);
   }
   k_cell_start<<<(kCells + 1 + 255) / 256, 256, 0, st>>>(n, sorted_cell, cell_start);
 }

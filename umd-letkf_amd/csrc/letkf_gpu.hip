@@ -54,9 +54,8 @@ struct letkf_gpu_t {
   // observations (raw copies, then sorted)
   int64_t nobs = 0;
   double2* d_opos = nullptr;   // unit vectors and index hashes, 2 per obs
-  float *d_ozdim = nullptr, *d_oerr = nullptr, *d_odep = nullptr, *d_otime = nullptr;
+  float *d_ozdim = nullptr, *d_oerr = nullptr, *d_otime = nullptr;
   int32_t *d_oidx = nullptr, *d_oobsid = nullptr, *d_oplatid = nullptr;
-  float* d_ohx = nullptr;
   float* d_ohxp = nullptr;   // padded operand columns (kp, n)
   int kp = 0;
   int cols_kt = 0;           // the order of its rows (column_entry)
@@ -412,8 +411,8 @@ int letkf_gpu_destroy(letkf_gpu_t* h) {
   dfree(h, h->d_state); dfree(h, h->d_mean); dfree(h, h->d_sprd); dfree(h, h->d_lat); dfree(h, h->d_lon);
   dfree(h, h->d_mask); dfree(h, h->d_gx); dfree(h, h->d_gy); dfree(h, h->d_gz);
   dfree(h, h->d_opos); dfree(h, h->d_ovt); dfree(h, h->d_ozdim); dfree(h, h->d_oerr);
-  dfree(h, h->d_odep); dfree(h, h->d_otime); dfree(h, h->d_oidx); dfree(h, h->d_oobsid);
-  dfree(h, h->d_oplatid); dfree(h, h->d_ohx); dfree(h, h->d_ohxp); dfree(h, h->d_cell_start); dfree(h, h->d_osurf);
+  dfree(h, h->d_otime); dfree(h, h->d_oidx); dfree(h, h->d_oobsid);
+  dfree(h, h->d_oplatid); dfree(h, h->d_ohxp); dfree(h, h->d_cell_start); dfree(h, h->d_osurf);
   dfree(h, h->d_otwp); dfree(h, h->d_otws);
   dfree(h, h->d_slab_var); dfree(h, h->d_slab_lev); dfree(h, h->d_inc_max); dfree(h, h->d_bounds);
   dfree(h, h->d_lev_depth);
@@ -669,7 +668,7 @@ static int set_obs_impl(letkf_gpu_t* h, int64_t n, const float* lat, const float
   float *r_val = nullptr, *r_err = nullptr, *r_hx = nullptr, *r_hxm = nullptr;
   int32_t *r_obsid = nullptr, *r_platid = nullptr, *cell = nullptr, *scell = nullptr;
   int32_t *iota = nullptr, *perm = nullptr, *r_qc = nullptr, *sel = nullptr, *nsel_d = nullptr;
-  float* r_full = nullptr;
+  float *r_full = nullptr, *dep = nullptr;
   uint8_t* keep = nullptr;
   ObsFields cf{};
   void* tmp = nullptr;
@@ -679,7 +678,7 @@ static int set_obs_impl(letkf_gpu_t* h, int64_t n, const float* lat, const float
     dfree(h, r_lat); dfree(h, r_lon); dfree(h, r_zdim); dfree(h, r_time); dfree(h, r_val); dfree(h, r_err);
     dfree(h, r_hx); dfree(h, r_hxm); dfree(h, r_obsid); dfree(h, r_platid); dfree(h, cell); dfree(h, scell);
     dfree(h, iota); dfree(h, perm); dfree(h, r_qc); dfree(h, sel); dfree(h, nsel_d); dfree(h, r_full);
-    dfree(h, keep);
+    dfree(h, keep); dfree(h, dep);
     for (auto& f : cf.f) dfree(h, f);
     for (auto& f : cf.i) dfree(h, f);
     dfree(h, cf.hx);
@@ -765,16 +764,16 @@ static int set_obs_impl(letkf_gpu_t* h, int64_t n, const float* lat, const float
     const size_t c = (size_t)cap;
     h->obs_cap = 0;
     OBSCHK(dalloc(h, &h->d_opos, 2 * c));
-    OBSCHK(dalloc(h, &h->d_ozdim, c)); OBSCHK(dalloc(h, &h->d_oerr, c)); OBSCHK(dalloc(h, &h->d_odep, c));
+    OBSCHK(dalloc(h, &h->d_ozdim, c)); OBSCHK(dalloc(h, &h->d_oerr, c));
     OBSCHK(dalloc(h, &h->d_otime, c)); OBSCHK(dalloc(h, &h->d_oidx, c)); OBSCHK(dalloc(h, &h->d_oobsid, c));
-    OBSCHK(dalloc(h, &h->d_oplatid, c)); OBSCHK(dalloc(h, &h->d_ohx, c * k));
+    OBSCHK(dalloc(h, &h->d_oplatid, c));
     OBSCHK(dalloc(h, &h->d_osurf, c)); OBSCHK(dalloc(h, &h->d_otwp, c)); OBSCHK(dalloc(h, &h->d_otws, c));
     OBSCHK(dalloc(h, &h->d_ohxp, c * h->kp));
     h->obs_cap = cap;
   }
   OBSCHK(dalloc_once(h, &h->d_cell_start, (size_t)kCells + 1));
   OBSCHK(dalloc(h, &cell, nn)); OBSCHK(dalloc(h, &scell, nn));
-  OBSCHK(dalloc(h, &iota, nn)); OBSCHK(dalloc(h, &perm, nn));
+  OBSCHK(dalloc(h, &iota, nn)); OBSCHK(dalloc(h, &perm, nn)); OBSCHK(dalloc(h, &dep, nn));
   if (n > 0) {
     launch_obs_prep(st, n, (int)k, r_lat, r_lon, cell, iota);
     OBSCHK(hipGetLastError());
@@ -784,11 +783,11 @@ static int set_obs_impl(letkf_gpu_t* h, int64_t n, const float* lat, const float
     OBSCHK(hipcub::DeviceRadixSort::SortPairs(tmp, tb, cell, scell, iota, perm, (int)n, 0, 17, st));
   }
   launch_obs_gather(st, n, (int)k, perm, r_lat, r_lon, r_zdim, r_time, r_val, r_err,
-                    r_obsid, r_platid, r_hx, r_hxm, scell, h->d_opos, h->d_ozdim, h->d_oerr, h->d_odep, h->d_oidx, h->d_oobsid,
-                    h->d_oplatid, h->d_otime, h->d_ohx, h->d_cell_start);
+                    r_obsid, r_platid, r_hxm, scell, h->d_opos, h->d_ozdim, h->d_oerr, dep,
+                    h->d_oidx, h->d_oobsid, h->d_oplatid, h->d_otime, h->d_cell_start);
   OBSCHK(hipGetLastError());
   h->cols_kt = columns_wanted(h);
-  launch_obs_pad_hx(st, n, (int)k, h->kp, h->cols_kt, h->d_ohx, h->d_odep, h->d_ohxp);
+  launch_obs_pad_hx(st, n, (int)k, h->kp, h->cols_kt, perm, r_hx, dep, h->d_ohxp);
   OBSCHK(hipGetLastError());
   OBSCHK(hipStreamSynchronize(st));
   cleanup();
@@ -1189,8 +1188,8 @@ static RunViews run_views(const letkf_gpu_t* h) {
   return RunViews{
       StateDev{h->k, h->ns, h->nij, h->d_state, h->d_mean, h->d_sprd, h->d_lat, h->d_lon,
                h->d_mask, h->d_gx, h->d_gy, h->d_gz},
-      ObsDev{h->obs_cap, h->d_opos, h->d_ozdim, h->d_oerr, h->d_odep, h->d_osurf, h->d_otwp,
-             h->d_otws, h->d_ohx, h->d_cell_start, h->d_ovt, h->d_ohxp, h->kp},
+      ObsDev{h->obs_cap, h->d_opos, h->d_ozdim, h->d_oerr, h->d_osurf, h->d_otwp, h->d_otws,
+             h->d_cell_start, h->d_ovt, h->d_ohxp, h->kp},
       VarsDev{h->nvars, h->d_slab_var, h->d_slab_lev, h->d_inc_max, h->d_bounds,
               h->d_lev_depth},
       DiagDev{h->d_maxhz, h->d_obscount, h->d_lgm, h->d_lgloc, h->d_lghash, h->d_mld,

@@ -41,11 +41,9 @@ struct ObsDev {
   const double2* pos;        // 2 per obs: (x, y), (z, bits of mix64(original index))
   const float* zdim;
   const float* err;
-  const float* dep;          // val - hx_mean in FP32
   const uint8_t* surf;       // LOC_OCEAN surface flag
   const float* tw_prof;      // GC(time, tloc_prof) or 1
   const float* tw_sat;
-  const float* hx;           // (k, n) perturbations, sorted columns
   const int32_t* cell_start; // kCells + 1
   const float* vt;           // LOC_VGAUSS (n, nlev): vertical weights, or nullptr
   const float* hxp;          // (kp, n): hx rows, departure in row k, zero rows,
@@ -195,11 +193,11 @@ void launch_obs_gather(hipStream_t st, int64_t n, int k, const int32_t* perm,
                        const float* lat, const float* lon, const float* zdim,
                        const float* time, const float* val, const float* err,
                        const int32_t* obsid, const int32_t* platid,
-                       const float* hx, const float* hxmean,
+                       const float* hxmean,
                        const int32_t* sorted_cell, double2* pos, float* ozdim,
                        float* oerr, float* odep,
                        int32_t* oidx, int32_t* oobsid, int32_t* oplatid,
-                       float* otime, float* ohx, int32_t* cell_start);
+                       float* otime, int32_t* cell_start);
 void launch_obs_flags(hipStream_t st, const LocDev& L, int64_t n,
                       const int32_t* obsid, const int32_t* platid,
                       const float* time, const int32_t* sat_obs, int n_sat_obs,
@@ -208,8 +206,9 @@ void launch_obs_flags(hipStream_t st, const LocDev& L, int64_t n,
 // vertical weights of LOC_VGAUSS: vt[g * ld + s] for every level g
 void launch_obs_vt(hipStream_t st, int64_t n, int64_t ld, int nlev, float vt_scale,
                    const float* zdim, const float* lev_depth, float* vt);
-void launch_obs_pad_hx(hipStream_t st, int64_t n, int k, int kp, int kt, const float* ohx,
-                       const float* odep, float* hxp);
+// hxp's column s from hx's column perm[s] and the sorted departures odep
+void launch_obs_pad_hx(hipStream_t st, int64_t n, int k, int kp, int kt, const int32_t* perm,
+                       const float* hx, const float* odep, float* hxp);
 // columns in the order `from` put in the order `to`
 void launch_obs_reorder(hipStream_t st, int64_t n, int kp, int from, int to, float* hxp);
 // observation arrays of set_obs in input order: lat, lon, zdim, time, val,
