@@ -1,14 +1,19 @@
 // back_apply.hip -- the transform of a group of many slabs for k < 64 without
 // an eigensolve: M = sqrt(k-1) Tri^(-1/2) as a matrix, W = Q M Q^T from the
-// stored reflectors, wbar = W (W b) / (k-1), and x_a = W x_b + wbar . x_b for
+// stored reflectors, wbar = Q Tri^-1 Q^T b, and x_a = W x_b + wbar . x_b for
 // every slab of the group (src/letkf_core.F90:100-141,
 // src/letkf_solver.F90:284-290), all in FP64.
 //
 //  k_small_rational  the lower triangle of M from the two-term recurrences of
 //                    the inverses (Tri + s_n I)^-1 (see kernels_transform.hip,
-//                    k_mat_rational), one wave per problem;
+//                    k_mat_rational), one wave per problem, and Tri^-1 Q^T b;
 //  k_back_apply      the two-sided back-transform and the apply with the
 //                    matrix one row a lane, as tridiag_pair.h keeps it.
+//
+// wbar is A^-1 b and not W (W b) / (k-1): W is right to some units of 2^-53 of
+// its largest entries, and b lies where W is smallest, so that the second form
+// loses the square of the condition number (at 3e8, k = 50 with 12 slabs, the
+// mean's increment was 9e-5 off, at 3e10 it was wrong; 4e-9 and 2e-7 so).
 //
 // They take the place of implicit QL with recorded rotations, the replay of
 // the records into eigenvectors and two mat-vecs a slab (k_tql, k_replay,
@@ -37,20 +42,24 @@ constexpr int kGroupNodes = 16;   // nodes of one pass over the rows (18 KB of
 // 199 us at 11 855 problems of k = 40, 44 -> 24 us at 33 problems of k = 50.
 __global__ __launch_bounds__(64) void k_small_rational(int k, int K, ChunkDev C,
                                                        double* __restrict__ B,
+                                                       double* __restrict__ U,
                                                        const double* __restrict__ dd,
                                                        const double* __restrict__ ee, RatTab R) {
   constexpr int NG = kGroupNodes;
   constexpr int LD = NG + 2;        // 16-byte rows, lanes' own rows in different banks
   __shared__ double sd[66], se[66];
-  // by row: U of the nodes' bottom-up pivots, and their top-down pivots
+  // by row: U of the nodes' bottom-up pivots, and their top-down pivots; in the
+  // two columns of Us that no node has, Q^T b and what its solve needs
   __shared__ __align__(16) double Us[66][LD], Gs[64][LD];
   const int64_t pair = blockIdx.x;
   if (!C.solve[pair]) return;
   const int l = threadIdx.x;
+  double* Up = U + pair * K;
   const double m = (double)(k - 1);
   sd[l] = l < k ? dd[pair * K + l] : 0.0;
   se[l] = l < k - 1 ? ee[pair * K + l] : 0.0;
-  if (l < 2) { sd[64 + l] = 0.0; se[64 + l] = 0.0; }
+  Us[l][NG] = l < k ? Up[l] : 0.0;
+  if (l < 2) { sd[64 + l] = 0.0; se[64 + l] = 0.0; Us[64 + l][NG] = 0.0; }
   __syncthreads();
   double gm = l < k ? sd[l] + (l > 0 ? fabs(se[l - 1]) : 0.0) + fabs(se[l]) : 0.0;
   gm = p_max<64>(gm);
@@ -63,21 +72,29 @@ __global__ __launch_bounds__(64) void k_small_rational(int k, int K, ChunkDev C,
   double* Bp = B + pair * (int64_t)k * k;
   for (int n0 = 0; n0 < nn; n0 += NG) {
     // the pivots: lanes 0..15 top-down, lanes 16..31 bottom-up, a node each
-    // (a node past the last has a pivot of at least m and weight 0)
-    if (l < 2 * NG) {
+    // (a node past the last has a pivot of at least m and weight 0).  Lane 32
+    // goes with the first ones for Tri x = Q^T b: the pivots of Tri itself, and
+    // the forward substitution by them.
+    const bool sol = n0 == 0 && l == 2 * NG;
+    if (l < 2 * NG || sol) {
       const int n = l & (NG - 1);
-      const double sg = n0 + n < nn ? m * sn[n0 + n] : m;
+      const double sg = sol ? 0.0 : (n0 + n < nn ? m * sn[n0 + n] : m);
       double f = 0.0, e0 = 0.0;           // e0: the row before's off-diagonal
-      if (l < NG) {
-        double d = sd[0], e1 = se[0];
+      if (l < NG || sol) {
+        double d = sd[0], e1 = se[0], b = Us[0][NG], z = 0.0;
+        double* out = sol ? &Us[0][NG] : &Gs[0][n];
         for (int i = 0; i < k; ++i) {
-          const double d2 = sd[i + 1], e2 = se[i + 1];
+          const double d2 = sd[i + 1], e2 = se[i + 1], b2 = Us[i + 1][NG];
           const double D = fma(-e0, f, d + sg);
-          Gs[i][n] = D;
-          f = e1 * rcp_cubic(D);
+          const double ri = rcp_cubic(D);
+          z = fma(-f, z, b);
+          out[i * LD] = sol ? z * ri : D;
+          f = e1 * ri;
+          if (sol) Us[i][NG + 1] = f;
           e0 = e1;
           d = d2;
           e1 = e2;
+          b = b2;
         }
       } else {
         double d = sd[k - 1], e1 = se[k - 2];
@@ -93,6 +110,15 @@ __global__ __launch_bounds__(64) void k_small_rational(int k, int K, ChunkDev C,
       }
     }
     __syncthreads();
+    if (n0 == 0) {                        // x, entry l in lane l
+      double x = 0.0, mine = 0.0;
+#pragma unroll 4
+      for (int i = k - 1; i >= 0; --i) {
+        x = fma(-Us[i][NG + 1], x, Us[i][NG]);
+        mine = l == i ? x : mine;
+      }
+      if (l < k) Up[l] = mine;
+    }
     // the inverse's diagonal 1 / (D+_i + D-_i - (d_i + s)) = 1 / (D+_i - e_i U_(i+1)),
     // where column l starts
     double cf[NG], x[NG], u[NG];
@@ -135,16 +161,18 @@ __global__ __launch_bounds__(64) void k_small_rational(int k, int K, ChunkDev C,
 // entry j, so the blocks of 16 columns below it need no product and only the
 // v_r w_c part of the update.  That is one loop for each block, not a branch
 // in the step: the matrix stays in place in its registers (with the branch
-// the compiler kept two copies of it and spilled).
+// the compiler kept two copies of it and spilled).  x = Tri^-1 Q^T b rides along
+// as row k, where v is zero: the product's row sum is v . x and the update
+// x <- H x, so that the row ends as wbar.
 template <int KQ, int P, int RPL>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2)))
 void k_back_apply(int k, int K, int64_t np, const int32_t* __restrict__ perm, LocDev L, StateDev S,
                   VarsDev V, ChunkDev C, DiagDev D, const double* __restrict__ B,
-                  const double* __restrict__ bvec, const double* __restrict__ tau,
+                  const double* __restrict__ U, const double* __restrict__ tau,
                   double* __restrict__ ana) {
   constexpr int NPW = 64 / P;
   constexpr int NT = (KQ + 15) / 16;
-  __shared__ unsigned short sl[NPW][2048];
+  __shared__ __align__(8) unsigned short sl[NPW][2048];
   const int lane = threadIdx.x;
   const int hh = P == 32 ? lane >> 5 : 0;
   const int r = lane & (P - 1), r1 = r + 32;
@@ -156,22 +184,33 @@ void k_back_apply(int k, int K, int64_t np, const int32_t* __restrict__ perm, Lo
   const int64_t pq = act ? pair : 0;
   const double* Bp = B + pq * (int64_t)k * k;
   const bool in0 = act && r < k, in1 = act && RPL == 2 && r1 < k;
+  // the lane of row k (two rows a lane only for k >= 32)
+  const bool bx = act && (RPL == 2 ? r1 : r) == k;
+  const bool b0 = RPL == 1 && bx, b1 = RPL == 2 && bx;
   // every load is made, from an address inside the problem, and masked after
   const int rc = min(r, k - 1), rc1 = min(r1, k - 1);
-  __shared__ double st[NPW][64];
+  __shared__ double st[NPW][64];    // tau, then wbar
   for (int i = r; i < 64; i += P) st[hh][i] = act && i < k - 1 ? tau[pq * K + i] : 0.0;
-  // M, symmetric, from its lower triangle (row-major in B)
+  // M, symmetric, from its lower triangle (row-major in B), and row k from U:
+  // chosen by the address (a lane that wrote over its row in a branch made the
+  // compiler keep a second copy of the matrix, and spill)
   double a0[KQ], a1[RPL == 2 ? KQ : 1];
+  const double* from0 = b0 ? U + pq * K : Bp;
+  const double* from1 = b1 ? U + pq * K : Bp;
+  const int d0 = b0 ? k : rc, o0 = b0 ? 0 : rc * k;      // entries up to the diagonal
+  const int d1 = b1 ? k : rc1, o1 = b1 ? 0 : rc1 * k;
 #pragma unroll
   for (int c = 0; c < KQ; ++c) {
     const int cc = min(c, k - 1);
-    a0[c] = Bp[max(rc, cc) * k + min(rc, cc)];
-    if constexpr (RPL == 2) a1[c] = Bp[max(rc1, cc) * k + min(rc1, cc)];
+    a0[c] = from0[cc <= d0 ? o0 + cc : cc * k + rc];
+    if constexpr (RPL == 2) a1[c] = from1[cc <= d1 ? o1 + cc : cc * k + rc1];
+    // bounds how many addresses are formed ahead
+    if (c % 8 == 7) asm volatile("" ::: "memory");
   }
 #pragma unroll
   for (int c = 0; c < KQ; ++c) {
-    a0[c] = in0 && c < k ? a0[c] : 0.0;
-    if constexpr (RPL == 2) a1[c] = in1 && c < k ? a1[c] : 0.0;
+    a0[c] = (in0 || b0) && c < k ? a0[c] : 0.0;
+    if constexpr (RPL == 2) a1[c] = (in1 || b1) && c < k ? a1[c] : 0.0;
   }
   __syncthreads();
   double n0 = 0.0, n1 = 0.0;
@@ -212,7 +251,25 @@ void k_back_apply(int k, int K, int64_t np, const int32_t* __restrict__ perm, Lo
       });
     }
   });
-  // wbar = W (W b) / (k-1), added to every row: T = W + 1 wbar^T
+  // wbar, an entry a lane, added to every row: T = W + 1 wbar^T.  Every lane
+  // writes its row, the others' where the slabs' list will be (a store in a
+  // branch made the compiler spill).
+  __syncthreads();
+  {
+    double* to = bx ? &st[hh][0] : reinterpret_cast<double*>(&sl[0][0]) + lane;
+#pragma unroll
+    for (int c = 0; c < KQ; ++c) to[c] = RPL == 2 ? a1[RPL == 2 ? c : 0] : a0[c];
+  }
+  __syncthreads();
+  {
+    double wq[4];
+    spread<P, RPL, NT>(in0 ? st[hh][r] : 0.0, in1 ? st[hh][r1 & 63] : 0.0, wq);
+    static_for<NT>([&](auto T) __attribute__((always_inline)) {
+      constexpr int tt = decltype(T)::value;
+      block_upd<KQ, tt, false>(a0, wq[tt], 0.0, 1.0, 0.0);
+      if constexpr (RPL == 2) block_upd<KQ, tt, false>(a1, wq[tt], 0.0, 1.0, 0.0);
+    });
+  }
   auto mul = [&](double x0, double x1, double* o0, double* o1) __attribute__((always_inline)) {
     double xq[4], p[4] = {0.0, 0.0, 0.0, 0.0};
     spread<P, RPL, NT>(x0, x1, xq);
@@ -223,19 +280,6 @@ void k_back_apply(int k, int K, int64_t np, const int32_t* __restrict__ perm, Lo
     *o0 = p[0] + p[1];
     *o1 = p[2] + p[3];
   };
-  {
-    double w0, w1;
-    mul(in0 ? bvec[pq * (int64_t)k + r] : 0.0, in1 ? bvec[pq * (int64_t)k + r1] : 0.0, &w0, &w1);
-    mul(w0, w1, &w0, &w1);
-    const double m = (double)(k - 1);
-    double wq[4];
-    spread<P, RPL, NT>(w0 / m, w1 / m, wq);
-    static_for<NT>([&](auto T) __attribute__((always_inline)) {
-      constexpr int tt = decltype(T)::value;
-      block_upd<KQ, tt, false>(a0, wq[tt], 0.0, 1.0, 0.0);
-      if constexpr (RPL == 2) block_upd<KQ, tt, false>(a1, wq[tt], 0.0, 1.0, 0.0);
-    });
-  }
   // slabs of each problem's group in ascending order
   const int64_t t_gp = pq / C.G;
   const int g = (int)(pq - t_gp * C.G);
@@ -275,23 +319,24 @@ void k_back_apply(int k, int K, int64_t np, const int32_t* __restrict__ perm, Lo
   }
 }
 
-// the reduction has left T in dd and ee and the reflectors in B and tau (K
-// entries a problem); perm: the order of the problems, nullptr for 0..np-1
+// the reduction has left T in dd and ee, the reflectors in B and tau and Q^T b in
+// U (K entries a problem); perm: the order of the problems, nullptr for 0..np-1.
+// Row k has to be one of a problem's rows: k = 32 takes two rows a lane.
 void launch_back_apply(hipStream_t st, const LocDev& L, const StateDev& S, const VarsDev& V,
-                       const ChunkDev& C, const DiagDev& D, double* B, const double* bvec,
+                       const ChunkDev& C, const DiagDev& D, double* B, double* U,
                        const double* tau, const double* dd, const double* ee, int K,
                        const RatTab& R, double* ana, const int32_t* perm) {
   const int64_t np = C.ngp * C.G;
   if (np <= 0) return;
   const int k = (int)S.k;
-  k_small_rational<<<(unsigned)np, 64, 0, st>>>(k, K, C, B, dd, ee, R);
+  k_small_rational<<<(unsigned)np, 64, 0, st>>>(k, K, C, B, U, dd, ee, R);
   const unsigned two = (unsigned)((np + 1) / 2);
 #define LK_BACK(KQ, P, RPL, nb)                                                              \
-  k_back_apply<KQ, P, RPL><<<nb, 64, 0, st>>>(k, K, np, perm, L, S, V, C, D, B, bvec, tau, ana)
+  k_back_apply<KQ, P, RPL><<<nb, 64, 0, st>>>(k, K, np, perm, L, S, V, C, D, B, U, tau, ana)
   if (k <= 8) LK_BACK(8, 32, 1, two);
   else if (k <= 16) LK_BACK(16, 32, 1, two);
   else if (k <= 24) LK_BACK(24, 32, 1, two);
-  else if (k <= 32) LK_BACK(32, 32, 1, two);
+  else if (k <= 31) LK_BACK(32, 32, 1, two);
   else if (k <= 40) LK_BACK(40, 32, 2, two);
   else if (k <= 48) LK_BACK(48, 32, 2, two);
   else if (k <= 50) LK_BACK(50, 32, 2, two);

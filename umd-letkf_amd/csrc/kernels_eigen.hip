@@ -85,8 +85,8 @@ __global__ __launch_bounds__(64) void k_tridiag(int k, LocDev L, StateDev S, Var
     const int64_t t_gp = pair / C.G;
     const int g = (int)(pair - t_gp * C.G);
     const int64_t ij = C.i0 + t_gp;
-    const int mld = D.mld[ij];
-    for (int s0 = 0; s0 < S.ns; s0 += K) {
+    const int mld = NV > 1 ? D.mld[ij] : 0;
+    for (int s0 = 0; NV > 1 && s0 < S.ns; s0 += K) {
       const int s = s0 + r;
       const bool in = s < S.ns && slab_group(L, V, s, mld) == g;
       const unsigned long long bal = __ballot(in);
@@ -162,8 +162,8 @@ __global__ __launch_bounds__(64) void k_tridiag(int k, LocDev L, StateDev S, Var
 #pragma unroll
     for (int q = 0; q < NV; ++q) Up[q * K + r] = xv[q];
     if (r == 0) {
-      nvec[pair] = nsl;
-      status[pair] = nsl > NV - 1 ? 3 : 0;     // more slabs than carried: Jacobi
+      if (NV > 1) nvec[pair] = nsl;
+      status[pair] = NV > 1 && nsl > NV - 1 ? 3 : 0;     // more slabs than carried: Jacobi
     }
   } else if (r == 0) {
     status[pair] = 0;
@@ -789,8 +789,9 @@ static void pipeline(hipStream_t st, const LocDev& L, const StateDev& S, const V
   // the rational solve may run inside the two-problem tridiagonalization
   const RatTab RF = (NV > 0 && fuse) ? R : RatTab{};
   int tri = 1;
-  switch (NV) {
+  switch (NV == 0 && R.nb > 0 ? 1 : NV) {   // the matrix transform takes Q^T b alone
     case 0: tri = tridiag_launch<K, 0>(st, nb, lds, k, L, S, V, C, D, B, bvec, tau, dd, ee, U, nvec, status, reg, perm, RF); break;
+    case 1: tri = tridiag_launch<K, 1>(st, nb, lds, k, L, S, V, C, D, B, bvec, tau, dd, ee, U, nvec, status, reg, perm, RF); break;
     case 2: tri = tridiag_launch<K, 2>(st, nb, lds, k, L, S, V, C, D, B, bvec, tau, dd, ee, U, nvec, status, reg, perm, RF); break;
     case 3: tri = tridiag_launch<K, 3>(st, nb, lds, k, L, S, V, C, D, B, bvec, tau, dd, ee, U, nvec, status, reg, perm, RF); break;
     case 5: tri = tridiag_launch<K, 5>(st, nb, lds, k, L, S, V, C, D, B, bvec, tau, dd, ee, U, nvec, status, reg, perm, RF); break;
@@ -819,7 +820,7 @@ static void pipeline(hipStream_t st, const LocDev& L, const StateDev& S, const V
     return;
   }
   if (R.nb > 0) {
-    launch_back_apply(st, L, S, V, C, D, B, bvec, tau, dd, ee, K, R, ana, perm);
+    launch_back_apply(st, L, S, V, C, D, B, U, tau, dd, ee, K, R, ana, perm);
     return;
   }
   tql_launch<K, K>(st, nl, k, np, C, dd, ee, rot, cap_rot, itr, cap_it, nit, status);

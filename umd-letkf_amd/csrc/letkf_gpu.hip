@@ -1073,7 +1073,7 @@ static int ensure_outputs(letkf_gpu_t* h) {
   if (h->eigK && !h->use_rat) eigen_caps((int)k, &h->cap_rot, &h->cap_it);
   const int64_t per_pair = 8 * k * k + 8 * k + 3 * 8 * (int64_t)(use_mat ? 128 : h->eigK) +
                            (nv ? 8 * (int64_t)nv * h->eigK
-                               : h->use_rat ? 0 : 8 * (int64_t)h->eigK * h->eigK) +
+                               : 8 * (int64_t)h->eigK * (h->use_rat ? 1 : h->eigK)) +
                            16 * (int64_t)h->cap_rot + 16 * (int64_t)h->cap_it + 40;
   int64_t pairs = std::max<int64_t>(
       1, std::min<int64_t>(1ll << h->tune_chunk_log2, (32ll << 30) / per_pair));
@@ -1106,9 +1106,11 @@ static int ensure_outputs(letkf_gpu_t* h) {
       dfree(h, h->d_Z);
       HIPCHK(h, dalloc(h, &h->d_U, (size_t)(np * nv * h->eigK)));
       HIPCHK(h, dalloc(h, &h->d_nvec, (size_t)np));
+    } else if (h->use_rat) {
+      HIPCHK(h, dalloc(h, &h->d_U, (size_t)(np * h->eigK)));   // Q^T b
     } else {
       dfree(h, h->d_U);
-      if (!h->use_rat) HIPCHK(h, dalloc(h, &h->d_Z, (size_t)(np * h->eigK * h->eigK)));
+      HIPCHK(h, dalloc(h, &h->d_Z, (size_t)(np * h->eigK * h->eigK)));
     }
   }
   size_t tb = 0;

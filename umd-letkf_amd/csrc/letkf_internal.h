@@ -294,10 +294,10 @@ int launch_tridiag_pair(hipStream_t st, int64_t np, const int32_t* perm, int KQ,
                         const ChunkDev& C, const DiagDev& D, double* B, const double* bvec,
                         double* tau, double* dd, double* ee, double* U, int* nvec,
                         int* status, const RatTab& R);
-// the transform of groups of many slabs from the reduction's T and
-// reflectors (k < 64): M, the back-transform and the apply (back_apply.hip)
+// the transform of groups of many slabs from the reduction's T, reflectors and
+// Q^T b (k < 64): M, the back-transform and the apply (back_apply.hip)
 void launch_back_apply(hipStream_t st, const LocDev& L, const StateDev& S, const VarsDev& V,
-                       const ChunkDev& C, const DiagDev& D, double* B, const double* bvec,
+                       const ChunkDev& C, const DiagDev& D, double* B, double* U,
                        const double* tau, const double* dd, const double* ee, int K,
                        const RatTab& R, double* ana, const int32_t* perm);
 int eigen_pipeline_K(int k);

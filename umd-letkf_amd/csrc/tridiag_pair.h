@@ -29,7 +29,8 @@ namespace lk {
 // The vectors the transform needs (b = Yb^T R^-1 d and x_b of the group's
 // slabs, NV of them) ride along as rows k .. k + NV - 1 of the matrix, rows
 // that are there anyway: the product's row sum is v . x, and the rank-2
-// update with v = 0 and w = t v . x on that row is x <- H x.
+// update with v = 0 and w = t v . x on that row is x <- H x.  NV = 1: b alone
+// (groups of many slabs, whose transform is formed as a matrix).
 //
 // A half past the end or on an unsolved problem computes on zeros and stores
 // nothing; a step whose column is already reduced is a no-op by v = w =
@@ -99,8 +100,8 @@ void k_tridiag_pair(int k, int K, int64_t np, const int32_t* __restrict__ perm, 
     const int64_t t_gp = pq / C.G;
     const int g = (int)(pq - t_gp * C.G);
     const int64_t ij = C.i0 + t_gp;
-    const int mld = act ? D.mld[ij] : 0;
-    for (int s0 = 0; s0 < S.ns; s0 += P) {
+    const int mld = act && NV > 1 ? D.mld[ij] : 0;
+    for (int s0 = 0; NV > 1 && s0 < S.ns; s0 += P) {
       const int s = s0 + r;
       const bool in = act && s < S.ns && slab_group(L, V, s, mld) == g;
       const unsigned long long bal = __ballot(in);
@@ -332,8 +333,8 @@ void k_tridiag_pair(int k, int K, int64_t np, const int32_t* __restrict__ perm, 
         if (i < K) Up[qv * K + i] = i < k ? su[qv * LDH + i] : 0.0;
   }
   if (r == 0) {
-    if (NV > 0) nvec[pq] = nsl;
-    status[pq] = NV > 0 && nsl > NV - 1 ? 3 : 0;   // more slabs than carried: Jacobi
+    if (NV > 1) nvec[pq] = nsl;
+    status[pq] = NV > 1 && nsl > NV - 1 ? 3 : 0;   // more slabs than carried: Jacobi
   }
 }
 
@@ -346,7 +347,7 @@ int launch_tridiag_pair_nv(hipStream_t st, int64_t np, const int32_t* perm, int 
                            double* tau, double* dd, double* ee, double* U, int* nvec,
                            int* status, const RatTab& R) {
   const unsigned nb = P == 32 ? (unsigned)((np + 1) / 2) : (unsigned)np;
-  if constexpr (NV > 0 && P == 32) {
+  if constexpr (NV > 1 && P == 32) {
     if (R.nb > 0) {
       k_tridiag_pair<KQ, NV, true, P, RPL, XS><<<nb, 64, 0, st>>>(
           k, K, np, perm, L, S, V, C, D, B, bvec, tau, dd, ee, U, nvec, status, R);
@@ -377,13 +378,19 @@ int launch_tridiag_pair_kq(hipStream_t st, int64_t np, const int32_t* perm, int 
   }
   if constexpr (KQ > 50) {
     if (NV == 0) LK_GO(0, 64, 1, false);
+    if (NV == 1) LK_GO(1, 64, 1, false);   // k <= 63
     if (k + NV > 64) LK_NV(64, 1, true)
     LK_NV(64, 1, false)
   } else if constexpr (KQ > 32) {
     if (NV == 0) LK_GO(0, 32, 2, false);
+    if (NV == 1) LK_GO(1, 32, 2, false);
     LK_NV(32, 2, false)   // k + NV <= 59
   } else {
     if (NV == 0) LK_GO(0, 32, 1, false);
+    if (NV == 1 && k < 32) LK_GO(1, 32, 1, false);
+    if constexpr (KQ == 32) {
+      if (NV == 1) LK_GO(1, 32, 2, false);
+    }
     if (k + NV <= 32) LK_NV(32, 1, false)
     if constexpr (KQ > 16) LK_NV(32, 2, false)
     return 0;             // not reached: k + NV <= 16 + 9

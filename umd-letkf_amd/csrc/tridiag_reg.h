@@ -44,8 +44,8 @@ void k_tridiag_reg(int k, int K, LocDev L, StateDev S, VarsDev V, ChunkDev C, Di
     const int64_t t_gp = pair / C.G;
     const int g = (int)(pair - t_gp * C.G);
     const int64_t ij = C.i0 + t_gp;
-    const int mld = D.mld[ij];
-    for (int s0 = 0; s0 < S.ns; s0 += 64) {
+    const int mld = NV > 1 ? D.mld[ij] : 0;
+    for (int s0 = 0; NV > 1 && s0 < S.ns; s0 += 64) {
       const int s = s0 + r;
       const bool in = s < S.ns && slab_group(L, V, s, mld) == g;
       const unsigned long long bal = __ballot(in);
@@ -131,8 +131,8 @@ void k_tridiag_reg(int k, int K, LocDev L, StateDev S, VarsDev V, ChunkDev C, Di
     for (int q = 0; q < NV; ++q)
       if (r < K) Up[q * K + r] = xv[q];
     if (r == 0) {
-      nvec[pair] = nsl;
-      status[pair] = nsl > NV - 1 ? 3 : 0;
+      if (NV > 1) nvec[pair] = nsl;
+      status[pair] = NV > 1 && nsl > NV - 1 ? 3 : 0;
     }
   } else if (r == 0) {
     status[pair] = 0;
@@ -146,6 +146,7 @@ bool launch_tridiag_reg_kq(hipStream_t st, unsigned nb, int NV, int k, int K, co
                            double* dd, double* ee, double* U, int* nvec, int* status) {
   switch (NV) {
     case 0: k_tridiag_reg<KQ, 0><<<nb, 64, 0, st>>>(k, K, L, S, V, C, D, B, bvec, tau, dd, ee, U, nvec, status); return true;
+    case 1: k_tridiag_reg<KQ, 1><<<nb, 64, 0, st>>>(k, K, L, S, V, C, D, B, bvec, tau, dd, ee, U, nvec, status); return true;
     case 2: k_tridiag_reg<KQ, 2><<<nb, 64, 0, st>>>(k, K, L, S, V, C, D, B, bvec, tau, dd, ee, U, nvec, status); return true;
     case 3: k_tridiag_reg<KQ, 3><<<nb, 64, 0, st>>>(k, K, L, S, V, C, D, B, bvec, tau, dd, ee, U, nvec, status); return true;
     case 5: k_tridiag_reg<KQ, 5><<<nb, 64, 0, st>>>(k, K, L, S, V, C, D, B, bvec, tau, dd, ee, U, nvec, status); return true;
