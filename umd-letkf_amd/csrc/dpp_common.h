@@ -102,6 +102,12 @@ __device__ __forceinline__ void wave_sums4(double (&q)[4]) {
   }
 }
 
+// sums of two values over the wave for the price of one: a's in lanes 0..31,
+// b's in lanes 32..63
+__device__ __forceinline__ double wave_sums2(double a, double b) {
+  return p_sum<32>(swap_sum32(a, b));
+}
+
 // largest value over the P lanes, in every lane
 template <int P>
 __device__ __forceinline__ double p_max(double x) {

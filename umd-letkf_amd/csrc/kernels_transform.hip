@@ -31,7 +31,8 @@ LK_NR(40) LK_NR(48) LK_NR(56) LK_NR(64)
 // k_blk_tridiag / k_blk_back launchers (one file per block size)
 #define LK_BS(n)                                                                          \
   void launch_blk_tridiag_bs##n(hipStream_t st, unsigned nb, int k, const ChunkDev& C,    \
-                                double* B, double* tau, double* dd, double* ee);          \
+                                double* B, double* bvec, double* tau, double* dd,         \
+                                double* ee);                                              \
   void launch_blk_back_bs##n(hipStream_t st, unsigned nb, int k, const ChunkDev& C,       \
                              double* B, const double* bvec, const double* tau);
 LK_BS(7) LK_BS(8)
@@ -39,9 +40,10 @@ LK_BS(7) LK_BS(8)
 // k_row_tridiag / k_row_back launchers (one file per row length)
 #define LK_KQ(n)                                                                          \
   void launch_row_tridiag_kq##n(hipStream_t st, unsigned nb, int k, const ChunkDev& C,    \
-                                double* B, double* tau, double* dd, double* ee);          \
+                                double* B, double* bvec, double* tau, double* dd,         \
+                                double* ee);                                              \
   void launch_row_back_kq##n(hipStream_t st, unsigned nb, int k, const ChunkDev& C,       \
-                             double* B, const double* bvec, const double* tau);
+                             double* B, double* bvec, const double* tau);
 LK_KQ(72) LK_KQ(80) LK_KQ(88) LK_KQ(96) LK_KQ(104)
 #undef LK_KQ
 
@@ -64,7 +66,9 @@ __device__ __forceinline__ double uniform_f64(double v) {
 // its node count is known (uniform over the block).
 //
 // The first wave's lanes run the nodes' top-down pivots, the second's the
-// bottom-up ones, a node each.  Then a thread takes a column: x starts at the
+// bottom-up ones, a node each; lanes 62 and 63 of the first go with them for
+// Tri x = Q^T b, the pivots of Tri itself and the forward substitution, and
+// x takes the place of Q^T b in bvec.  Then a thread takes a column: x starts at the
 // inverse's diagonal in row c and follows x <- -U_r x below; a row's U values,
 // the same for all lanes, are read two at a time and a row ahead, and the
 // multiplications run on the lanes below the diagonal alone.  11 900 problems
@@ -72,6 +76,7 @@ __device__ __forceinline__ double uniform_f64(double v) {
 // U read node by node and a select for each, 456 us now.
 template <int NNL, int NNLO>
 __global__ __launch_bounds__(128) void k_mat_rational(int k, ChunkDev C, double* __restrict__ B,
+                                                      double* __restrict__ bvec,
                                                       const double* __restrict__ dd,
                                                       const double* __restrict__ ee,
                                                       const double* __restrict__ tab,
@@ -80,7 +85,8 @@ __global__ __launch_bounds__(128) void k_mat_rational(int k, ChunkDev C, double*
   static_assert(NNL % 8 == 0 && NNL <= kMaxNodes, "node class");
   constexpr int LD = NNL + 2;       // 16-byte rows, lanes' own rows in different banks
   __shared__ double sd[130], se[130];
-  // by row: U of the nodes' bottom-up pivots, and their top-down pivots
+  // by row: U of the nodes' bottom-up pivots, and their top-down pivots; in the
+  // two columns of Us that no node has, Q^T b and what its solve needs
   __shared__ __align__(16) double Us[128][LD], Gs[128][LD];
   __shared__ double sgm[2];
   const int64_t pair = blockIdx.x;
@@ -89,6 +95,8 @@ __global__ __launch_bounds__(128) void k_mat_rational(int k, ChunkDev C, double*
   const double m = (double)(k - 1);
   sd[tid] = tid < k ? dd[pair * kMatStride + tid] : 0.0;
   se[tid] = tid < k - 1 ? ee[pair * kMatStride + tid] : 0.0;
+  double* bp = bvec + pair * (int64_t)k;
+  Us[tid][NNL] = tid < k ? bp[tid] : 0.0;
   if (tid < 2) { sd[128 + tid] = 0.0; se[128 + tid] = 0.0; }
   __syncthreads();
   double gm = 0.0;
@@ -107,19 +115,23 @@ __global__ __launch_bounds__(128) void k_mat_rational(int k, ChunkDev C, double*
   const double* sn = tab + bk * kRatLd;
   const double* wn = sn + kRatLd / 2;
   // a node past the last has a pivot of at least m and weight 0
-  if (l < NNL) {
-    const double sg = l < nn ? m * sn[l] : m;
+  const bool fwd = tid == 62, sol = fwd || tid == 63;
+  if (l < NNL || sol) {
+    const double sg = sol ? 0.0 : (l < nn ? m * sn[l] : m);
     double f = 0.0, e0 = 0.0;             // e0: the row before's off-diagonal
     if (tid < 64) {
-      double d = sd[0], e1 = se[0];
+      double d = sd[0], e1 = se[0], b = Us[0][NNL], z = 0.0;
+      double* out = sol ? &Us[0][tid == 63 ? NNL + 1 : NNL] : &Gs[0][l];
       for (int i = 0; i < k; ++i) {
-        const double d2 = sd[i + 1], e2 = se[i + 1];
+        const double d2 = sd[i + 1], e2 = se[i + 1], b2 = Us[min(i + 1, k - 1)][NNL];
         const double D = fma(-e0, f, d + sg);
-        Gs[i][l] = D;
+        z = fma(-f, z, b);
+        out[i * LD] = fwd ? z : D;        // lane 62 over what it has read of Q^T b
         f = e1 * rcp_cubic(D);
         e0 = e1;
         d = d2;
         e1 = e2;
+        b = b2;
       }
     } else {
       double d = sd[k - 1], e1 = se[k - 2];
@@ -135,6 +147,21 @@ __global__ __launch_bounds__(128) void k_mat_rational(int k, ChunkDev C, double*
     }
   }
   __syncthreads();
+  if (tid < k) {                          // z_i / D_i and e_i / D_i
+    const double ri = rcp_cubic(Us[tid][NNL + 1]);
+    Us[tid][NNL] *= ri;
+    Us[tid][NNL + 1] = se[tid] * ri;
+  }
+  __syncthreads();
+  {
+    double x = 0.0, mine = 0.0;
+#pragma unroll 4
+    for (int i = k - 1; i >= 0; --i) {
+      x = fma(-Us[i][NNL + 1], x, Us[i][NNL]);
+      mine = tid == i ? x : mine;
+    }
+    if (tid < k) bp[tid] = mine;
+  }
   const int c = tid;
   if (c >= k) return;
   // the inverse's diagonal 1 / (D+_c + D-_c - (d_c + s)) = 1 / (D+_c - e_c U_(c+1))
@@ -164,6 +191,51 @@ __global__ __launch_bounds__(128) void k_mat_rational(int k, ChunkDev C, double*
 #pragma unroll
     for (int n = 0; n < NNL; ++n) u[n] = un[n];
   }
+}
+
+// b <- Q^T b (FWD: reflectors 0 .. k - 3 in turn) or b <- Q b (the other way
+// round), one wave per problem, two entries a lane.  It reads the reflectors
+// once, half of a problem's B, eight of them ahead of the one that is applied:
+// 11 900 problems of k = 100 take 200 and 220 us, one ahead took 265 and 289.
+template <bool FWD>
+__global__ __launch_bounds__(64) void k_reflect_vec(int k, ChunkDev C, const double* __restrict__ B,
+                                                    double* __restrict__ bvec,
+                                                    const double* __restrict__ tau) {
+  constexpr int AHEAD = 8;
+  const int64_t pair = blockIdx.x;
+  if (!C.solve[pair]) return;
+  const int l = threadIdx.x, l1 = l + 64;
+  const double* Bp = B + pair * (int64_t)k * k;
+  const double* tp = tau + pair * kMatStride;
+  double* bp = bvec + pair * (int64_t)k;
+  double x0 = l < k ? bp[l] : 0.0, x1 = l1 < k ? bp[l1] : 0.0;
+  const int c0 = min(l, k - 1), c1 = min(l1, k - 1), n = k - 2;
+  double n0[AHEAD], n1[AHEAD], tn[AHEAD];
+  // step q's reflector, or the last one's again
+  auto fetch = [&](int q, int s) __attribute__((always_inline)) {
+    const int j = FWD ? min(q, n - 1) : max(n - 1 - q, 0);
+    n0[s] = Bp[j * k + c0];
+    n1[s] = Bp[j * k + c1];
+    tn[s] = tp[j];
+  };
+#pragma unroll
+  for (int s = 0; s < AHEAD; ++s) fetch(s, s);
+  for (int q0 = 0; q0 < n; q0 += AHEAD) {
+#pragma unroll
+    for (int s = 0; s < AHEAD; ++s) {
+      const int q = q0 + s, j = FWD ? q : n - 1 - q;
+      const double t = q < n ? tn[s] : 0.0;
+      // an unused reflector (t = 0) may not have been stored
+      const double v0 = l > j && l < k && t != 0.0 ? n0[s] : 0.0;
+      const double v1 = l1 > j && l1 < k && t != 0.0 ? n1[s] : 0.0;
+      fetch(q + AHEAD, s);
+      const double d = -t * p_sum<64>(fma(v0, x0, v1 * x1));
+      x0 = fma(d, v0, x0);
+      x1 = fma(d, v1, x1);
+    }
+  }
+  if (l < k) bp[l] = x0;
+  if (l1 < k) bp[l1] = x1;
 }
 
 // sum over a slab of the tile: the lane's registers (summed by the caller),
@@ -572,7 +644,7 @@ bool transform_mat_fuses_finalize(int prec) { return prec != LETKF_PREC_FP64; }
 
 void launch_transform_mat(hipStream_t st, int prec, const LocDev& L, const StateDev& S,
                           const VarsDev& V, const ChunkDev& C, const DiagDev& D, double* B,
-                          const double* bvec, double* tau, double* dd, double* ee,
+                          double* bvec, double* tau, double* dd, double* ee,
                           const RatTab& R, double* ana, bool blk, const FinArgs* fin) {
   const int64_t np = C.ngp * C.G;
   if (np <= 0) return;
@@ -583,20 +655,23 @@ void launch_transform_mat(hipStream_t st, int prec, const LocDev& L, const State
   // column-half kernels, rows per half k <= 2 NR
   const int nr = (k + 1) / 2;
   if (blk) {
-    if (k <= 72) launch_row_tridiag_kq72(st, nb, k, C, B, tau, dd, ee);
-    else if (k <= 80) launch_row_tridiag_kq80(st, nb, k, C, B, tau, dd, ee);
-    else if (k <= 88) launch_row_tridiag_kq88(st, nb, k, C, B, tau, dd, ee);
-    else if (k <= 96) launch_row_tridiag_kq96(st, nb, k, C, B, tau, dd, ee);
-    else if (k <= 104) launch_row_tridiag_kq104(st, nb, k, C, B, tau, dd, ee);
-    else if (k <= 112) launch_blk_tridiag_bs7(st, nb, k, C, B, tau, dd, ee);
-    else launch_blk_tridiag_bs8(st, nb, k, C, B, tau, dd, ee);
+    if (k <= 72) launch_row_tridiag_kq72(st, nb, k, C, B, bvec, tau, dd, ee);
+    else if (k <= 80) launch_row_tridiag_kq80(st, nb, k, C, B, bvec, tau, dd, ee);
+    else if (k <= 88) launch_row_tridiag_kq88(st, nb, k, C, B, bvec, tau, dd, ee);
+    else if (k <= 96) launch_row_tridiag_kq96(st, nb, k, C, B, bvec, tau, dd, ee);
+    else if (k <= 104) launch_row_tridiag_kq104(st, nb, k, C, B, bvec, tau, dd, ee);
+    else if (k <= 112) launch_blk_tridiag_bs7(st, nb, k, C, B, bvec, tau, dd, ee);
+    else launch_blk_tridiag_bs8(st, nb, k, C, B, bvec, tau, dd, ee);
   } else if (nr <= 40) launch_mat_tridiag_nr40(st, nb, k, C, B, tau, dd, ee);
   else if (nr <= 48) launch_mat_tridiag_nr48(st, nb, k, C, B, tau, dd, ee);
   else if (nr <= 56) launch_mat_tridiag_nr56(st, nb, k, C, B, tau, dd, ee);
   else launch_mat_tridiag_nr64(st, nb, k, C, B, tau, dd, ee);
-  k_mat_rational<16, 0><<<nb, 128, 0, st>>>(k, C, B, dd, ee, R.tab, R.n, R.nb);
-  k_mat_rational<24, 16><<<nb, 128, 0, st>>>(k, C, B, dd, ee, R.tab, R.n, R.nb);
-  k_mat_rational<kMaxNodes, 24><<<nb, 128, 0, st>>>(k, C, B, dd, ee, R.tab, R.n, R.nb);
+  // the others take b along in the reduction and the back-transform
+  if (!blk) k_reflect_vec<true><<<nb, 64, 0, st>>>(k, C, B, bvec, tau);
+  k_mat_rational<16, 0><<<nb, 128, 0, st>>>(k, C, B, bvec, dd, ee, R.tab, R.n, R.nb);
+  k_mat_rational<24, 16><<<nb, 128, 0, st>>>(k, C, B, bvec, dd, ee, R.tab, R.n, R.nb);
+  k_mat_rational<kMaxNodes, 24><<<nb, 128, 0, st>>>(k, C, B, bvec, dd, ee, R.tab, R.n, R.nb);
+  if (!blk) k_reflect_vec<false><<<nb, 64, 0, st>>>(k, C, B, bvec, tau);
   if (blk) {
     if (k <= 72) launch_row_back_kq72(st, nb, k, C, B, bvec, tau);
     else if (k <= 80) launch_row_back_kq80(st, nb, k, C, B, bvec, tau);

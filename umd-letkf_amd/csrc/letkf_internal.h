@@ -330,7 +330,7 @@ struct FinArgs {
 bool transform_mat_fuses_finalize(int prec);
 void launch_transform_mat(hipStream_t st, int prec, const LocDev& L, const StateDev& S,
                           const VarsDev& V, const ChunkDev& C, const DiagDev& D, double* B,
-                          const double* bvec, double* tau, double* dd, double* ee,
+                          double* bvec, double* tau, double* dd, double* ee,
                           const RatTab& R, double* ana, bool blk, const FinArgs* fin);
 // skip_solved: only masked gridpoints and the slabs of groups without a
 // solved problem (the rest were post-processed by the fused apply)

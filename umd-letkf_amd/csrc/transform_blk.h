@@ -1,7 +1,7 @@
 // transform_blk.h -- the reduction and the back-transform of the explicit
-// transform matrix (105 <= k <= 128, see transform_mat.h; transform_row.h
-// serves smaller ones) with A distributed over a 256-thread block in 2D: the matrix, padded to N = 16 BS, is a 16 x 16
-// grid of BS x BS blocks, and thread t holds block (I, J) = (t / 16, t % 16)
+// transform matrix (105 <= k <= 127, see transform_mat.h; transform_row.h
+// serves smaller ones) with A distributed over a 256-thread block in 2D: the
+// matrix, padded to N = 16 BS, is a 16 x 16 grid of BS x BS blocks, and thread t holds block (I, J) = (t / 16, t % 16)
 // in registers.  Per step a thread needs v and w only for its BS rows and
 // its BS columns (4 BS values from LDS), where the column layout of
 // transform_mat.h needs v and w for all of its NR rows, broadcast to every
@@ -12,21 +12,25 @@
 // barriers per step: after the column is in LDS, and after p = t A v and the
 // partial sums of v.p are; the back-transform, whose reflectors are known in
 // advance, only the second (its LDS arrays double buffered by step).  In the
-// reduction the column goes to LDS with its
-// reduced rows zeroed and the wholly reduced waves keep their p entries at
+// reduction the column goes to LDS with its reduced rows zeroed and the wholly reduced waves keep their p entries at
 // zero, so v = x sc and w = p - kc v need no row tests.
 //
 //  k_blk_tridiag<BS>  A = Q Tri Q^T (LAPACK dsytd2, lower), the outputs of
 //                     k_mat_tridiag: reflector j in row j of B (columns > j),
-//                     tau, d and e.  Waves whose rows are all reduced skip
-//                     the arithmetic of a step.
+//                     tau, d and e; Q^T b over b.  Waves whose rows are all
+//                     reduced skip the arithmetic of a step.
 //  k_blk_back<BS>     W = Q M Q^T from M in the lower triangle of B, then
-//                     wbar = W (W b) / (k-1) and T = W + 1 wbar^T over B, the
-//                     outputs of k_mat_back.
+//                     T = W + 1 wbar^T over B, the outputs of k_mat_back.
+//                     wbar from Tri^-1 Q^T b in bvec.
+//
+// b goes along an entry a lane, the one that finishes the row's product: its
+// v . b is summed with v . p (wave_sums2).  k_reflect_vec in its place: the
+// eigen stage of 11 952 problems of k = 105 / 127 9.18 / 12.75 ms, so 9.11 / 12.66.
 #pragma once
 
 #include <hip/hip_runtime.h>
 
+#include "dpp_common.h"
 #include "eigen_common.h"
 #include "letkf_internal.h"
 
@@ -40,15 +44,6 @@ __device__ __forceinline__ double blk_dpp(double v) {
   const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xf, 0xf, true);
   const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xf, 0xf, true);
   return __hiloint2double(hi, lo);
-}
-
-// sum over the 16 lanes of this lane's DPP row, complete in the row's lane 15
-__device__ __forceinline__ double row16_sum(double x) {
-  x += blk_dpp<0x111>(x);
-  x += blk_dpp<0x112>(x);
-  x += blk_dpp<0x114>(x);
-  x += blk_dpp<0x118>(x);
-  return x;
 }
 
 // sums of BS <= 8 values over the 16 lanes of this lane's DPP row, scattered:
@@ -83,13 +78,15 @@ __device__ __forceinline__ double row16_scatter_sums(const double (&s)[BS], int 
 
 template <int BS>
 __global__ __launch_bounds__(256) void k_blk_tridiag(int k, ChunkDev C, double* __restrict__ B,
+                                                     double* __restrict__ bvec,
                                                      double* __restrict__ tau,
                                                      double* __restrict__ dd,
                                                      double* __restrict__ ee) {
   static_assert(16 * BS <= 128, "at most 128 rows");
   __shared__ double sx[128];        // column j of A
   __shared__ double sp[128];        // p = t A v
-  __shared__ double skc[4];         // per-wave sums of v . p
+  __shared__ double skc[2][4];      // per-wave sums of v . p and of v . b
+  __shared__ double sb[128];        // b: an entry to the lane that owns the row
   __shared__ double se[128], stau[128];
   const int64_t pair = blockIdx.x;
   if (!C.solve[pair]) return;
@@ -118,6 +115,7 @@ __global__ __launch_bounds__(256) void k_blk_tridiag(int k, ChunkDev C, double* 
       a[x][y] = (r == c && r < k) ? v + m : v;
     }
   if (tid < 128) { sx[tid] = 0.0; sp[tid] = 0.0; se[tid] = 0.0; stau[tid] = 0.0; }
+  if (tid < 128) sb[tid] = tid < k ? bvec[pair * (int64_t)k + tid] : 0.0;
   __syncthreads();
   const int jend = k - 2;
   // last row of this wave's grid rows (wave-uniform)
@@ -164,6 +162,7 @@ __global__ __launch_bounds__(256) void k_blk_tridiag(int k, ChunkDev C, double* 
         }
       }
       const bool live = wlast > j;   // this wave still has rows below j
+      double vrow = 0.0;             // v in the row that this lane owns
       if (live) {
         // row sums of this block's part of A v, completed over the grid row:
         // lane J holds row R0 + J / 2 (the even lane writes it)
@@ -180,9 +179,9 @@ __global__ __launch_bounds__(256) void k_blk_tridiag(int k, ChunkDev C, double* 
         const bool own = (J & 1) == 0 && xr < BS;
         const double px = r > j ? t * pz : 0.0;
         if (own) sp[r] = px;
-        const double vrow = r == j1 ? 1.0 : sx[min(r, 127)] * sc;
-        const double ws = wave_sum_dpp(own ? px * vrow : 0.0);
-        if (l == 0) skc[wv] = ws;
+        if (own) vrow = r == j1 ? 1.0 : sx[r] * sc;
+        const double ws = wave_sums2(px * vrow, vrow * sb[min(r, 127)]);
+        if ((l & 31) == 0) skc[l >> 5][wv] = ws;
       } else {
         // every row of this wave is reduced: its p entries stay zero, so
         // that w = p - kc v needs no row test
@@ -190,7 +189,7 @@ __global__ __launch_bounds__(256) void k_blk_tridiag(int k, ChunkDev C, double* 
 #pragma unroll
           for (int x = 0; x < BS; ++x) sp[R0 + x] = 0.0;
         }
-        if (l == 0) skc[wv] = 0.0;
+        if ((l & 31) == 0) skc[l >> 5][wv] = 0.0;
       }
       // reflector j (columns > j), one entry per thread of the first two
       // waves (one store each instead of BS predicated stores in the first
@@ -199,7 +198,10 @@ __global__ __launch_bounds__(256) void k_blk_tridiag(int k, ChunkDev C, double* 
       if (tid == 0) { stau[j] = t; se[j] = beta; }
       __syncthreads();
       if (live) {
-        const double kc = 0.5 * t * ((skc[0] + skc[1]) + (skc[2] + skc[3]));
+        const double kc = 0.5 * t * ((skc[0][0] + skc[0][1]) + (skc[0][2] + skc[0][3]));
+        const int r = R0 + (J >> 1);
+        if ((J & 1) == 0 && (J >> 1) < BS)
+          sb[r] = fma(-t * ((skc[1][0] + skc[1][1]) + (skc[1][2] + skc[1][3])), vrow, sb[r]);
         // p and v are zero in the reduced rows, and so is w
         double wr[BS], wc[BS];
 #pragma unroll
@@ -232,6 +234,7 @@ __global__ __launch_bounds__(256) void k_blk_tridiag(int k, ChunkDev C, double* 
     ep[tid] = se[tid];
     tau[pair * kBlkStride + tid] = stau[tid];
   }
+  if (tid < k) bvec[pair * (int64_t)k + tid] = sb[tid];
 }
 
 template <int BS>
@@ -243,8 +246,9 @@ __global__ __launch_bounds__(256) void k_blk_back(int k, ChunkDev C, double* __r
   // buffered by step, and the next step's reflector goes to LDS during this
   // step's product
   __shared__ double sv[2][128];     // reflectors of this step and the next
-  __shared__ double sp[2][128];     // p = t A v; then W b, W (W b)
-  __shared__ double skc[2][4];
+  __shared__ double sp[2][128];     // p = t A v
+  __shared__ double skc[2][2][4];   // per-wave sums of v . p and of v . x
+  __shared__ double sb[128];        // x = Tri^-1 Q^T b, then wbar: an entry a lane
   __shared__ double stau[128];
   const int64_t pair = blockIdx.x;
   if (!C.solve[pair]) return;
@@ -252,7 +256,6 @@ __global__ __launch_bounds__(256) void k_blk_back(int k, ChunkDev C, double* __r
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int I = tid >> 4, J = tid & 15;
   const int R0 = BS * I, C0 = BS * J;
-  const double m = (double)(k - 1);
   double* Bp = B + pair * (int64_t)k * k;
   // M from the lower triangle of B (symmetric); all loads issued first
   double a[BS][BS];
@@ -272,6 +275,7 @@ __global__ __launch_bounds__(256) void k_blk_back(int k, ChunkDev C, double* __r
     stau[tid] = tid < k - 2 ? tau[pair * kBlkStride + tid] : 0.0;
     sp[0][tid] = 0.0;
     sp[1][tid] = 0.0;
+    sb[tid] = tid < k ? bvec[pair * (int64_t)k + tid] : 0.0;
   }
   // reflector rows go through LDS: reflector k-3 now, and threads 0..127
   // hold entry tid of the one after next (loaded two steps ahead)
@@ -307,8 +311,9 @@ __global__ __launch_bounds__(256) void k_blk_back(int k, ChunkDev C, double* __r
     const bool own = (J & 1) == 0 && xr < BS;
     const double px = t * pz;
     if (own) sp[buf][r] = px;
-    const double ws = wave_sum_dpp(own ? px * sv[buf][min(r, 127)] : 0.0);
-    if (l == 0) skc[buf][wv] = ws;
+    const double vrow = own ? sv[buf][r] : 0.0;
+    const double ws = wave_sums2(px * vrow, vrow * sb[min(r, 127)]);
+    if ((l & 31) == 0) skc[buf][l >> 5][wv] = ws;
     // reflector j-1 into the other buffer (its last reader, step j+1, has
     // passed the barrier of step j+1); reflector j-2 loaded
     if (tid < 128 && j > 0) {
@@ -317,7 +322,9 @@ __global__ __launch_bounds__(256) void k_blk_back(int k, ChunkDev C, double* __r
       if (jn >= 0) vnext = (tid > jn && tid < k) ? Bp[(int64_t)jn * k + tid] : 0.0;
     }
     __syncthreads();
-    const double kc = 0.5 * t * ((skc[buf][0] + skc[buf][1]) + (skc[buf][2] + skc[buf][3]));
+    const double(&s)[2][4] = skc[buf];
+    const double kc = 0.5 * t * ((s[0][0] + s[0][1]) + (s[0][2] + s[0][3]));
+    if (own) sb[r] = fma(-t * ((s[1][0] + s[1][1]) + (s[1][2] + s[1][3])), vrow, sb[r]);
     double wr[BS], wc[BS];
 #pragma unroll
     for (int x = 0; x < BS; ++x) {
@@ -329,41 +336,21 @@ __global__ __launch_bounds__(256) void k_blk_back(int k, ChunkDev C, double* __r
 #pragma unroll
       for (int y = 0; y < BS; ++y) a[x][y] = fma(-vr[x], wc[y], fma(-wr[x], vc[y], a[x][y]));
   }
-  // wbar = W (W b) / (k-1); T = W + 1 wbar^T, row major over B
+  // T = W + 1 wbar^T, row major over B
   __syncthreads();
-  if (tid < 128) sv[0][tid] = tid < k ? bvec[pair * (int64_t)k + tid] : 0.0;
-  __syncthreads();
-#pragma unroll
-  for (int pass = 0; pass < 2; ++pass) {
-    double vc[BS];
-#pragma unroll
-    for (int y = 0; y < BS; ++y) vc[y] = sv[pass][C0 + y];
-#pragma unroll
-    for (int x = 0; x < BS; ++x) {
-      double s0 = 0.0;
-#pragma unroll
-      for (int y = 0; y < BS; ++y) s0 = fma(a[x][y], vc[y], s0);
-      s0 = row16_sum(s0);
-      if (J == 15) {
-        if (pass == 0) sv[1][R0 + x] = s0;
-        else sp[0][R0 + x] = s0 / m;
-      }
-    }
-    __syncthreads();
-  }
 #pragma unroll
   for (int x = 0; x < BS; ++x)
 #pragma unroll
     for (int y = 0; y < BS; ++y) {
       const int r = R0 + x, c = C0 + y;
-      if (r < k && c < k) Bp[(int64_t)r * k + c] = a[x][y] + sp[0][c];
+      if (r < k && c < k) Bp[(int64_t)r * k + c] = a[x][y] + sb[c];
     }
 }
 
 template <int BS>
 void launch_blk_tridiag_bs(hipStream_t st, unsigned nb, int k, const ChunkDev& C, double* B,
-                           double* tau, double* dd, double* ee) {
-  k_blk_tridiag<BS><<<nb, 256, 0, st>>>(k, C, B, tau, dd, ee);
+                           double* bvec, double* tau, double* dd, double* ee) {
+  k_blk_tridiag<BS><<<nb, 256, 0, st>>>(k, C, B, bvec, tau, dd, ee);
 }
 template <int BS>
 void launch_blk_back_bs(hipStream_t st, unsigned nb, int k, const ChunkDev& C, double* B,

@@ -5,8 +5,8 @@
 namespace lk {
 
 void launch_blk_tridiag_bs7(hipStream_t st, unsigned nb, int k, const ChunkDev& C, double* B,
-                             double* tau, double* dd, double* ee) {
-  launch_blk_tridiag_bs<7>(st, nb, k, C, B, tau, dd, ee);
+                             double* bvec, double* tau, double* dd, double* ee) {
+  launch_blk_tridiag_bs<7>(st, nb, k, C, B, bvec, tau, dd, ee);
 }
 
 void launch_blk_back_bs7(hipStream_t st, unsigned nb, int k, const ChunkDev& C, double* B,

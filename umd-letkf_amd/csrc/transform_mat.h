@@ -27,7 +27,14 @@
 //  k_mat_back<NR>     the register layout of k_mat_tridiag: W = Q M Q^T by
 //                     the reflectors applied from both sides in reverse
 //                     order (the same two-sided rank-2 update), then
-//                     wbar = W (W b) / (k-1) and T = W + 1 wbar^T over B.
+//                     T = W + 1 wbar^T over B.
+//  k_reflect_vec      one wave per problem (the layouts of transform_row.h and
+//                     transform_blk.h take b along): b <- Q^T b after the reduction, and
+//                     after k_mat_rational has made it Tri^-1 Q^T b, b <- Q b,
+//                     which is wbar.  (W (W b) / (k-1) is the same but loses
+//                     the square of the condition number: W is right to
+//                     rounding of its largest entries, and b lies where W is
+//                     smallest.)
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -164,7 +171,6 @@ template <int NR>
 __global__ __launch_bounds__(256) void k_mat_back(int k, ChunkDev C, double* __restrict__ B,
                                                   const double* __restrict__ bvec,
                                                   const double* __restrict__ tau) {
-  __shared__ double sx[128];
   __shared__ double2 svw[2][128];
   __shared__ double pp[2][128];
   __shared__ double stau[128];
@@ -173,7 +179,6 @@ __global__ __launch_bounds__(256) void k_mat_back(int k, ChunkDev C, double* __r
   const int tid = threadIdx.x, l = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int h = wv >> 1, c = l + 64 * (wv & 1);
-  const double m = (double)(k - 1);
   double* Bp = B + pair * (int64_t)k * k;
   int r0 = NR * h;
   // M from the lower triangle of B (symmetric)
@@ -218,32 +223,8 @@ __global__ __launch_bounds__(256) void k_mat_back(int k, ChunkDev C, double* __r
       if ((s & (kFenceRows - 1)) == kFenceRows - 1) LK_FENCE(a[s]);
     }
   }
-  // wbar = W (W b) / (k-1); T = W + 1 wbar^T, row major over B
-  asm volatile("" : "+s"(r0));
-  __syncthreads();
-  if (h == 0) sx[c] = c < k ? bvec[pair * (int64_t)k + c] : 0.0;
-  __syncthreads();
-  double q = 0.0;
-#pragma unroll
-  for (int s = 0; s < NR; ++s) {
-    q = fma(a[s], sx[r0 + s], q);
-    if ((s & (kFenceRows - 1)) == kFenceRows - 1) LK_FENCE(q);
-  }
-  pp[h][c] = q;
-  __syncthreads();
-  const double t1 = pp[0][c] + pp[1][c];
-  __syncthreads();
-  if (h == 0) sx[c] = t1;
-  __syncthreads();
-  q = 0.0;
-#pragma unroll
-  for (int s = 0; s < NR; ++s) {
-    q = fma(a[s], sx[r0 + s], q);
-    if ((s & (kFenceRows - 1)) == kFenceRows - 1) LK_FENCE(q);
-  }
-  pp[h][c] = q;
-  __syncthreads();
-  const double wb = (pp[0][c] + pp[1][c]) / m;
+  // T = W + 1 wbar^T, row major over B
+  const double wb = c < k ? bvec[pair * (int64_t)k + c] : 0.0;
   asm volatile("" : "+s"(r0));
 #pragma unroll
   for (int s = 0; s < NR; ++s) {

@@ -23,9 +23,16 @@
 // this way, the back-transform 3.2 and 1.8.
 //
 //  k_row_tridiag<KQ>  A = Q Tri Q^T (LAPACK dsytd2, lower): reflector j in row
-//                     j of B (columns > j), tau, d and e.
-//  k_row_back<KQ>     W = Q M Q^T from M in the lower triangle of B, then
-//                     wbar = W (W b) / (k-1) and T = W + 1 wbar^T over B.
+//                     j of B (columns > j), tau, d and e; Q^T b over b.
+//  k_row_back<KQ>     W = Q M Q^T from M in the lower triangle of B, wbar from
+//                     Tri^-1 Q^T b in b, and T = W + 1 wbar^T over B.
+//
+// b goes along an entry a lane, in LDS for the reduction, where a register
+// more spills: its v . b is summed with v . p (wave_sums2).  As a row of the
+// matrix, as tridiag_pair.h has it, it made rows of 88 and more spill.  The
+// eigen stage of 11 952 problems at k = 64 / 80 / 100 / 104: 2.64 / 3.26 /
+// 4.53 / 4.56 ms with W (W b) / (k - 1), which loses the square of the
+// condition number, 2.71 / 3.35 / 4.58 / 4.74 ms now.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -53,12 +60,13 @@ __device__ __forceinline__ double row_pick(const double (&a)[KQ], int e) {
 
 template <int KQ>
 __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2)))
-void k_row_tridiag(int k, ChunkDev C, double* __restrict__ B, double* __restrict__ tau,
-                   double* __restrict__ dd, double* __restrict__ ee) {
+void k_row_tridiag(int k, ChunkDev C, double* __restrict__ B, double* __restrict__ bvec,
+                   double* __restrict__ tau, double* __restrict__ dd, double* __restrict__ ee) {
   constexpr int NT = (KQ + 15) / 16;
   __shared__ double sx[128];        // column j of A below the diagonal
   __shared__ double sp[128];        // p = t A v
-  __shared__ double ss[2], sd[2];   // the waves' sums of x . x and v . p
+  __shared__ double ss[2], sd[2][2];   // the waves' sums of x . x; of v . p and v . b
+  __shared__ double sb[128];        // b: an entry to the lane that holds the row
   const int64_t pair = blockIdx.x;
   if (!C.solve[pair]) return;
   const int r = threadIdx.x, lane = r & 63, i = r & 15;
@@ -78,6 +86,7 @@ void k_row_tridiag(int k, ChunkDev C, double* __restrict__ B, double* __restrict
     a[c] = r < k && c == r ? a[c] + (double)(k - 1) : a[c];
   }
   const double none[1] = {0.0};
+  sb[r] = r < k ? bvec[pair * (int64_t)k + r] : 0.0;
   const int jend = k - 2;
   const int jl = wv == 0 ? min(64, jend) : jend;   // the wave's rows are reduced from here
   static_for<NT>([&](auto I) __attribute__((always_inline)) {
@@ -126,8 +135,8 @@ void k_row_tridiag(int k, ChunkDev C, double* __restrict__ B, double* __restrict
       });
       const double pr = t * (p[0] + p[1]);
       sp[r] = pr;
-      const double vp = p_sum<64>(pr * v);
-      if (lane == 0) sd[wv] = vp;
+      const double vp = wave_sums2(pr * v, v * sb[r]);
+      if ((lane & 31) == 0) sd[lane >> 5][wv] = vp;
       // the reflector, and what only one row knows
       if (r > j && r < k) Bp[j * k + r] = v;
       if (r == j1) {
@@ -135,7 +144,8 @@ void k_row_tridiag(int k, ChunkDev C, double* __restrict__ B, double* __restrict
         ep[j] = beta;
       }
       __syncthreads();
-      const double kc = 0.5 * t * (sd[0] + sd[1]);
+      const double kc = 0.5 * t * (sd[0][0] + sd[0][1]);
+      sb[r] = fma(-t * (sd[1][0] + sd[1][1]), v, sb[r]);
       const double w = fma(-kc, v, pr);
 #pragma unroll
       for (int q = blk; q < NT; ++q) wq[q] = fma(-kc, vq[q], sp[16 * q + i]);
@@ -150,7 +160,7 @@ void k_row_tridiag(int k, ChunkDev C, double* __restrict__ B, double* __restrict
   if (jl < jend && lane == 0) ss[wv] = 0.0;
   for (int j = jl; j < jend; ++j) {
     __syncthreads();
-    if (j == jl && lane == 0) sd[wv] = 0.0;
+    if (j == jl && (lane & 31) == 0) sd[lane >> 5][wv] = 0.0;
     __syncthreads();
   }
   // the last two diagonal entries and the last subdiagonal one
@@ -162,16 +172,17 @@ void k_row_tridiag(int k, ChunkDev C, double* __restrict__ B, double* __restrict
     }
     if (c == k - 1 && r == k - 1) dp[k - 1] = a[c];
   }
+  if (r < k) bvec[pair * (int64_t)k + r] = sb[r];
 }
 
 template <int KQ>
 __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2)))
-void k_row_back(int k, ChunkDev C, double* __restrict__ B, const double* __restrict__ bvec,
+void k_row_back(int k, ChunkDev C, double* __restrict__ B, double* bvec,
                 const double* __restrict__ tau) {
   constexpr int NT = (KQ + 15) / 16;
   __shared__ double sv[2][128];     // the reflector of this step and of the next
-  __shared__ double sp[2][128];     // p = t A v; then W b
-  __shared__ double sd[2][2];       // the waves' sums of v . p
+  __shared__ double sp[2][128];     // p = t A v
+  __shared__ double sd[2][2][2];    // the waves' sums of v . p and of v . x
   __shared__ double st[128];
   const int64_t pair = blockIdx.x;
   if (!C.solve[pair]) return;
@@ -188,6 +199,7 @@ void k_row_back(int k, ChunkDev C, double* __restrict__ B, const double* __restr
     a[c] = Bp[max(rc, cc) * k + min(rc, cc)];
   }
   st[r] = r < k - 2 ? tau[pair * kRowStride + r] : 0.0;
+  double x = in ? bvec[pair * (int64_t)k + r] : 0.0;   // Tri^-1 Q^T b, then wbar
   // v: reflector j's entry r; vn: the next step's, as loaded
   double v = in && r > k - 3 ? Bp[(k - 3) * k + rc] : 0.0;
   double vn = Bp[max(k - 4, 0) * k + rc];
@@ -213,15 +225,16 @@ void k_row_back(int k, ChunkDev C, double* __restrict__ B, const double* __restr
       });
       const double pr = t * (p[0] + p[1]);
       sp[buf][r] = pr;
-      const double vp = p_sum<64>(pr * v);
-      if (lane == 0) sd[buf][wv] = vp;
+      const double vp = wave_sums2(pr * v, v * x);
+      if ((lane & 31) == 0) sd[buf][lane >> 5][wv] = vp;
       // the next reflector (the other buffer's readers, of step j + 1, have
       // passed that step's barrier), and the load of the one after it
       const double vx = in && r > j - 1 ? vn : 0.0;
       sv[buf ^ 1][r] = vx;
       vn = Bp[max(j - 2, 0) * k + rc];
       __syncthreads();
-      const double kc = 0.5 * t * (sd[buf][0] + sd[buf][1]);
+      const double kc = 0.5 * t * (sd[buf][0][0] + sd[buf][0][1]);
+      x = fma(-t * (sd[buf][1][0] + sd[buf][1][1]), v, x);
       const double w = fma(-kc, v, pr);
 #pragma unroll
       for (int q = 0; q < NT; ++q) {
@@ -235,21 +248,12 @@ void k_row_back(int k, ChunkDev C, double* __restrict__ B, const double* __restr
       v = vx;
     }
   });
-  // wbar = W (W b) / (k-1); T = W + 1 wbar^T.  W is symmetric, so the lane
-  // that holds row r writes column r, to which it adds wbar_r.
-  auto mul = [&](double x) __attribute__((always_inline)) {
-    __syncthreads();
-    sp[0][r] = x;
-    __syncthreads();
-    double p[4] = {0.0, 0.0, 0.0, 0.0};
-    static_for<NT>([&](auto T) __attribute__((always_inline)) {
-      constexpr int q = decltype(T)::value;
-      block_prod<KQ, 1, q>(p, sp[0][16 * q + i], a, none);
-    });
-    return p[0] + p[1];
-  };
-  const double y = mul(in ? bvec[pair * (int64_t)k + r] : 0.0);
-  const double wb = mul(y) / (double)(k - 1);
+  // wbar to memory and back: with x itself in the sums below the matrix's rows
+  // spill (rows of 104: 0 -> 52 registers, 1.74 -> 1.84 ms at 11 952 problems)
+  if (in) bvec[pair * (int64_t)k + r] = x;
+  const double wb = in ? bvec[pair * (int64_t)k + r] : 0.0;
+  // T = W + 1 wbar^T.  W is symmetric, so the lane that holds row r writes
+  // column r, to which it adds wbar_r.
 #pragma unroll
   for (int c = 0; c < KQ; ++c)
     if (in && c < k) Bp[c * k + r] = a[c] + wb;
@@ -257,12 +261,12 @@ void k_row_back(int k, ChunkDev C, double* __restrict__ B, const double* __restr
 
 template <int KQ>
 void launch_row_tridiag_kq(hipStream_t st, unsigned nb, int k, const ChunkDev& C, double* B,
-                           double* tau, double* dd, double* ee) {
-  k_row_tridiag<KQ><<<nb, 128, 0, st>>>(k, C, B, tau, dd, ee);
+                           double* bvec, double* tau, double* dd, double* ee) {
+  k_row_tridiag<KQ><<<nb, 128, 0, st>>>(k, C, B, bvec, tau, dd, ee);
 }
 template <int KQ>
 void launch_row_back_kq(hipStream_t st, unsigned nb, int k, const ChunkDev& C, double* B,
-                        const double* bvec, const double* tau) {
+                        double* bvec, const double* tau) {
   k_row_back<KQ><<<nb, 128, 0, st>>>(k, C, B, bvec, tau);
 }
 

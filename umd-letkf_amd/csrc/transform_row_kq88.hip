@@ -5,12 +5,12 @@
 namespace lk {
 
 void launch_row_tridiag_kq88(hipStream_t st, unsigned nb, int k, const ChunkDev& C, double* B,
-                              double* tau, double* dd, double* ee) {
-  launch_row_tridiag_kq<88>(st, nb, k, C, B, tau, dd, ee);
+                              double* bvec, double* tau, double* dd, double* ee) {
+  launch_row_tridiag_kq<88>(st, nb, k, C, B, bvec, tau, dd, ee);
 }
 
 void launch_row_back_kq88(hipStream_t st, unsigned nb, int k, const ChunkDev& C, double* B,
-                           const double* bvec, const double* tau) {
+                           double* bvec, const double* tau) {
   launch_row_back_kq<88>(st, nb, k, C, B, bvec, tau);
 }
 
