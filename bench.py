@@ -758,35 +758,6 @@ def main():
                                            "finalize": round(rt["finalize_ms"], 3)}}
         out["speedup_vs_fp64_plain"] = round(out["value"] / out["fp64_plain"]["value"], 3)
         log(f"[bench] fp64 plain: {out['fp64_plain']}")
-        if prob.k < 64:
-            # the plain FP64 path with the batched path's transform (the
-            # rational A^(-1/2) instead of the QL eigensolve): the speed-up of
-            # the precision alone
-            os.environ["LETKF_GPU_RAT"] = "2"
-            try:
-                ref = LetkfGpuSolver(prob, precision="fp64", path="plain")
-            finally:
-                del os.environ["LETKF_GPU_RAT"]
-            if not args.no_autotune:
-                ref.autotune(repeats=1)
-            for _ in range(args.warmup):
-                ref.run()
-            t0 = time.perf_counter()
-            for _ in range(args.steps):
-                ref.run()
-            dt = time.perf_counter() - t0
-            rt = ref.timing()
-            ref.final()
-            out["fp64_plain_rational"] = {
-                "value": round(prob.nij * args.steps / dt, 1),
-                "ms_per_step": round(1e3 * dt / args.steps, 3),
-                "phases_ms": {"search": round(rt["search_ms"], 3),
-                              "product": round(rt["product_ms"], 3),
-                              "transform": round(rt["eigen_ms"], 3),
-                              "finalize": round(rt["finalize_ms"], 3)}}
-            out["speedup_vs_fp64_plain_same_transform"] = round(
-                out["value"] / out["fp64_plain_rational"]["value"], 3)
-            log(f"[bench] fp64 plain, rational transform: {out['fp64_plain_rational']}")
     print(json.dumps(out), flush=True)
 
 
