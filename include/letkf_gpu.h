@@ -44,12 +44,12 @@ extern "C" {
 
 /* ---- arithmetic of the local analysis ---------------------------------- */
 #define LETKF_PREC_FP64     0  /* everything in FP64                        */
-#define LETKF_PREC_FP32     1  /* products in FP32, eigensolve in FP64      */
+#define LETKF_PREC_FP32     1  /* products in FP32, transform in FP64       */
 #define LETKF_PREC_BF16X3   2  /* products split-BF16 (3 MFMA terms), FP32
-                                  accumulation; eigensolve in FP64          */
+                                  accumulation; transform in FP64           */
 #define LETKF_PREC_BF16     3  /* products plain BF16, FP32 accumulation     */
 #define LETKF_PREC_BF16X4   4  /* products split-BF16 with all 4 MFMA terms,
-                                  compensated FP32 accumulation; eigensolve
+                                  compensated FP32 accumulation; transform
                                   in FP64 (FP32 products are compensated
                                   the same way)                             */
 
@@ -128,7 +128,7 @@ typedef struct letkf_gpu_diag {
 typedef struct letkf_gpu_timing {
   double search_ms;    /* local-obs search + localization          */
   double product_ms;   /* Yb^T R^-1 Yb and Yb^T R^-1 d              */
-  double eigen_ms;     /* eigensolve, transform, application        */
+  double eigen_ms;     /* reduction, transform, application         */
   double finalize_ms;  /* recenter / clip / inflation / spread      */
   double total_ms;
   int64_t n_problems;  /* (gridpoint, group) solves with m > 0       */

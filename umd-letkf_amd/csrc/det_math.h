@@ -221,7 +221,6 @@ DM_FN float gc(float z, float L) {
   return (float)res;
 }
 
-// linearinterp_lat get_dist on an already-completed table (n >= 1)
 // The same float results as dist() and gc() by shorter arithmetic (the search
 // is bound by its instructions: 99% of its cycles issue one; at 1.65e9
 // candidates 11.9 ms with the full forms, 10.1 with these), with a
@@ -300,6 +299,7 @@ DM_FN float gc_fast(float z, const GcScale& g, bool* sure) {
   return out ? 0.0f : lo;
 }
 
+// linearinterp_lat get_dist on an already-completed table (n >= 1)
 DM_FN float interp(int n, const float* lat, const float* dist, float x) {
 #pragma clang fp contract(off)
   const float a = fabsf(x);

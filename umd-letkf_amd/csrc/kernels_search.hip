@@ -228,7 +228,7 @@ __device__ __forceinline__ float list_weight(float w, float err) {
 }
 
 // the one-group fill pass (the common case) keeps one group in LDS, which
-// leaves six waves per SIMD to hide the candidates' load latency
+// leaves five waves per SIMD to hide the candidates' load latency
 template <int PASS, int CLS>
 __global__ __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(PASS == 3 ? 5 : 1, 8))) void k_search(LocDev L, ObsDev O, StateDev S,

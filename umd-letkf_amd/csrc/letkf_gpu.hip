@@ -3,7 +3,7 @@
 // letkf_gpu_run() replaces letkf_solver_run (src/letkf_solver.F90:150-389).
 // Gridpoints are processed in chunks so that the per-(gridpoint, group)
 // work arrays stay bounded; each chunk runs
-//   search count -> offsets scan -> search fill -> products -> eigensolve
+//   search count -> offsets scan -> search fill -> products -> transform
 //   and application -> post-processing
 // on the handle's stream.  Inputs stay untouched on the device, so a run can
 // be repeated (benchmarks, cycling).
@@ -168,7 +168,8 @@ struct letkf_gpu_t {
   int tune_chunk_log2 = 20;   // at most 2^n problems per chunk (17..20)
   int tune_vec = 1;       // vector path when every group has few slabs
   int tune_fuse = 1;      // rational solve inside the two-problem tridiagonalization
-  int tune_matblk = 1;    // 64 <= k <= 128: 2D-block reduction and back-transform
+  int tune_matblk = 1;    // 64 <= k <= 127: row-per-lane (k <= 104) or 2D-block reduction
+                          // and back-transform (0: column halves)
   int tune_fusefin = 1;   // 64 <= k <= 128, mixed: post-processing inside the apply
   int tune_rat = 1;       // k < 64: rational A^(-1/2), no eigensolve (0 off)
   int tune_mat = 1;       // batched, 64 <= k <= 128: explicit T applied on MFMA
@@ -1049,7 +1050,7 @@ static int ensure_outputs(letkf_gpu_t* h) {
   HIPCHK(h, dalloc_once(h, &h->d_mld, (size_t)nij));
   HIPCHK(h, dalloc_once(h, &h->d_ctr, (size_t)kCtrSlots * kCtrStride));
   // LETKF_GPU_EIGEN=jacobi selects the parallel Jacobi solver for every
-  // problem (reference solver for tests); default: tridiagonal QL pipeline
+  // problem (reference solver for tests); default: reduction to tridiagonal form
   const char* ev = getenv("LETKF_GPU_EIGEN");
   const bool force_jacobi = ev && strcmp(ev, "jacobi") == 0;
   // 64 <= k <= 128: explicit transform matrix, applied on MFMA (batched)

@@ -1,4 +1,4 @@
-// tridiag_pair_kq56.hip -- two-problem tridiagonalization, rows of 56.
+// tridiag_pair_kq56.hip -- one-problem tridiagonalization, rows of 56.
 #include "tridiag_pair.h"
 
 namespace lk {

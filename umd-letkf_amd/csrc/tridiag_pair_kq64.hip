@@ -1,4 +1,4 @@
-// tridiag_pair_kq64.hip -- two-problem tridiagonalization, rows of 64.
+// tridiag_pair_kq64.hip -- one-problem tridiagonalization, rows of 64.
 #include "tridiag_pair.h"
 
 namespace lk {
